@@ -186,3 +186,64 @@ def tolerance(case):
         return {"rel": 5e-6}
     train = case["call"] == "train"
     return {"rel": (1.6e-2 if train else 7e-3) if case["dtype"] == "bfloat16" else (2e-3 if train else 1e-3)}
+
+
+class _ClampGrad(torch.autograd.Function):
+    """Identity whose cotangent is clamped to [-v, v]."""
+
+    @staticmethod
+    def forward(ctx, x, v):
+        ctx.v = v
+        return x.view_as(x)
+
+    @staticmethod
+    def backward(ctx, g):
+        return g.clamp(-ctx.v, ctx.v), None
+
+
+def _cell(function, x, y, b, s):
+    """One step of a cell.  The stabiliser of the sLSTM is held constant in its adjoint, and the guard max(n, 1) is
+    transparent there, as in the kernels."""
+    sig, tanh = torch.sigmoid, torch.tanh
+    if function == "elman":
+        return (tanh(x[0] + y[0] + b[0]),)
+    if function == "gru":
+        r, z = sig(x[0] + y[1] + b[1]), sig(x[1] + y[2] + b[2])
+        return (z * s[0] + (1 - z) * tanh(x[2] + b[3] + r * (y[0] + b[0])),)
+    i, f, z, o = (x[k] + y[k] + b[k] for k in range(4))
+    if function == "lstm":
+        c = sig(f) * s[1] + sig(i) * tanh(z)
+        return (sig(o) * tanh(c), c)
+    lf = torch.nn.functional.logsigmoid(f) + s[3].detach()
+    m = torch.where(s[2] == 0, i, torch.maximum(i, lf)).detach()
+    i, f = torch.exp(i - m), torch.exp(lf - m)
+    c, n = f * s[1] + i * tanh(z), f * s[2] + i
+    n = n + (n.clamp(min=1.0) - n).detach()
+    return (sig(o) * c / n, c, n, m)
+
+
+def exact(case, seed):
+    """What ``run`` returns, in 64 bits: the parameters and inputs as the kernels take them (rounded to the kernel type)."""
+    st = prepare(case, seed)
+    Gr, _, _, _, S = rnn_function_registry[case["function"]]["gates_states"]
+    kdt, (B, N, D) = DTYPE_DICT[case["dtype"]], (case["B"], case["N"], case["D"])
+    step, train = case["call"] == "step", case["call"] == "train"
+    leaf = {"Wx": torch.cat(st["Wx"], 1) if step else st["Wx"], "R": st["R"], "b": st["b"], "states": st["states"]}
+    leaf = {k: v.detach().to(kdt).double().requires_grad_(train) for k, v in leaf.items() if v is not None}
+    s = tuple(leaf["states"][:, :, 0].unbind(0)) if "states" in leaf else tuple(leaf["Wx"].new_zeros(B, N, D) for _ in range(S))
+    with torch.set_grad_enabled(train):
+        R = leaf["R"].permute(1, 3, 0, 2).reshape(N, D, Gr * D).contiguous()
+        b, out = leaf["b"].unbind(0), []
+        for t, wx in enumerate(leaf["Wx"].unbind(1)):
+            if case["clip"] and t:
+                s = (_ClampGrad.apply(s[0], case["clip"]),) + s[1:]
+            y = torch.bmm(s[0].transpose(0, 1), R).reshape(N, B, Gr, D).permute(2, 1, 0, 3)
+            s = _cell(case["function"], wx.unbind(1), y.unbind(0), b, s)
+            out.append(torch.stack(s))
+        states = torch.stack(out, 2)
+    if step:
+        return {"states": [x[:, :, None] for x in out], "carry": out[-1]}
+    if not train:
+        return {"states": states, "last": states[:, :, -1:]}
+    grads = torch.autograd.grad(states, list(leaf.values()), grad_outputs=st["dstates"].double())
+    return {"states": states.detach(), **{"d" + k: v for k, v in zip(leaf, grads)}}
