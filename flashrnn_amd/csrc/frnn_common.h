@@ -344,13 +344,18 @@ __device__ __forceinline__ u64 ll_pack(half_t*, float a, float b, int t) { retur
 __device__ __forceinline__ u64 ll_pack(float*, float a, int t) {
   return (u64)__float_as_uint(a) | ((u64)(unsigned)(t + 1) << 32);
 }
-__device__ __forceinline__ bool ll_ok16(u64 w, int t) {
-  unsigned tg = tag16(t);
-  return ((unsigned)(w >> 16) & 0xffffu) == tg && (unsigned)(w >> 48) == tg;
+// Bits under TagMask in which the tags of a word differ from those of step t (zero: the word has arrived).  As integers,
+// so that the words of a set are combined with bit operations and one compare votes on all of them; as comparisons,
+// each word's result went through the scalar unit and the vote through a select and another compare.
+template <typename TAG> struct TagMask { static constexpr unsigned value = 0xffff0000u; };
+__device__ __forceinline__ unsigned ll_diff16(u64 w, int t) {
+  const unsigned tg = tag16(t) << 16;
+  return ((unsigned)w ^ tg) | ((unsigned)(w >> 32) ^ tg);
 }
-__device__ __forceinline__ bool ll_ok(bf16_t*, u64 w, int t) { return ll_ok16(w, t); }
-__device__ __forceinline__ bool ll_ok(half_t*, u64 w, int t) { return ll_ok16(w, t); }
-__device__ __forceinline__ bool ll_ok(float*, u64 w, int t) { return (unsigned)(w >> 32) == (unsigned)(t + 1); }
+__device__ __forceinline__ unsigned ll_diff(bf16_t*, u64 w, int t) { return ll_diff16(w, t); }
+__device__ __forceinline__ unsigned ll_diff(half_t*, u64 w, int t) { return ll_diff16(w, t); }
+template <> struct TagMask<float> { static constexpr unsigned value = 0xffffffffu; };
+__device__ __forceinline__ unsigned ll_diff(float*, u64 w, int t) { return (unsigned)(w >> 32) ^ (unsigned)(t + 1); }
 // payload as the 32 bits that go to LDS (bf16: two elements; f32: one)
 __device__ __forceinline__ unsigned ll_payload16(u64 w) {
   return ((unsigned)w & 0xffffu) | (((unsigned)(w >> 32) & 0xffffu) << 16);
@@ -367,7 +372,8 @@ __device__ __forceinline__ unsigned ll_payload(float*, u64 w) { return (unsigned
 struct Part64 { typedef u64 Word; };
 struct Part32 { typedef unsigned Word; };
 __device__ __forceinline__ u64 part_pack(Part64*, float a, int t) { return (u64)__float_as_uint(a) | ((u64)(unsigned)(t + 1) << 32); }
-__device__ __forceinline__ bool ll_ok(Part64*, u64 w, int t) { return (unsigned)(w >> 32) == (unsigned)(t + 1); }
+template <> struct TagMask<Part64> { static constexpr unsigned value = 0xffffffffu; };
+__device__ __forceinline__ unsigned ll_diff(Part64*, u64 w, int t) { return (unsigned)(w >> 32) ^ (unsigned)(t + 1); }
 __device__ __forceinline__ float part_value(Part64*, u64 w) { return __uint_as_float((unsigned)w); }
 __device__ __forceinline__ unsigned tag8(int t) { return (unsigned)(t % 255) + 1u; }
 __device__ __forceinline__ unsigned part_pack(Part32*, float a, int t) {
@@ -376,7 +382,8 @@ __device__ __forceinline__ unsigned part_pack(Part32*, float a, int t) {
   const unsigned bits = __float_as_uint(a);
   return (tag8(t) << 24) | ((a != a ? bits : bits + 0x80u) >> 8);
 }
-__device__ __forceinline__ bool ll_ok(Part32*, unsigned w, int t) { return (w >> 24) == tag8(t); }
+template <> struct TagMask<Part32> { static constexpr unsigned value = 0xff000000u; };
+__device__ __forceinline__ unsigned ll_diff(Part32*, unsigned w, int t) { return w ^ (tag8(t) << 24); }
 __device__ __forceinline__ float part_value(Part32*, unsigned w) { return __uint_as_float(w << 8); }
 __device__ __forceinline__ unsigned ll_load(const unsigned* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

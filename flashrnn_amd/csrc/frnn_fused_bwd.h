@@ -559,7 +559,8 @@ fused_bwd_kernel(const BwdArgs a) {
     for (int k = 0; k < S; ++k) sn[u][k] = buf_load<ND_, SB>(rSt, st_v[u], ((unsigned)k * BS * Tn + (Tn - 1)) * ND * ES);
   // exchange stores may stay in the L2 of the XCD once the group is known to share one
   if (KW > 1 && w == 0) {
-    const int r = (a.xcd && !a.cut) ? xcd_handshake<KW>(a.xcd + (size_t)grp * 32, slice, lane, a.status, a.spin_limit) : 0;
+    // (a host-side test hook, spin_limit < -1: every wait counts as run out)
+    const int r = (!a.cut && a.spin_limit < -1) ? -1 : (a.xcd && !a.cut) ? xcd_handshake<KW>(a.xcd + (size_t)grp * 32, slice, lane, a.status, a.spin_limit) : 0;
     if (lane == 0) near_word = r;
   }
   __syncthreads();
@@ -658,7 +659,7 @@ fused_bwd_kernel(const BwdArgs a) {
     rebuild_gates(pre[0], Tn - 1);
   }
 
-  bool dead = near_i < 0, fail = false;
+  bool dead = near_i < 0;
   // does a step look at the workgroup's flag of a failed wait?  Heads of one workgroup never wait (the recompute-mode
   // kernels of the sLSTM and of 8 waves keep the flag all the same: any other form of their step spills)
   constexpr bool FLAG = KW > 1 || (RC && (F == FRNN_SLSTM || WAVES > 6));
@@ -777,7 +778,7 @@ fused_bwd_kernel(const BwdArgs a) {
         asm volatile("" : "+s"(never));
         if (never) { dead = true; return; }
       }
-    } else { if (barrier_or(fail, dead_flag)) { dead = true; return; } }
+    } else { if (barrier_or(dead_flag)) { dead = true; return; } }
     FRNN_STAMP(c2);
     if constexpr (PW) {
       // the operands of step t-1 from the producer wave's buffer (behind this step's barrier; used in the next step)
@@ -1060,6 +1061,7 @@ fused_bwd_kernel(const BwdArgs a) {
         }
       }
       // receive: KW-1 partial sums of the own tiles, PSRC sources at a time
+      Wait wait{a.status, dead_flag, a.spin_limit};
       const IW* const mine = inbox + (size_t)(t & 1) * INW + ((size_t)(slice * NPOS + wp) * UTW) * KW * 256 + lane;
       if constexpr (RSP) {
         const int rbeg = 1 + hf * SRC_W;  // (uniform) this wave's sources: rbeg .. rbeg + SRC_W - 1, below KW
@@ -1084,7 +1086,7 @@ fused_bwd_kernel(const BwdArgs a) {
                 need[(rr * UTW + u) * E + e] = rvalid && in;
               }
           }
-          if (!fail) fail = poll_words_staggered<PT, NWR>(mine, off, need, t, v, a.status, a.spin_limit, k0 == 0 ? a.poll_delay : 0);
+          poll_words_reload<PT, NWR>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0);
 #pragma unroll
           for (int rr = 0; rr < PSRC_W; ++rr) {
             const bool in = k0 + rr < SRC_W && rbeg + k0 + rr < KW;
@@ -1140,13 +1142,18 @@ fused_bwd_kernel(const BwdArgs a) {
           if (t > 0) rebuild_fetch(t - 1, rhq);
           __builtin_amdgcn_sched_barrier(0);
           for (int i = 0; i < a.poll_delay; ++i) __builtin_amdgcn_s_sleep(1);
-          IW pv[NWR];
-          poll_issue<NWR>(mine, off, pv);
+          poll_issue<NWR>(mine, off, v);
           __builtin_amdgcn_sched_barrier(0);
           if (t > 0) { rebuild_product(rhq, racc); rebuild_math(pm, racc); }
-          if (!fail) fail = poll_finish<PT, NWR>(mine, off, need, t, pv, v, a.status, a.spin_limit);
+          poll_finish<PT, NWR, (TR < 16)>(mine, off, need, t, v, wait);
+          if constexpr (TR == 16) {
+            // (never taken, which the compiler does not know: without an exit here the sLSTM's D = 128 kernel spills)
+            int never = 0;
+            asm volatile("" : "+s"(never));
+            if (never) { dead = true; return; }
+          }
         } else {
-          if (!fail) fail = poll_words_staggered<PT, NWR>(mine, off, need, t, v, a.status, a.spin_limit, r0 == 1 ? a.poll_delay : 0);
+          poll_words_reload<PT, NWR>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0);
         }
 #pragma unroll
         for (int rr = 0; rr < PSRC; ++rr)
@@ -1218,7 +1225,7 @@ fused_bwd_kernel(const BwdArgs a) {
       if (!dead && t - j >= 0) step(std::false_type{}, t - j, pre[j], pre[j], pre[(j + PD) % (PD + 1)]);
   }
   if constexpr (!FLAG) lds_barrier();  // (the producer wave takes part in it)
-  else { if (!dead && barrier_or(fail, dead_flag)) dead = true; }
+  else { if (!dead && barrier_or(dead_flag)) dead = true; }
 #ifdef FRNN_TRACE
   if (lane == 0 && a.trace) {
     long long* o = a.trace + ((size_t)blockIdx.x * WAVES + w) * 8;

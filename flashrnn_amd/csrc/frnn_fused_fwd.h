@@ -235,7 +235,7 @@ fused_fwd_kernel(const FwdArgs a) {
       auto iter = [&](int t, const Dw<4> (&next)[NCH], Dw<4> (&refill)[NCH]) __attribute__((always_inline)) {
         if (t > 0) {
           if constexpr (OWN_FIRST) lds_barrier();
-          if constexpr (KW > 1) { if (barrier_or(false, &dead_flag)) { pdead = true; return; } }
+          if constexpr (KW > 1) { if (barrier_or(&dead_flag)) { pdead = true; return; } }
           else lds_barrier();
         }
         put(next, t + 1);
@@ -430,7 +430,8 @@ fused_fwd_kernel(const FwdArgs a) {
   // exchange stores may stay in the L2 of the XCD once the group is known to share one (a single step sends
   // nothing that is read)
   if (KW > 1 && w == 0) {
-    const int r = (a.xcd && Tn > 1 && !a.step) ? xcd_handshake<KW>(a.xcd + (size_t)grp * 32, slice, lane, a.status, a.spin_limit) : 0;
+    // (a host-side test hook, spin_limit < -1: every wait counts as run out)
+    const int r = (!MB && Tn > 1 && !a.step && a.spin_limit < -1) ? -1 : (a.xcd && Tn > 1 && !a.step) ? xcd_handshake<KW>(a.xcd + (size_t)grp * 32, slice, lane, a.status, a.spin_limit) : 0;
     if (lane == 0) near_word = r;
   }
   __syncthreads();
@@ -474,10 +475,10 @@ fused_fwd_kernel(const FwdArgs a) {
     }
     if (t > 0) {
       if (KW > 1) {
-        bool fail;
-        if constexpr (PAIRS) fail = ll_gather_pairs<T, NP>(rLL, (unsigned)((t - 1) & 1) * LLW * 8u, qpoll, t - 1, hbuf[cur], a.status, a.spin_limit, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
-        else fail = ll_gather<T, NP, M44>(llbase + (size_t)((t - 1) & 1) * LLW, qpoll, t - 1, hbuf[cur], a.status, a.spin_limit, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
-        if (barrier_or(fail, &dead_flag)) { dead = true; return; }
+        Wait w{a.status, &dead_flag, a.spin_limit};
+        if constexpr (PAIRS) ll_gather_pairs<T, NP>(rLL, (unsigned)((t - 1) & 1) * LLW * 8u, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
+        else ll_gather<T, NP, M44>(llbase + (size_t)((t - 1) & 1) * LLW, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
+        if (barrier_or(&dead_flag)) { dead = true; return; }
       } else {
         lds_barrier();
       }
