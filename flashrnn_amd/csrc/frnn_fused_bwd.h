@@ -680,6 +680,11 @@ fused_bwd_kernel(const BwdArgs a) {
     // partial sums are sent, where they fill the wait for the other workgroups instead of delaying
     // the barrier (a vector memory instruction costs ~30 cycles to issue)
     constexpr bool DW_LATE = KW > 1 && GW > 1;  // (a single store, Elman, measured no better behind the send)
+    // Kernels with a producer wave, gated cells: dWx_t is stored, and the operands of the next step are read from LDS, behind
+    // the requests for the fragments of the step, in the ~120 cycles until the first of them arrives, instead of in front
+    // of the barrier and of the requests (reverse kernel, bf16: GRU B16 T2048 N4 D128 1.037 -> 0.985 ms, LSTM B16 T512 N12 D64 0.180 ->
+    // 0.176, N6 D128 0.323 -> 0.324; the Elman cell, one store per step, 0.103 -> 0.111 at N6 D128: not there)
+    constexpr bool MID = PW && GR >= 3, DW_MID = MID && !PST;
     Dw<ND_> dwp[UTW][GW], dxp[UTW];
     auto store_dw = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
@@ -729,7 +734,7 @@ fused_bwd_kernel(const BwdArgs a) {
 #pragma unroll
         for (int k = 0; k < S; ++k) ds[u][e][k] = bvalid ? ds[u][e][k] : 0.f;
       }
-      if constexpr (DW_LATE && !cut) {
+      if constexpr ((DW_LATE || DW_MID) && !cut) {
 #pragma unroll
         for (int g = 0; g < GW; ++g) dwp[u][g] = pack<E>(dgw[g], (T*)0);
         if (F == FRNN_GRU) dxp[u] = pack<E>(dgr[0], (T*)0);
@@ -780,8 +785,9 @@ fused_bwd_kernel(const BwdArgs a) {
       }
     } else { if (barrier_or(dead_flag)) { dead = true; return; } }
     FRNN_STAMP(c2);
-    if constexpr (PW) {
-      // the operands of step t-1 from the producer wave's buffer (behind this step's barrier; used in the next step)
+    // operands of step t-1 from the producer wave's buffer (behind this step's barrier; used in the next step)
+    auto take_operands = [&]() __attribute__((always_inline)) {
+      if constexpr (PW) {
       static_assert(E == 1 && ND_ == 1 && PD == 1, "4-row tiles: one element per lane and tile, one step ahead");
       const T* const pb = pbuf + ((Tn - t) & 1) * PB;
 #pragma unroll
@@ -799,9 +805,11 @@ fused_bwd_kernel(const BwdArgs a) {
         }
       }
     }
-
+    };
+    if constexpr (!MID) take_operands();
     // one accumulator per tile: splitting a lone chain over several accumulators (as the forward
-    // kernel does) measured 3-8 % slower here, before and after the barrier was made LDS-only
+    // kernel does) measured 3-8 % slower here, before and after the barrier was made LDS-only, and 0-5 % for the lone chains of
+    // heads of one workgroup (LSTM B16 T512 N12 D64 0.176 -> 0.184 ms, GRU N4 D128 the same)
     constexpr int NACC = 1;
     // With 3 and more workgroups per head the products that other workgroups wait for come first
     // and are sent at once; the product for the own tiles follows while those words travel (it
@@ -851,6 +859,14 @@ fused_bwd_kernel(const BwdArgs a) {
       for (int rr = 0; rr < RLD; ++rr)
 #pragma unroll
         for (int u = 0; u < UTW; ++u) la_next[rr][u] = rl[((rr * UTW + u) * KS) * 64];
+    }
+    if constexpr (MID) {
+      take_operands();
+      if constexpr (!PST && !cut) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UTW; ++u) store_dw(u);
+      }
     }
     // keep the reads up here: issued just in time they would expose the LDS latency once per chunk
     __builtin_amdgcn_sched_barrier(0);

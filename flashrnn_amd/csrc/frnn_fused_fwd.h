@@ -495,6 +495,12 @@ fused_fwd_kernel(const FwdArgs a) {
     };
     if constexpr (MB) mb_probe();
     Dw<ND_> wcl[PW ? UTW : 1][PW ? GW : 1];  // this step's Wx from the producer wave's buffer
+    // Heads of one workgroup read them behind the requests for the fragments, which the MFMAs wait for (forward, bf16, GRU B16
+    // T2048 N4 D128 0.825 -> 0.793 ms, B40 T512 N8 D96 0.189 -> 0.185, LSTM fp16 B33 T515 N8 D96 0.245 -> 0.241, N12 D64 no change; but 8
+    // waves of a 4-gate cell, LSTM and sLSTM N6 D128, +0.5 and +1.0 %, and heads of several workgroups 0 to +0.6 %: not there).
+    // The outputs of a step stored at the same place, one step late, instead of behind the new h: +2 to +11 %.
+    constexpr bool WX_MID = KW == 1 && !(GR == 4 && WAVES >= 8);
+    auto take_wx = [&]() __attribute__((always_inline)) {
     if constexpr (PW) {
       // (the lane's E consecutive units of a gate: 2, 4 or 8 bytes)
       const T* const wb = wbuf + cur * WBUF;
@@ -508,6 +514,8 @@ fused_fwd_kernel(const FwdArgs a) {
           else { const uint2 v = *reinterpret_cast<const uint2*>(src); wcl[u][g].v[0] = v.x; wcl[u][g].v[1] = v.y; }
         }
     }
+    };
+    if constexpr (!WX_MID) take_wx();
 
     // h fragments are read KC k-steps ahead of the MFMAs that use them, so LDS latency is paid once
     f32x4 acc[UTW][GR];
@@ -563,6 +571,7 @@ fused_fwd_kernel(const FwdArgs a) {
 #pragma unroll
         for (int g = 0; g < GR; ++g) la_next[u][g] = rl[(u * GR + g) * 64];
     }
+    if constexpr (WX_MID) take_wx();
     // keep the reads up here: issued just in time they would expose the LDS latency once per chunk
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
