@@ -753,14 +753,9 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   const FusedBwdWs w = carve_fused_bwd(workspace, fx, dtype, B, T, N, D, p);
   if (workspace_bytes < w.total) return fail(FRNN_E_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, w.total);
   hipStream_t st = (hipStream_t)stream;
-  if (p.kw > 1) {  // (as in the forward call)
-    prof_begin("fill_zero_kernel", st);
-    e = launch_fill_zero(workspace, w.zero_bytes, st);
-    prof_end(st);
-    if (e) return hip_fail(e, "workspace clear");
-  }
+  // (heads of several workgroups: the launch that transposes R clears the status word and the exchange words as well)
   prof_begin("transpose_r_kernel", st);
-  e = launch_transpose_r(dtype, R, w.Rt, N, D, c.GR, st);
+  e = launch_transpose_r(dtype, R, w.Rt, N, D, c.GR, st, workspace, p.kw > 1 ? w.zero_bytes : 0);
   prof_end(st);
   if (e) return hip_fail(e, "R transpose");
   const int tr = tile_rows_for(B, N, p.kw, p.waves, p.max_tr, dtype);

@@ -15,7 +15,8 @@ struct GradGemmArgs {
   int rows_per_split;    // filled in by launch_grad_gemm
 };
 
-int launch_transpose_r(int dtype, const void* R, void* Rt, int N, int D, int GR, hipStream_t st);
+// Rt = R transposed per head; zero_bytes > 0: the same launch clears that many bytes at `zero` (16-byte aligned, whole words)
+int launch_transpose_r(int dtype, const void* R, void* Rt, int N, int D, int GR, hipStream_t st, void* zero = nullptr, size_t zero_bytes = 0);
 int grad_gemm_splits(int dtype, int B, int T, int N, int D, int GR);
 int launch_grad_gemm(int dtype, GradGemmArgs a, int splits, hipStream_t st);
 int launch_grad_reduce(const float* part_r, int splits_r, size_t n_r, float* dR,
