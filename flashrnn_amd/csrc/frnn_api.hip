@@ -133,9 +133,11 @@ static bool near_stores_allowed() { return env_int("FRNN_AGENT_STORES", 0) == 0;
 // value differs by cell and tiling.  Measured on MI355X (bf16, T = 1024, exchange stores kept in the XCD's
 // L2; a unit off costs up to 1-3 %, most curves are flat within 2 units):
 //   kernels that multiply the own slice in front of the wait, 4-row tiles: lstm D=256 0, D=320 0, D=512 1, D=640 1;
-//   slstm D=192, 256 0, D=640 1; gru D=256, 384, 640 1, D=768 2, D=1024 (16 workgroups) 6; elman D=512, 1024 0,
-//   D=640 2, fp32 0; 8- and 16-row tiles 2-4 (flat);
-//   lstm, slstm D=768 (12 workgroups) 0-1;  the others: lstm D=1024 (32 workgroups of 2 waves) 3-6.
+//   slstm D=192, 256 0, D=640 1; gru D=256, 384, 640, 768 1 (D=768, 512 steps, 0.652 ms with 2, 0.642 with 1), D=1024 (16
+//   workgroups) 6; elman D=320, 512 (4 waves) 1 (0.321 / 0.395 ms with 0, 0.314 / 0.386 with 1), D=1024 (8 waves) 0, D=640 0
+//   (0.441 ms with 2, 0.429 with 0), fp32 0; 8- and 16-row tiles 2-4 (flat);
+//   lstm, slstm D=768 (12 workgroups) 0-1, D=1024 (32 workgroups) 1 (0.862 / 0.891 ms with 6, 0.812 / 0.844 with 1; 8-row tiles
+//   B64 T256 0.563 with 6, 0.556 with 2; 16-row tiles B128 T128 0.429 with 6, 0.434 with 2);  fp32 with the operand in the 4x4x1 form 6 (D=384, 512 +2 to +7 % with 0-3).
 static int fwd_poll_delay_default(int function, int dtype, const Plan& p, int tile_rows) {
   if (p.kw <= 1) return 0;
   // groups that span the device exchange through memory, at agent scope: a round trip takes several times as long as
@@ -145,14 +147,15 @@ static int fwd_poll_delay_default(int function, int dtype, const Plan& p, int ti
   const bool elman = function == FRNN_ELMAN || function == FRNN_ELMAN_CLIP;
   // kernels that multiply the workgroup's own slice in front of the wait: little is left to sleep through
   if (fwd_own_slice_first(cell_dims(function).GR, p.D, p.waves, p.utw, p.kw, tile_rows, dtype == FRNN_F32 ? 4 : 2)) {
-    if (elman) return p.kw > 8 && dtype != FRNN_F32 ? 2 : 0;
-    if (p.kw > 8) return p.kw >= 16 ? 6 : p.kw < 12 ? 1 : function == FRNN_GRU ? 2 : 0;
+    if (elman) return p.kw <= 8 && p.waves <= 4 && tile_rows == 4 && dtype != FRNN_F32 ? 1 : 0;
+    if (p.kw > 8) return p.kw >= 16 ? 6 : p.kw < 12 ? 1 : function == FRNN_GRU ? 1 : 0;
     return tile_rows >= 8 ? 2 : (function == FRNN_GRU || p.kw > 5) ? 1 : 0;
   }
   if (elman) return p.waves > 4 ? 2 : 6;
   if (p.kw == 3) return 2;
   if (p.kw == 6) return 4;
   if (p.kw == 10) return 5;
+  if (p.kw >= 32 && dtype != FRNN_F32 && tile_rows <= 8) return tile_rows == 8 ? 2 : 1;
   if (p.kw >= 12) return 6;
   if (p.kw == 4 && function == FRNN_GRU) return 4;
   return 3;
@@ -776,9 +779,13 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   p.cooperative = env_int("FRNN_COOPERATIVE", 0);
   // measured best, as in the forward call (exchange stores kept in the XCD's L2): the gated cells 0-2 units at every
   // head dim from 192 to 1024 (their dWx stores are issued between the send and the first probe, which is part of
-  // their delay), elman D = 512 4, D = 1024 8; recompute mode sends its first probe behind the LDS reads of the
-  // rebuild: best without a delay for every cell
-  a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", o.rc ? 0 : c.GR == 1 ? (p.kw > 4 ? 8 : 4) : 2);
+  // their delay), 0 from 10 workgroups per head on in the 16-bit types at 4-row tiles (at 8 rows 0 to +1 %) and with 32
+  // (512 steps, with 2 and with 0: lstm D = 640 0.824 /
+  // 0.801 ms, D = 1024 1.038 / 1.013, B64 T256 0.700 / 0.683, slstm D = 768 0.950 / 0.929, gru D = 768 0.765 / 0.751); elman D = 512 4,
+  // D = 1024 8 (8 waves), the kernels of 4 waves 2 (D = 320 0.435 ms with 8, 0.375 with 2; D = 640 0.547 / 0.495); recompute
+  // mode sends its first probe behind the LDS reads of the rebuild: best without a delay for every cell
+  const bool half = dtype != FRNN_F32;
+  a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", o.rc ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && (tr == 4 || p.kw >= 32) ? 0 : 2);
   a.g_clip = o.g_clip; a.cut = o.cut;
   // producer-wave stores of dWx, under the same condition (reverse kernel: LSTM N12 D64 B256 1.16 against 1.26 ms, B128
   // 0.64 / 0.76, B64 0.48 / 0.49, B16 0.41 / 0.41; GRU N12 D64 B256 0.79 / 0.97; sLSTM N12 D64 B128 0.80 / 1.00; LSTM N24 D32
