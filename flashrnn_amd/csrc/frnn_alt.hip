@@ -42,7 +42,7 @@ struct AltStepFwdArgs {
                     // caller carries the state of an earlier call in sfp)
 };
 
-template <int F, typename T>
+template <int F, typename T, int RND>
 __global__ void __launch_bounds__(256) alt_step_fwd_kernel(const AltStepFwdArgs a) {
   typedef Cell<F> C;
   typedef ST<T> X;
@@ -121,12 +121,12 @@ __global__ void __launch_bounds__(256) alt_step_fwd_kernel(const AltStepFwdArgs 
           }
       }
     }
-    // 4 k-steps of this wave per round: all their fragments are requested before the first MFMA,
-    // so a round costs one trip to L2 instead of four
-    for (int ks0 = w; ks0 < (sizeof(T) == 4 ? 0 : KS); ks0 += 16) {
-      Frag vf[4], af[4][GR];
+    // RND k-steps of this wave per round: all their fragments are requested before the first MFMA,
+    // so a round costs one trip to L2 instead of RND (which RND: see alt_fwd_round_of_8)
+    for (int ks0 = w; ks0 < (sizeof(T) == 4 ? 0 : KS); ks0 += 4 * RND) {
+      Frag vf[RND], af[RND][GR];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < RND; ++j) {
         const int ks = ks0 + 4 * j;
         vf[j] = Frag{};
 #pragma unroll
@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(256) alt_step_fwd_kernel(const AltStepFwdArgs 
         }
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < RND; ++j)
 #pragma unroll
         for (int g = 0; g < GR; ++g) acc[g] = X::mfma(af[j][g], vf[j], acc[g]);
     }
@@ -329,13 +329,26 @@ __global__ void __launch_bounds__(256) alt_bias_kernel(const AltBiasArgs a) {
 // ---------------------------------------------------------------------------------------------
 // host drivers
 // ---------------------------------------------------------------------------------------------
+// k-steps that a wave of the 16-bit forward step requests per round.  8 for a cell with one recurrent gate whose waves have more
+// than 4 each (heads beyond 512 units): the launch then waits for one trip to memory instead of two (Elman bf16, us per
+// launch: B32 D1024 4.21 -> 4.10, B16 D640 3.49 -> 3.37); 4 otherwise: with nothing to request in the upper half of the
+// round its branches are on the way (Elman N3 D256 2.73 -> 2.76), and with four gates the 4-step rounds already have 20
+// loads each in flight (LSTM D1024 7.24 -> 7.34).
+static bool alt_fwd_round_of_8(int D) { return D > 512; }
+
 template <int F, typename T>
 static int alt_forward_t(const AltProblem& p, const AltFwdBuffers& bf, hipStream_t st) {
   const dim3 grid(p.D / 16, p.N, (p.B + 15) / 16);
+  [[maybe_unused]] const bool wide = alt_fwd_round_of_8(p.D);
   for (int t = 0; t < p.T; ++t) {
     AltStepFwdArgs a{bf.Wx, bf.R, bf.b, bf.s0, bf.states, bf.cache, bf.sfp, p.B, p.T, p.N, p.D, t, p.training, p.h_clip,
                      (t > 0 || p.use_carry) ? 1 : 0};
-    hipLaunchKernelGGL((alt_step_fwd_kernel<F, T>), grid, dim3(256), 0, st, a);
+    if constexpr (Cell<F>::GR == 1 && sizeof(T) == 2) {
+      if (wide) hipLaunchKernelGGL((alt_step_fwd_kernel<F, T, 8>), grid, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL((alt_step_fwd_kernel<F, T, 4>), grid, dim3(256), 0, st, a);
+    } else {
+      hipLaunchKernelGGL((alt_step_fwd_kernel<F, T, 4>), grid, dim3(256), 0, st, a);
+    }
     const int e = (int)hipGetLastError();
     if (e) return e;
   }
