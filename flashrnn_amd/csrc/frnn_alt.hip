@@ -194,8 +194,11 @@ __global__ void __launch_bounds__(256) alt_step_bwd_kernel(const AltStepBwdArgs 
   const int D = a.D, N = a.N, B = a.B, Tn = a.T, t = a.t;
   const size_t ND = (size_t)N * D, BND = (size_t)B * ND;
 
-  // operands of the adjoint first (thread -> unit d0 + tid % 16 of batch row bt*16 + tid / 16), so
-  // that their latency hides behind the product
+  // operands of the adjoint (thread -> unit d0 + tid % 16 of batch row bt*16 + tid / 16), requested before the MFMAs so that
+  // their latency hides behind the product, but behind the fragments of the first round: loads return in order, these come
+  // from HBM and the fragments from closer by, so in front of them they hold up the product (16-bit types, us per step of a
+  // pass, forward and backward: Elman B32 D1024 10.01 -> 9.55, N3 D256 7.50 -> 7.16, LSTM D1024 19.38 -> 18.68, D256 8.95 ->
+  // 8.56, sLSTM N2 D384 12.47 -> 12.26, GRU D768 14.37 -> 14.39)
   const int u = tid & 15, bl = tid >> 4;
   const int b = bt * 16 + bl, d = d0 + u;
   const bool evalid = b < B;
@@ -205,20 +208,24 @@ __global__ void __launch_bounds__(256) alt_step_bwd_kernel(const AltStepBwdArgs 
   const T* states = static_cast<const T*>(a.states);
   const T* dstates = static_cast<const T*>(a.dstates);
   float cc[NC > 0 ? NC : 1], sp[S], sn[S], dso[S], ds[S], gr[GR], gw[GW], gb[GT];
+  auto operands = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int k = 0; k < S; ++k) ds[k] = a.dsr[(size_t)k * BND + idx];
-  if (t >= 0) {  // uniform
-    const T* cache = static_cast<const T*>(a.cache) + (((size_t)t * B + be) * N + n) * NC * D + d;
+    for (int k = 0; k < S; ++k) ds[k] = a.dsr[(size_t)k * BND + idx];
+    if (t >= 0) {  // uniform
+      const T* cache = static_cast<const T*>(a.cache) + (((size_t)t * B + be) * N + n) * NC * D + d;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) cc[c] = ld(cache + (size_t)c * D);
+      for (int c = 0; c < NC; ++c) cc[c] = ld(cache + (size_t)c * D);
 #pragma unroll
-    for (int k = 0; k < S; ++k) {
-      const size_t so = (((size_t)k * B + be) * Tn + t) * ND + (size_t)n * D + d;
-      sn[k] = ld(states + so);
-      dso[k] = ld(dstates + so);
-      sp[k] = t > 0 ? ld(states + so - ND) : ld(s0 + ((size_t)k * B + be) * ND + (size_t)n * D + d);
+      for (int k = 0; k < S; ++k) {
+        const size_t so = (((size_t)k * B + be) * Tn + t) * ND + (size_t)n * D + d;
+        sn[k] = ld(states + so);
+        dso[k] = ld(dstates + so);
+        sp[k] = t > 0 ? ld(states + so - ND) : ld(s0 + ((size_t)k * B + be) * ND + (size_t)n * D + d);
+      }
     }
-  }
+  };
+  const bool product_first = sizeof(T) == 2 && a.has_dg && GR * D >= 4 * X::KM;  // uniform; every wave has a k-step
+  if (!product_first) operands();
 
   if (a.has_dg) {  // uniform
     const int bm = bt * 16 + r16;
@@ -257,6 +264,9 @@ __global__ void __launch_bounds__(256) alt_step_bwd_kernel(const AltStepBwdArgs 
         af[j] = load_frag<T>(arow, kc, q4);
         if (!bvalid || ks >= KS) vf[j] = Frag{};
       }
+      __builtin_amdgcn_sched_barrier(0);
+      if (product_first && ks0 == w) operands();
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 8; j += 2) {
         acc = X::mfma(af[j], vf[j], acc);
