@@ -249,18 +249,35 @@ fused_bwd_kernel(const BwdArgs a) {
         s0o[i] = oks ? (((unsigned)(pk * BS + bt * TR + pr) * ND + col) * ES) : kInvalidOff;
         sl[i] = c < SP_TOT ? ((pk * UT_WG + ptile) * TR + pr) * 16 + half * 8 : -1;
       }
+      // The compiler counts the operations in flight behind each load exactly, but where two paths meet it takes the lower
+      // count: at the head of a loop that follows the first fetches directly, with the loads of two iterations interleaved
+      // by its scheduler, the first of every three iterations waited for loads sent one iteration before (vmcnt 1 where 11
+      // may stay in flight: a trip to HBM within the step).  ORDERED: loads in program order, and the first three
+      // iterations in front of the loop, so that the counts hold on every turn.  Where it pays: the sLSTM's kernels of 4
+      // and 6 waves (reverse kernel, T = 512, without and with: bf16 B128 N12 D64 0.396 -> 0.373 ms, B224 N10 D64 0.693
+      // -> 0.626, B256 N8 D64 0.494 -> 0.479, B128 N6 D96 0.347 -> 0.309); its kernels of 2 waves +4 to +8 % at small batches
+      // and of 8 waves +-1 %, the other gated cells -5 to +3 %, the Elman cell +15 % (B16 N12 D64)
+      constexpr bool ORDERED = F == FRNN_SLSTM && WAVES >= 4 && WAVES <= 6;
+      auto in_order = []() __attribute__((always_inline)) { if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0); };
       struct Ops { Dw<4> ca[NPC > 0 ? NPC : 1], sp[NPS], dso[NPS]; };
       Ops set[3];
       auto fetch = [&](Ops& o, int j) __attribute__((always_inline)) {
-        const int t = Tn - 1 - j > 0 ? Tn - 1 - j : 0;  // (beyond the last step: the operands of step 0 again, unused)
+        int t = Tn - 1 - j > 0 ? Tn - 1 - j : 0;  // (beyond the last step: the operands of step 0 again, unused)
+        if constexpr (ORDERED) t = __builtin_amdgcn_readfirstlane(t);  // (as in the steps: no vector arithmetic on a scalar offset)
         const bool first = t == 0;
         const rsrc_t rPrev = first ? rS0 : rSt;
+        in_order();
 #pragma unroll
-        for (int i = 0; i < NPC; ++i) o.ca[i] = buf_load<4>(rCa, cvo[i], (((unsigned)t * N + n) * (D / 16)) * Bpad * 16 * NCP * ES);
+        for (int i = 0; i < NPC; ++i) {
+          o.ca[i] = buf_load<4>(rCa, cvo[i], (((unsigned)t * N + n) * (D / 16)) * Bpad * 16 * NCP * ES);
+          in_order();
+        }
 #pragma unroll
         for (int i = 0; i < NPS; ++i) {
           o.dso[i] = buf_load<4>(rDs, svo[i], (unsigned)t * ND * ES);
+          in_order();
           o.sp[i] = buf_load<4>(rPrev, first ? s0o[i] : spo[i], first ? 0u : (unsigned)(t - 1) * ND * ES);
+          in_order();
         }
       };
       // (no branch on the lane: behind one the compiler waits for every load in flight, the latest ones included;
@@ -325,7 +342,17 @@ fused_bwd_kernel(const BwdArgs a) {
 #endif
         };
         int i = 0;
-        for (; i + 2 < Tn; i += 3) {
+        if (ORDERED && Tn >= 3) {
+          iter(0, set[2], set[1]);
+          iter(1, set[0], set[2]);
+          iter(2, set[1], set[0]);
+          for (i = 3; i + 2 < Tn; i += 3) {
+            iter(i, set[2], set[1]);
+            iter(i + 1, set[0], set[2]);
+            iter(i + 2, set[1], set[0]);
+          }
+        }
+        for (; !ORDERED && i + 2 < Tn; i += 3) {
           iter(i, set[2], set[1]);
           iter(i + 1, set[0], set[2]);
           iter(i + 2, set[1], set[0]);

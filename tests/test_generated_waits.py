@@ -1,0 +1,50 @@
+"""Waits in the generated code of kernels whose loads have to stay in flight over a step.  What a source line asks for can be
+lost in the compiler's counting of outstanding loads (it takes the lower count where two paths meet), which shows in no
+result, only in the time; so the built device code is read back."""
+import os
+import re
+
+import pytest
+
+from test_kernel_resources import LLVM, ROOT, _disassemble
+
+BUILD = os.path.join(ROOT, "flashrnn_amd", "csrc", "build")
+
+
+def _functions(obj, tmp):
+    path = os.path.join(BUILD, obj)
+    if not os.path.exists(path):
+        pytest.fail(f"{path} is missing: build the library first (make -C flashrnn_amd/csrc)")
+    if not os.path.exists(f"{LLVM}/llvm-objdump"):
+        pytest.skip("no llvm-objdump in this image")
+    out, name = {}, None
+    for line in _disassemble(path, str(tmp)).splitlines():
+        m = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+        if m:
+            name = m.group(1)
+            out[name] = []
+        elif name and line.strip():
+            out[name].append(line.split("//")[0].strip())
+    return out
+
+
+def _vmcnt(lines):
+    return [int(m.group(1)) for t in lines for m in [re.search(r"s_waitcnt .*vmcnt\((\d+)\)", t)] if m]
+
+
+@pytest.mark.parametrize("obj", ["fused_bwd_1_0.o", "fused_bwd_1_2.o"])
+def test_producer_wave_of_the_slstm_waits_for_no_load_of_the_last_iteration(obj, tmp_path):
+    """Between two barriers the producer wave hands over operands that it requested two iterations before and requests new
+    ones: with n loads per iteration at least n are in flight, whatever path led there, and no wait may ask for fewer."""
+    kernels = {k: v for k, v in _functions(obj, tmp_path).items()
+               if re.search(r"fused_bwd_kernelILi1E\w+?Li(64ELi4|96ELi6)ELi1ELi1ELi4ELb0ELb[01]E", k)}
+    assert len(kernels) == 4, sorted(kernels)
+    for name, code in kernels.items():
+        bars = [i for i, t in enumerate(code) if t.startswith("s_barrier")]
+        steps = [code[a:b] for a, b in zip(bars, bars[1:])]
+        steps = [s for s in steps if any("ds_write_b128" in t for t in s) and any("buffer_load_dwordx4" in t for t in s)]
+        loads = [sum("buffer_load_dwordx4" in t for t in s) for s in steps]
+        n = min(loads)
+        assert n >= 6 and loads.count(n) >= 3 and set(loads) <= {n, 3 * n}, (name, loads)  # (3n: the first requests)
+        short = [w for s, m in zip(steps, loads) for w in _vmcnt(s) if m == n and w < n]
+        assert not short, f"{name}: waits of vmcnt {short} with {n} loads per iteration"
