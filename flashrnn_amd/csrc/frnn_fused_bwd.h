@@ -1104,6 +1104,11 @@ fused_bwd_kernel(const BwdArgs a) {
         }
       }
       // receive: KW-1 partial sums of the own tiles, PSRC sources at a time
+      // LANES: Elman heads of 8 workgroups of 8 waves (D = 1024), which sit at the register limit, combine the tests of a probe
+      // as lane conditions and ask whether to give up before they send the next one (reverse kernel, T = 256, integers and
+      // send first against LANES: bf16 B16 0.374 -> 0.346 ms, B96 0.408 -> 0.372; with forward_clipval bf16 B96 4.8 %, fp16
+      // 12 % less; fp16 without it 2 % more: not there.  The other Elman tilings: integers 1 to 8 % ahead)
+      constexpr bool LANES = GR == 1 && WAVES == 8 && KW == 8 && !(F == FRNN_ELMAN && std::is_same_v<T, half_t>);
       Wait wait{a.status, dead_flag, a.spin_limit};
       const IW* const mine = inbox + (size_t)(t & 1) * INW + ((size_t)(slice * NPOS + wp) * UTW) * KW * 256 + lane;
       if constexpr (RSP) {
@@ -1129,7 +1134,7 @@ fused_bwd_kernel(const BwdArgs a) {
                 need[(rr * UTW + u) * E + e] = rvalid && in;
               }
           }
-          poll_words_reload<PT, NWR>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0);
+          poll_words_reload<PT, NWR, true, true>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0);
 #pragma unroll
           for (int rr = 0; rr < PSRC_W; ++rr) {
             const bool in = k0 + rr < SRC_W && rbeg + k0 + rr < KW;
@@ -1188,7 +1193,7 @@ fused_bwd_kernel(const BwdArgs a) {
           poll_issue<NWR>(mine, off, v);
           __builtin_amdgcn_sched_barrier(0);
           if (t > 0) { rebuild_product(rhq, racc); rebuild_math(pm, racc); }
-          poll_finish<PT, NWR, (TR < 16)>(mine, off, need, t, v, wait);
+          poll_finish<PT, NWR, (TR < 16), true>(mine, off, need, t, v, wait);
           if constexpr (TR == 16) {
             // (never taken, which the compiler does not know: without an exit here the sLSTM's D = 128 kernel spills)
             int never = 0;
@@ -1196,7 +1201,7 @@ fused_bwd_kernel(const BwdArgs a) {
             if (never) { dead = true; return; }
           }
         } else {
-          poll_words_reload<PT, NWR>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0);
+          poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0);
         }
 #pragma unroll
         for (int rr = 0; rr < PSRC; ++rr)
