@@ -48,3 +48,13 @@ def test_producer_wave_of_the_slstm_waits_for_no_load_of_the_last_iteration(obj,
         assert n >= 6 and loads.count(n) >= 3 and set(loads) <= {n, 3 * n}, (name, loads)  # (3n: the first requests)
         short = [w for s, m in zip(steps, loads) for w in _vmcnt(s) if m == n and w < n]
         assert not short, f"{name}: waits of vmcnt {short} with {n} loads per iteration"
+
+
+def test_alternating_lstm_step_in_fp32_requests_its_product_before_it_waits(tmp_path):
+    """The operands of the adjoint are requested in front of the product and waited for behind it: on the way to the block of
+    its first MFMA, which waits for the fragments, there is no wait for a load."""
+    (code,) = [v for k, v in _functions("frnn_alt.o", tmp_path).items() if "alt_step_bwd_kernelILi0EfE" in k]
+    first = next(i for i, t in enumerate(code) if "mfma" in t)
+    waits = [i for i, t in enumerate(code[:first]) if re.search(r"vmcnt\(", t)]
+    early = [i for i in waits if first - i > 20]
+    assert not early, code[early[0] - 5:early[0] + 3]
