@@ -1,6 +1,6 @@
 """Alternating backend: head dims around the lines at which its step kernels change the order and the number of the
 fragments that a wave requests at once (forward: more than 512 units of a one-gate cell, 8 k-steps of 32 units per round
-and 4 waves; backward: at least 4 k-steps, one for each wave)."""
+and 4 waves; backward: at least 4 k-steps, one for each wave, and for the GRU no more than the 32 of a round)."""
 import pytest
 
 from parity import check_case
@@ -21,6 +21,7 @@ CASES = [
     ("gru", 17, 9, 2, 32, "bfloat16"),
     ("lstm", 17, 9, 2, 32, "float16"),
     ("slstm", 1, 9, 3, 32, "bfloat16"),
+    ("gru", 3, 9, 1, 320, "bfloat16"),
     ("gru", 3, 9, 1, 352, "bfloat16"),
 ]
 
