@@ -206,142 +206,6 @@ __global__ void __launch_bounds__(256) alt_step_bwd_kernel(const AltStepBwdArgs 
   const bool evalid = b < B;
   const int be = evalid ? b : 0;
   const size_t idx = ((size_t)be * N + n) * D + d;
-  float ry[GR], wx[GW], bb[GT - GR + 1], s[S], cc[NC > 0 ? NC : 1];
-#pragma unroll
-  for (int g = 0; g < GR; ++g) ry[g] = ld(bias + (size_t)(g * N + n) * D + d);
-#pragma unroll
-  for (int g = 0; g < GW; ++g) wx[g] = ld(Wx + (((size_t)be * Tn + t) * GW + g) * ND + (size_t)n * D + d);
-#pragma unroll
-  for (int g = GR; g < GT; ++g) bb[g - GR] = ld(bias + (size_t)(g * N + n) * D + d);
-#pragma unroll
-  for (int k = 0; k < S; ++k)
-    s[k] = a.from_sfp ? a.sfp[(size_t)k * BND + idx] : ld(s0 + ((size_t)k * B + be) * ND + (size_t)n * D + d);
-
-  // ---- R h_{t-1} of the tile: acc[g] = rows (g, n, d0..d0+15) x batch rows bt*16..+15 ----
-  {
-    const int bm = bt * 16 + r16;
-    const bool bvalid = bm < B;
-    const T* vrow = (t > 0 ? states + (size_t)(bvalid ? bm : 0) * Tn * ND + (size_t)(t - 1) * ND
-                           : s0 + (size_t)(bvalid ? bm : 0) * ND) + (size_t)n * D;
-    const int KS = D / X::KM;
-    f32x4 acc[GR];
-#pragma unroll
-    for (int g = 0; g < GR; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // fp32: a fragment of v_mfma_f32_16x16x4_f32 is one float per lane, and a load of 4 bytes per lane and k-step
-    // left the step waiting for hundreds of tiny loads (LSTM fp32 D = 1024: 52 us per step).  A lane takes 4
-    // consecutive k with one 16-byte load instead (k = 16 kg + 4 q4 .. + 3) and MFMA i of the group uses element i of
-    // every lane: both operands are read the same way, so every k still meets itself, in another order.
-    if constexpr (sizeof(T) == 4) {
-      const int KG = D / 16;
-      for (int kg0 = w; kg0 < KG; kg0 += 16) {  // 4 groups of this wave per round, requested together
-        float4 vf[4], af[4][GR];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int kg = kg0 + 4 * j;
-          vf[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-          for (int g = 0; g < GR; ++g) af[j][g] = make_float4(0.f, 0.f, 0.f, 0.f);
-          if (kg < KG) {  // uniform over the wave
-            if (bvalid) vf[j] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(vrow) + kg * 16 + q4 * 4);
-#pragma unroll
-            for (int g = 0; g < GR; ++g)
-              af[j][g] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(R) + ((size_t)(g * N + n) * D + d0 + r16) * D + kg * 16 + q4 * 4);
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int g = 0; g < GR; ++g) {
-            acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[j][g].x, vf[j].x, acc[g], 0, 0, 0);
-            acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[j][g].y, vf[j].y, acc[g], 0, 0, 0);
-            acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[j][g].z, vf[j].z, acc[g], 0, 0, 0);
-            acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[j][g].w, vf[j].w, acc[g], 0, 0, 0);
-          }
-      }
-    }
-    // RND k-steps of this wave per round: all their fragments are requested before the first MFMA,
-    // so a round costs one trip to L2 instead of RND (which RND: see alt_fwd_round_of_8)
-    for (int ks0 = w; ks0 < (sizeof(T) == 4 ? 0 : KS); ks0 += 4 * RND) {
-      Frag vf[RND], af[RND][GR];
-#pragma unroll
-      for (int j = 0; j < RND; ++j) {
-        const int ks = ks0 + 4 * j;
-        vf[j] = Frag{};
-#pragma unroll
-        for (int g = 0; g < GR; ++g) af[j][g] = Frag{};
-        if (ks < KS) {  // uniform over the wave
-          vf[j] = load_frag<T>(vrow, ks, q4);
-#pragma unroll
-          for (int g = 0; g < GR; ++g) af[j][g] = load_frag<T>(R + ((size_t)(g * N + n) * D + d0 + r16) * D, ks, q4);
-          if (!bvalid) vf[j] = Frag{};
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < RND; ++j)
-#pragma unroll
-        for (int g = 0; g < GR; ++g) acc[g] = X::mfma(af[j][g], vf[j], acc[g]);
-    }
-#pragma unroll
-    for (int g = 0; g < GR; ++g) *reinterpret_cast<f32x4*>(&red[w][g][lane * 4]) = acc[g];
-  }
-  __syncthreads();
-  if (!evalid) return;
-  const int src = red_index(u, bl);
-#pragma unroll
-  for (int g = 0; g < GR; ++g) ry[g] += red[0][g][src] + red[1][g][src] + red[2][g][src] + red[3][g][src];
-  CM::fwd(ry, wx, bb, s, cc);
-  s[0] = clamp_if(s[0], a.h_clip);
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    st_(states + (((size_t)k * B + b) * Tn + t) * ND + (size_t)n * D + d, s[k]);
-    if (a.sfp) a.sfp[(size_t)k * BND + idx] = s[k];
-  }
-  if (a.training && NC > 0) {
-    T* cache = static_cast<T*>(a.cache) + (((size_t)t * B + b) * N + n) * NC * D + d;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) st_(cache + (size_t)c * D, cc[c]);
-  }
-}
-
-// Reverse step t: the recurrent term R^T dg_{t+1} of the tile's 16 units (dg of the step above
-// comes from the previous launch, in the storage type, as the product's operand), then the
-// adjoint of step t for the same units, which leaves dg_t for the next launch.  t == -1: only the
-// recurrent term of step 0, added to the running cotangent to give ds0.
-struct AltStepBwdArgs {
-  const void* Rt; const void* s0; const void* states; const void* cache; const void* dstates;
-  void* dWx; void* dgx; void* ds0;
-  const void* dg_in;  // [B][N][G_r*D] of step t+1
-  void* dg_out;       // same for step t (the other of two buffers)
-  float* dsr;         // [S][B][N][D] running cotangent without the recurrent term
-  int B, T, N, D, t;
-  int has_dg;         // 0: no recurrent term (first reverse step, or gradient_recurrent_cut)
-  float g_clip;       // > 0: cotangent carried into h_t clamped to [-g_clip, g_clip]
-};
-
-template <int F, typename T>
-__global__ void __launch_bounds__(256) alt_step_bwd_kernel(const AltStepBwdArgs a) {
-  typedef Cell<F> C;
-  typedef ST<T> X;
-  typedef typename X::Frag Frag;
-  typedef CellMath<F, X::FAST> CM;
-  constexpr int GR = C::GR, GW = C::GW, GT = C::GT, S = C::S, NC = C::NC;
-  __shared__ __attribute__((aligned(16))) float red[4][256];
-  const int d0 = blockIdx.x * 16, n = blockIdx.y, bt = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int r16 = lane & 15, q4 = lane >> 4;
-  const int D = a.D, N = a.N, B = a.B, Tn = a.T, t = a.t;
-  const size_t ND = (size_t)N * D, BND = (size_t)B * ND;
-
-  // operands of the adjoint (thread -> unit d0 + tid % 16 of batch row bt*16 + tid / 16), requested before the MFMAs so that
-  // their latency hides behind the product, but behind the fragments of the first round: loads return in order, these come
-  // from HBM and the fragments from closer by, so in front of them they hold up the product (16-bit types, us per step of a
-  // pass, forward and backward: Elman B32 D1024 10.01 -> 9.55, N3 D256 7.50 -> 7.16, LSTM D1024 19.38 -> 18.68, D256 8.95 ->
-  // 8.56, sLSTM N2 D384 12.47 -> 12.26, GRU D768 14.37 -> 14.39)
-  const int u = tid & 15, bl = tid >> 4;
-  const int b = bt * 16 + bl, d = d0 + u;
-  const bool evalid = b < B;
-  const int be = evalid ? b : 0;
-  const size_t idx = ((size_t)be * N + n) * D + d;
   const T* s0 = static_cast<const T*>(a.s0);
   const T* states = static_cast<const T*>(a.states);
   const T* dstates = static_cast<const T*>(a.dstates);
