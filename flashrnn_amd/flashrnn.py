@@ -714,8 +714,10 @@ def flashrnn_step(
 
 
 def make_carry(states: torch.Tensor) -> torch.Tensor:
-    """The fp32 carry of ``flashrnn_step`` for a chain that starts at ``states`` [S,B,1,N,D]."""
-    return states[:, :, 0].to(torch.float32).contiguous()
+    """The fp32 carry of ``flashrnn_step`` for a chain that starts at ``states`` [S,B,1,N,D]: memory of its own also for
+    states that are fp32 already, since a step rewrites it while workgroups of the same head still read h from ``states``."""
+    return states[:, :, 0].to(torch.float32, copy=True, memory_format=torch.contiguous_format)
+
 
 class FlashRNNDecoder:
     """A decode session: the fused forward kernel of the head dimension stays on the device, R in its registers and the
