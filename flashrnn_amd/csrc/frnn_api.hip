@@ -127,6 +127,17 @@ static int env_int(const char* name, int dflt) {
 // check the placement themselves, see xcd_handshake).  FRNN_AGENT_STORES=1 keeps every store at agent scope.
 static bool near_stores_allowed() { return env_int("FRNN_AGENT_STORES", 0) == 0; }
 
+// FRNN_SPIN_LIMIT: probes before a wait between the workgroups of a head gives up.  Two values are there for tests of the failure
+// path.  -2: the fused scans take the wait at their start as run out and enter no time step.  -3: the launches leave out the
+// last workgroup of their last (up to 8) groups, for which the others of its group then wait 256 probes in vain, in their first
+// step that waits (or, with FRNN_AGENT_STORES=0, in the handshake at the start); every kernel still ends by its own bounds.
+static int spin_limit_of(Plan* p, bool waits) {
+  const int limit = env_int("FRNN_SPIN_LIMIT", 1 << 22);
+  if (limit != -3) return limit;
+  if (waits && p->kw > 1) p->left_out = p->kw > kXcdWorkgroups ? 1 : 8;  // (the last slice of 8 consecutive groups: see decode_block)
+  return 256;
+}
+
 // s_sleep units before the first probe of a forward step.  A probe that reaches memory before the
 // data costs a whole extra round trip and adds traffic, one that comes late costs its lateness; where
 // the data arrives depends on how long the other workgroups' gate math and stores take, so the best
@@ -656,7 +667,7 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   a.carry = carry; a.step = step;
   a.B = B; a.BS = o.bs ? o.bs : B; a.T = T; a.N = N; a.groups_total = groups; a.tile_rows = tr;
   a.training = need_cache ? 1 : 0;
-  a.spin_limit = env_int("FRNN_SPIN_LIMIT", 1 << 22);
+  a.spin_limit = spin_limit_of(&p, !step && T > 1);
   p.cooperative = env_int("FRNN_COOPERATIVE", 0);
   a.poll_delay = env_int("FRNN_POLL_DELAY", fwd_poll_delay_default(fx, dtype, p, tr));
   a.h_clip = o.h_clip;
@@ -775,7 +786,7 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   a.ll = w.ll; a.status = w.status;
   a.xcd = (near_stores_possible(p) && near_stores_allowed()) ? w.xcd : nullptr;
   a.B = B; a.BS = o.bs ? o.bs : B; a.T = T; a.N = N; a.groups_total = groups; a.tile_rows = tr;
-  a.spin_limit = env_int("FRNN_SPIN_LIMIT", 1 << 22);
+  a.spin_limit = spin_limit_of(&p, !o.cut);
   p.cooperative = env_int("FRNN_COOPERATIVE", 0);
   // measured best, as in the forward call (exchange stores kept in the XCD's L2): the gated cells 0-2 units at every
   // head dim from 192 to 1024 (their dWx stores are issued between the send and the first probe, which is part of

@@ -22,7 +22,7 @@ template <int Dv, int W, int U, int K, int MTR> static void (*fwd_kernel_for(int
 
 template <>
 int fused_fwd_launch<FRNN_F, FRNN_DT>(const Plan& p, const FwdArgs& a, hipStream_t st) {
-  const dim3 grid(grid_for(a.groups, p.kw));
+  const dim3 grid(grid_for(a.groups, p.kw) - p.left_out);
 #define FRNN_CASE(Dv, VAR, W, U, K, MTR)                                                     \
   if (p.D == Dv && p.waves == W && p.utw == U && p.kw == K) {                                 \
     auto kern = fwd_kernel_for<Dv, W, U, K, MTR>(a.tile_rows, a.pst);                                \

@@ -1,8 +1,8 @@
 """The waits between the workgroups of a head are bounded: when one runs out, every kernel still
 ends normally, the status word says so, the affected outputs are NaN and the Python layer raises
 RuntimeError at the next call or at check_status().  The condition is forced from the host with
-FRNN_SPIN_LIMIT=-2 (every wait then gives up at once, before its first probe); nothing on the GPU
-faults or hangs."""
+FRNN_SPIN_LIMIT=-2 (the scans then take the wait at their start as run out and report it without a single time step;
+waits that run out within the time loop: test_gpu_wait_runs_out.py); nothing on the GPU faults or hangs."""
 import pytest
 import torch
 
@@ -12,8 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 KDT = {"bfloat16": torch.bfloat16, "float32": torch.float32}
-# (the fp32 case and bf16 D = 1024: the kernels whose waves work in pairs, 14 and 32 workgroups per head, where the second
-# wave of a pair takes part in every barrier of the first and must leave the time loop with it)
+# (the fp32 case and bf16 D = 1024: the kernels whose waves work in pairs, 14 and 32 workgroups per head)
 SHAPES = [("bfloat16", 256), ("float32", 448), ("bfloat16", 1024), ("float32", 1024)]
 
 
@@ -46,7 +45,7 @@ def test_expired_wait_in_forward_raises_at_the_next_call(gpu, monkeypatch, dtype
     assert torch.isfinite(good).all()
 
     monkeypatch.setenv("FRNN_SPIN_LIMIT", "-2")
-    bad, _ = _call(gpu, inp, False, dtype)             # returns: every wave left its time loop
+    bad, _ = _call(gpu, inp, False, dtype)             # returns: every wave passed its time loop by
     assert torch.isnan(bad[0]).all()                   # h of every workgroup: all of them gave up
     assert last_status("forward") == 1
     monkeypatch.delenv("FRNN_SPIN_LIMIT")
