@@ -687,9 +687,9 @@ fused_bwd_kernel(const BwdArgs a) {
   }
 
   bool dead = near_i < 0;
-  // does a step look at the workgroup's flag of a failed wait?  Heads of one workgroup never wait (the recompute-mode
-  // kernels of the sLSTM and of 8 waves keep the flag all the same: any other form of their step spills)
-  constexpr bool FLAG = KW > 1 || (RC && (F == FRNN_SLSTM || WAVES > 6));
+  // does a step look at the workgroup's flag of a failed wait?  Heads of one workgroup never wait, and nobody sets it (the
+  // recompute-mode kernel of the sLSTM at D = 96 reads it all the same: in fp16 any other form of its step spills)
+  constexpr bool FLAG = KW > 1 || (RC && F == FRNN_SLSTM && WAVES > 4);
   static_assert(!(PW && FLAG), "the producer wave reads no flag");
   // one reverse step: consumes `pc` (operands of step t), prefetches those of step t-1 into `pn`.
   // CUT (a std::bool_constant): truncated backpropagation, the step ends with the pointwise carry;
@@ -803,12 +803,8 @@ fused_bwd_kernel(const BwdArgs a) {
     // mode 0.555 -> 0.540, GRU bf16 B16 T2048 N4 D128 1.043 -> 1.032)
     if constexpr (!FLAG) {
       lds_barrier();
-      if constexpr (RC || TR > 4) {
-        // (never taken, which the compiler does not know: without an exit here it schedules these kernels, which sit at the
-        // register limit, into spills)
-        int never = 0;
-        asm volatile("" : "+s"(never));
-        if (never) { dead = true; return; }
+      if constexpr (RC || TR > 4) {  // (without an exit here: spills)
+        if (never()) { dead = true; return; }
       }
     } else { if (barrier_or(dead_flag)) { dead = true; return; } }
     FRNN_STAMP(c2);
@@ -1195,10 +1191,7 @@ fused_bwd_kernel(const BwdArgs a) {
           if (t > 0) { rebuild_product(rhq, racc); rebuild_math(pm, racc); }
           poll_finish<PT, NWR, (TR < 16), true>(mine, off, need, t, v, wait);
           if constexpr (TR == 16) {
-            // (never taken, which the compiler does not know: without an exit here the sLSTM's D = 128 kernel spills)
-            int never = 0;
-            asm volatile("" : "+s"(never));
-            if (never) { dead = true; return; }
+            if (never()) { dead = true; return; }  // (without an exit here the sLSTM's D = 128 kernel spills)
           }
         } else {
           poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0);
