@@ -182,7 +182,7 @@ struct Wait {
 typedef __attribute__((address_space(3))) int lds_flag_t;  // (an explicit LDS pointer: see barrier_or)
 // Does every word that the wave needs carry the tag of step t?  Straight-line (a short-circuit && turns into a chain of
 // divergent branches with a wait inside each).  BITS: the differences are combined as integers, one compare at the end;
-// otherwise as lane conditions in scalar registers, for the kernels at the register limit, where the masks spill.
+// otherwise as lane conditions in scalar registers, for the kernels at the register limit, where the integers spill to memory.
 template <typename TAG, int NW, bool BITS, typename W>
 __device__ __forceinline__ bool all_arrived(const W* v, const bool* need, int t) {
   if constexpr (BITS) {
@@ -213,7 +213,7 @@ __device__ __forceinline__ bool give_up(Wait& w, int spins) {
 // Poll NW tagged words (addresses base + off[i]; every lane polls NW words, lanes or entries
 // with nothing to wait for pass need[i] = false and may point anywhere valid) until all carry the
 // tag of step t.  Loads are unconditional and the exit test is a wave vote.
-template <typename TAG, int NW>
+template <typename TAG, int NW, bool BITS>
 __device__ __forceinline__ void poll_words(const u64* base, const int* off, const bool* need, int t, u64* out, Wait& w, int first_delay) {
   // (one probe of the set in flight: more only add congestion, measured again with exact waits)
   // the producers finish their step at about the same time as this wave: a probe sent at once
@@ -222,7 +222,7 @@ __device__ __forceinline__ void poll_words(const u64* base, const int* off, cons
   for (int spins = 0;; ++spins) {
 #pragma unroll
     for (int i = 0; i < NW; ++i) out[i] = ll_load(base + off[i]);
-    if (__builtin_expect(all_arrived<TAG, NW, (NW < 16)>(out, need, t), 1)) break;
+    if (__builtin_expect(all_arrived<TAG, NW, BITS>(out, need, t), 1)) break;
     if (give_up(w, spins)) break;
   }
 }
@@ -260,7 +260,7 @@ __device__ __forceinline__ void poll_words_reload(const W* base, const int* off,
 // The same wait for pairs of adjacent words, each pair fetched with one 16-byte agent-scope load
 // (raw buffer load, cache policy sc1): half the memory instructions per probe.  A 16-byte load is
 // not one atomic access, which the protocol does not need: every 32-bit half carries its own tag.
-template <typename TAG, int NW>
+template <typename TAG, int NW, bool BITS>
 __device__ __forceinline__ void poll_pairs(rsrc_t slot, unsigned soff, const int* off, const bool* need, int t, u64* out, Wait& w, int first_delay) {
   static_assert(NW % 2 == 0, "pairs");
   for (int i = 0; i < first_delay; ++i) __builtin_amdgcn_s_sleep(1);
@@ -271,7 +271,7 @@ __device__ __forceinline__ void poll_pairs(rsrc_t slot, unsigned soff, const int
       out[i] = (u64)v.x | ((u64)v.y << 32);
       out[i + 1] = (u64)v.z | ((u64)v.w << 32);
     }
-    if (__builtin_expect(all_arrived<TAG, NW, (NW < 16)>(out, need, t), 1)) break;
+    if (__builtin_expect(all_arrived<TAG, NW, BITS>(out, need, t), 1)) break;
     if (give_up(w, spins)) break;
   }
 }
@@ -281,7 +281,7 @@ __device__ __forceinline__ unsigned lds_rotated(int off, int rot, int tot) {
   const unsigned d = (unsigned)(off - rot);
   return tot ? min(d, d + (unsigned)tot) : (unsigned)off;  // (off < rot: d wraps, d + tot is the index)
 }
-template <typename T, int NP>
+template <typename T, int NP, bool BITS>
 __device__ __forceinline__ void ll_gather_pairs(rsrc_t slots, unsigned soff, const int* q, int t, T* lds_dst, Wait& w,
                                                 int first_delay, int rot = 0, int tot = 0) {
   constexpr int CH = NP < 16 ? NP : 16;  // words polled together
@@ -291,7 +291,7 @@ __device__ __forceinline__ void ll_gather_pairs(rsrc_t slots, unsigned soff, con
     int off[CH]; bool need[CH]; u64 v[CH];
 #pragma unroll
     for (int i = 0; i < CH; ++i) { need[i] = q[c0 + i] >= 0; off[i] = need[i] ? q[c0 + i] : 0; }
-    poll_pairs<T, CH>(slots, soff, off, need, t, v, w, c0 == 0 ? first_delay : 0);
+    poll_pairs<T, CH, BITS>(slots, soff, off, need, t, v, w, c0 == 0 ? first_delay : 0);
     // (the list is a whole number of pairs: its length, rows x columns / 2, is even)
 #pragma unroll
     for (int i = 0; i < CH; i += 2)
@@ -303,7 +303,7 @@ __device__ __forceinline__ void ll_gather_pairs(rsrc_t slots, unsigned soff, con
 
 // Forward gather: poll the planned words of slot, then copy their payloads to LDS.
 // C4: the LDS vector is kept as [k][4 rows] (the fp32 4-row tiles, see lds_index4) instead of fragment order
-template <typename T, int NP, bool C4 = false>
+template <typename T, int NP, bool BITS, bool C4 = false>
 __device__ __forceinline__ void ll_gather(const u64* slot, const int* q, int t, T* lds_dst, Wait& w,
                                           int first_delay, int rot = 0, int tot = 0) {
   constexpr int CH = NP < 16 ? NP : 16;  // words polled together
@@ -313,7 +313,7 @@ __device__ __forceinline__ void ll_gather(const u64* slot, const int* q, int t, 
     int off[CH]; bool need[CH]; u64 v[CH];
 #pragma unroll
     for (int i = 0; i < CH; ++i) { need[i] = q[c0 + i] >= 0; off[i] = need[i] ? q[c0 + i] : 0; }
-    poll_words<T, CH>(slot, off, need, t, v, w, c0 == 0 ? first_delay : 0);
+    poll_words<T, CH, BITS>(slot, off, need, t, v, w, c0 == 0 ? first_delay : 0);
 #pragma unroll
     for (int i = 0; i < CH; ++i)
       if (need[i]) reinterpret_cast<unsigned*>(lds_dst)[C4 ? lds_index4_of_word(off[i]) : lds_rotated(off[i], rot, tot)] = ll_payload((T*)0, v[i]);

@@ -90,6 +90,14 @@ fused_fwd_kernel(const FwdArgs a) {
   // 16-bit types fetch two adjacent words with one 16-byte load when a thread polls more than one
   constexpr bool PAIRS = X::EPW == 2 && NP_ > 1;
   constexpr int NP = NP_ <= 16 ? (PAIRS ? (NP_ + 1) / 2 * 2 : NP_) : (NP_ + 15) / 16 * 16;
+  // The words of a probe are tested as integers, also where a probe has 16 of them.  As lane conditions the tests keep a second set
+  // of masks, the inverse of the one under which the words are copied to LDS; with 16 words and more the two sets overflow the
+  // scalar registers, and between the arrival of the words and the barrier each mask of the copy is fetched back from a vector
+  // register (54 v_readlane per step).  That had cost the 16-row tiles of the GRU at D = 768 and of the fp32 Elman cell 1 to 2 %
+  // (forward, T = 256, B256 N2, lane conditions and integers: GRU bf16 D768 1.400 and 1.242 ms, Elman fp32 D512 1.238 and
+  // 1.128, D448 1.065 and 0.974; LSTM bf16 D1024 -12 %, D640 -6 %).
+  // Lane conditions where the integers spill to memory: the 16-bit 16-row tiles of the sLSTM at D = 640 and of the GRU at D = 1024.
+  constexpr bool LANE_TESTS = sizeof(T) == 2 && TR == 16 && ((F == FRNN_SLSTM && D == 640) || (F == FRNN_GRU && D == 1024));
   // (values per element of a cache line: the cell's NC and, where cache_carried_state says so, one state of step t-1)
   constexpr int CXS = cache_carried_state(F, (int)sizeof(T), D), NCX = NC + (CXS >= 0 ? 1 : 0);
   constexpr int NCA = NCX > 0 ? NCX : 1;
@@ -476,8 +484,8 @@ fused_fwd_kernel(const FwdArgs a) {
     if (t > 0) {
       if (KW > 1) {
         Wait w{a.status, &dead_flag, a.spin_limit};
-        if constexpr (PAIRS) ll_gather_pairs<T, NP>(rLL, (unsigned)((t - 1) & 1) * LLW * 8u, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
-        else ll_gather<T, NP, M44>(llbase + (size_t)((t - 1) & 1) * LLW, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
+        if constexpr (PAIRS) ll_gather_pairs<T, NP, !LANE_TESTS>(rLL, (unsigned)((t - 1) & 1) * LLW * 8u, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
+        else ll_gather<T, NP, !LANE_TESTS, M44>(llbase + (size_t)((t - 1) & 1) * LLW, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
         if (barrier_or(&dead_flag)) { dead = true; return; }
       } else {
         lds_barrier();

@@ -50,6 +50,23 @@ def test_producer_wave_of_the_slstm_waits_for_no_load_of_the_last_iteration(obj,
         assert not short, f"{name}: waits of vmcnt {short} with {n} loads per iteration"
 
 
+@pytest.mark.parametrize("obj,kernel", [
+    ("fused_fwd_3_1.o", r"ILi3EfLi(448|512|640)ELi4E\w+?Li16E"), ("fused_fwd_2_0.o", r"ILi2E\w+?Li768ELi4E\w+?Li16E"),
+    ("fused_fwd_2_2.o", r"ILi2E\w+?Li768ELi4E\w+?Li16E")])
+def test_masks_of_a_probe_of_16_words_stay_in_scalar_registers(obj, kernel, tmp_path):
+    """Forward, tallest tiles: from the last request of a probe to the barrier behind the copy of its words to LDS no mask is
+    fetched back from a vector register, to which the compiler moves scalar values that it has no room for."""
+    kernels = {k: v for k, v in _functions(obj, tmp_path).items() if re.search("fused_fwd_kernel" + kernel, k)}
+    assert kernels
+    for name, code in kernels.items():
+        probes = [i for i, (a, b) in enumerate(zip(code, code[1:])) if "load_dwordx" in a and "sc1" in a and not ("load_dwordx" in b and "sc1" in b)]
+        assert len(probes) >= 4, name  # (two rounds of a step, two steps per turn of the loop)
+        for i in probes:
+            end = next(j for j in range(i, len(code)) if code[j].startswith("s_barrier") or (j > i and "sc1" in code[j] and "dwordx" in code[j]))
+            back = sum("v_readlane" in t for t in code[i:end])
+            assert back <= 4, f"{name}: {back} masks fetched back behind the probe at {i}"
+
+
 def test_alternating_lstm_step_in_fp32_requests_its_product_before_it_waits(tmp_path):
     """The operands of the adjoint are requested in front of the product and waited for behind it: on the way to the block of
     its first MFMA, which waits for the fragments, there is no wait for a load."""
