@@ -148,7 +148,9 @@ static int spin_limit_of(Plan* p, bool waits) {
 //   workgroups) 6; elman D=320, 512 (4 waves) 1 (0.321 / 0.395 ms with 0, 0.314 / 0.386 with 1), D=1024 (8 waves) 0, D=640 0
 //   (0.441 ms with 2, 0.429 with 0), fp32 0; 8- and 16-row tiles 2-4 (flat);
 //   lstm, slstm D=768 (12 workgroups) 0-1, D=1024 (32 workgroups) 1 (0.862 / 0.891 ms with 6, 0.812 / 0.844 with 1; 8-row tiles
-//   B64 T256 0.563 with 6, 0.556 with 2; 16-row tiles B128 T128 0.429 with 6, 0.434 with 2);  fp32 with the operand in the 4x4x1 form 6 (D=384, 512 +2 to +7 % with 0-3).
+//   B64 T256 0.563 with 6, 0.556 with 2; 16-row tiles B128 T128 0.429 with 6, 0.434 with 2);  fp32 with the operand in the 4x4x1 form 6 (D=384, 512 +2 to +7 % with 0-3),
+//   but the sLSTM 8 (with 6 and 8, 256 steps: B5 D=384 0.507 / 0.498 ms, D=448 0.566 / 0.545, D=512 0.619 / 0.594, B64 N2 D=512 1.285 / 1.266;
+//   with the shorter waits 6 had become its slowest place between 0 and 12).
 static int fwd_poll_delay_default(int function, int dtype, const Plan& p, int tile_rows) {
   if (p.kw <= 1) return 0;
   // groups that span the device exchange through memory, at agent scope: a round trip takes several times as long as
@@ -167,7 +169,7 @@ static int fwd_poll_delay_default(int function, int dtype, const Plan& p, int ti
   if (p.kw == 6) return 4;
   if (p.kw == 10) return 5;
   if (p.kw >= 32 && dtype != FRNN_F32 && tile_rows <= 8) return tile_rows == 8 ? 2 : 1;
-  if (p.kw >= 12) return 6;
+  if (p.kw >= 12) return function == FRNN_SLSTM && dtype == FRNN_F32 ? 8 : 6;
   if (p.kw == 4 && function == FRNN_GRU) return 4;
   return 3;
 }
