@@ -796,9 +796,12 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   // (512 steps, with 2 and with 0: lstm D = 640 0.824 /
   // 0.801 ms, D = 1024 1.038 / 1.013, B64 T256 0.700 / 0.683, slstm D = 768 0.950 / 0.929, gru D = 768 0.765 / 0.751); elman D = 512 4,
   // D = 1024 8 (8 waves), the kernels of 4 waves 2 (D = 320 0.435 ms with 8, 0.375 with 2; D = 640 0.547 / 0.495); recompute
-  // mode sends its first probe behind the LDS reads of the rebuild: best without a delay for every cell
+  // mode sends its first probe behind the LDS reads of the rebuild: best without a delay for every cell; heads of 40 workgroups
+  // (fp32 D = 640), whose words come through memory, 14 (with 2 and 14, 256 steps: lstm B4 N1 0.866 / 0.829 ms, B16 N2 2.19 / 2.15, B64 N2
+  // 7.37 / 7.31, gru 0.797 / 0.760, 2.02 / 1.99, 6.76 / 6.68); with 48 and 64 the best place differs by batch size (D = 1024: B8 N1 -4 %
+  // with 24, B4 N1 +10 %)
   const bool half = dtype != FRNN_F32;
-  a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", o.rc ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && (tr == 4 || p.kw >= 32) ? 0 : 2);
+  a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", o.rc ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && (tr == 4 || p.kw >= 32) ? 0 : p.kw == 40 ? 14 : 2);
   a.g_clip = o.g_clip; a.cut = o.cut;
   // producer-wave stores of dWx, under the same condition (reverse kernel: LSTM N12 D64 B256 1.16 against 1.26 ms, B128
   // 0.64 / 0.76, B64 0.48 / 0.49, B16 0.41 / 0.41; GRU N12 D64 B256 0.79 / 0.97; sLSTM N12 D64 B128 0.80 / 1.00; LSTM N24 D32

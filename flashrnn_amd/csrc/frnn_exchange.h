@@ -237,11 +237,13 @@ __device__ __forceinline__ void poll_issue(const W* base, const int* off, W* v) 
 }
 // SEND_FIRST: the next probe is sent before it is asked whether the wait gives up (a few scalar instructions earlier, but the
 // way out with loads in flight puts waits for them behind the loop).
-template <typename TAG, int NW, bool BITS, bool SEND_FIRST, typename W>
+// PAUSE: s_sleep units in front of the next probe, for heads whose probes go to memory and share its queues with many others.
+template <typename TAG, int NW, bool BITS, bool SEND_FIRST, int PAUSE = 0, typename W>
 __device__ __forceinline__ void poll_finish(const W* base, const int* off, const bool* need, int t, W* v, Wait& w) {
   for (int spins = 0;; ++spins) {
     if (__builtin_expect(all_arrived<TAG, NW, BITS>(v, need, t), 1)) break;
     if constexpr (!SEND_FIRST) { if (give_up(w, spins)) break; }
+    if constexpr (PAUSE > 0) __builtin_amdgcn_s_sleep(PAUSE);
 #pragma unroll
     for (int i = 0; i < NW; ++i) v[i] = ll_load(base + off[i]);
     if constexpr (SEND_FIRST) { if (give_up(w, spins)) break; }
@@ -249,12 +251,12 @@ __device__ __forceinline__ void poll_finish(const W* base, const int* off, const
 }
 
 // The two halves back to back.
-template <typename TAG, int NW, bool BITS, bool SEND_FIRST, typename W>
+template <typename TAG, int NW, bool BITS, bool SEND_FIRST, int PAUSE = 0, typename W>
 __device__ __forceinline__ void poll_words_reload(const W* base, const int* off, const bool* need, int t, W* v, Wait& w, int first_delay) {
   for (int i = 0; i < first_delay; ++i) __builtin_amdgcn_s_sleep(1);
 #pragma unroll
   for (int i = 0; i < NW; ++i) v[i] = ll_load(base + off[i]);
-  poll_finish<TAG, NW, BITS, SEND_FIRST>(base, off, need, t, v, w);
+  poll_finish<TAG, NW, BITS, SEND_FIRST, PAUSE>(base, off, need, t, v, w);
 }
 
 // The same wait for pairs of adjacent words, each pair fetched with one 16-byte agent-scope load

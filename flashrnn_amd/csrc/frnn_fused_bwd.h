@@ -1130,7 +1130,10 @@ fused_bwd_kernel(const BwdArgs a) {
                 need[(rr * UTW + u) * E + e] = rvalid && in;
               }
           }
-          poll_words_reload<PT, NWR, true, true>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0);
+          // (groups that span the device probe memory: the shorter waits had them probe more often, at D = 640 in front of the words;
+          // a pause between the probes 0.4 to 1.5 % at every batch size, two units less, four and eight slower; see also the
+          // first-probe delay)
+          poll_words_reload<PT, NWR, true, true, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0);
 #pragma unroll
           for (int rr = 0; rr < PSRC_W; ++rr) {
             const bool in = k0 + rr < SRC_W && rbeg + k0 + rr < KW;
