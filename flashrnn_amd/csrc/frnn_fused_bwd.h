@@ -1107,6 +1107,9 @@ fused_bwd_kernel(const BwdArgs a) {
       constexpr bool LANES = GR == 1 && WAVES == 8 && KW == 8 && !(F == FRNN_ELMAN && std::is_same_v<T, half_t>);
       Wait wait{a.status, dead_flag, a.spin_limit};
       const IW* const mine = inbox + (size_t)(t & 1) * INW + ((size_t)(slice * NPOS + wp) * UTW) * KW * 256 + lane;
+      // fp32 wave pairs of the GRU, 14 and 16 workgroups per head: asked in front of the next probe (reverse kernel, T = 256, B8 N2, next
+      // probe first against this: D = 512 0.668 -> 0.659 ms, where the shorter waits had cost 2 %, D = 448 0.605 -> 0.590)
+      constexpr bool SEND_FIRST = !(F == FRNN_GRU && sizeof(T) == 4 && DSP == 2 && KW >= 14);
       if constexpr (RSP) {
         const int rbeg = 1 + hf * SRC_W;  // (uniform) this wave's sources: rbeg .. rbeg + SRC_W - 1, below KW
         float rs[UTW][E];
@@ -1133,7 +1136,7 @@ fused_bwd_kernel(const BwdArgs a) {
           // (groups that span the device probe memory: the shorter waits had them probe more often, at D = 640 in front of the words;
           // a pause between the probes 0.4 to 1.5 % at every batch size, two units less, four and eight slower; see also the
           // first-probe delay)
-          poll_words_reload<PT, NWR, true, true, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0);
+          poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0);
 #pragma unroll
           for (int rr = 0; rr < PSRC_W; ++rr) {
             const bool in = k0 + rr < SRC_W && rbeg + k0 + rr < KW;
