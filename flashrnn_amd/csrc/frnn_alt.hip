@@ -346,16 +346,18 @@ __global__ void __launch_bounds__(256) alt_bias_kernel(const AltBiasArgs a) {
 // host drivers
 // ---------------------------------------------------------------------------------------------
 // k-steps that a wave of the 16-bit forward step requests per round.  8 for a cell with one recurrent gate whose waves have more
-// than 4 each (heads beyond 512 units): the launch then waits for one trip to memory instead of two (Elman bf16, us per
-// launch: B32 D1024 4.21 -> 4.10, B16 D640 3.49 -> 3.37); 4 otherwise: with nothing to request in the upper half of the
-// round its branches are on the way (Elman N3 D256 2.73 -> 2.76), and with four gates the 4-step rounds already have 20
-// loads each in flight (LSTM D1024 7.24 -> 7.34).
-static bool alt_fwd_round_of_8(int D) { return D > 512; }
+// than 4 each (heads beyond 512 units): the launch then waits for one trip to memory instead of two (Elman bf16 B16 N1, ms per 256 steps,
+// 4 and 8: D544 0.800 / 0.772, D640 0.886 / 0.853, D768 0.940 / 0.908, D1024 1.051 / 1.017), while a compute unit has about one
+// workgroup (the device has 256): a second one hides the second trip (B64 N2: D544, 272 workgroups, 0.960 / 0.951; D640, 320, 1.148 / 1.155;
+// D1024, 512, 1.500 / 1.510).  4 otherwise: with nothing to request in the upper half of the round its branches are on the way (D384
+// 0.735 / 0.742, D512 0.787 / 0.795), and with four gates the 4-step rounds already have 20 loads each in flight (LSTM
+// D1024, us per launch, 7.24 / 7.34).
+static bool alt_fwd_round_of_8(int D, unsigned workgroups) { return D > 512 && workgroups <= 288; }
 
 template <int F, typename T>
 static int alt_forward_t(const AltProblem& p, const AltFwdBuffers& bf, hipStream_t st) {
   const dim3 grid(p.D / 16, p.N, (p.B + 15) / 16);
-  [[maybe_unused]] const bool wide = alt_fwd_round_of_8(p.D);
+  [[maybe_unused]] const bool wide = alt_fwd_round_of_8(p.D, grid.x * grid.y * grid.z);
   for (int t = 0; t < p.T; ++t) {
     AltStepFwdArgs a{bf.Wx, bf.R, bf.b, bf.s0, bf.states, bf.cache, bf.sfp, p.B, p.T, p.N, p.D, t, p.training, p.h_clip,
                      (t > 0 || p.use_carry) ? 1 : 0};

@@ -15,6 +15,10 @@ CASES = [
     ("elman", 5, 9, 1, 544, "float16"),
     ("elman", 33, 9, 1, 1024, "bfloat16"),
     ("elman", 2, 9, 1, 1056, "bfloat16"),
+    # ... and the 4-step rounds again where the launch has more than 288 workgroups of 16 units x 16 rows: 272, 306 and 320 of them
+    ("elman", 64, 5, 2, 544, "bfloat16"),
+    ("elman", 129, 5, 1, 544, "float16"),
+    ("elman", 65, 5, 1, 1024, "bfloat16"),
     # backward: k-steps (gates x units / 32) below, at and above one for each wave, and one into the second round
     ("elman", 5, 9, 2, 96, "bfloat16"),
     ("elman", 5, 9, 2, 128, "bfloat16"),
