@@ -795,7 +795,8 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   // their delay), 0 from 10 workgroups per head on in the 16-bit types at 4-row tiles (at 8 rows 0 to +1 %) and with 32
   // (512 steps, with 2 and with 0: lstm D = 640 0.824 /
   // 0.801 ms, D = 1024 1.038 / 1.013, B64 T256 0.700 / 0.683, slstm D = 768 0.950 / 0.929, gru D = 768 0.765 / 0.751); elman D = 512 4,
-  // D = 1024 8 (8 waves), the kernels of 4 waves 2 (D = 320 0.435 ms with 8, 0.375 with 2; D = 640 0.547 / 0.495); recompute
+  // D = 1024 8 (8 waves), the kernels of 4 waves 2 (D = 320 0.435 ms with 8, 0.375 with 2; D = 640
+  // 0.547 / 0.495; at 8- and 16-row tiles of D = 320, 448 and 640 within 1 % of the best, 8 +3 to +9 %); recompute
   // mode sends its first probe behind the LDS reads of the rebuild: best without a delay for every cell; heads of 40 workgroups
   // (fp32 D = 640), whose words come through memory, 14 (with 2 and 14, 256 steps: lstm B4 N1 0.866 / 0.829 ms, B16 N2 2.19 / 2.15, B64 N2
   // 7.37 / 7.31, gru 0.797 / 0.760, 2.02 / 1.99, 6.76 / 6.68); with 48 and 64 the best place differs by batch size (D = 1024: B8 N1 -4 %

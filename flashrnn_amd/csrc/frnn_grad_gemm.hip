@@ -18,8 +18,8 @@ namespace frnn {
 // The first tiles * tiles * GR * N workgroups transpose one 32 x 32 tile each; the others clear 4 KB each of the exchange
 // words that the reverse scan behind this launch needs at zero (heads of several workgroups).  Both are far too short to
 // fill the device (4-5 us each, most of it the launch), so one launch does both
-// (forward + backward, LSTM bf16 B100 T200 N1 D640 0.956 -> 0.950 ms, Elman B64 T256 D640 0.607 -> 0.602, LSTM B128 T128 D1024,
-// 11 MB to clear, 1.444 -> 1.430).
+// (forward + backward, LSTM bf16 B100 T200 N1 D640 0.956 -> 0.950 ms, LSTM B128 T128 D1024, 11 MB to clear, 1.444 -> 1.430: 0.6 to 1 %,
+// little more than two runs differ).
 template <typename T>
 __global__ void __launch_bounds__(256) transpose_r_kernel(const T* __restrict__ R, T* __restrict__ Rt, int N, int D, int GR,
                                                           unsigned transposing, u32x4* __restrict__ zero, size_t zero_pieces) {

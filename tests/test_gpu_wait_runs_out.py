@@ -18,7 +18,7 @@ CASES = [
     ("lstm", "bfloat16", 8, 256, 4, False),
     ("slstm", "bfloat16", 16, 768, 8, False),
     ("slstm", "bfloat16", 8, 192, 4, False),
-    # ... 16 words per probe (lane conditions), in one round and in several, with and without the own slice in front
+    # ... 16 words per probe, in one round and in several, with and without the own slice in front (GRU at 16 rows: lane conditions)
     ("gru", "bfloat16", 5, 1024, 4, False),
     ("gru", "float16", 20, 1024, 8, False),
     ("gru", "bfloat16", 17, 1024, 16, False),
@@ -36,7 +36,7 @@ CASES = [
     ("lstm", "float16", 16, 192, 16, True),
     ("slstm", "bfloat16", 16, 128, 16, True),
     ("gru", "bfloat16", 16, 256, 16, True),
-    # fp32: the 4x4x1 form, without a split, in wave pairs, in fours over the device (24 and 32 workgroups: lane conditions)
+    # fp32: the 4x4x1 form, without a split, in wave pairs, in fours over the device (with a pause between reverse probes)
     ("gru", "float32", 4, 256, 4, False),
     ("lstm", "float32", 4, 320, 4, False),
     ("lstm", "float32", 4, 384, 4, False),
