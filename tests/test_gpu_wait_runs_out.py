@@ -23,6 +23,7 @@ CASES = [
     ("gru", "float16", 20, 1024, 8, False),
     ("gru", "bfloat16", 17, 1024, 16, False),
     ("lstm", "bfloat16", 16, 640, 16, False),
+    ("slstm", "bfloat16", 16, 640, 16, False),
     # ... wave pairs that split k forward, the destinations and the sources in reverse, in one round and in several
     ("lstm", "bfloat16", 9, 1024, 4, False),
     ("slstm", "float16", 16, 1024, 8, False),
@@ -41,6 +42,7 @@ CASES = [
     ("lstm", "float32", 4, 320, 4, False),
     ("lstm", "float32", 4, 384, 4, False),
     ("slstm", "float32", 3, 512, 4, False),
+    ("gru", "float32", 4, 512, 4, False),
     ("gru", "float32", 3, 640, 4, False),
     ("lstm", "float32", 4, 1024, 4, False),
     # ... the 16x16x4 form: one round and several, few words and 16 per probe
