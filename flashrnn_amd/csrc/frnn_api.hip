@@ -158,6 +158,19 @@ static int fwd_poll_delay_default(int function, int dtype, const Plan& p, int ti
   // (the other cells and D = 768 also best at 24, within 1 %; 40 workgroups per head, D = 640: 18 2.64 ms, 24 2.74)
   if (p.kw > kXcdWorkgroups) return p.kw <= 40 ? 18 : 24;
   const bool elman = function == FRNN_ELMAN || function == FRNN_ELMAN_CLIP;
+  // heads spread by splitting k between the waves of a tile (variants 2 and 3 of the tables), T = 256, B4 N1 and B16 N2, delays 0 to
+  // 12 swept: fp32, fours: D=128 flat from 0 to 4 (6 +3 %), D=192 gru 6 (0.271 ms; 0 0.274), the others 0, D=256 lstm and gru 6 (0.311; 0
+  // 0.320), slstm 0 (0.326; 6 0.348), D=320 8, D=384 .. 512 8 (D=512 0.462; 6 0.470, 12 0.476), slstm 10; 16-bit pairs flat from 0 to 2
+  const int ksp = fwd_k_split(p.D, p.waves, p.utw, p.kw);
+  if (dtype != FRNN_F32 && ksp > 1 && p.D < 1024) return 1;
+  if (dtype != FRNN_F32 && ksp > 1 && function == FRNN_GRU) return 1;
+  if (dtype == FRNN_F32 && ksp == 4) {
+    if (p.kw <= 8) return 4;
+    if (p.kw <= 12) return function == FRNN_GRU ? 6 : 0;
+    if (p.kw <= 16) return function == FRNN_SLSTM ? 0 : 6;
+    return function == FRNN_SLSTM && p.kw > 20 ? 10 : 8;
+  }
+  if (dtype == FRNN_F32 && ksp == 2 && p.kw <= 10) return function == FRNN_SLSTM ? 0 : p.kw >= 8 ? 6 : 4;  // (D=320 slstm 0.431 ms, with 5 0.447)
   // kernels that multiply the workgroup's own slice in front of the wait: little is left to sleep through
   if (fwd_own_slice_first(cell_dims(function).GR, p.D, p.waves, p.utw, p.kw, tile_rows, dtype == FRNN_F32 ? 4 : 2)) {
     if (elman) return p.kw <= 8 && p.waves <= 4 && tile_rows == 4 && dtype != FRNN_F32 ? 1 : 0;
@@ -196,16 +209,22 @@ static int groups_per_launch(int kw) { return kw > kXcdWorkgroups ? device_cus()
 // (such groups never share an XCD: no handshake, every exchange store at agent scope)
 static bool near_stores_possible(const Plan& p) { return p.kw > 1 && p.kw <= kXcdWorkgroups; }
 
-// The tiling of a call: the table's default for the head dim, or its small-batch alternative (variant 2) while all
-// groups of the call fit one launch with 4-row tiles.  FRNN_FUSED_VARIANT picks a variant by hand.
+// The tiling of a call: the table's default for the head dim, or the widest of its small-batch alternatives (variant 3, else 2) for
+// which all groups of the call fit one launch with 4-row tiles (not where FRNN_TILE_ROWS asks for taller tiles than it has).
+// FRNN_FUSED_VARIANT picks a variant by hand.
 static bool pick_plan(int function, int dtype, int B, int N, int D, int backward, Plan* p) {
   const int variant = env_int("FRNN_FUSED_VARIANT", 0);
   if (!find_plan(function, dtype, D, variant, backward, p)) return false;
   if (variant == 0) {
-    Plan q;
-    if (find_plan(function, dtype, D, 2, backward, &q) && q.variant == 2 && q.kw > 1 &&
-        (long)N * ((B + 3) / 4) <= groups_per_launch(q.kw))
-      *p = q;
+    const int rows = env_int("FRNN_TILE_ROWS", 0);
+    for (int v = 3; v >= 2; --v) {
+      Plan q;
+      if (find_plan(function, dtype, D, v, backward, &q) && q.variant == v && q.kw > 1 && rows <= q.max_tr &&
+          (long)N * ((B + 3) / 4) <= groups_per_launch(q.kw)) {
+        *p = q;
+        break;
+      }
+    }
   }
   return true;
 }
@@ -367,7 +386,7 @@ static FusedBwdWs carve_fused_bwd(void* ws, int function, int dtype, int B, int 
   w.status = (int*)bp.take(256);
   const int tr = tile_rows_for(B, N, p.kw, p.waves, p.max_tr, dtype);
   const size_t bt = (B + tr - 1) / tr, groups = (size_t)N * bt;
-  w.ll = (u64*)bp.take(p.kw > 1 ? groups * 3 * bwd_inbox_words(D, p.kw) * 8 : 0);
+  w.ll = (u64*)bp.take(p.kw > 1 ? groups * 3 * bwd_inbox_words(D, p.kw, tr) * (dtype == FRNN_F32 ? 8 : 4) : 0);
   w.xcd = (int*)bp.take(p.kw > 1 ? groups * 32 * 4 : 0);  // words of xcd_handshake
   w.zero_bytes = bp.off;
 #ifdef FRNN_TRACE
@@ -460,7 +479,8 @@ static int decode_plan(int function, int dtype, int B, int N, int D, int slots, 
   int e = check_problem(function, dtype, B, 1, N, D);
   if (e) return e;
   if (slots != 2 && slots != 4 && slots != 8 && slots != 16) return fail(FRNN_E_ARG, "slots must be 2, 4, 8 or 16 (got %d)", slots);
-  if (!find_plan(function, dtype, D, 0, 0, &out->p))
+  // (the tiling of a sequence call of this size: the order of a step's sums, and so the bits, are those of the sequence)
+  if (!pick_plan(function, dtype, B, N, D, 0, &out->p))
     return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
   const Plan& p = out->p;
   out->groups = N * ((B + 3) / 4);
@@ -801,8 +821,14 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   // (fp32 D = 640), whose words come through memory, 14 (with 2 and 14, 256 steps: lstm B4 N1 0.866 / 0.829 ms, B16 N2 2.19 / 2.15, B64 N2
   // 7.37 / 7.31, gru 0.797 / 0.760, 2.02 / 1.99, 6.76 / 6.68); with 48 and 64 the best place differs by batch size (D = 1024: B8 N1 -4 %
   // with 24, B4 N1 +10 %)
+  // heads spread by splitting the destinations (variants 2 and 3 of the tables), swept as in the forward call: 16-bit pairs 2 up to
+  // 14 workgroups (1 at 8, D=256 0.240 ms, with 2 0.247), 0 from 16 on (lstm D=512, 256 steps, 0.323 ms with 0, 0.330 with 2; D=768 0.433 / 0.446; D=320 0.249 with 2, 0.257 with
+  // 0); fp32 fours 4 from 10 to 16 workgroups, 6 from 20 to 28 (D=320 0.443 ms, with 2 0.450), 0 at 4, else 2
   const bool half = dtype != FRNN_F32;
-  a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", o.rc ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && (tr == 4 || p.kw >= 32) ? 0 : p.kw == 40 ? 14 : 2);
+  const int dsp = bwd_dest_split(p.D, p.waves, p.utw, p.kw);
+  const int wide_delay = half && dsp > 1 ? (p.kw <= 4 || p.kw >= 16 ? 0 : p.kw == 8 ? 1 : 2) : half || dsp != 4 ? 2
+                       : p.kw <= 4 ? 0 : p.kw < 10 ? 2 : p.kw <= 16 ? 4 : p.kw <= 28 ? 6 : 2;
+  a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", o.rc ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && dsp == 1 && tr == 4 || half && p.kw >= 32 ? 0 : p.kw == 40 ? 14 : wide_delay);
   a.g_clip = o.g_clip; a.cut = o.cut;
   // producer-wave stores of dWx, under the same condition (reverse kernel: LSTM N12 D64 B256 1.16 against 1.26 ms, B128
   // 0.64 / 0.76, B64 0.48 / 0.49, B16 0.41 / 0.41; GRU N12 D64 B256 0.79 / 0.97; sLSTM N12 D64 B128 0.80 / 1.00; LSTM N24 D32

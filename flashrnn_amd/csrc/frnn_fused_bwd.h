@@ -59,8 +59,8 @@ struct BwdArgs {
 };
 
 // words (64-bit for fp32 storage, 32-bit otherwise) of one inbox area of one group:
-// [dst wg][wave][tile][src wg][element 4][lane 64]
-constexpr size_t bwd_inbox_words(int D, int KW) { return (size_t)KW * (D / 16) * 256; }
+// [dst wg][wave][tile][src wg][element TR / 4][lane 64]
+constexpr size_t bwd_inbox_words(int D, int KW, int TR) { return (size_t)KW * (D / 16) * 64 * (TR / 4); }
 
 // Resident operand of the reverse product: a wave holds KW*UTW*KS fragments of the transposed R (all
 // destination tiles at its position, its workgroup's gate rows).  At 4 waves per workgroup a wave has
@@ -109,7 +109,7 @@ fused_bwd_kernel(const BwdArgs a) {
   typedef Own<TR> O;
   constexpr int GR = C::GR, GW = C::GW, GT = C::GT, S = C::S, NC = C::NC;
   // (DSP = 2: pairs of waves share a tile position and split the destinations between them, see bwd_dest_split)
-  constexpr int DSP = bwd_dest_split(GR, D, WAVES, UTW, KW, TR, (int)sizeof(T), RC), NPOS = WAVES / DSP;
+  constexpr int DSP = bwd_dest_split(D, WAVES, UTW, KW), NPOS = WAVES / DSP;
   constexpr int NT = WAVES * 64, UT_WG = NPOS * UTW;
   static_assert(UT_WG * KW * 16 == D, "tiling must cover the head");
   constexpr int DL = D / KW;            // units owned by this workgroup
@@ -129,13 +129,14 @@ fused_bwd_kernel(const BwdArgs a) {
   constexpr int RC_MAX = RCW / (UTW * (TR / 4)) > 0 ? RCW / (UTW * (TR / 4)) : 1;
   constexpr int ROUNDS = KW == 1 ? 1 : (KW - 1 + RC_MAX - 1) / RC_MAX;
   constexpr int PSRC = KW == 1 ? 1 : (KW - 1 + ROUNDS - 1) / ROUNDS;  // sources polled per round
-  constexpr size_t INW = bwd_inbox_words(D, KW);
+  constexpr size_t INW = bwd_inbox_words(D, KW, TR);
+  constexpr int EW = 64 * O::E;  // words of one (tile, source)
   // Waves that split the destinations of a tile position (DSP > 1) also split its sources where one wave would poll them
   // in several rounds, each a trip to memory and back: wave hf polls sources 1 + hf * SRC_W .. and hands its sum to the
   // first wave through LDS.  Measured, reverse kernel, 1024 steps: LSTM fp32 D = 1024 (63 sources at agent scope, 4 rounds of
   // 16 become one per wave) 8.68 -> 6.30 ms, bf16 D = 1024 B16 2.67 -> 2.39; also from 13 sources on, where one round
   // shrinks to half the words: fp32 D = 512 2.62 -> 2.52, D = 448 2.61 -> 2.55 (D = 384, 11 sources: 2.49 -> 2.54, left alone).
-  constexpr bool RSP = DSP > 1 && (ROUNDS > 1 || KW >= 14);
+  constexpr bool RSP = DSP > 1 && (ROUNDS > 1 || (sizeof(T) == 4 && KW >= 14));
   constexpr int SRC_W = RSP ? (KW - 1 + DSP - 1) / DSP : 1;                    // sources per wave
   constexpr int ROUNDS_W = (SRC_W + RC_MAX - 1) / RC_MAX, PSRC_W = (SRC_W + ROUNDS_W - 1) / ROUNDS_W;
   constexpr int E = O::E, ND_ = NDW<T, E>::value;
@@ -841,7 +842,7 @@ fused_bwd_kernel(const BwdArgs a) {
     // More than 8 remote destinations (10 and more workgroups per head): their products run in groups
     // of 4 destinations (4 independent MFMA chains), each group sent as soon as it is complete, so that
     // 16 accumulator registers are live instead of 4 per destination (128 at 32 workgroups per head).
-    constexpr bool GROUPED = OWN_LAST && KW - 1 > 8;
+    constexpr bool GROUPED = OWN_LAST && (KW - 1 > 8 || DS16);
     constexpr int RI = 4;
     static_assert(!GROUPED || RLD % RI == 0, "LDS-resident destinations come in whole groups");
     static_assert(!DS16 || GROUPED, "wave pairs split the destinations of the grouped product only");
@@ -904,7 +905,7 @@ fused_bwd_kernel(const BwdArgs a) {
 #pragma unroll
             for (int rr = 0; rr < RI; ++rr) {
               const int x = (slice + hfo + r0 + rr) % KW;
-              base[rr] = inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * 256;
+              base[rr] = inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * EW;
               float part[E];
               own_elems<TR>(ag[rr][u], part);
 #pragma unroll
@@ -926,7 +927,7 @@ fused_bwd_kernel(const BwdArgs a) {
 #pragma unroll
             for (int e = 0; e < E; ++e) wv[e] = part_pack((PT*)0, part[e], t);
             // (the destination's place in the area is uniform and goes into the scalar base; the lane's offset is the same for all)
-            ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * 256, sslot, wv, near_m);
+            ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * EW, sslot, wv, near_m);
           }
         }
       };
@@ -1052,7 +1053,7 @@ fused_bwd_kernel(const BwdArgs a) {
             for (int u = 0; u < UTW; ++u) {
               IW wv[E];
               wv[0] = part_pack((PT*)0, p44[q][u][j], t);
-              ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * 256, sslot, wv, near_m);
+              ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * EW, sslot, wv, near_m);
             }
           }
       }
@@ -1068,7 +1069,7 @@ fused_bwd_kernel(const BwdArgs a) {
 #pragma unroll
           for (int e = 0; e < E; ++e) wv[e] = part_pack((PT*)0, part[e], t);
           // (the destination's place in the area is uniform and goes into the scalar base; the lane's offset is the same for all)
-            ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * 256, sslot, wv, near_m);
+            ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * EW, sslot, wv, near_m);
         }
       }
       if constexpr (DW_LATE) {
@@ -1092,7 +1093,7 @@ fused_bwd_kernel(const BwdArgs a) {
             IW wv[E];
 #pragma unroll
             for (int e = 0; e < E; ++e) wv[e] = part_pack((PT*)0, own[e], t);
-            ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((((slice + hfo) % KW) * NPOS + wp_u) * UTW + u) * KW + slice) * 256, sslot, wv, near_m);
+            ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((((slice + hfo) % KW) * NPOS + wp_u) * UTW + u) * KW + slice) * EW, sslot, wv, near_m);
           } else {
 #pragma unroll
             for (int e = 0; e < E; ++e) ds[u][e][0] += own[e];
@@ -1106,7 +1107,7 @@ fused_bwd_kernel(const BwdArgs a) {
       // 12 % less; fp16 without it 2 % more: not there.  The other Elman tilings: integers 1 to 8 % ahead)
       constexpr bool LANES = GR == 1 && WAVES == 8 && KW == 8 && !(F == FRNN_ELMAN && std::is_same_v<T, half_t>);
       Wait wait{a.status, dead_flag, a.spin_limit};
-      const IW* const mine = inbox + (size_t)(t & 1) * INW + ((size_t)(slice * NPOS + wp) * UTW) * KW * 256 + lane;
+      const IW* const mine = inbox + (size_t)(t & 1) * INW + ((size_t)(slice * NPOS + wp) * UTW) * KW * EW + lane;
       // fp32 wave pairs of the GRU, 14 and 16 workgroups per head: asked in front of the next probe (reverse kernel, T = 256, B8 N2, next
       // probe first against this: D = 512 0.668 -> 0.659 ms, where the shorter waits had cost 2 %, D = 448 0.605 -> 0.590)
       constexpr bool SEND_FIRST = !(F == FRNN_GRU && sizeof(T) == 4 && DSP == 2 && KW >= 14);
@@ -1129,7 +1130,7 @@ fused_bwd_kernel(const BwdArgs a) {
             for (int u = 0; u < UTW; ++u)
 #pragma unroll
               for (int e = 0; e < E; ++e) {
-                off[(rr * UTW + u) * E + e] = (u * KW + src) * 256 + e * 64;
+                off[(rr * UTW + u) * E + e] = (u * KW + src) * EW + e * 64;
                 need[(rr * UTW + u) * E + e] = rvalid && in;
               }
           }
@@ -1177,7 +1178,7 @@ fused_bwd_kernel(const BwdArgs a) {
           for (int u = 0; u < UTW; ++u)
 #pragma unroll
             for (int e = 0; e < E; ++e) {
-              off[(rr * UTW + u) * E + e] = (u * KW + src) * 256 + e * 64;
+              off[(rr * UTW + u) * E + e] = (u * KW + src) * EW + e * 64;
               need[(rr * UTW + u) * E + e] = bvalid && (r0 + rr < KW);
             }
         }

@@ -78,10 +78,11 @@ fused_fwd_kernel(const FwdArgs a) {
   typedef typename X::Frag Frag;
   typedef Own<TR> O;
   constexpr int GR = C::GR, GW = C::GW, GT = C::GT, S = C::S, NC = C::NC;
-  // (KSP = 2: the fp32 4x4x1 form of heads from 384 units on, two waves per tile, each with one half of k; 4 beyond 512 units)
-  constexpr int KSP = fwd_k_split(GR, D, WAVES, UTW, TR, (int)sizeof(T)), DK = D / KSP;
+  // (KSP waves per tile, each with its part of k)
+  constexpr int KSP = fwd_k_split(D, WAVES, UTW, KW), DK = D / KSP;
   constexpr int KS = D / X::KM, NT = WAVES * 64, UT_WG = WAVES * UTW / KSP;
-  static_assert(UT_WG * KW * 16 == D, "tiling must cover the head");
+  static_assert(UT_WG * KW * 16 == D && WAVES % KSP == 0, "tiling must cover the head");
+  static_assert(KSP == 1 || sizeof(T) == 2 || DK % 16 == 0, "fp32: a wave reads its part of h 16 k at a time");
   static_assert(KSP <= 2 || (sizeof(T) == 4 && UTW == 1), "more than two waves per tile: the fp32 4x4x1 form only");
   constexpr int LLW = 16 * D / X::EPW;  // 64-bit words per exchange slot
   // words a thread polls per step: the TR rows of the tile, without the workgroup's own slice
@@ -111,8 +112,8 @@ fused_fwd_kernel(const FwdArgs a) {
   // instruction computes 16 columns, 12 of them padding, at the same rate).  Block = unit of the tile, the 4
   // columns of a block = the gates of that unit, A = h (the values of one block broadcast to all 16), one
   // instruction per k: D instructions of 8 cycles per tile and step instead of G_r * D / 4 of 32.
-  constexpr bool M44 = fwd_form_4x4x1(GR, D, WAVES, UTW, TR, (int)sizeof(T));  // (the whole operand, D registers per tile, in registers)
-  constexpr bool KS16 = fwd_k_split16(GR, D, WAVES, UTW, TR, (int)sizeof(T));  // 16-bit kernels whose wave pairs split k
+  constexpr bool M44 = fwd_form_4x4x1(GR, D, WAVES, UTW, KW, TR, (int)sizeof(T));  // (the whole operand, D registers per tile, in registers)
+  constexpr bool KS16 = fwd_k_split16(D, WAVES, UTW, KW, (int)sizeof(T));  // 16-bit kernels whose wave pairs split k
   constexpr int KSW = KS16 ? KS / KSP : KS;  // k-steps of a wave
   constexpr int RLK = M44 || KS16 ? 0 : fwd_lds_ksteps(GR, D, WAVES, UTW, (int)sizeof(T)), KSR = KSW - RLK;
   // Own slice first: of the h_(t-1) a step multiplies with, the workgroup's own D / KW units are in LDS as soon as
@@ -257,6 +258,7 @@ fused_fwd_kernel(const FwdArgs a) {
         fetch(refill, t + 3);
         if constexpr (PST) { if (t > 0) drain(t - 1); }
 #endif
+        if constexpr (KSP > 1) lds_barrier();  // (the one at which the waves of a tile hand their sums over)
       };
       int t = 0;
       for (; t + 2 < Tn && !pdead; t += 3) {
@@ -516,7 +518,7 @@ fused_fwd_kernel(const FwdArgs a) {
       for (int u = 0; u < UTW; ++u)
 #pragma unroll
         for (int g = 0; g < GW; ++g) {
-          const T* const src = wb + (((w * UTW + u) * GW + g) * TR + brow) * 16 + esub;
+          const T* const src = wb + (((wt * UTW + u) * GW + g) * TR + brow) * 16 + esub;
           if constexpr (E == 1) wcl[u][g].v[0] = *reinterpret_cast<const unsigned short*>(src);
           else if constexpr (E == 2) wcl[u][g].v[0] = *reinterpret_cast<const unsigned*>(src);
           else { const uint2 v = *reinterpret_cast<const uint2*>(src); wcl[u][g].v[0] = v.x; wcl[u][g].v[1] = v.y; }

@@ -9,10 +9,10 @@
 // compiler's resource report of every instantiation.
 //   R registers per lane = UTW * G_r * D / 8 (bf16) or UTW * G_r * D / 4 (f32); a workgroup of
 //   4 waves (one per SIMD) may use up to 512 VGPRs per lane, one of 8 waves 256, of 16 waves 128.
-// VARIANT 0 is the default.  VARIANT 2, where a head dim has one, spreads the head over more workgroups: it is
-// used instead of the default while every workgroup of the call still gets a compute unit of its own with 4-row
-// batch tiles (measured faster there, slower once the device is full).  To try another tiling add an
-// X(D, 1, ...) entry and run with FRNN_FUSED_VARIANT=1.  The alternatives that were measured and lost (4 waves x 2 tiles for
+// VARIANT 0 is the default.  VARIANTS 2 and 3, where a head dim has them, spread the head over more workgroups: 3, the
+// wider one, or else 2, is used instead of the default while all groups of the call fit one launch with 4-row
+// batch tiles (measured faster up to a launch that fills the device, slower where the default still takes one launch and
+// they would take two).  To try another tiling add an X(D, 1, ...) entry and run with FRNN_FUSED_VARIANT=1.  The alternatives that were measured and lost (4 waves x 2 tiles for
 // D = 128, 2 x 8 waves or 8 x 2 waves for D = 256, ...) are not compiled in.
 // Forward and backward tile independently (the gate cache layout does not depend on the plan).
 #pragma once
@@ -38,28 +38,29 @@ constexpr int fwd_lds_ksteps(int GR, int D, int WAVES, int UTW, int esize) {
   return want < room ? want : room;
 }
 
-// Forward kernel, fp32 at 4-row tiles, cells with 3 or 4 recurrent gates: the product runs on v_mfma_f32_4x4x1_16B_f32
-// (see the kernel), when the whole operand, D registers per tile in that form, fits the registers of a wave
-// (workgroups of up to 4 waves: 512 registers each).
-// Heads from 384 units on: the four waves of a workgroup pair up over two tiles, each wave of a pair keeps R for one half
-// of k (D / 2 registers) and multiplies it with that half of h; the second wave hands its partial sums to the first
-// through LDS, which alone does the gate math of the tile.  D = 16 * (WAVES / 2) * KW for these tilings.
-// The same split for the 16-bit kernels of the 4-gate cells at D = 1024 (16x16x32 form: a tile of R is 512 registers, with
-// the split 256 per wave, nothing of it in LDS, and room for the working sets of the 8- and 16-row tiles): the second
-// wave hands over its G_r accumulators.
-// fp32 heads beyond 512 units: all four waves share one tile, a quarter of k each (D / 4 registers), and three of them hand
-// their sums over; D = 16 * KW (D = 640, 768, 1024: 40, 48, 64 workgroups per head), more than the 32 compute units of an XCD: such a group
+// Waves per unit tile, forward: tilings with 16 * UTW * WAVES * KW = KSP * D, KSP = 2 or 4, have KSP waves of a workgroup share
+// a tile.  Each keeps R for one part of k (D / KSP of it) and multiplies it with that part of h; all but the first hand their
+// sums to the first through LDS, which alone does the gate math of the tile.  Two reasons to do so:
+//   the operand of a tile is more than the 512 registers of a wave hold (16-bit D = 1024; fp32 from D = 384 on), or
+//   the product of a step is long against the exchange: the head then takes KSP times the workgroups and multiplies for 1 / KSP
+//   of the time.  fp32 (8 cycles per k, see fwd_form_4x4x1), LSTM B16 N1 T256, forward: D = 512 as 16 workgroups
+//   of pairs 0.543 ms, as 32 of fours 0.470; D = 256 as 4 / 8 / 16 workgroups 0.441 / 0.369 / 0.312; D = 128 as 2 / 4 / 8 0.300 /
+//   0.279 / 0.254.  16-bit (16 cycles per gate and 32 k) from D = 384 on: LSTM D = 384 0.282 -> 0.274, D = 512 0.317 -> 0.292,
+//   D = 640 0.363 -> 0.340, D = 768 0.394 -> 0.363; sLSTM 0.298 -> 0.285 .. 0.409 -> 0.381; GRU D = 1024 0.430 -> 0.364, D = 768 0.334 ->
+//   0.319, D = 640 0.315 -> 0.298 (D = 512 and less no gain); below that the pairs lose what they cannot do, multiply the own slice in
+//   front of the wait (D = 256 0.217 -> 0.244).
+// fp32 heads beyond 512 units take D / 16 = 40, 48 or 64 workgroups, more than the 32 compute units of an XCD: such a group
 // spreads over the device (decode_block) and exchanges at agent scope.
-constexpr int fwd_k_split(int GR, int D, int WAVES, int UTW, int TR, int esize) {
-  if (esize == 2) return GR == 4 && D == 1024 && WAVES == 4 && UTW == 1 ? 2 : 1;
-  return esize == 4 && TR == 4 && GR >= 3 && WAVES == 4 && UTW == 1 && D >= 384 ? (D > 512 ? 4 : 2) : 1;
-}
-constexpr bool fwd_form_4x4x1(int GR, int D, int WAVES, int UTW, int TR, int esize) {
-  return esize == 4 && TR == 4 && GR >= 3 && WAVES <= 4 && UTW * D / fwd_k_split(GR, D, WAVES, UTW, TR, esize) <= 384;
+constexpr int fwd_k_split(int D, int WAVES, int UTW, int KW) { return 16 * WAVES * UTW * KW / D; }
+// Forward kernel, fp32 at 4-row tiles, cells with 3 or 4 recurrent gates: the product runs on v_mfma_f32_4x4x1_16B_f32
+// (see the kernel), when the whole operand, D / KSP registers per tile in that form, fits the registers of a wave (512 in
+// workgroups of up to 4 waves, 256 with up to 8: D = 96 as 6 waves).
+constexpr bool fwd_form_4x4x1(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize) {
+  return esize == 4 && TR == 4 && GR >= 3 && (WAVES <= 4 ? UTW * D / fwd_k_split(D, WAVES, UTW, KW) <= 384 : WAVES <= 8 && UTW * D <= 96);
 }
 // (16-bit kernels whose waves split k: the whole operand in registers)
-constexpr bool fwd_k_split16(int GR, int D, int WAVES, int UTW, int TR, int esize) {
-  return esize == 2 && fwd_k_split(GR, D, WAVES, UTW, TR, esize) > 1;
+constexpr bool fwd_k_split16(int D, int WAVES, int UTW, int KW, int esize) {
+  return esize == 2 && fwd_k_split(D, WAVES, UTW, KW) > 1;
 }
 // Forward kernel: one more wave per workgroup that fetches Wx for the compute waves.  A vector memory instruction that a
 // compute wave issues behind the exchange wait delays its MFMAs (~70 cycles each on the chain of dependent steps), one
@@ -72,8 +73,10 @@ constexpr bool fwd_k_split16(int GR, int D, int WAVES, int UTW, int TR, int esiz
 // D = 192 0.961 -> 0.914; the GRU (three loads per step to save) measured +1.5 % to -0.8 %, Elman the same to 0.3 %.
 constexpr bool fwd_producer_wave(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize) {
   // (heads of one workgroup: every load is on the chain; the Elman cell, one load per step, measured 0 to +10 % with the wave)
+  // (wave pairs that split k up to D = 512, 128 registers of R: forward, B8 N1 T256, without and with: LSTM D = 384 0.286 -> 0.273 ms,
+  // D = 512 0.327 -> 0.293; D = 640, 160 registers, spills with five waves)
   if (KW == 1) return esize == 2 && GR >= 3 && TR == 4 && WAVES <= 8 && UTW == 1;
-  return esize == 2 && GR == 4 && KW > 1 && TR <= 8 && WAVES == 4 && UTW * GR * (D / 32) * 4 <= (TR == 4 ? 160 : 128);
+  return esize == 2 && GR == 4 && KW > 1 && TR <= 8 && WAVES == 4 && UTW * GR * (D / 32) * 4 / fwd_k_split(D, WAVES, UTW, KW) <= (TR == 4 && fwd_k_split(D, WAVES, UTW, KW) == 1 ? 160 : 128);
 }
 // Forward kernel: may the producer wave also store the outputs of a step (16-byte pieces, one step late) instead of the
 // compute lanes (2 bytes per state and lane at 4-row tiles)?  Exists for the heads that run as one workgroup with a
@@ -105,17 +108,18 @@ constexpr int bwd_producer_bytes(int nc, int s, int ut_wg, int TR, int esize) {
 constexpr bool bwd_producer_stores(int GR, int nc, int D, int WAVES, int UTW, int KW, int TR, int esize, bool rc) {
   return bwd_producer_wave(GR, nc, D, WAVES, UTW, KW, TR, esize, rc) && WAVES <= 6;
 }
-// Backward kernel, fp32 4x4x1 form, gated cells at heads from 384 units on: the four waves of a workgroup pair up over two
-// tile positions, and each wave of a pair keeps R^T (own gate rows x destinations) for every second group of 4
-// destination workgroups (G_r * D / 8 registers instead of G_r * D / 4) and sends those groups' partial sums itself;
-// the first wave of a pair alone owns the pair's elements (gate math, loads, stores, receive).  D = 16 * (WAVES / 2) * KW.
-// The same for the 16-bit kernels of the 4-gate cells at D = 1024 (16x16x32 form, every tile height): each wave of a
-// pair keeps the fragments of one half of the 32 destination workgroups, 256 registers, none of them in LDS.
-// fp32 heads beyond 512 units: one tile position, every fourth group of 4 destinations per wave (G_r * D / 16 registers).
-constexpr int bwd_dest_split(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize, bool rc) {
-  if (esize == 2) return !rc && GR == 4 && D == 1024 && WAVES == 4 && UTW == 1 && KW == 32 ? 2 : 1;
-  return esize == 4 && TR == 4 && !rc && GR >= 3 && WAVES == 4 && UTW == 1 && D >= 384 && KW >= 8 ? (D > 512 ? 4 : 2) : 1;
-}
+// Waves per tile position, backward: with 16 * UTW * WAVES * KW = DSP * D, DSP = 2 or 4 waves of a workgroup share a position
+// and split the destinations of the reverse product between them.  fp32 (4x4x1 form): each keeps R^T (own gate rows x
+// destinations) for every DSP-th group of 4 destination workgroups, G_r * D / (4 DSP) registers; 16-bit (16x16x32 form): for one
+// half of the destination workgroups.  Each sends the partial sums it computes itself; the first wave alone owns the
+// position's elements (gate math, loads, stores).  There is no sum to hand over (but see RSP in the kernel), so the split pays from
+// smaller heads on than forward.  Reverse kernel, B8 N1 T256: 16-bit LSTM D = 192 as 6 workgroups of pairs instead of 3 0.227 -> 0.214 ms,
+// D = 256 0.257 -> 0.241, D = 320 0.279 -> 0.249, D = 384 0.305 -> 0.276, D = 448 0.333 -> 0.297, D = 512 0.359 -> 0.323, D = 640 0.411 ->
+// 0.382, D = 768 0.455 -> 0.432; sLSTM the same within 2 %, but D = 256 slower with 8 workgroups (0.263 -> 0.289) and 0.247 with 16 of
+// fours; GRU D = 320 0.248 -> 0.232, D = 512 0.316 -> 0.299, D = 1024 0.508 -> 0.477, the others no gain.
+// fp32 LSTM B16 N1 T256: D = 128 as 2 / 4 / 8 workgroups 0.422 / 0.325 / 0.278, D = 256 as 4 / 8 / 16 0.462 / 0.368 / 0.321, D = 512
+// as 16 / 32 0.623 / 0.528.
+constexpr int bwd_dest_split(int D, int WAVES, int UTW, int KW) { return 16 * WAVES * UTW * KW / D; }
 // Backward kernel: LDS bytes of the two dWx hand-over buffers of the producer-store instantiations
 // ([gate][row][unit], and [row][unit] for the GRU's g-gate cotangent), behind the operand hand-over buffers
 constexpr int bwd_producer_store_bytes(int gw, bool gru, int D, int TR, int esize) {
@@ -127,7 +131,7 @@ constexpr int bwd_producer_store_bytes(int gw, bool gru, int D, int TR, int esiz
 // (with the two-part product they spill).  The host reads this for the delay of the first probe.
 constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize) {
   const int KM = esize == 4 ? 4 : 32, KS = D / KM;
-  return KW > 1 && KW <= 16 && !fwd_form_4x4x1(GR, D, WAVES, UTW, TR, esize) && !fwd_k_split16(GR, D, WAVES, UTW, TR, esize) &&
+  return KW > 1 && KW <= 16 && !fwd_form_4x4x1(GR, D, WAVES, UTW, KW, TR, esize) && !fwd_k_split16(D, WAVES, UTW, KW, esize) &&
          (fwd_lds_ksteps(GR, D, WAVES, UTW, esize) == 0 || KW <= 12) && (D / KW) % KM == 0 &&
          !(esize == 4 && UTW * GR * KS >= 256 && TR >= (KW > 8 ? 8 : 16));
 }
@@ -142,19 +146,22 @@ constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, in
 // stop at 8-row tiles: at 16 rows the sLSTM's, with four states, and the fp16 LSTM's spill, and the bf16 LSTM's, which
 // does not, takes twice as long per launch as at 8 rows: LSTM bf16 B256 T512 12.5 against 12.8 ms)
 #define FRNN_PLANS_GR4_BF16(X) \
+  X(384, 2, 4, 1, 12, 4) X(448, 2, 4, 1, 14, 4) X(512, 2, 4, 1, 16, 4) X(640, 2, 4, 1, 20, 4) X(768, 2, 4, 1, 24, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 8, 1, 1, 16) X(160, 0, 10, 1, 1, 8) X(192, 0, 12, 1, 1, 4) \
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 8) X(1024, 0, 4, 1, 32, 16)
 #define FRNN_BWD_PLANS_GR4_BF16(X) \
+  X(192, 2, 4, 1, 6, 4) X(256, 2, 4, 1, 8, 4) X(320, 2, 4, 1, 10, 4) X(384, 2, 4, 1, 12, 4) X(448, 2, 4, 1, 14, 4) X(512, 2, 4, 1, 16, 4) X(640, 2, 4, 1, 20, 4) X(768, 2, 4, 1, 24, 4) \
   X(160, 2, 2, 1, 5, 16) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 8, 1, 1, 16) X(160, 0, 10, 1, 1, 4) X(192, 0, 4, 1, 3, 16) \
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 8) X(1024, 0, 4, 1, 32, 8)
 // slstm backward: as above, but D = 160 as 5 workgroups of 2 waves (10 waves of 168 registers each spill at every tile height)
 #define FRNN_BWD_PLANS_SLSTM_BF16(X) \
-  X(128, 2, 4, 1, 2, 16) \
+  X(128, 2, 4, 1, 2, 16) X(128, 3, 4, 1, 4, 4) X(192, 2, 4, 1, 6, 4) X(256, 2, 4, 1, 16, 4) X(320, 2, 4, 1, 10, 4) X(384, 2, 4, 1, 12, 4) X(448, 2, 4, 1, 14, 4) X(512, 2, 4, 1, 16, 4) X(640, 2, 4, 1, 20, 4) X(768, 2, 4, 1, 24, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 8) X(128, 0, 8, 1, 1, 8) X(160, 0, 2, 1, 5, 16) X(192, 0, 4, 1, 3, 16) \
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 8) X(1024, 0, 4, 1, 32, 8)
 // slstm: its heavier gate math tips D = 192 forward to 3 workgroups of 4 waves (1.19 against 1.26 ms)
 #define FRNN_PLANS_SLSTM_BF16(X) \
+  X(384, 2, 4, 1, 12, 4) X(448, 2, 4, 1, 14, 4) X(512, 2, 4, 1, 16, 4) X(640, 2, 4, 1, 20, 4) X(768, 2, 4, 1, 24, 4) \
   X(160, 2, 2, 1, 5, 16) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 8, 1, 1, 16) X(160, 0, 10, 1, 1, 8) X(192, 0, 4, 1, 3, 16) \
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 8) X(1024, 0, 4, 1, 32, 16)
@@ -162,37 +169,44 @@ constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, in
 // Forward, D = 384 .. 512: workgroups of two wave pairs, 4-row tiles only (see fwd_k_split; D = 16 * (WAVES / 2) * KW);
 // D = 640 .. 1024: one tile per workgroup, k split over its four waves, groups that span the device (D = 16 * KW)
 #define FRNN_PLANS_GR4_F32(X) \
+  X(128, 2, 4, 1, 4, 4) X(128, 3, 4, 1, 8, 4) X(160, 2, 4, 1, 5, 4) X(192, 2, 4, 1, 6, 4) X(192, 3, 4, 1, 12, 4) X(256, 2, 4, 1, 8, 4) X(256, 3, 4, 1, 16, 4) \
+  X(320, 2, 4, 1, 10, 4) X(320, 3, 4, 1, 20, 4) X(384, 3, 4, 1, 24, 4) X(448, 3, 4, 1, 28, 4) X(512, 3, 4, 1, 32, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 4, 1, 2, 16) X(160, 0, 2, 1, 5, 16) X(192, 0, 4, 1, 3, 16) X(256, 0, 4, 1, 4, 16) \
   X(320, 0, 4, 1, 5, 8) X(384, 0, 4, 1, 12, 4) X(448, 0, 4, 1, 14, 4) X(512, 0, 4, 1, 16, 4) \
   X(640, 0, 4, 1, 40, 4) X(768, 0, 4, 1, 48, 4) X(1024, 0, 4, 1, 64, 4)
 // (backward, D = 384 .. 512: workgroups of two wave pairs, D = 640 .. 1024: one tile position per workgroup, 4-row tiles
 // only; see bwd_dest_split)
 #define FRNN_BWD_PLANS_GR4_F32(X) \
-  X(320, 2, 1, 1, 20, 4) \
-  X(64, 2, 2, 1, 2, 16) \
+  X(64, 2, 2, 1, 2, 16) X(64, 3, 4, 1, 4, 4) X(96, 3, 4, 1, 6, 4) X(128, 2, 4, 1, 4, 4) X(128, 3, 4, 1, 8, 4) X(160, 2, 4, 1, 5, 4) X(160, 3, 4, 1, 10, 4) X(192, 2, 4, 1, 6, 4) X(192, 3, 4, 1, 12, 4) \
+  X(256, 2, 4, 1, 8, 4) X(256, 3, 4, 1, 16, 4) X(320, 2, 4, 1, 10, 4) X(320, 3, 4, 1, 20, 4) X(384, 3, 4, 1, 24, 4) X(448, 3, 4, 1, 28, 4) X(512, 3, 4, 1, 32, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 8) X(96, 0, 2, 1, 3, 16) X(128, 0, 4, 1, 2, 16) X(160, 0, 2, 1, 5, 16) X(192, 0, 4, 1, 3, 16) X(256, 0, 4, 1, 4, 8) \
   X(320, 0, 4, 1, 5, 8) X(384, 0, 4, 1, 12, 4) X(448, 0, 4, 1, 14, 4) X(512, 0, 4, 1, 16, 4) \
   X(640, 0, 4, 1, 40, 4) X(768, 0, 4, 1, 48, 4) X(1024, 0, 4, 1, 64, 4)
 // slstm fp32 backward: the same without the 20-workgroup tiling of D = 320 (with four states its kernel spills)
 #define FRNN_BWD_PLANS_SLSTM_F32(X) \
-  X(64, 2, 2, 1, 2, 16) \
+  X(64, 2, 2, 1, 2, 16) X(64, 3, 4, 1, 4, 4) X(96, 3, 4, 1, 6, 4) X(128, 2, 4, 1, 4, 4) X(128, 3, 4, 1, 8, 4) X(160, 2, 4, 1, 5, 4) X(160, 3, 4, 1, 10, 4) X(192, 2, 4, 1, 6, 4) X(192, 3, 4, 1, 12, 4) \
+  X(256, 2, 4, 1, 8, 4) X(256, 3, 4, 1, 16, 4) X(320, 2, 4, 1, 10, 4) X(320, 3, 4, 1, 20, 4) X(384, 3, 4, 1, 24, 4) X(448, 3, 4, 1, 28, 4) X(512, 3, 4, 1, 32, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 8) X(96, 0, 2, 1, 3, 16) X(128, 0, 4, 1, 2, 16) X(160, 0, 2, 1, 5, 16) X(192, 0, 4, 1, 3, 16) X(256, 0, 4, 1, 4, 8) \
   X(320, 0, 4, 1, 5, 8) X(384, 0, 4, 1, 12, 4) X(448, 0, 4, 1, 14, 4) X(512, 0, 4, 1, 16, 4) \
   X(640, 0, 4, 1, 40, 4) X(768, 0, 4, 1, 48, 4) X(1024, 0, 4, 1, 64, 4)
 // ---- 3 recurrent gate rows per unit (gru) ----------------------------------------------------
 #define FRNN_PLANS_GR3_BF16(X) \
+  X(640, 2, 4, 1, 20, 4) X(768, 2, 4, 1, 24, 4) X(1024, 2, 4, 1, 32, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 8, 1, 1, 16) X(160, 0, 10, 1, 1, 16) X(192, 0, 12, 1, 1, 16) \
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 16) X(1024, 0, 4, 1, 16, 16)
 #define FRNN_BWD_PLANS_GR3_BF16(X) \
-  X(192, 2, 4, 1, 3, 16) \
+  X(192, 2, 4, 1, 3, 16) X(320, 2, 4, 1, 10, 4) X(512, 2, 4, 1, 16, 4) X(1024, 2, 4, 1, 32, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 8, 1, 1, 16) X(160, 0, 10, 1, 1, 8) X(192, 0, 12, 1, 1, 4) \
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 8) X(1024, 0, 4, 1, 16, 16)
 #define FRNN_PLANS_GR3_F32(X) \
+  X(128, 2, 4, 1, 4, 4) X(128, 3, 4, 1, 8, 4) X(160, 2, 4, 1, 5, 4) X(192, 2, 4, 1, 6, 4) X(192, 3, 4, 1, 12, 4) X(256, 2, 4, 1, 8, 4) X(256, 3, 4, 1, 16, 4) \
+  X(320, 2, 4, 1, 10, 4) X(320, 3, 4, 1, 20, 4) X(384, 3, 4, 1, 24, 4) X(448, 3, 4, 1, 28, 4) X(512, 3, 4, 1, 32, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 4, 1, 2, 16) X(160, 0, 2, 1, 5, 16) X(192, 0, 4, 1, 3, 16) X(256, 0, 4, 1, 4, 16) \
   X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 12, 4) X(448, 0, 4, 1, 14, 4) X(512, 0, 4, 1, 16, 4) \
   X(640, 0, 4, 1, 40, 4) X(768, 0, 4, 1, 48, 4) X(1024, 0, 4, 1, 64, 4)
 #define FRNN_BWD_PLANS_GR3_F32(X) \
-  X(64, 2, 2, 1, 2, 16) \
+  X(64, 2, 2, 1, 2, 16) X(64, 3, 4, 1, 4, 4) X(96, 3, 4, 1, 6, 4) X(128, 2, 4, 1, 4, 4) X(128, 3, 4, 1, 8, 4) X(160, 2, 4, 1, 5, 4) X(160, 3, 4, 1, 10, 4) X(192, 2, 4, 1, 6, 4) X(192, 3, 4, 1, 12, 4) \
+  X(256, 2, 4, 1, 8, 4) X(256, 3, 4, 1, 16, 4) X(320, 2, 4, 1, 10, 4) X(320, 3, 4, 1, 20, 4) X(384, 3, 4, 1, 24, 4) X(448, 3, 4, 1, 28, 4) X(512, 3, 4, 1, 32, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 2, 1, 3, 16) X(128, 0, 4, 1, 2, 16) X(160, 0, 2, 1, 5, 16) X(192, 0, 4, 1, 3, 16) X(256, 0, 4, 1, 4, 16) \
   X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 12, 4) X(448, 0, 4, 1, 14, 4) X(512, 0, 4, 1, 16, 4) \
   X(640, 0, 4, 1, 40, 4) X(768, 0, 4, 1, 48, 4) X(1024, 0, 4, 1, 64, 4)
