@@ -8,6 +8,7 @@ from ctypes import c_char_p, c_int, c_size_t, c_void_p, POINTER
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = None
+_HOST = None
 
 FUNCTION_IDS = {"lstm": 0, "slstm": 1, "gru": 2, "elman": 3}
 DTYPE_IDS = {"bfloat16": 0, "float32": 1, "float16": 2}
@@ -26,8 +27,14 @@ class Options(ctypes.Structure):
 
     def __init__(self, forward_clipval=0.0, gradient_recurrent_clipval=0.0, gradient_recurrent_cut=0, recompute=0,
                  batch_stride=0):
-        super().__init__(ctypes.sizeof(Options), forward_clipval, gradient_recurrent_clipval, gradient_recurrent_cut,
+        super().__init__(ctypes.sizeof(type(self)), forward_clipval, gradient_recurrent_clipval, gradient_recurrent_cut,
                          recompute, batch_stride)
+
+
+class OptionsReport(Options):
+    """With the fields behind those: the host words of a call that reports a failed wait."""
+
+    _fields_ = [("report", c_void_p), ("report_any", c_void_p)]
 
 
 _P6 = [c_int] * 6
@@ -36,6 +43,8 @@ _BWD = _P6 + [c_void_p] * 11 + [c_size_t, c_void_p]
 _SIGNATURES = {
     "frnn_last_error": (c_char_p, []),
     "frnn_version": (c_char_p, []),
+    "frnn_stream_capturing": (c_int, [c_void_p]),
+    "frnn_wait_launches": (None, []),
     "frnn_profile_enable": (None, [c_int]),
     "frnn_profile_reset": (None, []),
     "frnn_profile_count": (c_int, []),
@@ -106,6 +115,20 @@ def load_library():
             fn.restype, fn.argtypes = res, args
         _LIB = lib
     return _LIB
+
+
+def load_host():
+    """The host module (csrc/host_torch.cpp), bound to the library; raises if it is missing (no fallback)."""
+    global _HOST
+    if _HOST is None:
+        lib = load_library()
+        if not os.path.exists(os.path.join(_HERE, "_host.so")):
+            raise RuntimeError(f"{_HERE}/_host.so is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}`")
+        from . import _host
+
+        _host.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in _SIGNATURES})
+        _HOST = _host
+    return _HOST
 
 
 def last_error() -> str:

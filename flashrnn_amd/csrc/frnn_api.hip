@@ -301,9 +301,9 @@ static void gate_leave(LaunchGate* g, hipStream_t st, bool launched_ok = true, b
 // fx is the cell the kernels are instantiated for: the function itself, except that an Elman cell under
 // forward_clipval runs as FRNN_ELMAN_CLIP (one cached value per element: the unclamped h).
 // rc: the gate cache is left out (forward) / rebuilt (backward): only for cells that have one.
-struct Opts { float h_clip, g_clip; int cut; int fx; int rc; int bs; };
+struct Opts { float h_clip, g_clip; int cut; int fx; int rc; int bs; int *report, *report_any; };
 static int parse_opts(const frnn_options* o, int function, Opts* out) {
-  out->h_clip = 0.f; out->g_clip = 0.f; out->cut = 0; out->fx = function; out->rc = 0; out->bs = 0;
+  out->h_clip = 0.f; out->g_clip = 0.f; out->cut = 0; out->fx = function; out->rc = 0; out->bs = 0; out->report = out->report_any = nullptr;
   if (!o) return 0;
   // (the struct may grow at its end: struct_size says how much of it the caller's build knows)
   if (o->struct_size < offsetof(frnn_options, recompute))
@@ -317,6 +317,7 @@ static int parse_opts(const frnn_options* o, int function, Opts* out) {
   if (function == FRNN_ELMAN && out->h_clip > 0.f) out->fx = FRNN_ELMAN_CLIP;
   out->rc = recompute != 0 && function != FRNN_ELMAN;
   out->bs = o->struct_size >= offsetof(frnn_options, batch_stride) + sizeof(int) ? o->batch_stride : 0;
+  if (o->struct_size >= offsetof(frnn_options, report_any) + sizeof(int*)) { out->report = o->report; out->report_any = o->report_any; }
   if (out->bs < 0) return fail(FRNN_E_ARG, "batch_stride must be 0 (= B) or the number of rows of the whole batch (got %d)", out->bs);  // (elman caches nothing, or one value under forward_clipval)
   return 0;
 }
@@ -530,6 +531,18 @@ extern "C" {
 const char* frnn_last_error(void) { return g_err; }
 const char* frnn_version(void) { return "flashrnn_hip 0.1 (gfx950)"; }
 
+int frnn_stream_capturing(void* stream) { return stream_capturing((hipStream_t)stream) ? 1 : 0; }
+void frnn_wait_launches(void) {
+  for (LaunchGate& g : g_gate) {
+    hipEvent_t ev = nullptr;
+    {
+      std::lock_guard<std::mutex> lk(g.mu);
+      if (g.have) ev = g.ev;  // (events are never destroyed; one recorded again meanwhile stands for a later launch)
+    }
+    if (ev && hipEventSynchronize(ev) != hipSuccess) (void)hipGetLastError();
+  }
+}
+
 void frnn_profile_enable(int on) { g_prof_on = on ? 1 : 0; g_prof_n = 0; }
 void frnn_profile_reset(void) { g_prof_n = 0; }
 int frnn_profile_count(void) { return (int)(g_prof_n < kProfMax ? g_prof_n : kProfMax); }
@@ -689,6 +702,7 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   a.carry = carry; a.step = step;
   a.B = B; a.BS = o.bs ? o.bs : B; a.T = T; a.N = N; a.groups_total = groups; a.tile_rows = tr;
   a.training = need_cache ? 1 : 0;
+  a.report = o.report; a.report_any = o.report_any;
   a.spin_limit = spin_limit_of(&p, !step && T > 1);
   p.cooperative = env_int("FRNN_COOPERATIVE", 0);
   a.poll_delay = env_int("FRNN_POLL_DELAY", fwd_poll_delay_default(fx, dtype, p, tr));
@@ -808,6 +822,7 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   a.ll = w.ll; a.status = w.status;
   a.xcd = (near_stores_possible(p) && near_stores_allowed()) ? w.xcd : nullptr;
   a.B = B; a.BS = o.bs ? o.bs : B; a.T = T; a.N = N; a.groups_total = groups; a.tile_rows = tr;
+  a.report = o.report; a.report_any = o.report_any;
   a.spin_limit = spin_limit_of(&p, !o.cut);
   p.cooperative = env_int("FRNN_COOPERATIVE", 0);
   // measured best, as in the forward call (exchange stores kept in the XCD's L2): the gated cells 0-2 units at every
@@ -983,7 +998,7 @@ int frnn_fused_decode_open(int function, int dtype, int B, int N, int D,
   a.xcd = (near_stores_possible(p) && near_stores_allowed()) ? (int*)(mb + dp.l.xcd_off) : nullptr;
   a.carry = carry; a.step = 0;
   a.B = B; a.BS = B; a.T = max_tokens; a.N = N; a.grp0 = 0; a.groups = dp.groups; a.groups_total = dp.groups; a.tile_rows = 4;
-  a.training = 0;
+  a.training = 0; a.report = a.report_any = nullptr;
   a.spin_limit = env_int("FRNN_SPIN_LIMIT", 1 << 22);
   a.poll_delay = env_int("FRNN_POLL_DELAY", fwd_poll_delay_default(function, dtype, p, 4));
   a.h_clip = o.h_clip; a.pst = 0;

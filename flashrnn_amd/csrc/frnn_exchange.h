@@ -210,6 +210,12 @@ __device__ __forceinline__ bool give_up(Wait& w, int spins) {
   return true;
 }
 
+// the host words of a call that failed (frnn_options.report, report_any)
+__device__ __forceinline__ void report_failure(int* one, int* any) {
+  if (one) __hip_atomic_store(one, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (any) __hip_atomic_store(any, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Poll NW tagged words (addresses base + off[i]; every lane polls NW words, lanes or entries
 // with nothing to wait for pass need[i] = false and may point anywhere valid) until all carry the
 // tag of step t.  Loads are unconditional and the exit test is a wave vote.

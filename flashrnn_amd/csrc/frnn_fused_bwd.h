@@ -49,6 +49,7 @@ struct BwdArgs {
   int BS;  // rows between the state planes of s0, states, dstates and ds0 ([S, BS, ...]); B unless the call covers a range of a larger batch
   int grp0, groups, groups_total, tile_rows;
   int spin_limit, poll_delay;
+  int *report, *report_any;  // frnn_options: host words set beside the status word, or null
   float g_clip;  // > 0: cotangent carried into h_t clamped to [-g_clip, g_clip] (gradient_recurrent_clipval)
   int cut;       // != 0: no gradient through R h (gradient_recurrent_cut)
   long long* trace;  // phase cycle sums per wave; only written by -DFRNN_TRACE builds
@@ -1282,7 +1283,10 @@ fused_bwd_kernel(const BwdArgs a) {
 #endif
 
   if (dead) {
-    if (tid == 0) __hip_atomic_store(a.status, (int)STATUS_WAIT_EXPIRED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) {
+      __hip_atomic_store(a.status, (int)STATUS_WAIT_EXPIRED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      report_failure(a.report, a.report_any);
+    }
 #pragma unroll
     for (int u = 0; u < UTW; ++u)
 #pragma unroll

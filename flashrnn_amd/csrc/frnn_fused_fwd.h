@@ -41,6 +41,7 @@ struct FwdArgs {
   // fp32 registers); h for the recurrent product still comes from s0, in the storage type, as in the time loop.
   // step != 0: all groups send their (unread) exchange words to one area
   float* carry; int step;
+  int *report, *report_any;  // frnn_options: host words set beside the status word, or null
   float h_clip;      // > 0: new h clamped to [-h_clip, h_clip] (forward_clipval)
   int pst;           // host side only: launch the instantiation whose producer wave stores the outputs (fwd_producer_stores)
   // resident decode kernel (the MB instantiations): T = the most tokens the launch serves; the Wx of token t is taken
@@ -815,7 +816,10 @@ fused_fwd_kernel(const FwdArgs a) {
   if (dead) {
     // bounded wait ran out: report, and make the damage visible (NaN in every h of this
     // workgroup's units; the step that failed is not known exactly, so all steps are marked)
-    if (tid == 0) __hip_atomic_store(a.status, (int)STATUS_WAIT_EXPIRED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) {
+      __hip_atomic_store(a.status, (int)STATUS_WAIT_EXPIRED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      report_failure(a.report, a.report_any);
+    }
     float nanv[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) nanv[e] = __uint_as_float(0x7fc00000u);

@@ -1,0 +1,364 @@
+// _host.so: the host side of flashrnn() and flashrnn_step() for the usual call (see flashrnn.py: plain tensors in the kernels'
+// layouts, no transform, tracing or dispatch mode active), and the record of failed waits of every fused call.
+//
+// A short call is bound by the host: LSTM bf16 B5 T19 N3 D256, forward and backward, takes ~70 us on the device.  With an
+// autograd function and ctypes calls in Python it took 300 us of host time (a copy, an event and a tensor view per call to fetch
+// its status word, a dozen ctypes calls, the interpreter on the autograd worker thread); here it takes 111, of which an autograd
+// node of torch's own takes 42.  The forward alone 57 -> 18 us, flashrnn_step 9.6 -> 5.8 us a call.
+// The entry points of libflashrnn_hip.so are handed over as addresses (bind), so the library that FLASHRNN_HIP_LIBRARY names is
+// the one that runs, and this file needs no HIP symbol of its own.
+#include <torch/extension.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+
+#include <c10/hip/HIPStream.h>
+
+#include <atomic>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include "../../include/flashrnn_hip.h"
+
+namespace {
+
+using torch::Tensor;
+
+struct Api {
+  decltype(&frnn_last_error) last_error;
+  decltype(&frnn_fused_supported) fused_supported, alt_supported, recompute_supported;
+  decltype(&frnn_fused_max_batch) max_batch;
+  decltype(&frnn_fused_cache_bytes_opt) fused_cache_bytes, alt_cache_bytes;
+  decltype(&frnn_fused_workspace_bytes_opt) fused_workspace_bytes;
+  decltype(&frnn_alt_workspace_bytes) alt_workspace_bytes;
+  decltype(&frnn_fused_forward_opt) fused_forward, alt_forward;
+  decltype(&frnn_fused_backward_opt) fused_backward, alt_backward;
+  decltype(&frnn_fused_backward_recompute) backward_recompute;
+  decltype(&frnn_fused_step) fused_step, alt_step;
+  decltype(&frnn_stream_capturing) stream_capturing;
+  decltype(&frnn_wait_launches) wait_launches;
+};
+Api api{};
+
+void bind(const std::unordered_map<std::string, uintptr_t>& f) {
+  auto get = [&](auto& p, const char* name) { p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(f.at(name)); };
+  get(api.last_error, "frnn_last_error");
+  get(api.fused_supported, "frnn_fused_supported");
+  get(api.alt_supported, "frnn_alt_supported");
+  get(api.recompute_supported, "frnn_fused_recompute_supported");
+  get(api.max_batch, "frnn_fused_max_batch");
+  get(api.fused_cache_bytes, "frnn_fused_cache_bytes_opt");
+  get(api.alt_cache_bytes, "frnn_alt_cache_bytes_opt");
+  get(api.fused_workspace_bytes, "frnn_fused_workspace_bytes_opt");
+  get(api.alt_workspace_bytes, "frnn_alt_workspace_bytes");
+  get(api.fused_forward, "frnn_fused_forward_opt");
+  get(api.alt_forward, "frnn_alt_forward_opt");
+  get(api.fused_backward, "frnn_fused_backward_opt");
+  get(api.alt_backward, "frnn_alt_backward_opt");
+  get(api.backward_recompute, "frnn_fused_backward_recompute");
+  get(api.fused_step, "frnn_fused_step");
+  get(api.alt_step, "frnn_alt_step");
+  get(api.stream_capturing, "frnn_stream_capturing");
+  get(api.wait_launches, "frnn_wait_launches");
+}
+
+// (as _raise in flashrnn.py: the reference raises ValueError when no tiling exists)
+void check_rc(int rc, bool fused, const char* what) {
+  if (rc == 0) return;
+  const std::string msg = std::string(fused ? "hip_fused" : "hip") + " " + what + ": " + api.last_error() + " (code " + std::to_string(rc) + ")";
+  TORCH_CHECK_VALUE(rc != FRNN_E_UNSUPPORTED, msg);
+  TORCH_CHECK(false, msg);
+}
+
+// ---- failed waits -------------------------------------------------------------------------------------------------
+// A fused kernel whose bounded wait between workgroups ran out fills its outputs with NaN and sets the status word of its
+// workspace.  It also sets two words of pinned host memory that the call was given (frnn_options.report / report_any): one that
+// belongs to the call, in a ring of kSlots, and one that all calls share.  So nothing is copied or recorded per call: a later call
+// reads the shared word, and only where it is set looks for the calls that set theirs, once the launches so far have ended.
+// A slot is used again after kSlots calls; the ring first waits for the launches so far there.
+constexpr int kSlots = 4096;
+const char* const kNames[4] = {"lstm", "slstm", "gru", "elman"};
+struct CallInfo { int kind, function, B, T, N, D; };
+struct StatusRing {
+  std::mutex mu;
+  Tensor words;              // pinned: [kSlots] and the shared word
+  std::vector<CallInfo> info;
+  long taken = 0;
+  long last[2] = {-1, -1};   // the most recent call of each kind (forward, backward)
+  std::vector<std::string> older;  // failed calls whose slots were used again before anyone asked
+
+  volatile int* any() { return words.defined() ? words.data_ptr<int>() + kSlots : nullptr; }
+  // the words of a call on `stream`; calls under capture are not recorded: a replay repeats the kernels, not this
+  void take(const CallInfo& c, void* stream, frnn_options& o) {
+    o.report = o.report_any = nullptr;
+    if (api.stream_capturing(stream)) return;
+    std::lock_guard<std::mutex> lk(mu);
+    if (!words.defined()) {
+      words = torch::zeros({kSlots + 1}, torch::TensorOptions().dtype(torch::kInt).pinned_memory(true));
+      info.resize(kSlots);
+    }
+    const long s = taken++;
+    if (s >= kSlots && s % kSlots == 0) {
+      api.wait_launches();
+      gather(older);
+      *any() = older.empty() ? 0 : 1;
+      for (int i = 0; i < kSlots; ++i) words.data_ptr<int>()[i] = 0;
+    }
+    info[s % kSlots] = c;
+    last[c.kind] = s;
+    int* w = words.data_ptr<int>();
+    o.report = w + s % kSlots;
+    o.report_any = w + kSlots;
+  }
+  // descriptions of the calls whose word is set, once each
+  std::vector<std::string> collect() {
+    std::lock_guard<std::mutex> lk(mu);
+    std::vector<std::string> failed;
+    if (!words.defined()) return failed;
+    if (*any() != 0) api.wait_launches();  // (the other workgroups of a call that reported may still be on their way out)
+    failed.swap(older);
+    gather(failed);
+    return failed;
+  }
+  void gather(std::vector<std::string>& failed) {  // (the launches so far have ended, mu is held)
+    if (*any() == 0) return;
+    *any() = 0;
+    volatile int* w = words.data_ptr<int>();
+    const long n = std::min<long>(taken, kSlots);
+    for (long i = taken - n; i < taken; ++i) {
+      if (w[i % kSlots] != 1) continue;
+      w[i % kSlots] = 2;  // (reported; still what last() returns)
+      const CallInfo& c = info[i % kSlots];
+      failed.push_back(std::string(c.kind ? "backward" : "forward") + " of " + kNames[c.function] + " B" + std::to_string(c.B) + " T" +
+                       std::to_string(c.T) + " N" + std::to_string(c.N) + " D" + std::to_string(c.D));
+    }
+  }
+  void poll(bool wait, void* stream) {
+    const volatile int* a = any();
+    if (!a || (!wait && *a == 0) || api.stream_capturing(stream)) return;
+    if (wait) api.wait_launches();
+    const auto failed = collect();
+    if (failed.empty()) return;
+    std::string what;
+    for (const auto& f : failed) what += (what.empty() ? "" : "; ") + f;
+    TORCH_CHECK(false, "flashrnn_amd: a bounded wait between the workgroups of a head ran out in an earlier fused call (", what,
+                "): its outputs are NaN.  The workgroups of a head must all be resident; another process's kernels on the same device "
+                "can prevent that");
+  }
+  int last_word(int kind) {
+    api.wait_launches();
+    std::lock_guard<std::mutex> lk(mu);
+    if (last[kind] < 0 || taken - last[kind] > kSlots) return 0;
+    return words.data_ptr<int>()[last[kind] % kSlots] != 0 ? 1 : 0;
+  }
+};
+StatusRing& ring() { static StatusRing* r = new StatusRing; return *r; }  // (never destroyed: calls may end after static destruction began)
+
+void* stream_of(const Tensor& x) { return c10::hip::getCurrentHIPStream(x.device().index()).stream(); }
+
+constexpr int kGr[4] = {4, 4, 3, 1}, kGw[4] = {4, 4, 3, 1}, kGt[4] = {4, 4, 4, 1}, kS[4] = {2, 4, 1, 1};
+c10::ScalarType kernel_type(int d) { return d == FRNN_BF16 ? torch::kBFloat16 : d == FRNN_F16 ? torch::kHalf : torch::kFloat; }
+
+// what a call was configured with (frnn_options and the rest of FlashRNNConfig that reaches the kernels)
+struct Call : torch::CustomClassHolder {
+  int function, dtype;
+  bool fused, amp, training;
+  frnn_options o;
+};
+using CallPtr = c10::intrusive_ptr<Call>;
+CallPtr make_call(int function, int dtype, bool fused, double h_clip, double g_clip, bool cut, bool rc, bool amp) {
+  auto c = c10::make_intrusive<Call>();
+  c->function = function; c->dtype = dtype; c->fused = fused; c->amp = amp; c->training = false;
+  c->o = frnn_options{};
+  c->o.struct_size = sizeof(frnn_options);
+  c->o.forward_clipval = (float)h_clip; c->o.gradient_recurrent_clipval = (float)g_clip;
+  c->o.gradient_recurrent_cut = cut; c->o.recompute = rc && fused;
+  return c;
+}
+
+Tensor cast(const Tensor& x, const char* name, const Call& c) {
+  const auto k = kernel_type(c.dtype);
+  TORCH_CHECK_TYPE(c.amp || x.scalar_type() == k, name, " is ", x.scalar_type(), ", the kernel type is ", k,
+                   " and enable_automatic_mixed_precision is off");
+  return x.detach().to(k).contiguous();
+}
+
+struct Saved { Tensor R, b, s0, states, cache, Wx; };
+
+// one forward call of the library (as _run_forward in flashrnn.py)
+Saved run_forward(const Tensor& Wx_, const Tensor& R_, const Tensor& b_, const Tensor& s0_, const Call& c) {
+  Saved v;
+  const int64_t B = Wx_.size(0), T = Wx_.size(1), N = Wx_.size(3), D = Wx_.size(4), S = kS[c.function];
+  v.Wx = cast(Wx_, "Wx", c); v.R = cast(R_, "R", c); v.b = cast(b_, "b", c);
+  v.s0 = cast(s0_, "states", c);
+  c10::DeviceGuard guard(v.Wx.device());
+  check_rc((c.fused ? api.fused_supported : api.alt_supported)(c.function, c.dtype, B, N, D), c.fused, "backend");
+  if (c.o.recompute) check_rc(api.recompute_supported(c.function, c.dtype, B, N, D), c.fused, "backend");
+  const auto bytes = v.Wx.options().dtype(torch::kByte);
+  v.states = torch::empty({S, B, T, N, D}, v.Wx.options());
+  const size_t cache = c.training ? (c.fused ? api.fused_cache_bytes : api.alt_cache_bytes)(c.function, c.dtype, B, T, N, D, &c.o) : 0;
+  v.cache = torch::empty({(int64_t)std::max<size_t>(cache, 16)}, bytes);
+  const size_t wsb = std::max<size_t>(256, c.fused ? api.fused_workspace_bytes(c.function, c.dtype, B, T, N, D, 0, &c.o)
+                                                   : api.alt_workspace_bytes(c.function, c.dtype, B, T, N, D, 0));
+  const Tensor ws = torch::empty({(int64_t)wsb}, bytes);
+  void* st = stream_of(v.Wx);
+  frnn_options o = c.o;
+  if (c.fused) ring().take({0, c.function, (int)B, (int)T, (int)N, (int)D}, st, o);
+  check_rc((c.fused ? api.fused_forward : api.alt_forward)(
+               c.function, c.dtype, c.training, B, T, N, D, v.Wx.data_ptr(), v.R.data_ptr(), v.b.data_ptr(), v.s0.data_ptr(),
+               v.states.data_ptr(), c.training ? v.cache.data_ptr() : nullptr, ws.data_ptr(), wsb, st, &o),
+           c.fused, "forward");
+  return v;
+}
+
+struct Function : torch::autograd::Function<Function> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& Wx, const Tensor& R, const Tensor& b, const Tensor& s0, CallPtr c) {
+    Saved v = run_forward(Wx, R, b, s0, *c);
+    ctx->saved_data["call"] = c10::IValue::make_capsule(c);
+    // (recompute mode reads Wx again in the backward pass; it is the caller's tensor unless it was cast)
+    ctx->save_for_backward({v.R, v.b, v.s0, v.states, v.cache, c->o.recompute ? v.Wx : v.cache});
+    return v.states;
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto c = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
+    const auto v = ctx->get_saved_variables();
+    const bool again = torch::GradMode::is_enabled() && grads[0].requires_grad();
+    torch::autograd::variable_list out;
+    {
+      torch::NoGradGuard no_grad;
+      out = run(*c, v, grads[0]);
+    }
+    if (again) {  // the reverse scan is not differentiable: an error where a second derivative is asked for, not a silent zero
+      auto err = std::make_shared<torch::autograd::DelayedError>(
+          "trying to differentiate twice a function that was marked with @once_differentiable", (int64_t)out.size());
+      for (auto& g : out) { g = g.detach(); g.set_requires_grad(true); }
+      out = (*err)(std::move(out));
+    }
+    out.emplace_back();  // (the call)
+    return out;
+  }
+
+  static torch::autograd::variable_list run(const Call& c, const torch::autograd::variable_list& v, const Tensor& dstates) {
+    const Tensor &R = v[0], &b = v[1], &s0 = v[2], &states = v[3], &cache = v[4], &Wx = v[5];
+    const int64_t S = states.size(0), B = states.size(1), T = states.size(2), N = states.size(3), D = states.size(4);
+    const int64_t Gr = kGr[c.function], Gw = kGw[c.function], Gt = kGt[c.function];
+    c10::DeviceGuard guard(states.device());
+    void* st = stream_of(states);
+    ring().poll(false, st);
+    const Tensor ds = dstates.to(states.scalar_type()).contiguous();
+    const auto k = states.options(), f = k.dtype(torch::kFloat);
+    const Tensor dWx = torch::empty({B, T, Gw, N, D}, k), ds0 = torch::empty({S, B, N, D}, k);
+    const Tensor dR = torch::empty({Gr, N, D, D}, f), db = torch::empty({Gt, N, D}, f);
+    const size_t wsb = std::max<size_t>(256, c.fused ? api.fused_workspace_bytes(c.function, c.dtype, B, T, N, D, 1, &c.o)
+                                                     : api.alt_workspace_bytes(c.function, c.dtype, B, T, N, D, 1));
+    const Tensor ws = torch::empty({(int64_t)wsb}, k.dtype(torch::kByte));
+    frnn_options o = c.o;
+    if (c.fused) ring().take({1, c.function, (int)B, (int)T, (int)N, (int)D}, st, o);
+    int rc;
+    if (c.o.recompute)
+      rc = api.backward_recompute(c.function, c.dtype, B, T, N, D, Wx.data_ptr(), R.data_ptr(), b.data_ptr(), s0.data_ptr(), states.data_ptr(),
+                                  ds.data_ptr(), dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr<float>(), db.data_ptr<float>(), ws.data_ptr(), wsb, st, &o);
+    else
+      rc = (c.fused ? api.fused_backward : api.alt_backward)(
+          c.function, c.dtype, B, T, N, D, R.data_ptr(), b.data_ptr(), s0.data_ptr(), states.data_ptr(), cache.data_ptr(), ds.data_ptr(),
+          dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr<float>(), db.data_ptr<float>(), ws.data_ptr(), wsb, st, &o);
+    check_rc(rc, c.fused, "backward");
+    // dR / db stay fp32: autograd casts them to the dtype of the leaf they belong to, so fp32 master weights receive
+    // unrounded gradients
+    return {dWx, dR, db, ds0.view({S, B, 1, N, D})};
+  }
+};
+
+std::string shape(const Tensor& x) {  // as Python prints a tuple
+  std::string s = "(";
+  for (int64_t i = 0; i < x.dim(); ++i) s += (i ? ", " : "") + std::to_string(x.size(i));
+  return s + (x.dim() == 1 ? ",)" : ")");
+}
+
+// flashrnn() on tensors in the kernels' layouts; None where the call needs the general path (two heads per head of 32 units,
+// ranges of the batch).
+py::object call(const Tensor& Wx, const Tensor& R, const Tensor& b, const std::optional<Tensor>& states, int function, int dtype, bool fused,
+                double h_clip, double g_clip, bool cut, bool rc, bool amp) {
+  const int64_t Gr = kGr[function], Gw = kGw[function], Gt = kGt[function], S = kS[function];
+  TORCH_CHECK_VALUE(Wx.dim() == 5 && Wx.size(2) == Gw, "Wx must be [B,T,", Gw, ",N,D], got ", shape(Wx));
+  const int64_t B = Wx.size(0), T = Wx.size(1), N = Wx.size(3), D = Wx.size(4);
+  TORCH_CHECK_VALUE(R.sizes() == torch::IntArrayRef({Gr, N, D, D}), "R must be [", Gr, ",", N, ",", D, ",", D, "], got ", shape(R));
+  TORCH_CHECK_VALUE(b.sizes() == torch::IntArrayRef({Gt, N, D}), "b must be [", Gt, ",", N, ",", D, "], got ", shape(b));
+  TORCH_CHECK_VALUE(!states || states->sizes() == torch::IntArrayRef({S, B, 1, N, D}), "states must be [", S, ",", B, ",1,", N, ",", D, "], got ",
+                    states ? shape(*states) : "");
+  if (D == 16 || !Wx.is_cuda() || (rc && !fused) || B > INT_MAX || T > INT_MAX || N > INT_MAX || D > INT_MAX) return py::none();
+  auto c = make_call(function, dtype, fused, h_clip, g_clip, cut, rc, amp);
+  c->training = torch::GradMode::is_enabled() &&
+                (Wx.requires_grad() || R.requires_grad() || b.requires_grad() || (states && states->requires_grad()));
+  if (fused) {
+    long rows = api.max_batch(function, dtype, T, N, D, 0, c->training, &c->o);
+    if (const char* limit = getenv("FRNN_TEST_MAX_BATCH")) rows = std::min(rows, atol(limit));  // (tests: see _apply_in_batch_ranges)
+    if (rows < B) return py::none();
+  }
+  Tensor out, last;
+  {
+    py::gil_scoped_release nogil;
+    ring().poll(false, stream_of(Wx));
+    Tensor s0;
+    if (states) s0 = *states;
+    else {
+      c10::DeviceGuard guard(Wx.device());
+      s0 = torch::zeros({S, B, 1, N, D}, Wx.options().requires_grad(false));
+    }
+    out = c->training ? Function::apply(Wx, R, b, s0, c) : run_forward(Wx, R, b, s0, *c).states;
+    last = out.narrow(2, T - 1, 1);
+  }
+  return py::make_tuple(out, last);
+}
+
+Tensor step(const Tensor& Wx, const Tensor& R, const Tensor& b, const Tensor& states, int function, int dtype, bool fused, double h_clip,
+            double g_clip, bool cut, bool rc, const std::optional<Tensor>& carry) {
+  const int64_t Gr = kGr[function], Gw = kGw[function], Gt = kGt[function], S = kS[function];
+  TORCH_CHECK_VALUE(Wx.dim() == 5 && Wx.size(1) == 1 && Wx.size(2) == Gw, "Wx must be [B,1,", Gw, ",N,D], got ", shape(Wx));
+  const int64_t B = Wx.size(0), N = Wx.size(3), D = Wx.size(4);
+  TORCH_CHECK_VALUE(R.sizes() == torch::IntArrayRef({Gr, N, D, D}) && b.sizes() == torch::IntArrayRef({Gt, N, D}) &&
+                        states.sizes() == torch::IntArrayRef({S, B, 1, N, D}),
+                    "R, b, states must be [", Gr, ",", N, ",", D, ",", D, "], [", Gt, ",", N, ",", D, "], [", S, ",", B, ",1,", N, ",", D, "]; got ",
+                    shape(R), ", ", shape(b), ", ", shape(states));
+  const auto k = kernel_type(dtype);
+  const std::pair<const char*, const Tensor&> in[] = {{"Wx", Wx}, {"R", R}, {"b", b}, {"states", states}};
+  for (const auto& [name, x] : in) {
+    TORCH_CHECK(x.is_cuda(), "flashrnn_amd runs on a GPU only (got a CPU tensor); there is no CPU fallback");
+    TORCH_CHECK_TYPE(x.scalar_type() == k && x.is_contiguous(), name, " must be a contiguous ", k, " tensor (the step path casts and copies nothing)");
+  }
+  TORCH_CHECK_TYPE(!carry || (carry->scalar_type() == torch::kFloat && carry->sizes() == torch::IntArrayRef({S, B, N, D}) &&
+                              carry->is_contiguous() && carry->device() == Wx.device()),
+                   "carry must be a contiguous float32 tensor [", S, ",", B, ",", N, ",", D, "] on the device of Wx");
+  py::gil_scoped_release nogil;
+  c10::DeviceGuard guard(Wx.device());
+  const Tensor out = torch::empty({S, B, 1, N, D}, Wx.options().requires_grad(false));
+  const auto c = make_call(function, dtype, fused, h_clip, g_clip, cut, rc, true);
+  check_rc((fused ? api.fused_step : api.alt_step)(function, dtype, B, N, D, Wx.data_ptr(), R.data_ptr(), b.data_ptr(), states.data_ptr(),
+                                                   out.data_ptr(), carry ? carry->data_ptr<float>() : nullptr, stream_of(Wx), &c->o),
+           fused, "step");
+  return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+  m.def("bind", &bind);
+  m.def("call", &call);
+  m.def("step", &step);
+  // (the general path's calls, made from Python: addresses of the two words, 0 under capture)
+  m.def("status_take", [](int kind, int function, int B, int T, int N, int D, uintptr_t stream) {
+    frnn_options o{};
+    ring().take({kind, function, B, T, N, D}, reinterpret_cast<void*>(stream), o);
+    return std::make_pair(reinterpret_cast<uintptr_t>(o.report), reinterpret_cast<uintptr_t>(o.report_any));
+  });
+  m.def("status_poll", [](bool wait, uintptr_t stream) { ring().poll(wait, reinterpret_cast<void*>(stream)); }, py::call_guard<py::gil_scoped_release>());
+  m.def("status_last", [](int kind) { return ring().last_word(kind); }, py::call_guard<py::gil_scoped_release>());
+  m.def("status_drain", []() {
+    api.wait_launches();
+    auto failed = ring().collect();
+    std::lock_guard<std::mutex> lk(ring().mu);
+    ring().words.reset();  // (pinned memory goes back while the HIP runtime is up)
+    ring().taken = 0; ring().last[0] = ring().last[1] = -1;
+    return failed;
+  }, py::call_guard<py::gil_scoped_release>());
+}

@@ -13,7 +13,6 @@ for the backward pass (:746) or slice dWx (:789-796).
 from __future__ import annotations
 
 import atexit
-import functools
 import os
 from dataclasses import dataclass
 from typing import Optional, Sequence, Union
@@ -163,12 +162,14 @@ def _entry(backend: str, name: str):
     return getattr(_lib.load_library(), prefix + name)
 
 
-def _options(cfg: "FlashRNNConfig", batch_stride: int = 0):
+def _options(cfg: "FlashRNNConfig", batch_stride: int = 0, words=(None, None)):
     import ctypes
 
-    return ctypes.byref(_lib.Options(float(cfg.forward_clipval or 0.0), float(cfg.gradient_recurrent_clipval or 0.0),
-                                     int(bool(cfg.gradient_recurrent_cut)),
-                                     int(bool(cfg.recompute_gates) and cfg.backend == "hip_fused"), int(batch_stride)))
+    o = _lib.OptionsReport(float(cfg.forward_clipval or 0.0), float(cfg.gradient_recurrent_clipval or 0.0),
+                           int(bool(cfg.gradient_recurrent_cut)),
+                           int(bool(cfg.recompute_gates) and cfg.backend == "hip_fused"), int(batch_stride))
+    o.report, o.report_any = words
+    return ctypes.byref(o)
 
 
 def _workspace_bytes(cfg: "FlashRNNConfig", f_id, d_id, B, T, N, D, backward: int) -> int:
@@ -185,90 +186,30 @@ def _raise(code: int, what: str):
 
 
 class _StatusLog:
-    """Status words of the fused calls, checked without a device-wide synchronisation.
+    """Failed waits of the fused calls, found without a synchronisation and without copying anything per call.
 
-    A fused kernel whose bounded wait between workgroups ran out fills its outputs with NaN and sets the
-    status word at the head of its workspace.  Every fused call copies that word to pinned host memory
-    behind the kernels (4 bytes, asynchronous) and records an event; the entries whose event has
-    completed are read at the start of every later call (forward or backward, any stream), and a non-zero
-    one raises RuntimeError there.  ``check_status()`` waits for the entries still pending (their events
-    only) and does the same.  Entries made under stream capture are not logged: a replay repeats the
-    kernels, not this bookkeeping.  The pinned words and events of entries that have been read are used again
-    (except the most recent entry of each kind, which ``last()`` may still be asked for)."""
+    A fused kernel whose bounded wait between workgroups ran out fills its outputs with NaN and sets the status word at the head
+    of its workspace, and with it two words of pinned host memory: the call's own and one that all calls share (csrc/host_torch.cpp).
+    The shared word is read at the start of every later call (forward or backward, any stream); where it is set, the calls that
+    failed are named in a RuntimeError raised there.  ``check_status()`` waits for the launches so far (an event behind the last of
+    them, not the device) and does the same.  Calls under stream capture are not recorded: a replay repeats the kernels, not this
+    bookkeeping."""
 
-    def __init__(self):
-        import collections
-        import threading
-
-        self._lock = threading.Lock()
-        self._pending = collections.deque()
-        self._last = {}
-        self._free = []
-
-    def log(self, kind: str, ws: torch.Tensor, what: str):
-        if torch.cuda.is_current_stream_capturing():
-            return
-        with self._lock:
-            host, ev = self._free.pop() if self._free else (None, None)
-        if host is None:
-            host, ev = torch.empty(1, dtype=torch.int32, pin_memory=True), torch.cuda.Event()
-        host.copy_(ws[:4].view(torch.int32), non_blocking=True)
-        ev.record()
-        entry = (kind, what, host, ev)
-        with self._lock:
-            self._pending.append(entry)
-            self._last[kind] = entry
-
-    def note_ok(self, kind: str):
-        """A call that cannot fail this way (heads of one workgroup: nothing waits): nothing to fetch."""
-        with self._lock:
-            self._last[kind] = None
+    def words(self, kind: str, cfg: "FlashRNNConfig", B: int, T: int, N: int, D: int, stream: int):
+        """The two words of a call (addresses; 0 under capture)."""
+        return _lib.load_host().status_take(int(kind == "backward"), _lib.FUNCTION_IDS[cfg.function], B, T, N, D, stream)
 
     def poll(self, wait: bool = False):
-        if torch.cuda.is_current_stream_capturing():
-            return  # (querying an event is not allowed while this thread captures)
-        failed = []
-        with self._lock:
-            keep = []
-            while self._pending:
-                entry = self._pending.popleft()
-                kind, what, host, ev = entry
-                if wait:
-                    ev.synchronize()
-                if ev.query():
-                    if int(host[0]) != 0:
-                        failed.append(f"{kind} of {what}")
-                    if self._last.get(kind) is not entry and len(self._free) < 64:
-                        self._free.append((host, ev))
-                else:
-                    keep.append(entry)
-            self._pending.extend(keep)
-        if failed:
-            raise RuntimeError(
-                "flashrnn_amd: a bounded wait between the workgroups of a head ran out in an earlier fused call ("
-                + "; ".join(failed) + "): its outputs are NaN.  The workgroups of a head must all be resident; "
-                "another process's kernels on the same device can prevent that")
+        if torch.cuda.is_initialized():
+            _lib.load_host().status_poll(wait, torch.cuda.current_stream().cuda_stream)
 
     def last(self, kind: str) -> int:
-        with self._lock:
-            entry = self._last.get(kind)
-        if entry is None:
-            return 0
-        entry[3].synchronize()
-        return int(entry[2][0])
+        return _lib.load_host().status_last(int(kind == "backward"))
 
     def drain(self) -> list:
-        """Waits for every pending entry, then lets go of all events and pinned words (while the HIP runtime is
-        still up).  Returns the descriptions of the calls whose status word was set."""
-        with self._lock:
-            pending, self._pending = list(self._pending), type(self._pending)()
-            self._last, self._free = {}, []
-        failed = []
-        for kind, what, host, ev in pending:
-            ev.synchronize()
-            if int(host[0]) != 0:
-                failed.append(f"{kind} of {what}")
-        return failed
+        """Waits for the launches so far, then lets go of the pinned words (while the HIP runtime is still up).  Returns the
+        descriptions of the calls that failed."""
+        return _lib._HOST.status_drain() if _lib._HOST is not None else []
 
 
 _status = _StatusLog()
@@ -351,20 +292,6 @@ def fused_plan(function: str, dtype: str, B: int, N: int, D: int, backward: bool
     return tuple(o.value for o in out)
 
 
-@functools.lru_cache(maxsize=None)
-def _heads_wait_cached(function: str, dtype: str, B: int, N: int, D: int, backward: bool, variant) -> bool:
-    return fused_plan(function, dtype, B, N, D, backward)[2] > 1
-
-
-def _heads_wait(cfg: FlashRNNConfig, B: int, N: int, D: int, backward: bool) -> bool:
-    """Whether the heads of this fused call run as several workgroups that wait for each other: only then can the
-    status word of the call become non-zero, and only then is it fetched (a copy on the stream per call).  The
-    recompute-mode reverse kernels have tilings of their own, so their calls always fetch it."""
-    if cfg.recompute_gates and backward:
-        return True
-    return _heads_wait_cached(cfg.function, cfg.dtype, B, N, D, backward, os.environ.get("FRNN_FUSED_VARIANT"))
-
-
 def _cast_inputs(Wx, R, b, s0, cfg: FlashRNNConfig):
     """The inputs in the kernel type and the kernels' layouts, as the reference's custom_fwd(cast_inputs=...) does
     (flashrnn.py:690-695); s0 comes back as [S,B,N,D]."""
@@ -403,17 +330,13 @@ def _run_forward(Wx_k, R_k, b_k, s0_k, cfg: FlashRNNConfig, training: bool, out=
         ws_bytes = _workspace_bytes(cfg, f_id, d_id, B, T, N, D, 0)
         ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=Wx_k.device)
         stream = _raw_stream(Wx_k.device)
+        words = _status.words("forward", cfg, B, T, N, D, stream) if cfg.backend == "hip_fused" else (None, None)
         rc = _entry(cfg.backend, "forward_opt")(
             f_id, d_id, int(training), B, T, N, D, Wx_k.data_ptr(), R_k.data_ptr(), b_k.data_ptr(),
             s0_k.data_ptr(), states.data_ptr(), cache.data_ptr() if training else None,
-            ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride))
+            ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride, words))
         if rc != 0:
             _raise(rc, f"{cfg.backend} forward")
-        if cfg.backend == "hip_fused":
-            if _heads_wait(cfg, B, N, D, False):
-                _status.log("forward", ws, f"{cfg.function} B{B} T{T} N{N} D{D}")
-            else:
-                _status.note_ok("forward")
     return states, cache
 
 
@@ -434,23 +357,19 @@ def _run_backward(cfg: FlashRNNConfig, R_k, b_k, s0_k, states, cache, Wx_k, ds, 
         ws_bytes = _workspace_bytes(cfg, f_id, d_id, B, T, N, D, 1)
         ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
         stream = _raw_stream(dev)
+        words = _status.words("backward", cfg, B, T, N, D, stream) if cfg.backend == "hip_fused" else (None, None)
         if cfg.recompute_gates:
             rc = _lib.load_library().frnn_fused_backward_recompute(
                 f_id, d_id, B, T, N, D, Wx_k.data_ptr(), R_k.data_ptr(), b_k.data_ptr(), s0_k.data_ptr(),
                 states.data_ptr(), ds.data_ptr(), dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr(), db.data_ptr(),
-                ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride))
+                ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride, words))
         else:
             rc = _entry(cfg.backend, "backward_opt")(
                 f_id, d_id, B, T, N, D, R_k.data_ptr(), b_k.data_ptr(), s0_k.data_ptr(), states.data_ptr(),
                 cache.data_ptr(), ds.data_ptr(), dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr(), db.data_ptr(),
-                ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride))
+                ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride, words))
         if rc != 0:
             _raise(rc, f"{cfg.backend} backward")
-        if cfg.backend == "hip_fused":
-            if _heads_wait(cfg, B, N, D, True):
-                _status.log("backward", ws, f"{cfg.function} B{B} T{T} N{N} D{D}")
-            else:
-                _status.note_ok("backward")
     return dR, db, ds0
 
 
@@ -611,6 +530,17 @@ def flashrnn(
     kernel for the head dimension (as the reference does when no tiling exists)."""
     if config is None:
         config = _get_config(Wx, R, b, function, backend, dtype)
+    if _plain(config, Wx, R, b, states):
+        out = _lib.load_host().call(
+            Wx, R, b, states, _lib.FUNCTION_IDS[config.function], _lib.DTYPE_IDS[config.dtype], config.backend == "hip_fused",
+            config.forward_clipval or 0.0, config.gradient_recurrent_clipval or 0.0, bool(config.gradient_recurrent_cut),
+            bool(config.recompute_gates), bool(config.enable_automatic_mixed_precision))
+        if out is not None:
+            index = Wx.get_device()
+            _used_devices.add(index)
+            if out[0].requires_grad:
+                _backward_devices.add(index)
+            return out
     # to the layouts the kernels read (views; nothing is copied for the default layouts)
     Wx = _permuted(Wx, config.input_shape, "BTGHD")
     R = _permuted(R, config.recurrent_shape, "GHDP")
@@ -635,6 +565,22 @@ def flashrnn(
     else:
         out = _apply_in_batch_ranges(Wx, R, b, states, config, training)
     return _permuted(out, "SBTHD", config.output_shape), _permuted(out[:, :, -1:], "SBTHD", config.output_shape)
+
+
+_plain_types = (torch.Tensor, torch.nn.Parameter, type(None))
+
+
+def _plain(config: FlashRNNConfig, Wx, R, b, states) -> bool:
+    """Whether a call can take the host module's path (csrc/host_torch.cpp): tensors in the kernels' layouts, the zero default
+    state, and nothing active that looks at the operations of an autograd function (transforms, forward-mode differentiation, tracing,
+    compilation, dispatch or function modes, tensor subclasses): those see _FlashRNNFunction."""
+    return (config.input_shape == "BTGHD" and config.output_shape == "SBTHD" and config.recurrent_shape == "GHDP" and config.bias_shape == "GHD"
+            and (states is not None or (isinstance(config.initial_val, (int, float)) and config.initial_val == 0.0))
+            and not torch.compiler.is_compiling()
+            and type(Wx) in _plain_types[:2] and type(R) in _plain_types[:2] and type(b) in _plain_types[:2] and type(states) in _plain_types
+            and torch._C._functorch.maybe_current_level() is None and torch._C._get_tracing_state() is None
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and torch.autograd.forward_ad._current_level < 0)
 
 
 def _apply_in_batch_ranges(Wx, R, b, states, config, training):
@@ -686,31 +632,11 @@ def flashrnn_step(
     ``states``."""
     if config is None:
         config = _get_config(Wx, R, b, function, backend, dtype)
-    kdt = DTYPE_DICT[config.dtype]
-    Gr, Gw, _, Gt, S = rnn_function_registry[config.function]["gates_states"]
-    if Wx.dim() != 5 or Wx.shape[1] != 1 or Wx.shape[2] != Gw:
-        raise ValueError(f"Wx must be [B,1,{Gw},N,D], got {tuple(Wx.shape)}")
-    B, _, _, N, D = Wx.shape
-    if tuple(R.shape) != (Gr, N, D, D) or tuple(b.shape) != (Gt, N, D) or tuple(states.shape) != (S, B, 1, N, D):
-        raise ValueError(f"R, b, states must be [{Gr},{N},{D},{D}], [{Gt},{N},{D}], [{S},{B},1,{N},{D}]; got "
-                         f"{tuple(R.shape)}, {tuple(b.shape)}, {tuple(states.shape)}")
-    for name, x in (("Wx", Wx), ("R", R), ("b", b), ("states", states)):
-        if not x.is_cuda:
-            raise RuntimeError("flashrnn_amd runs on a GPU only (got a CPU tensor); there is no CPU fallback")
-        if x.dtype != kdt or not x.is_contiguous():
-            raise TypeError(f"{name} must be a contiguous {kdt} tensor (the step path casts and copies nothing)")
-    if carry is not None and (carry.dtype != torch.float32 or tuple(carry.shape) != (S, B, N, D)
-                              or not carry.is_contiguous() or carry.device != Wx.device):
-        raise TypeError(f"carry must be a contiguous float32 tensor [{S},{B},{N},{D}] on the device of Wx")
-    f_id, d_id = _lib.FUNCTION_IDS[config.function], _lib.DTYPE_IDS[config.dtype]
-    with _on_device(Wx.device):
-        out = torch.empty((S, B, 1, N, D), dtype=kdt, device=Wx.device)
-        rc = _entry(config.backend, "step")(
-            f_id, d_id, B, N, D, Wx.data_ptr(), R.data_ptr(), b.data_ptr(), states.data_ptr(), out.data_ptr(),
-            carry.data_ptr() if carry is not None else None, _raw_stream(Wx.device), _options(config))
-        if rc != 0:
-            _raise(rc, f"{config.backend} step")
-    return out
+    # (every check on types, shapes and devices is made there)
+    return _lib.load_host().step(
+        Wx, R, b, states, _lib.FUNCTION_IDS[config.function], _lib.DTYPE_IDS[config.dtype], config.backend == "hip_fused",
+        config.forward_clipval or 0.0, config.gradient_recurrent_clipval or 0.0, bool(config.gradient_recurrent_cut),
+        bool(config.recompute_gates), carry)
 
 
 def make_carry(states: torch.Tensor) -> torch.Tensor:

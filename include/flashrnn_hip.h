@@ -180,7 +180,17 @@ typedef struct frnn_options {
                       * a contiguous block of its own (the gate cache is private to the call that wrote it); dR and db are
                       * the range's own sums.  This is how a batch whose tensors reach 2 GiB runs as several calls that
                       * read and write the caller's tensors in place. */
+  int* report;      /* fused forward / backward calls, or null: two words of host memory that the device can write (pinned).  A call */
+  int* report_any;  /* one of whose bounded waits ran out sets both to 1, beside the status word of its workspace: one word per call
+                      * and one for many calls tell the caller which call failed without copying the status word of each.  Valid
+                      * until the call has ended (frnn_wait_launches); the library only ever stores 1. */
 } frnn_options;
+
+/* Waits for the most recent fused launch of every device whose workgroups wait for each other (and so, these launches being
+ * ordered, for all of them made so far); calls under stream capture do not count.  What such a call reports is then final. */
+void frnn_wait_launches(void);
+/* 1 if `stream` is being captured, else 0. */
+int frnn_stream_capturing(void* stream);
 
 /* Gate-cache size under options: an Elman cell under forward_clipval caches the unclamped h (one value per
  * element, as elman_fused_pointwise.cuh:44-47), without it nothing.  opt == NULL: as the plain queries. */

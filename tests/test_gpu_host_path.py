@@ -1,0 +1,126 @@
+"""flashrnn() through the host module (csrc/host_torch.cpp) against the autograd function in Python, which every call takes that the
+module does not: the same bits, and the same behaviour towards autograd."""
+import pytest
+import torch
+
+from oracle import make_inputs
+
+
+class _Mode(torch.overrides.TorchFunctionMode):
+    """Any active mode sends a call down the general path."""
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def _leaves(gpu, function="lstm", B=5, T=7, N=2, D=64, dtype=torch.bfloat16, weights=None):
+    inp = make_inputs(function, B, T, N, D, 3, init="randn", round_to=torch.bfloat16)
+    return [inp["Wx"].to(gpu, dtype).requires_grad_(), inp["R"].to(gpu, weights or dtype).requires_grad_(),
+            inp["b"].to(gpu, weights or dtype).requires_grad_(), inp["states"].to(gpu, dtype).requires_grad_()]
+
+
+def test_only_plain_calls_take_the_host_module():
+    import importlib
+
+    fr = importlib.import_module("flashrnn_amd.flashrnn")
+    cfg = fr.FlashRNNConfig(head_dim=32, num_heads=1)
+    x = [torch.zeros(2, 3, 4, 1, 32), torch.nn.Parameter(torch.zeros(4, 1, 32, 32)), torch.zeros(4, 1, 32)]
+    assert fr._plain(cfg, *x, None) and fr._plain(cfg, *x, torch.zeros(2, 2, 1, 1, 32))
+    assert not fr._plain(fr.FlashRNNConfig(head_dim=32, num_heads=1, input_shape="TBGHD"), *x, None)
+    assert not fr._plain(fr.FlashRNNConfig(head_dim=32, num_heads=1, initial_val=0.5), *x, None)
+    assert not fr._plain(cfg, x[0].as_subclass(type("Sub", (torch.Tensor,), {})), x[1], x[2], None)
+    with _Mode():
+        assert not fr._plain(cfg, *x, None)
+    with torch.autograd.forward_ad.dual_level():
+        assert not fr._plain(cfg, *x, None)
+    seen = []
+    torch.func.vmap(lambda w: (seen.append(fr._plain(cfg, w, x[1], x[2], None)), w)[1])(x[0][None])
+    torch.jit.trace(lambda w: (seen.append(fr._plain(cfg, w, x[1], x[2], None)), w + 1)[1], x[0], check_trace=False)
+    assert seen == [False, False]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("function,D,backend,options,dtype,weights", [
+    ("lstm", 256, "hip_fused", {}, torch.bfloat16, None), ("gru", 64, "hip", {}, torch.bfloat16, None),
+    ("slstm", 64, "hip_fused", {"recompute_gates": True}, torch.float16, torch.float32),
+    ("lstm", 64, "hip_fused", {"gradient_recurrent_clipval": 0.5, "forward_clipval": 0.7}, torch.float32, None),
+    ("elman", 32, "hip", {"gradient_recurrent_cut": True}, torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("given", [True, False])
+def test_both_paths_give_the_same_bits(gpu, function, D, backend, options, dtype, weights, given):
+    from flashrnn_amd import FlashRNNConfig, flashrnn
+
+    name = {torch.bfloat16: "bfloat16", torch.float16: "float16", torch.float32: "float32"}[dtype]
+    print(f"case host path {function} D{D} {backend} {options} {name}", flush=True)
+    cfg = FlashRNNConfig(backend=backend, function=function, dtype=name, head_dim=D, num_heads=2, **options)
+    leaves = _leaves(gpu, function, D=D, dtype=dtype, weights=weights)
+    leaves[0] = torch.cat([leaves[0].detach()] * 2, dim=1)[:, ::2].requires_grad_()  # (not contiguous)
+    if not given:
+        leaves = leaves[:3]
+
+    def run():
+        out, last = flashrnn(*leaves, config=cfg)
+        g = torch.autograd.grad([out, last], leaves, [out.detach(), last.detach()])
+        return [out.detach(), last.detach(), *g]
+
+    got = run()
+    with _Mode():
+        ref = run()
+    with torch.no_grad():
+        plain = flashrnn(*leaves, config=cfg)
+    for x, y in zip(got + list(plain), ref + ref[:2]):
+        assert x.dtype == y.dtype and torch.equal(x, y)
+
+
+@pytest.mark.gpu
+def test_autograd_meets_the_function_it_knows(gpu):
+    from flashrnn_amd import flashrnn
+
+    print("case host path autograd", flush=True)
+    leaves = _leaves(gpu)
+    out, _ = flashrnn(*leaves)
+    one = torch.autograd.grad(out.float().sum(), leaves, retain_graph=True)
+    two = torch.autograd.grad(out.float().sum(), leaves[1:2])  # (a part of the inputs, and the graph a second time)
+    assert torch.equal(one[1], two[0])
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out.float().sum(), leaves)
+    out, _ = flashrnn(*leaves)  # no second derivative: an error where it is asked for
+    g = torch.autograd.grad((out.float() ** 2).sum(), leaves[0], create_graph=True)[0]
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        g.float().sum().backward()
+    packed = []  # saved-tensor hooks see what the function saves, and the reverse pass what they give back
+    with torch.autograd.graph.saved_tensors_hooks(lambda x: (packed.append(x.shape), x.cpu())[1], lambda x: x.to(gpu)):
+        out, _ = flashrnn(*leaves)
+    hooked = torch.autograd.grad(out.float().sum(), leaves)
+    assert len(packed) >= 5 and all(torch.equal(x, y) for x, y in zip(one, hooked))
+    R = leaves[1].detach().clone().requires_grad_()
+    out, _ = flashrnn(leaves[0], R, *leaves[2:])
+    with torch.no_grad():
+        R.mul_(2.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(out.float().sum(), leaves[0])
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda w: flashrnn(w, *[x.detach() for x in leaves[1:]])[0])(leaves[0].detach()[None])
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError):
+        flashrnn(torch.autograd.forward_ad.make_dual(leaves[0].detach(), torch.ones_like(leaves[0])), *leaves[1:])
+    torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_a_failed_wait_is_named_behind_more_calls_than_the_ring_holds(gpu, monkeypatch):
+    from flashrnn_amd import check_status, flashrnn, last_status
+
+    print("case host path status ring", flush=True)
+    x = [v.detach() for v in _leaves(gpu, T=2, D=256)]
+    with torch.no_grad():
+        for _ in range(4100):
+            flashrnn(*x)
+        check_status()
+        monkeypatch.setenv("FRNN_SPIN_LIMIT", "-2")
+        flashrnn(*x)
+        monkeypatch.delenv("FRNN_SPIN_LIMIT")
+        assert last_status("forward") == 1
+        with pytest.raises(RuntimeError, match="forward of lstm B5 T2 N2 D256"):
+            flashrnn(*x)
+        flashrnn(*x)
+    check_status()
+    assert last_status("forward") == 0
