@@ -15,6 +15,7 @@
 #include "frnn_grad.h"
 #include "frnn_launch.h"
 #include "frnn_mailbox.h"
+#include "frnn_step.h"
 
 namespace frnn {
 
@@ -666,7 +667,8 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
     return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
   e = check_fused_sizes(fx, dtype, B, T, N, D, o.bs, training && !o.rc);
   if (e) return e;
-  CHECK_PTR(Wx) CHECK_PTR(R) CHECK_PTR(b) CHECK_PTR(s0) CHECK_PTR(states) CHECK_PTR(workspace)
+  CHECK_PTR(Wx) CHECK_PTR(R) CHECK_PTR(b) CHECK_PTR(s0) CHECK_PTR(states)
+  CHECK_PTR(workspace)
   if (o.rc) {
     Plan prc;
     if (!find_plan(fx, dtype, D, 0, 2, &prc))
@@ -675,6 +677,12 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   const bool need_cache = training && cell_dims(fx).NC > 0 && !o.rc;
   if (need_cache) CHECK_PTR(cache)
   hipStream_t st = (hipStream_t)stream;
+  if (step && dtype != FRNN_F32) {  // a kernel of its own, with the bits of this tiling
+    prof_begin("fused_step_kernel", st);
+    e = launch_fused_step(fx, dtype, p, tile_rows_for(B, N, p.kw, p.waves, p.max_tr, dtype), StepArgs{Wx, R, b, s0, states, carry, B, o.bs ? o.bs : B, N, D, o.h_clip}, st);
+    prof_end(st);
+    return e ? hip_fail(e, "fused step launch") : 0;
+  }
   FusedFwdWs w = carve_fused_fwd(workspace, dtype, B, N, D, p);
   if (!step) {
     if (workspace_bytes < w.total) return fail(FRNN_E_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, w.total);

@@ -707,6 +707,12 @@ fused_fwd_kernel(const FwdArgs a) {
         if constexpr (CXS >= 0) cc[NC] = s[u][e][CXS];  // (before the step overwrites it)
         CM::fwd(ry, wx, bx[u][e], s[u][e], cc);
         s[u][e][0] = clamp_if(s[u][e][0], a.h_clip);
+        // (fp16: the states are rounded to fp32 first.  Left alone, some kernels round product and conversion at once
+        // (v_fma_mixlo_f16), and 4e-5 of their states differ in the last bit from those of a single step)
+        if constexpr (X::ID == FRNN_F16) {
+#pragma unroll
+          for (int k = 0; k < S; ++k) asm("" : "+v"(s[u][e][k]));
+        }
 #pragma unroll
         for (int c = 0; c < NCX; ++c) cv[c][e] = cc[c];
 #pragma unroll

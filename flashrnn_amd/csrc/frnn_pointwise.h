@@ -15,20 +15,31 @@
 
 namespace frnn {
 
+// Which product of a sum is contracted into a fused multiply-add is written out in the forward math, not left to the compiler
+// (whose choice between f * c + (i * z) and (f * c) + i * z differs from kernel to kernel): a step then rounds the same way in every
+// tiling, tile height and kernel, and single steps give the bits of a sequence whichever kernels run them.  The product that is ready
+// first is the one that is rounded.
 template <bool FAST> struct Math {
   static __device__ __forceinline__ float exp(float x) { return FAST ? __expf(x) : expf(x); }
   static __device__ __forceinline__ float rcp(float x) { return FAST ? __builtin_amdgcn_rcpf(x) : 1.0f / x; }
   static __device__ __forceinline__ float sigmoid(float x) { return rcp(1.0f + exp(-x)); }
   static __device__ __forceinline__ float tanh(float x) {
-    if (FAST) return 1.0f - 2.0f * rcp(1.0f + __expf(2.0f * x));
+    if (FAST) return __builtin_fmaf(-2.0f, rcp(1.0f + __expf(2.0f * x)), 1.0f);
     return tanhf(x);
   }
   // log(sigmoid(x)) = min(x,0) - log1p(exp(-|x|))
   static __device__ __forceinline__ float logsigmoid(float x) {
+#pragma clang fp contract(off)
     const float e = exp(-fabsf(x));
     return fminf(x, 0.0f) - (FAST ? __logf(1.0f + e) : log1pf(e));
   }
 };
+
+// a product that is rounded, whatever it is added to
+__device__ __forceinline__ float mul(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
 
 // fwd:  ry[GR] recurrent pre-activations WITH the bias of their gate slot already added (the
 //       fused kernels fold it into the MFMA accumulator), wx[GW], bx = biases of the gate slots
@@ -46,9 +57,9 @@ template <bool FAST> struct CellMath<FRNN_LSTM, FAST> {
     const float f = M::sigmoid(wx[1] + ry[1]);
     const float z = M::tanh(wx[2] + ry[2]);
     const float o = M::sigmoid(wx[3] + ry[3]);
-    const float c = f * s[1] + i * z;
+    const float c = __builtin_fmaf(i, z, mul(f, s[1]));
     s[1] = c;
-    s[0] = o * M::tanh(c);
+    s[0] = mul(o, M::tanh(c));
     cache[0] = i; cache[1] = f; cache[2] = z; cache[3] = o;
   }
   static __device__ __forceinline__ void bwd(const float* cache, const float* sp, const float* sn, const float* dso,
@@ -81,9 +92,9 @@ template <bool FAST> struct CellMath<FRNN_SLSTM, FAST> {
     const float mn = (s[2] == 0.0f) ? ir : fmaxf(ir, lfm);
     const float ig = M::exp(ir - mn);
     const float fg = M::exp(lfm - mn);
-    const float c = fg * s[1] + ig * z;
-    const float n = fmaxf(fg * s[2] + ig, 1.0f);
-    s[0] = o * c * M::rcp(n);
+    const float c = __builtin_fmaf(ig, z, mul(fg, s[1]));
+    const float n = fmaxf(__builtin_fmaf(fg, s[2], ig), 1.0f);
+    s[0] = mul(mul(o, c), M::rcp(n));
     s[1] = c; s[2] = n; s[3] = mn;
     cache[0] = ig; cache[1] = fg; cache[2] = z; cache[3] = o; cache[4] = M::sigmoid(-fr);
   }
@@ -112,8 +123,8 @@ template <bool FAST> struct CellMath<FRNN_GRU, FAST> {
     const float g = ry[0];
     const float r = M::sigmoid(wx[0] + ry[1]);
     const float z = M::sigmoid(wx[1] + ry[2]);
-    const float nv = M::tanh(wx[2] + b[0] + r * g);
-    s[0] = z * s[0] + (1.0f - z) * nv;
+    const float nv = M::tanh(__builtin_fmaf(r, g, wx[2] + b[0]));
+    s[0] = __builtin_fmaf(1.0f - z, nv, mul(z, s[0]));
     cache[0] = g; cache[1] = r; cache[2] = z; cache[3] = nv;  // the candidate itself: the adjoint needs no tanh
   }
   static __device__ __forceinline__ void bwd(const float* cache, const float* sp, const float* sn, const float* dso,
