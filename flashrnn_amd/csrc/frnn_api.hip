@@ -213,18 +213,35 @@ static bool near_stores_possible(const Plan& p) { return p.kw > 1 && p.kw <= kXc
 // The tiling of a call: the table's default for the head dim, or the widest of its small-batch alternatives (variant 3, else 2) for
 // which all groups of the call fit one launch with 4-row tiles (not where FRNN_TILE_ROWS asks for taller tiles than it has).
 // FRNN_FUSED_VARIANT picks a variant by hand.
-static bool pick_plan(int function, int dtype, int B, int N, int D, int backward, Plan* p) {
+//
+// `dense`: the call may take the dense alternative (kDenseVariant), 8 waves on half the workgroups.  Its launches hold
+// twice the groups, so where the default needs tiles of twice the height to fit, it does not; its own step is longer (the product
+// of two waves per SIMD).  Taken where the default would need 16-row tiles, the GRU's forward kernels also where it would need 8.
+// Forward / reverse kernel, T = 256, default and dense: 16 rows against 8, LSTM B256 N3 D256 0.510 / 0.509 and 0.447 / 0.550 ms (the reverse
+// kernel of 8 waves spills and is not compiled; sLSTM 0.620 and 0.597 forward), GRU B256 N3 D256 0.425 / 0.464 and 0.366 / 0.425, B192 0.407 /
+// 0.446 and 0.343 / 0.415, GRU B256 N2 D384 forward 0.453 and 0.378; 8 rows against 4, B128 N3 D256: GRU 0.296 / 0.295 and 0.285 / 0.317, B160 N2 D384
+// forward 0.326 and 0.305, LSTM forward 0.261 and 0.266, sLSTM 0.372 and 0.401; 4 rows against 4, LSTM B256 N1 D256 0.256 / 0.267 and 0.306 / 0.398.
+// Beyond one launch of 16-row tiles a dense launch takes 1.6 times as long as one of the default and holds twice the groups (pass of 128 steps,
+// default and dense: B512 N3 D256, 2 launches and 1, LSTM 1.192 and 1.077 ms, GRU 1.057 and 0.885; B1024, 3 and 2, 1.87 and 1.89, 1.65 and 1.69).
+static bool pick_plan(int function, int dtype, int B, int N, int D, int backward, Plan* p, bool dense = true) {
   const int variant = env_int("FRNN_FUSED_VARIANT", 0);
   if (!find_plan(function, dtype, D, variant, backward, p)) return false;
   if (variant == 0) {
     const int rows = env_int("FRNN_TILE_ROWS", 0);
+    Plan q;
     for (int v = 3; v >= 2; --v) {
-      Plan q;
       if (find_plan(function, dtype, D, v, backward, &q) && q.variant == v && q.kw > 1 && rows <= q.max_tr &&
           (long)N * ((B + 3) / 4) <= groups_per_launch(q.kw)) {
         *p = q;
-        break;
+        return true;
       }
+    }
+    const int lim = !backward && cell_dims(function).GR == 3 ? 4 : 8;  // the tallest tiles at which the default is the faster one
+    if (dense && rows == 0 && (long)N * ((B + lim - 1) / lim) > groups_per_launch(p->kw) &&
+        find_plan(function, dtype, D, kDenseVariant, backward, &q) && q.variant == kDenseVariant) {
+      const long g = (long)N * ((B + 15) / 16), room = groups_per_launch(p->kw), room_q = groups_per_launch(q.kw);
+      const long launches = (g + room - 1) / room, launches_q = (g + room_q - 1) / room_q;
+      if (launches <= 1 || 8 * launches_q < 5 * launches) *p = q;
     }
   }
   return true;
@@ -482,7 +499,8 @@ static int decode_plan(int function, int dtype, int B, int N, int D, int slots, 
   if (e) return e;
   if (slots != 2 && slots != 4 && slots != 8 && slots != 16) return fail(FRNN_E_ARG, "slots must be 2, 4, 8 or 16 (got %d)", slots);
   // (the tiling of a sequence call of this size: the order of a step's sums, and so the bits, are those of the sequence)
-  if (!pick_plan(function, dtype, B, N, D, 0, &out->p))
+  // (never the dense tiling: it is for calls with more groups than a session may have)
+  if (!pick_plan(function, dtype, B, N, D, 0, &out->p, false))
     return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
   const Plan& p = out->p;
   out->groups = N * ((B + 3) / 4);
@@ -654,7 +672,7 @@ int frnn_fused_forward(int function, int dtype, int training, int B, int T, int 
 static int fused_forward_impl(int function, int dtype, int training, int B, int T, int N, int D,
                               const void* Wx, const void* R, const void* b, const void* s0,
                               void* states, void* cache, void* workspace, size_t workspace_bytes, void* stream,
-                              const frnn_options* opt, int step = 0, float* carry = nullptr) {
+                              const frnn_options* opt, int step = 0, float* carry = nullptr, bool dense = true) {
   g_err[0] = 0;
   int e = check_problem(function, dtype, B, T, N, D);
   if (e) return e;
@@ -663,7 +681,7 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   if (e) return e;
   const int fx = o.fx;
   Plan p;
-  if (!pick_plan(fx, dtype, B, N, D, 0, &p))
+  if (!pick_plan(fx, dtype, B, N, D, 0, &p, dense))
     return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
   e = check_fused_sizes(fx, dtype, B, T, N, D, o.bs, training && !o.rc);
   if (e) return e;
@@ -761,9 +779,14 @@ int frnn_fused_forward_static(int function, int dtype, int training, int B, int 
   int e = check_problem(function, dtype, B, T, N, D);
   if (e) return e;
   Plan p;
-  if (!pick_plan(function, dtype, B, N, D, 0, &p))
-    return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
-  const size_t need = carve_fused_fwd(nullptr, dtype, B, N, D, p).total;
+  size_t need = 0;
+  bool dense = true;  // (the dense tiling has up to twice the groups, and exchange words, of the default)
+  for (;; dense = false) {
+    if (!pick_plan(function, dtype, B, N, D, 0, &p, dense))
+      return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
+    need = carve_fused_fwd(nullptr, dtype, B, N, D, p).total;
+    if (need <= kStaticForwardBytes || !dense) break;
+  }
   if (need > kStaticForwardBytes)
     return fail(FRNN_E_WORKSPACE, "this problem needs %zu bytes of workspace, the static scratch array holds %zu: "
                 "use frnn_fused_forward_opt with a workspace of the caller", need, kStaticForwardBytes);
@@ -771,7 +794,7 @@ int frnn_fused_forward_static(int function, int dtype, int training, int B, int 
   e = static_scratch(&ws);
   if (e) return e;
   return fused_forward_impl(function, dtype, training, B, T, N, D, Wx, R, b, s0, states, cache, ws,
-                            kStaticForwardBytes, stream, opt);
+                            kStaticForwardBytes, stream, opt, 0, nullptr, dense);
 }
 
 int frnn_fused_backward(int function, int dtype, int B, int T, int N, int D,

@@ -12,8 +12,9 @@
 // VARIANT 0 is the default.  VARIANTS 2 and 3, where a head dim has them, spread the head over more workgroups: 3, the
 // wider one, or else 2, is used instead of the default while all groups of the call fit one launch with 4-row
 // batch tiles (measured faster up to a launch that fills the device, slower where the default still takes one launch and
-// they would take two).  To try another tiling add an X(D, 1, ...) entry and run with FRNN_FUSED_VARIANT=1.  The alternatives that were measured and lost (4 waves x 2 tiles for
-// D = 128, 2 x 8 waves or 8 x 2 waves for D = 256, ...) are not compiled in.
+// they would take two).  VARIANT 4 packs the head into half the workgroups of the default, two waves per SIMD: a large batch then
+// runs on tiles of half the height (see pick_plan).  To try another tiling add an X(D, 1, ...) entry and run with FRNN_FUSED_VARIANT=1.  The alternatives that were measured and lost (4 waves x 2 tiles for
+// D = 128, 8 x 2 waves for D = 256, ...) are not compiled in.
 // Forward and backward tile independently (the gate cache layout does not depend on the plan).
 #pragma once
 
@@ -52,6 +53,8 @@ constexpr int fwd_lds_ksteps(int GR, int D, int WAVES, int UTW, int esize) {
 // fp32 heads beyond 512 units take D / 16 = 40, 48 or 64 workgroups, more than the 32 compute units of an XCD: such a group
 // spreads over the device (decode_block) and exchanges at agent scope.
 constexpr int fwd_k_split(int D, int WAVES, int UTW, int KW) { return 16 * WAVES * UTW * KW / D; }
+// the dense alternatives of the tables (host: pick_plan; not for the resident decode kernel, whose groups all have 4 rows)
+constexpr int kDenseVariant = 4;
 // Forward kernel, fp32 at 4-row tiles, cells with 3 or 4 recurrent gates: the product runs on v_mfma_f32_4x4x1_16B_f32
 // (see the kernel), when the whole operand, D / KSP registers per tile in that form, fits the registers of a wave (512 in
 // workgroups of up to 4 waves, 256 with up to 8: D = 96 as 6 waves).
@@ -146,6 +149,7 @@ constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, in
 // stop at 8-row tiles: at 16 rows the sLSTM's, with four states, and the fp16 LSTM's spill, and the bf16 LSTM's, which
 // does not, takes twice as long per launch as at 8 rows: LSTM bf16 B256 T512 12.5 against 12.8 ms)
 #define FRNN_PLANS_GR4_BF16(X) \
+  X(256, 4, 8, 1, 2, 16) \
   X(384, 2, 4, 1, 12, 4) X(448, 2, 4, 1, 14, 4) X(512, 2, 4, 1, 16, 4) X(640, 2, 4, 1, 20, 4) X(768, 2, 4, 1, 24, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 8, 1, 1, 16) X(160, 0, 10, 1, 1, 8) X(192, 0, 12, 1, 1, 4) \
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 8) X(1024, 0, 4, 1, 32, 16)
@@ -161,6 +165,7 @@ constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, in
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 8) X(1024, 0, 4, 1, 32, 8)
 // slstm: its heavier gate math tips D = 192 forward to 3 workgroups of 4 waves (1.19 against 1.26 ms)
 #define FRNN_PLANS_SLSTM_BF16(X) \
+  X(256, 4, 8, 1, 2, 16) \
   X(384, 2, 4, 1, 12, 4) X(448, 2, 4, 1, 14, 4) X(512, 2, 4, 1, 16, 4) X(640, 2, 4, 1, 20, 4) X(768, 2, 4, 1, 24, 4) \
   X(160, 2, 2, 1, 5, 16) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 8, 1, 1, 16) X(160, 0, 10, 1, 1, 8) X(192, 0, 4, 1, 3, 16) \
@@ -191,10 +196,12 @@ constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, in
   X(640, 0, 4, 1, 40, 4) X(768, 0, 4, 1, 48, 4) X(1024, 0, 4, 1, 64, 4)
 // ---- 3 recurrent gate rows per unit (gru) ----------------------------------------------------
 #define FRNN_PLANS_GR3_BF16(X) \
+  X(256, 4, 8, 1, 2, 16) X(384, 4, 8, 1, 3, 16) \
   X(640, 2, 4, 1, 20, 4) X(768, 2, 4, 1, 24, 4) X(1024, 2, 4, 1, 32, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 8, 1, 1, 16) X(160, 0, 10, 1, 1, 16) X(192, 0, 12, 1, 1, 16) \
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 16) X(1024, 0, 4, 1, 16, 16)
 #define FRNN_BWD_PLANS_GR3_BF16(X) \
+  X(256, 4, 8, 1, 2, 16) \
   X(192, 2, 4, 1, 3, 16) X(320, 2, 4, 1, 10, 4) X(512, 2, 4, 1, 16, 4) X(1024, 2, 4, 1, 32, 4) \
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 16) X(96, 0, 6, 1, 1, 16) X(128, 0, 8, 1, 1, 16) X(160, 0, 10, 1, 1, 8) X(192, 0, 12, 1, 1, 4) \
   X(256, 0, 4, 1, 4, 16) X(320, 0, 4, 1, 5, 16) X(384, 0, 4, 1, 6, 16) X(448, 0, 4, 1, 7, 16) X(512, 0, 4, 1, 8, 16) X(640, 0, 4, 1, 10, 16) X(768, 0, 4, 1, 12, 8) X(1024, 0, 4, 1, 16, 16)

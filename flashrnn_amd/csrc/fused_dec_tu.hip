@@ -6,12 +6,19 @@
 
 namespace frnn {
 
+template <int Dv, int VAR, int W, int U, int K> static void (*dec_kernel_for())(const FwdArgs) {
+  if constexpr (VAR == kDenseVariant) return nullptr;  // (never a session's tiling)
+  else return fused_fwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, 4, true>;
+}
+
 template <>
 int fused_dec_launch<FRNN_F, FRNN_DT>(const Plan& p, const FwdArgs& a, hipStream_t st) {
   const dim3 grid(grid_for(a.groups, p.kw));
 #define FRNN_CASE(Dv, VAR, W, U, K, MTR)                                                     \
   if (p.D == Dv && p.waves == W && p.utw == U && p.kw == K) {                                 \
-    hipLaunchKernelGGL((fused_fwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, 4, true>), grid, dim3(W * 64), 0, st, a); \
+    auto kern = dec_kernel_for<Dv, VAR, W, U, K>();                                           \
+    if (!kern) return FRNN_E_UNSUPPORTED;                                                     \
+    hipLaunchKernelGGL(kern, grid, dim3(W * 64), 0, st, a);                                   \
     return (int)hipGetLastError();                                                            \
   }
   FRNN_TU_PLANS(FRNN_CASE)

@@ -1,5 +1,6 @@
 """The rule that chooses a tiling (no GPU: the device counts as one of 256 compute units): the alternatives that spread a head are
-used only while all groups of the call fit one launch, and batch tiles that are asked for are kept."""
+used only while all groups of the call fit one launch, the dense ones only where the default would need taller tiles, and batch tiles
+that are asked for are kept."""
 import ctypes
 
 import pytest
@@ -30,6 +31,9 @@ def test_a_spread_tiling_always_fits_one_launch(monkeypatch, function, dtype):
                 monkeypatch.setenv("FRNN_FUSED_VARIANT", "1")  # (no such entry: the default)
                 q = _plan(function, dtype, B, N, D, backward)
                 assert 16 * p[0] * p[1] * p[2] % D == 0
+                if p[2] < q[2]:  # dense: half the workgroups per head, tiles of half the height or no more launches
+                    assert p[0] == 8 and 2 * p[2] == q[2] and p[3] <= max(q[3], 8 * (32 // p[2]) * p[2])
+                    continue
                 if p[:3] != q[:3]:
                     differ += 1
                     assert p[2] >= q[2] and 1 < p[2] <= 32 and N * -(-B // 4) <= 8 * (32 // p[2])
@@ -39,3 +43,29 @@ def test_a_spread_tiling_always_fits_one_launch(monkeypatch, function, dtype):
                     t = _plan(function, dtype, B, N, D, backward)
                     assert t[:3] == q[:3] or t[3] == N * -(-B // 16) * t[2]
     assert differ > 0 or function == "elman"
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("function,D,backward,lim,default,dense", [("lstm", 256, 0, 8, 4, 2), ("slstm", 256, 0, 8, 4, 2), ("gru", 256, 0, 4, 4, 2),
+                                                                   ("gru", 384, 0, 4, 6, 3), ("gru", 256, 1, 8, 4, 2)])
+def test_the_dense_tiling_begins_where_the_default_needs_taller_tiles(monkeypatch, function, dtype, D, backward, lim, default, dense):
+    room = 8 * (32 // default)
+    for N in (1, 2, 3, 40, 200):
+        last = room // N * lim  # rows of the largest batch that the default still takes with tiles of `lim` rows
+        for B in {1, max(1, last), last + 1, 2 * last + 2, 5 * last + 7}:
+            p = _plan(function, dtype, B, N, D, backward)
+            launches, packed = -(-N * -(-B // 16) // room), -(-N * -(-B // 16) // (8 * (32 // dense)))
+            assert p[2] == (dense if N * -(-B // lim) > room and (launches <= 1 or 8 * packed < 5 * launches) else default), (B, N, p)
+    B = room * lim + 1  # (never where a height is asked for)
+    monkeypatch.setenv("FRNN_TILE_ROWS", "16")
+    assert _plan(function, dtype, B, 1, D, backward)[2] == default
+
+
+def test_calls_that_fit_the_static_scratch_keep_fitting():
+    """The dense tiling's exchange words can exceed the library's static scratch where the default's do not: such a call keeps the
+    default there (null tensors: the size is checked first, then the pointers)."""
+    lib = load_library()
+    for function, B, N in (("lstm", 256, 3), ("slstm", 180, 3), ("gru", 100, 3)):
+        args = [FUNCTION_IDS[function], DTYPE_IDS["bfloat16"], 0, B, 4, N, 256] + [None] * 8
+        rc = lib.frnn_fused_forward_static(*args)
+        assert "static scratch" not in lib.frnn_last_error().decode(), (rc, lib.frnn_last_error())
