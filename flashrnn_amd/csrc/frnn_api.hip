@@ -415,7 +415,7 @@ static FusedBwdWs carve_fused_bwd(void* ws, int function, int dtype, int B, int 
   w.dgx = bp.take(function == FRNN_GRU ? (size_t)B * T * N * D * es : 0);
   w.dbp = (float*)bp.take(bt * c.GT * N * D * 4);
   w.splits = grad_gemm_splits(dtype, B, T, N, D, c.GR);
-  w.part = (float*)bp.take((size_t)w.splits * c.GR * N * D * D * 4);
+  w.part = (float*)bp.take(w.splits > 1 ? (size_t)w.splits * c.GR * N * D * D * 4 : 0);
   w.total = bp.off;
   return w;
 }
@@ -449,10 +449,15 @@ static int weight_grads(int function, int dtype, int B, int T, int N, int D, con
   }
   g.states_h = states; g.s0_h = s0; g.part = part;
   g.B = B; g.T = T; g.N = N; g.D = D; g.GR = c.GR;
+  if (splits == 1) {  // nothing is left to reduce
+    g.part = dR;
+    g.part_b = dbp; g.splits_b = db_splits; g.n_b = (long)((size_t)c.GT * ND); g.db = db;
+  }
   prof_begin("grad_gemm_kernel", st);
   int e = launch_grad_gemm(dtype, g, splits, st);
   prof_end(st);
   if (e) return hip_fail(e, "dR gemm");
+  if (splits == 1) return 0;
   prof_begin("grad_reduce_kernel", st);
   e = launch_grad_reduce(part, splits, (size_t)c.GR * N * D * D, dR, dbp, db_splits, (size_t)c.GT * ND, db, st);
   prof_end(st);
@@ -1120,7 +1125,7 @@ AltWs carve_alt(void* ws, int function, int dtype, int B, int T, int N, int D, i
     w.bsplits = rows < 256 ? (int)rows : 256;
     w.dbp = (float*)bp.take((size_t)w.bsplits * c.GT * ND * 4);
     w.splits = grad_gemm_splits(dtype, B, T, N, D, c.GR);
-    w.part = (float*)bp.take((size_t)w.splits * c.GR * ND * D * 4);
+    w.part = (float*)bp.take(w.splits > 1 ? (size_t)w.splits * c.GR * ND * D * 4 : 0);
   }
   w.total = bp.off;
   return w;

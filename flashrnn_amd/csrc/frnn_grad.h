@@ -13,6 +13,10 @@ struct GradGemmArgs {
   float* part;           // [splits][G_r][N][D][D] partial sums
   int B, T, N, D, GR;
   int rows_per_split;    // filled in by launch_grad_gemm
+  // one split: the GEMM's sums are dR itself (part = dR), and its workgroups also sum the bias partials
+  const float* part_b;   // [splits_b][n_b]
+  int splits_b; long n_b;
+  float* db;             // null: not here
 };
 
 // Rt = R transposed per head; zero_bytes > 0: the same launch clears that many bytes at `zero` (16-byte aligned, whole words)

@@ -97,6 +97,18 @@ __device__ __forceinline__ void gemm_store_partial(const GradGemmArgs& a, int TM
     }
 }
 
+// db of a call with one split, spread over all workgroups (the order of the sums is that of grad_reduce_kernel)
+__device__ __forceinline__ void gemm_sum_bias(const GradGemmArgs& a) {
+  if (!a.db) return;
+  const long lin = blockIdx.x + (long)gridDim.x * (blockIdx.y + (long)gridDim.y * blockIdx.z), all = (long)gridDim.x * gridDim.y * gridDim.z;
+  for (long i = lin * blockDim.x + threadIdx.x; i < a.n_b; i += all * blockDim.x) {
+    float s = 0.f;
+#pragma unroll 16
+    for (int k = 0; k < a.splits_b; ++k) s += a.part_b[(size_t)k * a.n_b + i];
+    a.db[i] = s;
+  }
+}
+
 // 16-bit storage types.  Both operands arrive with the contraction index as the slow one.  The stages are brought in
 // by direct global-to-LDS loads (global_load_lds_dwordx4: no registers, no LDS store instructions) and transposed on
 // their way OUT of LDS by ds_read_b64_tr_b16.  Workgroup tile TM x TM, WD x WD waves of (TM / WD)^2 each.
@@ -275,6 +287,7 @@ __global__ void __launch_bounds__(64 * WD * WD) grad_gemm16_kernel(const GradGem
     static_assert(NS <= 3, "the stage loop is written out for up to 3 buffers");
   }
   gemm_store_partial<WT>(a, TM, g, n, split, dt, pt, wm, wn, r16, q4, acc, TM / WD);
+  gemm_sum_bias(a);
 }
 
 // fp32 storage: the MFMA (16x16x4) takes the operands as they are stored, [row][unit]
@@ -352,17 +365,37 @@ __global__ void __launch_bounds__(256) grad_gemm32_kernel(const GradGemmArgs a) 
     }
   }
   gemm_store_partial<WT>(a, TM, g, n, split, dt, pt, wm, wn, r16, q4, acc, TM / WD);
+  gemm_sum_bias(a);
 }
 
 // side of the square workgroup tile: the largest of 256, 128 (16-bit types only), 64, 32 that divides D; 96 and 160
 // (16-bit types) for the head dims that only much smaller powers of two divide: every pair of tiles of a gate streams
 // both of its operand slabs, so D = 96 as 9 pairs of 32-unit tiles took 1.30 ms at B256 T1024 N8 against 0.40 for D = 64
-static int gemm_tile_side(int dtype, int D) {
+static int gemm_tile_side_of(int dtype, int D) {
   if (dtype != FRNN_F32 && D % 256 == 0) return 256;
   if (dtype != FRNN_F32 && D % 128 == 0) return 128;
   if (dtype != FRNN_F32 && D % 96 == 0 && D / 96 <= 2) return 96;     // 96, 192
   if (dtype != FRNN_F32 && D % 160 == 0 && D / 160 <= 3) return 160;  // 160, 320, 480
   return (D % 64 == 0) ? 64 : 32;
+}
+
+// One split: the GEMM writes dR itself and sums db on the side, so that the launch of the reduction (7 us behind a kernel of 7 to 15) and the
+// trip of the partial sums are saved; a workgroup then walks all stages, ~0.35 us each.  16-bit types up to 16 stages, up to 32 where
+// the tiles alone come to a good part of the device.  GEMM and reduction, two or more splits -> one: LSTM N3 D256 B5 T48 (8 stages) 14.7
+// + 6.9 -> 10.2 us, B8 T64 (16) 15.6 + 7.7 -> 12.8, B8 T128 (32) 15.3 + 10.0 -> 17.5, N1 D768 B16 T64 (32) 20.2 + 17.2 -> 25.5; not GRU N1
+// D128 B16 T64 (32 stages, 12 tiles) 8.7 + 6.7 / 18.8.  fp32: only where there were no two splits of 4 stages before.
+static bool gemm_one_split(int dtype, int B, int T, int N, int D, int GR) {
+  const long chunks = ((long)B * T + 31) / 32;
+  if (dtype == FRNN_F32) return chunks < 8;
+  return chunks <= 16 || (chunks <= 32 && (long)GR * N * (D / 64) * (D / 64) >= 96);
+}
+// ... in tiles small enough to occupy most of the device (LSTM N3 D256 B5 T19, 12 tiles of 256 units -> 192 of 64: 13.8 -> 8.6 us,
+// N1 D768 B4 T40 17.4 -> 12.8, Elman D512 B3 T40 13.4 -> 8.0)
+static int gemm_tile_side(int dtype, int B, int T, int N, int D, int GR) {
+  int TM = gemm_tile_side_of(dtype, D);
+  if (gemm_one_split(dtype, B, T, N, D, GR))
+    while (TM > 64 && D % 64 == 0 && (long)GR * N * (D / TM) * (D / TM) < 192) TM = TM == 256 ? 128 : 64;
+  return TM;
 }
 
 // split-K factor.  Tiles of up to 128 units (workgroups of 4 waves): a workgroup waits for its loads once per stage,
@@ -371,7 +404,7 @@ static int gemm_tile_side(int dtype, int D) {
 // one workgroup per compute unit, all in one round (measured at D = 256, 768, 1024: best at 190-260 workgroups).
 // Bounded by 4 stages per split and by 64 MiB of partial sums.
 int grad_gemm_splits(int dtype, int B, int T, int N, int D, int GR) {
-  const int TM = gemm_tile_side(dtype, D);
+  const int TM = gemm_tile_side(dtype, B, T, N, D, GR);
   const long tiles = (long)GR * (D / TM) * (D / TM) * N;
   const long chunks = ((long)B * T + 31) / 32;
   const long out_bytes = (long)GR * N * D * D * 4;
@@ -382,6 +415,7 @@ int grad_gemm_splits(int dtype, int B, int T, int N, int D, int GR) {
   if (s > 64) s = 64;
   if (s > (64l << 20) / out_bytes) s = (64l << 20) / out_bytes;
   if (s > chunks / 4) s = chunks / 4;
+  if (gemm_one_split(dtype, B, T, N, D, GR)) s = 1;
   if (const char* e = getenv("FRNN_GEMM_SPLITS")) s = atoi(e);
   if (s > 64) s = 64;
   if (s < 1) s = 1;
@@ -411,7 +445,7 @@ static int launch_gemm16_any(int TM, const GradGemmArgs& a, dim3 grid, hipStream
 }
 
 int launch_grad_gemm(int dtype, GradGemmArgs a, int splits, hipStream_t st) {
-  const int TM = gemm_tile_side(dtype, a.D);
+  const int TM = gemm_tile_side(dtype, a.B, a.T, a.N, a.D, a.GR);
   const long chunks = ((long)a.B * a.T + 31) / 32;
   a.rows_per_split = (int)(((chunks + splits - 1) / splits) * 32);
   const dim3 grid(a.GR * (a.D / TM) * (a.D / TM), a.N, splits);
