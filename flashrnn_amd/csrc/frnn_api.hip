@@ -319,9 +319,9 @@ static void gate_leave(LaunchGate* g, hipStream_t st, bool launched_ok = true, b
 // fx is the cell the kernels are instantiated for: the function itself, except that an Elman cell under
 // forward_clipval runs as FRNN_ELMAN_CLIP (one cached value per element: the unclamped h).
 // rc: the gate cache is left out (forward) / rebuilt (backward): only for cells that have one.
-struct Opts { float h_clip, g_clip; int cut; int fx; int rc; int bs; int *report, *report_any; };
+struct Opts { float h_clip, g_clip; int cut; int fx; int rc; int bs; int *report, *report_any; int narrow; void* clear; size_t clear_bytes; };
 static int parse_opts(const frnn_options* o, int function, Opts* out) {
-  out->h_clip = 0.f; out->g_clip = 0.f; out->cut = 0; out->fx = function; out->rc = 0; out->bs = 0; out->report = out->report_any = nullptr;
+  out->h_clip = 0.f; out->g_clip = 0.f; out->cut = 0; out->fx = function; out->rc = 0; out->bs = 0; out->report = out->report_any = nullptr; out->narrow = 0; out->clear = nullptr; out->clear_bytes = 0;
   if (!o) return 0;
   // (the struct may grow at its end: struct_size says how much of it the caller's build knows)
   if (o->struct_size < offsetof(frnn_options, recompute))
@@ -336,6 +336,12 @@ static int parse_opts(const frnn_options* o, int function, Opts* out) {
   out->rc = recompute != 0 && function != FRNN_ELMAN;
   out->bs = o->struct_size >= offsetof(frnn_options, batch_stride) + sizeof(int) ? o->batch_stride : 0;
   if (o->struct_size >= offsetof(frnn_options, report_any) + sizeof(int*)) { out->report = o->report; out->report_any = o->report_any; }
+  out->narrow = o->struct_size >= offsetof(frnn_options, weight_grads) + sizeof(int) ? o->weight_grads : 0;
+  if (out->narrow < 0 || out->narrow > 3) return fail(FRNN_E_ARG, "weight_grads must be 0 to 3 (got %d)", out->narrow);
+  if (o->struct_size >= offsetof(frnn_options, clear_bytes) + sizeof(size_t) && o->clear) {
+    if (((uintptr_t)o->clear | o->clear_bytes) & 3) return fail(FRNN_E_ALIGN, "frnn_options.clear: %zu bytes at %p are not whole dwords", o->clear_bytes, o->clear);
+    out->clear = o->clear; out->clear_bytes = o->clear_bytes;
+  }
   if (out->bs < 0) return fail(FRNN_E_ARG, "batch_stride must be 0 (= B) or the number of rows of the whole batch (got %d)", out->bs);  // (elman caches nothing, or one value under forward_clipval)
   return 0;
 }
@@ -432,7 +438,7 @@ template <int F> static int fused_bwd_dispatch(int dtype, const Plan& p, const B
 // common tail of both backward paths: dR GEMM, final reductions
 static int weight_grads(int function, int dtype, int B, int T, int N, int D, const void* s0, const void* states,
                         const void* dWx, const void* dgx, float* part, int splits, const float* dbp, int db_splits,
-                        float* dR, float* db, hipStream_t st) {
+                        float* dR, float* db, int narrow, hipStream_t st) {
   const CellDims c = cell_dims(function);
   const size_t es = dtype_size(dtype);
   const size_t ND = (size_t)N * D;
@@ -450,7 +456,7 @@ static int weight_grads(int function, int dtype, int B, int T, int N, int D, con
   g.states_h = states; g.s0_h = s0; g.part = part;
   g.B = B; g.T = T; g.N = N; g.D = D; g.GR = c.GR;
   if (splits == 1) {  // nothing is left to reduce
-    g.part = dR;
+    g.dR = dR; g.narrow = narrow;
     g.part_b = dbp; g.splits_b = db_splits; g.n_b = (long)((size_t)c.GT * ND); g.db = db;
   }
   prof_begin("grad_gemm_kernel", st);
@@ -459,7 +465,7 @@ static int weight_grads(int function, int dtype, int B, int T, int N, int D, con
   if (e) return hip_fail(e, "dR gemm");
   if (splits == 1) return 0;
   prof_begin("grad_reduce_kernel", st);
-  e = launch_grad_reduce(part, splits, (size_t)c.GR * N * D * D, dR, dbp, db_splits, (size_t)c.GT * ND, db, st);
+  e = launch_grad_reduce(dtype, narrow, part, splits, (size_t)c.GR * N * D * D, dR, dbp, db_splits, (size_t)c.GT * ND, db, st);
   prof_end(st);
   if (e) return hip_fail(e, "gradient reduction");
   return 0;
@@ -709,9 +715,9 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   FusedFwdWs w = carve_fused_fwd(workspace, dtype, B, N, D, p);
   if (!step) {
     if (workspace_bytes < w.total) return fail(FRNN_E_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, w.total);
-    if (p.kw > 1) {  // (a head of one workgroup has no exchange words, and its kernel sets the status word itself)
+    if (p.kw > 1 || o.clear) {  // (a head of one workgroup has no exchange words, and its kernel sets the status word itself)
       prof_begin("fill_zero_kernel", st);
-      e = launch_fill_zero(workspace, w.zero_bytes, st);
+      e = launch_fill_zero(workspace, p.kw > 1 ? w.zero_bytes : 0, st, o.clear, o.clear_bytes);
       prof_end(st);
       if (e) return hip_fail(e, "workspace clear");
     }
@@ -906,7 +912,7 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   }
   gate_leave(gate, st, e == 0);
   if (e) return hip_fail(e, "fused backward launch");
-  return weight_grads(fx, dtype, B, T, N, D, s0, states, dWx, w.dgx, w.part, w.splits, w.dbp, bt, dR, db, st);
+  return weight_grads(fx, dtype, B, T, N, D, s0, states, dWx, w.dgx, w.part, w.splits, w.dbp, bt, dR, db, o.narrow, st);
 }
 
 int frnn_fused_backward_opt(int function, int dtype, int B, int T, int N, int D,
@@ -1162,6 +1168,8 @@ int frnn_alt_forward_opt(int function, int dtype, int training, int B, int T, in
   if (workspace_bytes < w.total) return fail(FRNN_E_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, w.total);
   AltProblem p{o.fx, dtype, B, T, N, D, need_cache ? 1 : 0, o.h_clip, 0.f, 0, 0};
   AltFwdBuffers bf{Wx, R, b, s0, states, cache, w.sfp};
+  e = launch_fill_zero(nullptr, 0, (hipStream_t)stream, o.clear, o.clear_bytes);
+  if (e) return hip_fail(e, "clear");
   prof_begin("alt_forward_steps", (hipStream_t)stream);
   e = alt_forward(p, bf, (hipStream_t)stream);
   prof_end((hipStream_t)stream);
@@ -1256,7 +1264,7 @@ int frnn_alt_backward_opt(int function, int dtype, int B, int T, int N, int D,
   e = launch_bias_partial(dtype, src, ld, c.GT, N, D, (long)B * T, w.bsplits, w.dbp, st);
   prof_end(st);
   if (e) return hip_fail(e, "bias partial sums");
-  return weight_grads(fx, dtype, B, T, N, D, s0, states, dWx, w.dgx, w.part, w.splits, w.dbp, w.bsplits, dR, db, st);
+  return weight_grads(fx, dtype, B, T, N, D, s0, states, dWx, w.dgx, w.part, w.splits, w.dbp, w.bsplits, dR, db, o.narrow, st);
 }
 
 }  // extern "C"

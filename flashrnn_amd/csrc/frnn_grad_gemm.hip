@@ -81,10 +81,31 @@ __device__ __forceinline__ void gemm_tile_of(const GradGemmArgs& a, int TM, int&
   g = tile / tiles;
 }
 
-template <int WT>
+// a gradient in the storage type (16-bit types: rounded to nearest even) or in fp32
+template <typename T>
+__device__ __forceinline__ void store_grad(void* p, size_t i, float v, bool narrow) {
+  if constexpr (sizeof(T) == 2) {
+    if (narrow) { static_cast<unsigned short*>(p)[i] = (unsigned short)pack<1>(&v, (T*)nullptr).v[0]; return; }
+  }
+  static_cast<float*>(p)[i] = v;
+}
+
+template <typename T, int WT>
 __device__ __forceinline__ void gemm_store_partial(const GradGemmArgs& a, int TM, int g, int n, int split, int dt, int pt,
                                                    int wm, int wn, int r16, int q4, const f32x4 (&acc)[WT][WT], int span) {
   const int D = a.D;
+  if (a.dR) {  // (uniform)
+    const size_t at = (((size_t)g * a.N + n) * D) * D;
+#pragma unroll
+    for (int i = 0; i < WT; ++i)
+#pragma unroll
+      for (int j = 0; j < WT; ++j) {
+        const int d = dt * TM + wm * span + i * 16 + q4 * 4, p = pt * TM + wn * span + j * 16 + r16;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) store_grad<T>(a.dR, at + (size_t)(d + e) * D + p, acc[i][j][e], a.narrow & 1);
+      }
+    return;
+  }
   float* out = a.part + ((((size_t)split * a.GR + g) * a.N + n) * D) * D;
 #pragma unroll
   for (int i = 0; i < WT; ++i)
@@ -98,14 +119,15 @@ __device__ __forceinline__ void gemm_store_partial(const GradGemmArgs& a, int TM
 }
 
 // db of a call with one split, spread over all workgroups (the order of the sums is that of grad_reduce_kernel)
+template <typename T>
 __device__ __forceinline__ void gemm_sum_bias(const GradGemmArgs& a) {
-  if (!a.db) return;
+  if (!a.dR) return;
   const long lin = blockIdx.x + (long)gridDim.x * (blockIdx.y + (long)gridDim.y * blockIdx.z), all = (long)gridDim.x * gridDim.y * gridDim.z;
   for (long i = lin * blockDim.x + threadIdx.x; i < a.n_b; i += all * blockDim.x) {
     float s = 0.f;
 #pragma unroll 16
     for (int k = 0; k < a.splits_b; ++k) s += a.part_b[(size_t)k * a.n_b + i];
-    a.db[i] = s;
+    store_grad<T>(a.db, i, s, a.narrow & 2);
   }
 }
 
@@ -286,8 +308,8 @@ __global__ void __launch_bounds__(64 * WD * WD) grad_gemm16_kernel(const GradGem
     if (NS > 2 && s + 2 < nst) stage(s + 2, std::integral_constant<int, 2 % NS>{});
     static_assert(NS <= 3, "the stage loop is written out for up to 3 buffers");
   }
-  gemm_store_partial<WT>(a, TM, g, n, split, dt, pt, wm, wn, r16, q4, acc, TM / WD);
-  gemm_sum_bias(a);
+  gemm_store_partial<T, WT>(a, TM, g, n, split, dt, pt, wm, wn, r16, q4, acc, TM / WD);
+  gemm_sum_bias<T>(a);
 }
 
 // fp32 storage: the MFMA (16x16x4) takes the operands as they are stored, [row][unit]
@@ -364,8 +386,8 @@ __global__ void __launch_bounds__(256) grad_gemm32_kernel(const GradGemmArgs a) 
         for (int j = 0; j < WT; ++j) acc[i][j] = X::mfma(af[i], bfr[j], acc[i][j]);
     }
   }
-  gemm_store_partial<WT>(a, TM, g, n, split, dt, pt, wm, wn, r16, q4, acc, TM / WD);
-  gemm_sum_bias(a);
+  gemm_store_partial<T, WT>(a, TM, g, n, split, dt, pt, wm, wn, r16, q4, acc, TM / WD);
+  gemm_sum_bias<T>(a);
 }
 
 // side of the square workgroup tile: the largest of 256, 128 (16-bit types only), 64, 32 that divides D; 96 and 160
@@ -458,41 +480,45 @@ int launch_grad_gemm(int dtype, GradGemmArgs a, int splits, hipStream_t st) {
 
 // ---------------------------------------------------------------------------------------------
 // out[i] = sum_s part[s][i]: i < n_r for the dR partials (splits_r of them), then i - n_r < n_b
-// for the bias partials (splits_b of them).
+// for the bias partials (splits_b of them).  narrow: see launch_grad_reduce.  (Written in the type of the weights the results need no
+// launch that casts each of them.)
 // ---------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) grad_reduce_kernel(const float* __restrict__ part_r, int splits_r, size_t n_r, float* __restrict__ dR,
-                                                          const float* __restrict__ part_b, int splits_b, size_t n_b, float* __restrict__ db) {
+template <typename T>
+__global__ void __launch_bounds__(256) grad_reduce_kernel(int narrow, const float* __restrict__ part_r, int splits_r, size_t n_r, void* __restrict__ dR,
+                                                          const float* __restrict__ part_b, int splits_b, size_t n_b, void* __restrict__ db) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i < n_r) {
     float s = 0.f;
 #pragma unroll 16
     for (int k = 0; k < splits_r; ++k) s += part_r[(size_t)k * n_r + i];
-    dR[i] = s;
+    store_grad<T>(dR, i, s, narrow & 1);
   } else if (i - n_r < n_b) {
     const size_t j = i - n_r;
     float s = 0.f;
 #pragma unroll 16
     for (int k = 0; k < splits_b; ++k) s += part_b[(size_t)k * n_b + j];
-    db[j] = s;
+    store_grad<T>(db, j, s, narrow & 2);
   }
 }
 
-int launch_grad_reduce(const float* part_r, int splits_r, size_t n_r, float* dR,
-                       const float* part_b, int splits_b, size_t n_b, float* db, hipStream_t st) {
+int launch_grad_reduce(int dtype, int narrow, const float* part_r, int splits_r, size_t n_r, void* dR,
+                       const float* part_b, int splits_b, size_t n_b, void* db, hipStream_t st) {
   const size_t total = n_r + n_b;
-  hipLaunchKernelGGL(grad_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                     part_r, splits_r, n_r, dR, part_b, splits_b, n_b, db);
+  const auto kern = dtype == FRNN_BF16 ? grad_reduce_kernel<bf16_t> : dtype == FRNN_F16 ? grad_reduce_kernel<half_t> : grad_reduce_kernel<float>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
+                     narrow, part_r, splits_r, n_r, dR, part_b, splits_b, n_b, db);
   return (int)hipGetLastError();
 }
 
-__global__ void __launch_bounds__(256) fill_zero_kernel(unsigned* p, size_t words) {
+__global__ void __launch_bounds__(256) fill_zero_kernel(unsigned* p, size_t words, unsigned* p2, size_t words2) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i < words) p[i] = 0u;
+  else if (i - words < words2) p2[i - words] = 0u;
 }
-int launch_fill_zero(void* p, size_t bytes, hipStream_t st) {
-  const size_t words = (bytes + 3) / 4;
-  if (words == 0) return 0;
-  hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, (unsigned*)p, words);
+int launch_fill_zero(void* p, size_t bytes, hipStream_t st, void* p2, size_t bytes2) {
+  const size_t words = p ? (bytes + 3) / 4 : 0, words2 = p2 ? bytes2 / 4 : 0;
+  if (words + words2 == 0) return 0;
+  hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((words + words2 + 255) / 256)), dim3(256), 0, st, (unsigned*)p, words, (unsigned*)p2, words2);
   return (int)hipGetLastError();
 }
 

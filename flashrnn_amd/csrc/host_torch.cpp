@@ -162,6 +162,7 @@ c10::ScalarType kernel_type(int d) { return d == FRNN_BF16 ? torch::kBFloat16 : 
 struct Call : torch::CustomClassHolder {
   int function, dtype;
   bool fused, amp, training;
+  bool zero_s0 = false;  // s0 is this call's own, and its launches set it to zero
   frnn_options o;
 };
 using CallPtr = c10::intrusive_ptr<Call>;
@@ -202,6 +203,7 @@ Saved run_forward(const Tensor& Wx_, const Tensor& R_, const Tensor& b_, const T
   const Tensor ws = torch::empty({(int64_t)wsb}, bytes);
   void* st = stream_of(v.Wx);
   frnn_options o = c.o;
+  if (c.zero_s0) { o.clear = v.s0.data_ptr(); o.clear_bytes = v.s0.nbytes(); }
   if (c.fused) ring().take({0, c.function, (int)B, (int)T, (int)N, (int)D}, st, o);
   check_rc((c.fused ? api.fused_forward : api.alt_forward)(
                c.function, c.dtype, c.training, B, T, N, D, v.Wx.data_ptr(), v.R.data_ptr(), v.b.data_ptr(), v.s0.data_ptr(),
@@ -248,7 +250,7 @@ struct Function : torch::autograd::Function<Function> {
     const Tensor ds = dstates.to(states.scalar_type()).contiguous();
     const auto k = states.options(), f = k.dtype(torch::kFloat);
     const Tensor dWx = torch::empty({B, T, Gw, N, D}, k), ds0 = torch::empty({S, B, N, D}, k);
-    const Tensor dR = torch::empty({Gr, N, D, D}, f), db = torch::empty({Gt, N, D}, f);
+    const Tensor dR = torch::empty({Gr, N, D, D}, c.o.weight_grads & 1 ? k : f), db = torch::empty({Gt, N, D}, c.o.weight_grads & 2 ? k : f);
     const size_t wsb = std::max<size_t>(256, c.fused ? api.fused_workspace_bytes(c.function, c.dtype, B, T, N, D, 1, &c.o)
                                                      : api.alt_workspace_bytes(c.function, c.dtype, B, T, N, D, 1));
     const Tensor ws = torch::empty({(int64_t)wsb}, k.dtype(torch::kByte));
@@ -257,14 +259,14 @@ struct Function : torch::autograd::Function<Function> {
     int rc;
     if (c.o.recompute)
       rc = api.backward_recompute(c.function, c.dtype, B, T, N, D, Wx.data_ptr(), R.data_ptr(), b.data_ptr(), s0.data_ptr(), states.data_ptr(),
-                                  ds.data_ptr(), dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr<float>(), db.data_ptr<float>(), ws.data_ptr(), wsb, st, &o);
+                                  ds.data_ptr(), dWx.data_ptr(), ds0.data_ptr(), static_cast<float*>(dR.data_ptr()), static_cast<float*>(db.data_ptr()), ws.data_ptr(), wsb, st, &o);
     else
       rc = (c.fused ? api.fused_backward : api.alt_backward)(
           c.function, c.dtype, B, T, N, D, R.data_ptr(), b.data_ptr(), s0.data_ptr(), states.data_ptr(), cache.data_ptr(), ds.data_ptr(),
-          dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr<float>(), db.data_ptr<float>(), ws.data_ptr(), wsb, st, &o);
+          dWx.data_ptr(), ds0.data_ptr(), static_cast<float*>(dR.data_ptr()), static_cast<float*>(db.data_ptr()), ws.data_ptr(), wsb, st, &o);
     check_rc(rc, c.fused, "backward");
-    // dR / db stay fp32: autograd casts them to the dtype of the leaf they belong to, so fp32 master weights receive
-    // unrounded gradients
+    // dR / db of tensors in the kernel type come rounded from the kernels (autograd would cast each in a launch of its own); the
+    // others stay fp32, so that fp32 master weights receive unrounded gradients
     return {dWx, dR, db, ds0.view({S, B, 1, N, D})};
   }
 };
@@ -299,12 +301,15 @@ py::object call(const Tensor& Wx, const Tensor& R, const Tensor& b, const std::o
   {
     py::gil_scoped_release nogil;
     ring().poll(false, stream_of(Wx));
+    const auto k = kernel_type(dtype);
     Tensor s0;
     if (states) s0 = *states;
     else {
       c10::DeviceGuard guard(Wx.device());
-      s0 = torch::zeros({S, B, 1, N, D}, Wx.options().requires_grad(false));
+      s0 = torch::empty({S, B, 1, N, D}, Wx.options().dtype(k).requires_grad(false));
+      c->zero_s0 = true;
     }
+    if (k != torch::kFloat) c->o.weight_grads = (R.scalar_type() == k ? 1 : 0) | (b.scalar_type() == k ? 2 : 0);
     out = c->training ? Function::apply(Wx, R, b, s0, c) : run_forward(Wx, R, b, s0, *c).states;
     last = out.narrow(2, T - 1, 1);
   }

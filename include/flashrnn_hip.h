@@ -184,6 +184,10 @@ typedef struct frnn_options {
   int* report_any;  /* one of whose bounded waits ran out sets both to 1, beside the status word of its workspace: one word per call
                       * and one for many calls tell the caller which call failed without copying the status word of each.  Valid
                       * until the call has ended (frnn_wait_launches); the library only ever stores 1. */
+  int weight_grads; /* backward calls with a 16-bit storage type: 1 = dR, 2 = db, 3 = both are written in the storage type (the fp32
+                     * sums, rounded to nearest even) and point at tensors of it; 0 (and always in fp32): fp32 */
+  void* clear;      /* forward calls, or null: clear_bytes of device memory (whole dwords) that the call sets to zero in front of its */
+  size_t clear_bytes; /* kernels, where it can in the launch that clears its workspace: the s0 of a call that begins at zero */
 } frnn_options;
 
 /* Waits for the most recent fused launch of every device whose workgroups wait for each other (and so, these launches being
