@@ -81,12 +81,16 @@ struct CallInfo { int kind, function, B, T, N, D; };
 struct StatusRing {
   std::mutex mu;
   Tensor words;              // pinned: [kSlots] and the shared word
+  std::atomic<int*> base{nullptr};  // its memory, for threads that look at the shared word without holding mu
   std::vector<CallInfo> info;
   long taken = 0;
   long last[2] = {-1, -1};   // the most recent call of each kind (forward, backward)
   std::vector<std::string> older;  // failed calls whose slots were used again before anyone asked
 
-  volatile int* any() { return words.defined() ? words.data_ptr<int>() + kSlots : nullptr; }
+  volatile int* any() {
+    int* const w = base.load(std::memory_order_acquire);
+    return w ? w + kSlots : nullptr;
+  }
   // the words of a call on `stream`; calls under capture are not recorded: a replay repeats the kernels, not this
   void take(const CallInfo& c, void* stream, frnn_options& o) {
     o.report = o.report_any = nullptr;
@@ -95,6 +99,7 @@ struct StatusRing {
     if (!words.defined()) {
       words = torch::zeros({kSlots + 1}, torch::TensorOptions().dtype(torch::kInt).pinned_memory(true));
       info.resize(kSlots);
+      base.store(words.data_ptr<int>(), std::memory_order_release);
     }
     const long s = taken++;
     if (s >= kSlots && s % kSlots == 0) {
@@ -362,6 +367,7 @@ PYBIND11_MODULE(_host, m) {
     api.wait_launches();
     auto failed = ring().collect();
     std::lock_guard<std::mutex> lk(ring().mu);
+    ring().base.store(nullptr);
     ring().words.reset();  // (pinned memory goes back while the HIP runtime is up)
     ring().taken = 0; ring().last[0] = ring().last[1] = -1;
     return failed;

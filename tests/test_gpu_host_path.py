@@ -2,6 +2,7 @@
 module does not: the same bits, and the same behaviour towards autograd."""
 import pytest
 import torch
+import torch.utils.checkpoint
 
 from oracle import make_inputs
 
@@ -92,6 +93,9 @@ def test_autograd_meets_the_function_it_knows(gpu):
         out, _ = flashrnn(*leaves)
     hooked = torch.autograd.grad(out.float().sum(), leaves)
     assert len(packed) >= 5 and all(torch.equal(x, y) for x, y in zip(one, hooked))
+    out = torch.utils.checkpoint.checkpoint(lambda *x: flashrnn(*x)[0], *leaves, use_reentrant=False)  # (its hooks end the second call early)
+    again = torch.autograd.grad(out.float().sum(), leaves)
+    assert all(torch.equal(x, y) for x, y in zip(one, again))
     R = leaves[1].detach().clone().requires_grad_()
     out, _ = flashrnn(leaves[0], R, *leaves[2:])
     with torch.no_grad():
@@ -103,6 +107,31 @@ def test_autograd_meets_the_function_it_knows(gpu):
     with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError):
         flashrnn(torch.autograd.forward_ad.make_dual(leaves[0].detach(), torch.ones_like(leaves[0])), *leaves[1:])
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_threads_share_the_record_of_failed_waits(gpu):
+    import threading
+
+    from flashrnn_amd import check_status, flashrnn
+
+    print("case host path threads", flush=True)
+    x = [v.detach() for v in _leaves(gpu, D=256)]
+    ref, results = flashrnn(*x)[0], [None] * 4
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            results[i] = [flashrnn(*x)[0] for _ in range(50)]
+            torch.cuda.current_stream().synchronize()
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    check_status()
+    assert all(torch.equal(y, ref) for r in results for y in r)
 
 
 @pytest.mark.gpu
