@@ -211,12 +211,13 @@ fused_bwd_kernel(const BwdArgs a) {
   //      iteration i+2 into the other buffer and sends for those of iteration i+4 --------------------------------------
   constexpr bool PW = bwd_producer_wave(GR, NC, D, WAVES, UTW, KW, TR, (int)sizeof(T), RC);
   // one buffer: [cache: tile][row][16 units][NCP values] [s_(t-1): state][tile][row][16 units] [cotangent: the same]
-  constexpr int PB_CA = NC > 0 ? UT_WG * TR * 16 * NCP : 0, PB_ST = S * UT_WG * TR * 16, PB = PB_CA + 2 * PB_ST;
-  static_assert(!PW || 2 * PB * (int)sizeof(T) + 16 == bwd_producer_bytes(NCX, S, UT_WG, TR, (int)sizeof(T)), "hand-over buffer size");
+  // (recompute mode: [Wx: gate][tile][row][16 units] in the place of the cache; h_(t-1) goes to its buffers hb0 / hb1)
+  constexpr int PB_CA = RC ? UT_WG * TR * 16 * ((GW + 1) / 2 * 2) : NC > 0 ? UT_WG * TR * 16 * NCP : 0, PB_ST = S * UT_WG * TR * 16, PB = PB_CA + 2 * PB_ST;
+  static_assert(!PW || 2 * PB * (int)sizeof(T) + 16 == bwd_producer_bytes(RC ? GW : NCX, S, UT_WG, TR, (int)sizeof(T)), "hand-over buffer size");
   // the carried state comes out of the cache line instead of a load of its own (the kernels with a producer wave keep the
   // load: it is the producer's, off the compute waves' chain)
   constexpr bool CXU = CXS >= 0 && !PW;
-  T* const pbuf = reinterpret_cast<T*>(smem_raw + bwd_lds_bytes(GR, D, WAVES, UTW, KW, (int)sizeof(T)));
+  T* const pbuf = reinterpret_cast<T*>(smem_raw + bwd_lds_bytes(GR, D, WAVES, UTW, KW, (int)sizeof(T), RC));
   // Producer-wave stores (PSTV instantiations, chosen on the host for launches that fill the device; see the forward
   // kernel): the compute waves leave dWx_t (and the GRU's g-gate cotangent) in LDS as they lie in memory, two buffers by
   // iteration parity behind the hand-over buffers, and the producer wave stores them in 16-byte pieces behind the
@@ -229,11 +230,20 @@ fused_bwd_kernel(const BwdArgs a) {
   if constexpr (PW) {
     if (w == WAVES) {
       constexpr int CPR = NCP * 2;  // 16-byte pieces per (tile, batch row) of the cache
-      constexpr int CP_TOT = NC > 0 ? UT_WG * TR * CPR : 0, NPC = (CP_TOT + 63) / 64;
+      constexpr int CP_TOT = RC ? GW * UT_WG * TR * 2 : NC > 0 ? UT_WG * TR * CPR : 0, NPC = (CP_TOT + 63) / 64;  // recompute mode: of Wx, as of the states
+      constexpr int HP_TOT = RC ? TR * (D / 8) : 0, NPH = (HP_TOT + 63) / 64;  // recompute mode: pieces of 8 units of one row of h
       constexpr int SP_TOT = S * UT_WG * TR * 2, NPS = (SP_TOT + 63) / 64;  // pieces of 8 units of one state, tile and row
+      constexpr int SPM = RC && F == FRNN_SLSTM ? 0xf : C::SPM;  // (the rebuilt gates of the sLSTM need m as well)
       unsigned cvo[NPC > 0 ? NPC : 1], svo[NPS], spo[NPS], s0o[NPS]; int cl[NPC > 0 ? NPC : 1], sl[NPS];
 #pragma unroll
       for (int i = 0; i < NPC; ++i) {
+        if constexpr (RC) {
+          const int c = lane + 64 * i, half = c & 1, pr = (c >> 1) % TR, ptile = ((c >> 1) / TR) % UT_WG, pg = (c >> 1) / (TR * UT_WG);
+          const bool ok = c < CP_TOT && bt * TR + pr < B;
+          cvo[i] = ok ? (((unsigned)(bt * TR + pr) * Tn * GW + pg) * ND + n * D + ptile * 16 + half * 8) * ES : kInvalidOff;  // + t * GW * ND * ES
+          cl[i] = c < CP_TOT ? ((pg * UT_WG + ptile) * TR + pr) * 16 + half * 8 : -1;
+          continue;
+        }
         const int c = lane + 64 * i, q = c % CPR, pr = (c / CPR) % TR, ptile = c / (CPR * TR);
         const bool ok = c < CP_TOT && bt * TR + pr < B;
         cvo[i] = ok ? ((((unsigned)(slice * UT_WG + ptile) * Bpad + bt * TR + pr) * 16) * NCP * ES + q * 16) : kInvalidOff;
@@ -245,11 +255,20 @@ fused_bwd_kernel(const BwdArgs a) {
         const bool ok = c < SP_TOT && bt * TR + pr < B;
         const unsigned col = n * D + slice * DL + ptile * 16 + half * 8;
         // (planes that the cell's adjoint never reads: out of range, no memory traffic; their LDS slots hold zeros)
-        const bool oks = ok && ((C::SPM >> pk) & 1), okd = ok && ((C::DSM >> pk) & 1);
+        const bool oks = ok && ((SPM >> pk) & 1), okd = ok && ((C::DSM >> pk) & 1);
         svo[i] = okd ? ((((unsigned)(pk * BS + bt * TR + pr) * Tn) * ND + col) * ES) : kInvalidOff;   // + t * ND * ES
         spo[i] = oks ? ((((unsigned)(pk * BS + bt * TR + pr) * Tn) * ND + col) * ES) : kInvalidOff;
         s0o[i] = oks ? (((unsigned)(pk * BS + bt * TR + pr) * ND + col) * ES) : kInvalidOff;
         sl[i] = c < SP_TOT ? ((pk * UT_WG + ptile) * TR + pr) * 16 + half * 8 : -1;
+      }
+      unsigned hvo[NPH > 0 ? NPH : 1], h0o[NPH > 0 ? NPH : 1]; int hl[NPH > 0 ? NPH : 1];
+#pragma unroll
+      for (int i = 0; i < NPH; ++i) {  // (consecutive lanes take the rows of one piece position, as in stage_h)
+        const int c = lane + 64 * i, pr = c % TR, k0 = c / TR * 8;
+        const bool ok = c < HP_TOT && bt * TR + pr < B;
+        hvo[i] = ok ? ((unsigned)(bt * TR + pr) * Tn * ND + n * D + k0) * ES : kInvalidOff;
+        h0o[i] = ok ? ((unsigned)(bt * TR + pr) * ND + n * D + k0) * ES : kInvalidOff;
+        hl[i] = c < HP_TOT ? (int)X::frag_elem(pr, k0) : -1;
       }
       // The compiler counts the operations in flight behind each load exactly, but where two paths meet it takes the lower
       // count: at the head of a loop that follows the first fetches directly, with the loads of two iterations interleaved
@@ -259,9 +278,9 @@ fused_bwd_kernel(const BwdArgs a) {
       // and 6 waves (reverse kernel, T = 512, without and with: bf16 B128 N12 D64 0.396 -> 0.373 ms, B224 N10 D64 0.693
       // -> 0.626, B256 N8 D64 0.494 -> 0.479, B128 N6 D96 0.347 -> 0.309); its kernels of 2 waves +4 to +8 % at small batches
       // and of 8 waves +-1 %, the other gated cells -5 to +3 %, the Elman cell +15 % (B16 N12 D64)
-      constexpr bool ORDERED = F == FRNN_SLSTM && WAVES >= 4 && WAVES <= 6;
+      constexpr bool ORDERED = F == FRNN_SLSTM && WAVES >= 4 && WAVES <= 6 && !RC;
       auto in_order = []() __attribute__((always_inline)) { if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0); };
-      struct Ops { Dw<4> ca[NPC > 0 ? NPC : 1], sp[NPS], dso[NPS]; };
+      struct Ops { Dw<4> ca[NPC > 0 ? NPC : 1], sp[NPS], dso[NPS], h[NPH > 0 ? NPH : 1]; };
       Ops set[3];
       auto fetch = [&](Ops& o, int j) __attribute__((always_inline)) {
         int t = Tn - 1 - j > 0 ? Tn - 1 - j : 0;  // (beyond the last step: the operands of step 0 again, unused)
@@ -271,7 +290,13 @@ fused_bwd_kernel(const BwdArgs a) {
         in_order();
 #pragma unroll
         for (int i = 0; i < NPC; ++i) {
-          o.ca[i] = buf_load<4>(rCa, cvo[i], (((unsigned)t * N + n) * (D / 16)) * Bpad * 16 * NCP * ES);
+          if constexpr (RC) o.ca[i] = buf_load<4>(rWx, cvo[i], (unsigned)t * GW * ND * ES);
+          else o.ca[i] = buf_load<4>(rCa, cvo[i], (((unsigned)t * N + n) * (D / 16)) * Bpad * 16 * NCP * ES);
+          in_order();
+        }
+#pragma unroll
+        for (int i = 0; i < NPH; ++i) {
+          o.h[i] = buf_load<4>(rPrev, first ? h0o[i] : hvo[i], first ? 0u : (unsigned)(t - 1) * ND * ES);
           in_order();
         }
 #pragma unroll
@@ -287,6 +312,10 @@ fused_bwd_kernel(const BwdArgs a) {
       auto put = [&](const Ops& o, int j) __attribute__((always_inline)) {
         T* const pb = pbuf + (j & 1) * PB;
         T* const spare = pbuf + 2 * PB;
+        T* const hb = ((Tn - 1 - j) & 1) ? hb1 : hb0;
+#pragma unroll
+        for (int i = 0; i < NPH; ++i)
+          *reinterpret_cast<uint4*>(hl[i] >= 0 ? hb + hl[i] : spare) = make_uint4(o.h[i].v[0], o.h[i].v[1], o.h[i].v[2], o.h[i].v[3]);
 #pragma unroll
         for (int i = 0; i < NPC; ++i)
           *reinterpret_cast<uint4*>(cl[i] >= 0 ? pb + cl[i] : spare) = make_uint4(o.ca[i].v[0], o.ca[i].v[1], o.ca[i].v[2], o.ca[i].v[3]);
@@ -329,8 +358,9 @@ fused_bwd_kernel(const BwdArgs a) {
         }
       };
       fetch(set[1], 1); fetch(set[2], 2); fetch(set[0], 3);
+      if constexpr (RC) __syncthreads();  // (behind which the buffers of h are cleared)
       put(set[1], 1);
-      __syncthreads();  // (the one of the prologue below)
+      __syncthreads();  // (the one of the prologue below; recompute mode: the one in front of the first gates)
       if (!a.cut) {
         auto iter = [&](int i, const Ops& next, Ops& refill) __attribute__((always_inline)) {
           lds_barrier();
@@ -363,6 +393,8 @@ fused_bwd_kernel(const BwdArgs a) {
           iter(i, set[2], set[1]);
           if (i + 1 < Tn) iter(i + 1, set[0], set[2]);
         }
+      } else if constexpr (RC) {
+        for (int t = Tn - 1; t > 0; --t) lds_barrier();  // (the truncated scan hands h over to itself)
       }
       lds_barrier();  // (the one behind the time loop)
       return;
@@ -469,7 +501,8 @@ fused_bwd_kernel(const BwdArgs a) {
           // the chain of dependent steps, is the one to live in the accumulation registers, where the MFMA
           // reads it directly.  Left to the register allocator, fragments of both operands end up there as
           // spills, each copied back before its MFMA (measured: +400 cycles on the R^T product of a step)
-          asm volatile("" : "+a"(rfw[u][g][ks]));
+          // (with the producer wave both fit the architectural registers, of which a kernel with a pinned operand gets half)
+          if constexpr (!PW) asm volatile("" : "+a"(rfw[u][g][ks]));
 #endif
         }
         if constexpr (BIAS_C) {
@@ -689,9 +722,8 @@ fused_bwd_kernel(const BwdArgs a) {
   }
 
   bool dead = near_i < 0;
-  // does a step look at the workgroup's flag of a failed wait?  Heads of one workgroup never wait, and nobody sets it (the
-  // recompute-mode kernel of the sLSTM at D = 96 reads it all the same: in fp16 any other form of its step spills)
-  constexpr bool FLAG = KW > 1 || (RC && F == FRNN_SLSTM && WAVES > 4);
+  // does a step look at the workgroup's flag of a failed wait?  Heads of one workgroup never wait, and nobody sets it
+  constexpr bool FLAG = KW > 1;
   static_assert(!(PW && FLAG), "the producer wave reads no flag");
   // one reverse step: consumes `pc` (operands of step t), prefetches those of step t-1 into `pn`.
   // CUT (a std::bool_constant): truncated backpropagation, the step ends with the pointwise carry;
@@ -789,7 +821,8 @@ fused_bwd_kernel(const BwdArgs a) {
       }
     }
     }
-    if constexpr (RC) {
+    constexpr bool RCP = RC && PW && !cut;  // recompute mode with the producer wave, which stages h
+    if constexpr (RC && !RCP) {
       if (t > 0) stage_h(pm, t - 1);  // uniform
     }
     if constexpr (cut) {
@@ -802,10 +835,10 @@ fused_bwd_kernel(const BwdArgs a) {
     // the barrier also spreads a failed wait of the previous step to the whole workgroup; a head of one workgroup never
     // waits and has no flag to read: its fragments are requested right behind the barrier (without the flag's trip to LDS
     // and back in front of them: LSTM bf16 B256 T1024 N12 D64 reverse kernel 1.10 -> 0.98 ms, B16 0.405 -> 0.358, Elman B16 0.260 -> 0.159, fp16 B33 T515 N8 D96 recompute
-    // mode 0.555 -> 0.540, GRU bf16 B16 T2048 N4 D128 1.043 -> 1.032)
+    // mode (before its producer wave) 0.555 -> 0.540, GRU bf16 B16 T2048 N4 D128 1.043 -> 1.032)
     if constexpr (!FLAG) {
       lds_barrier();
-      if constexpr (RC || TR > 4) {  // (without an exit here: spills)
+      if constexpr ((RC && !PW) || TR > 4) {  // (without an exit here: spills)
         if (never()) { dead = true; return; }
       }
     } else { if (barrier_or(dead_flag)) { dead = true; return; } }
@@ -813,12 +846,15 @@ fused_bwd_kernel(const BwdArgs a) {
     // operands of step t-1 from the producer wave's buffer (behind this step's barrier; used in the next step)
     auto take_operands = [&]() __attribute__((always_inline)) {
       if constexpr (PW) {
-      static_assert(E == 1 && ND_ == 1 && PD == 1, "4-row tiles: one element per lane and tile, one step ahead");
+      static_assert(E == 1 && ND_ == 1 && (PD == 1 || RC), "4-row tiles: one element per lane and tile, one step ahead");
       const T* const pb = pbuf + ((Tn - t) & 1) * PB;
 #pragma unroll
       for (int u = 0; u < UTW; ++u) {
         const int el = ((w * UTW + u) * TR + brow) * 16 + esub;
-        if constexpr (NC > 0) {
+        if constexpr (RC) {
+#pragma unroll
+          for (int g = 0; g < GW; ++g) pn.wx[u][g].v[0] = reinterpret_cast<const unsigned short*>(pb)[g * UT_WG * TR * 16 + el];
+        } else if constexpr (NC > 0) {
           const unsigned* const pc_ = reinterpret_cast<const unsigned*>(pb) + el * NWC;
 #pragma unroll
           for (int i = 0; i < NWC; ++i) pn.cache[u].v[i] = pc_[i];
@@ -885,7 +921,10 @@ fused_bwd_kernel(const BwdArgs a) {
 #pragma unroll
         for (int u = 0; u < UTW; ++u) la_next[rr][u] = rl[((rr * UTW + u) * KS) * 64];
     }
+    Frag hq[RCP ? KSF : 1];
+    f32x4 racc[UTW][GR];
     if constexpr (MID) {
+      if constexpr (RCP) rebuild_fetch(t - 1, hq);
       take_operands();
       if constexpr (!PST && !cut) {
         __builtin_amdgcn_sched_barrier(0);
@@ -1013,9 +1052,18 @@ fused_bwd_kernel(const BwdArgs a) {
           for (int u = 0; u < UTW; ++u)
             accp[j][r][u] = X::mfma(r < KWR ? rtf[r < KWR ? r : 0][u][ks] : la[r < KWR ? 0 : r - KWR][u], gq[kc & 1][k],
                                     ks < NACC ? f32x4{0.f, 0.f, 0.f, 0.f} : accp[j][r][u]);
+        // (one gate row of the rebuilt product per k-step: it fills the gaps of the lone chain)
+        if constexpr (RCP) {
+#pragma unroll
+          for (int u = 0; u < UTW; ++u) {
+            const int g = ks % GR, kf = ks / GR;
+            racc[u][g] = X::mfma(rfw[u][g][kf], hq[kf], kf == 0 ? (BIAS_C ? biasc[u][g] : f32x4{0.f, 0.f, 0.f, 0.f}) : racc[u][g]);
+          }
+        }
         if (j == NACC - 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
+    static_assert(!RCP || KS == GR * KSF, "the two products have the same number of instructions");
     static_assert(NACC == 1, "one accumulator per tile");
     f32x4 acc[GROUPED ? 1 : KW][UTW];
 #pragma unroll
@@ -1215,7 +1263,8 @@ fused_bwd_kernel(const BwdArgs a) {
       }
       }
     }
-    if constexpr (RC && KW == 1) {
+    if constexpr (RCP) rebuild_math(pn, racc);  // (behind step 0: of nothing, unused)
+    else if constexpr (RC && KW == 1) {
       if (t > 0) rebuild_gates(pm, t - 1);
     }
 #ifdef FRNN_TRACE
@@ -1231,6 +1280,15 @@ fused_bwd_kernel(const BwdArgs a) {
     // ring of 3 sets: step t consumes set j (its own operands) and set j+1 (those of step t-1, for the
     // rebuild) and refills set j+2 with the operands of step t-2
     auto run = [&](auto CUT) __attribute__((always_inline)) {
+      if constexpr (PW && !decltype(CUT)::value) {  // two sets: the operands of step t-1 come from LDS within step t
+        for (; t >= 1 && !dead; t -= 2) {
+          step(CUT, t, pre[0], pre[1], pre[1]);
+          if (dead) break;
+          step(CUT, t - 1, pre[1], pre[0], pre[0]);
+        }
+        if (!dead && t == 0) step(CUT, 0, pre[0], pre[1], pre[1]);
+        return;
+      }
       for (; t >= 2 && !dead; t -= 3) {
         step(CUT, t, pre[0], pre[1], pre[2]);
         if (dead) break;

@@ -92,12 +92,18 @@ constexpr bool fwd_producer_stores(int GR, int D, int WAVES, int UTW, int KW, in
 // states), for the heads that run as one workgroup: there every load of the compute waves is on the chain of dependent
 // steps, and a step (~1600 cycles) is shorter than a fetch from HBM, which their one-step prefetch therefore waits for
 // (a timing-only build without these loads runs GRU D = 128 backward 35 % faster).  The producer wave loads four steps
-// ahead and leaves the operands of the next step in LDS.  Not in recompute mode, and not for truncated backpropagation
+// ahead and leaves the operands of the next step in LDS.  Not for truncated backpropagation
 // (no barrier per step to hand over at: that variant of the step keeps its own loads).  All four cells: GRU B16 T2048
 // N4 D128 1.396 -> 1.049 ms, Elman B16 T1024 N12 D64 0.312 -> 0.261, N6 D128 0.386 -> 0.301.
+// Recompute mode: Wx in the place of the gate cache, and h_(t-1) straight into the buffer that the rebuilt product reads, so the compute
+// waves load nothing, keep two operand sets instead of three and have the registers for both operands without accumulation registers.
+// Whole backward pass, T = 256, without and with: LSTM B33 N8 D96 (fp16, T515) 609 -> 490 us, sLSTM 392 -> 285, GRU 264 -> 201; B16 N12 D64 LSTM 223 ->
+// 152, sLSTM 261 -> 165, GRU 196 -> 125; B16 N4 D32 172 -> 116, 207 -> 126, 166 -> 101; B256 N12 D64, mostly bytes, 613 -> 534, 750 -> 572, 492 ->
+// 477; B256 N24 D32 709 -> 586, 818 -> 715, 583 -> 426.  Not the GRU's 8 waves at D = 128, which have 170 registers each beside a ninth.
 constexpr bool bwd_producer_wave(int GR, int nc, int D, int WAVES, int UTW, int KW, int TR, int esize, bool rc) {
   // (nc = 5, the sLSTM: its 8-wave kernel spills at the 170 registers that nine waves leave each)
-  return esize == 2 && !rc && KW == 1 && TR == 4 && (WAVES <= 6 || (WAVES <= 8 && nc <= 4)) && UTW == 1;
+  if (rc) return esize == 2 && KW == 1 && TR == 4 && WAVES <= 6 && UTW == 1;
+  return esize == 2 && KW == 1 && TR == 4 && (WAVES <= 6 || (WAVES <= 8 && nc <= 4)) && UTW == 1;
 }
 // LDS bytes of the hand-over buffers of that wave (two steps): the gate cache (nc values per element, padded to an even
 // number), s_(t-1) and the cotangent (s states each) of the workgroup's UT_WG tiles of TR rows x 16 units, and 16

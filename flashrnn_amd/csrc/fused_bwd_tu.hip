@@ -28,7 +28,7 @@ int fused_bwd_launch<FRNN_F, FRNN_DT>(const Plan& p, const BwdArgs& a, hipStream
   const bool ds16 = sizeof(FRNN_TU_T) == 2 && bwd_dest_split(p.D, p.waves, p.utw, p.kw) > 1;
   const size_t lds = (ds16 ? (size_t)2 * 16 * Cell<FRNN_F>::GR * (p.D / p.kw) * sizeof(FRNN_TU_T)
                            : bwd_lds_bytes(Cell<FRNN_F>::GR, p.D, p.waves, p.utw, p.kw, (int)sizeof(FRNN_TU_T), rc)) + 16 +
-                     (pw ? bwd_producer_bytes(Cell<FRNN_F>::NC + (cache_carried_state(FRNN_F, (int)sizeof(FRNN_TU_T), p.D) >= 0 ? 1 : 0), Cell<FRNN_F>::S, p.waves * p.utw, a.tile_rows, (int)sizeof(FRNN_TU_T)) : 0) +
+                     (pw ? bwd_producer_bytes(rc ? Cell<FRNN_F>::GW : Cell<FRNN_F>::NC + (cache_carried_state(FRNN_F, (int)sizeof(FRNN_TU_T), p.D) >= 0 ? 1 : 0), Cell<FRNN_F>::S, p.waves * p.utw, a.tile_rows, (int)sizeof(FRNN_TU_T)) : 0) +
                      (pst ? bwd_producer_store_bytes(Cell<FRNN_F>::GW, FRNN_F == FRNN_GRU, p.D, a.tile_rows, (int)sizeof(FRNN_TU_T)) : 0);
 #define FRNN_CASE_(RCV, Dv, VAR, W, U, K, MTR)                                                          \
   if (rc == RCV && p.D == Dv && p.waves == W && p.utw == U && p.kw == K) {                               \
