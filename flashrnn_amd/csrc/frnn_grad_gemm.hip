@@ -312,14 +312,19 @@ __global__ void __launch_bounds__(64 * WD * WD) grad_gemm16_kernel(const GradGem
   gemm_sum_bias<T>(a);
 }
 
-// fp32 storage: the MFMA (16x16x4) takes the operands as they are stored, [row][unit]
+// fp32 storage: the MFMA (16x16x4) takes the operands as they are stored, [row][unit].  Bound by that instruction, 32 cycles for
+// 1024 products: LSTM B16 T1024 N1 D512 takes 301 us, 114 of the 154 TFLOP/s that a large fp32 product reaches on this card.  What got it there from
+// 353: rows that lie in different banks, 16-byte pieces, no division per stage (330 together), tiles of 128 units where they divide D (half
+// the reads per product: 311) and registers for four workgroups per compute unit, whose waves cover each other's reads and barriers (301).  Two
+// LDS buffers with one barrier per stage (+2 to +15 % at 64 units) and fragments read one step ahead (359 us) were slower.
+// (a row of 16 floats more than a multiple of 64: the four rows that a fragment read touches lie in different banks)
 template <int TM> struct GemmStage32 {
-  static constexpr int LD = TM + 4;
+  static constexpr int LD = TM + (TM % 64 == 0 ? 16 : 48);
   float a[32][LD], b[32][LD];
 };
 
 template <int TM>
-__global__ void __launch_bounds__(256) grad_gemm32_kernel(const GradGemmArgs a) {
+__global__ void __launch_bounds__(256, 4) grad_gemm32_kernel(const GradGemmArgs a) {
   typedef float T;
   typedef ST<T> X;
   constexpr int EV = TM / 8;           // elements per thread per staged row
@@ -339,10 +344,12 @@ __global__ void __launch_bounds__(256) grad_gemm32_kernel(const GradGemmArgs a) 
   const long r_end = min(rows, r_begin + a.rows_per_split);
   const size_t ND = (size_t)N * D;
 
-  const T* __restrict__ G = static_cast<const T*>(a.gsrc[g]) + (size_t)n * D + dt * TM;
+  // thread -> row rr of the stage, pieces of 4 units, 32 apart
+  const int rr = tid / 8, cc = tid % 8 * 4;
+  const T* __restrict__ G = static_cast<const T*>(a.gsrc[g]) + (size_t)n * D + dt * TM + cc;
   const long gld = a.gld[g];
-  const T* __restrict__ H = static_cast<const T*>(a.states_h) + (size_t)n * D + pt * TM;
-  const T* __restrict__ H0 = static_cast<const T*>(a.s0_h) + (size_t)n * D + pt * TM;
+  const T* __restrict__ H = static_cast<const T*>(a.states_h) + (size_t)n * D + pt * TM + cc;
+  const T* __restrict__ H0 = static_cast<const T*>(a.s0_h) + (size_t)n * D + pt * TM + cc;
 
   f32x4 acc[WT][WT];
 #pragma unroll
@@ -350,26 +357,34 @@ __global__ void __launch_bounds__(256) grad_gemm32_kernel(const GradGemmArgs a) 
 #pragma unroll
     for (int j = 0; j < WT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int rr = tid / (TM / EV), cc = (tid % (TM / EV)) * EV;
-  T ga[EV], hb[EV];
+  // this thread's row as (batch row, time step), kept up to date instead of divided out per stage (B * T < 2^31, checked on the host)
+  unsigned fb = (unsigned)(r_begin + rr) / (unsigned)Tn, ft = (unsigned)(r_begin + rr) - fb * (unsigned)Tn;
+  f32x4 ga[EV / 4], hb[EV / 4];
   auto fetch = [&](long r0) __attribute__((always_inline)) {
     const long r = r0 + rr;
-    if (r < r_end) {
-      const long b = r / Tn, t = r - b * Tn;
-      const T* gp = G + (size_t)r * gld + cc;
-      const T* hp = (t > 0) ? H + (size_t)(r - 1) * ND + cc : H0 + (size_t)b * ND + cc;
+    const bool ok = r < r_end;
+    const T* gp = G + (size_t)(ok ? r : 0) * gld;
+    const T* hp = ok && ft > 0 ? H + (size_t)(r - 1) * ND : H0 + (size_t)(ok ? fb : 0) * ND;
 #pragma unroll
-      for (int e = 0; e < EV; ++e) { ga[e] = gp[e]; hb[e] = hp[e]; }
-    } else {
-#pragma unroll
-      for (int e = 0; e < EV; ++e) { ga[e] = 0.0f; hb[e] = 0.0f; }
+    for (int e = 0; e < EV / 4; ++e) {
+      ga[e] = *reinterpret_cast<const f32x4*>(gp + 32 * e);
+      hb[e] = *reinterpret_cast<const f32x4*>(hp + 32 * e);
     }
+    if (!ok) {  // (the last stage of a split) rows beyond the end count as zero
+#pragma unroll
+      for (int e = 0; e < EV / 4; ++e) ga[e] = hb[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    ft += 32;
+    while (ft >= (unsigned)Tn) { ft -= (unsigned)Tn; ++fb; }
   };
   fetch(r_begin);
   for (long r0 = r_begin; r0 < r_end; r0 += 32) {
     __syncthreads();  // previous stage fully consumed
 #pragma unroll
-    for (int e = 0; e < EV; ++e) { sm.a[rr][cc + e] = ga[e]; sm.b[rr][cc + e] = hb[e]; }
+    for (int e = 0; e < EV / 4; ++e) {
+      *reinterpret_cast<f32x4*>(&sm.a[rr][cc + 32 * e]) = ga[e];
+      *reinterpret_cast<f32x4*>(&sm.b[rr][cc + 32 * e]) = hb[e];
+    }
     __syncthreads();
     if (r0 + 32 < r_end) fetch(r0 + 32);
 #pragma unroll
@@ -390,12 +405,12 @@ __global__ void __launch_bounds__(256) grad_gemm32_kernel(const GradGemmArgs a) 
   gemm_sum_bias<T>(a);
 }
 
-// side of the square workgroup tile: the largest of 256, 128 (16-bit types only), 64, 32 that divides D; 96 and 160
+// side of the square workgroup tile: the largest of 256 (16-bit types only), 128, 64, 32 that divides D; 96 and 160
 // (16-bit types) for the head dims that only much smaller powers of two divide: every pair of tiles of a gate streams
 // both of its operand slabs, so D = 96 as 9 pairs of 32-unit tiles took 1.30 ms at B256 T1024 N8 against 0.40 for D = 64
 static int gemm_tile_side_of(int dtype, int D) {
   if (dtype != FRNN_F32 && D % 256 == 0) return 256;
-  if (dtype != FRNN_F32 && D % 128 == 0) return 128;
+  if (D % 128 == 0) return 128;
   if (dtype != FRNN_F32 && D % 96 == 0 && D / 96 <= 2) return 96;     // 96, 192
   if (dtype != FRNN_F32 && D % 160 == 0 && D / 160 <= 3) return 160;  // 160, 320, 480
   return (D % 64 == 0) ? 64 : 32;
@@ -473,7 +488,8 @@ int launch_grad_gemm(int dtype, GradGemmArgs a, int splits, hipStream_t st) {
   const dim3 grid(a.GR * (a.D / TM) * (a.D / TM), a.N, splits);
   if (dtype == FRNN_BF16) return launch_gemm16_any<bf16_t>(TM, a, grid, st);
   if (dtype == FRNN_F16) return launch_gemm16_any<half_t>(TM, a, grid, st);
-  if (TM == 64) hipLaunchKernelGGL((grad_gemm32_kernel<64>), grid, dim3(256), 0, st, a);
+  if (TM == 128) hipLaunchKernelGGL((grad_gemm32_kernel<128>), grid, dim3(256), 0, st, a);
+  else if (TM == 64) hipLaunchKernelGGL((grad_gemm32_kernel<64>), grid, dim3(256), 0, st, a);
   else hipLaunchKernelGGL((grad_gemm32_kernel<32>), grid, dim3(256), 0, st, a);
   return (int)hipGetLastError();
 }
