@@ -891,7 +891,11 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   // 0.64 / 0.76, B64 0.48 / 0.49, B16 0.41 / 0.41; GRU N12 D64 B256 0.79 / 0.97; sLSTM N12 D64 B128 0.80 / 1.00; LSTM N24 D32
   // B256 1.22 / 1.53.  With the stores issued in front of the loads of an iteration the same kernels lost up to 25 %:
   // a wave's memory operations complete in order, and the stores are acknowledged late)
-  a.pst = env_int("FRNN_PRODUCER_STORES", tr == 4 && p.kw == 1 && 2 * groups > device_cus() ? 1 : 0);
+  // recompute mode: at any size, the compute waves have the rebuild to do meanwhile (backward pass, T = 256, compute-wave stores and producer
+  // stores: LSTM fp16 B33 T515 N8 D96 489 / 474 us, B16 N12 D64 153 / 148, B256 N24 D32 620 / 587, sLSTM B33 N8 D96 285 / 277, GRU 204 / 197), but not
+  // the GRU of 64 units (B16 N12 125 / 125, B256 N12 409 / 478)
+  const bool pst = o.rc ? !(function == FRNN_GRU && D == 64) : 2 * groups > device_cus();
+  a.pst = env_int("FRNN_PRODUCER_STORES", tr == 4 && p.kw == 1 && pst ? 1 : 0);
   a.trace = nullptr;
 #ifdef FRNN_TRACE
   a.trace = (long long*)((char*)workspace + w.zero_bytes);
