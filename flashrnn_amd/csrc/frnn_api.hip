@@ -210,6 +210,36 @@ static int groups_per_launch(int kw) { return kw > kXcdWorkgroups ? device_cus()
 // (such groups never share an XCD: no handshake, every exchange store at agent scope)
 static bool near_stores_possible(const Plan& p) { return p.kw > 1 && p.kw <= kXcdWorkgroups; }
 
+// Whether the producer wave stores the outputs of a step (forward; 16-bit heads of one workgroup at 4-row tiles): it takes them off the compute
+// waves' chain and stores 16 bytes at a time, but adds a trip through LDS to a step.  It pays from the size on where the stores
+// delay a step, sooner the more a step writes (sLSTM with cache: 10 values per element, GRU without: one).  `units`: units of
+// all workgroups.  Forward, T = 256, 24 to 1280 groups of every cell and head dim, the change from compute-wave stores to the producer's, on either side
+// of the lines: with cache LSTM D=64 192 groups +7.0 %, 288 -28 %, D=96 144 +3.2, 192 -6.7, D=32 384 +0.3, 512 -5.2; sLSTM D=64 120 -13 (T = 512),
+// D=128 96 -21, D=96 96 +0.1, 144 -30, D=32 288 +3.3, 384 -9.9; GRU D=64 232 +6.2, 288 -18, D=96 232 +1.4, 288 -12, D=32 512 -1.3.  Without: LSTM D=64
+// 232 +6.6, 288 -0.4, 384 -8.7, D=32 768 +1.3, 1280 -12, D=96 and 128 +2 to +6 up to 768; sLSTM D=64 232 -0.9, 288 -21, D=96 144 0, 192 -14;
+// GRU D=64 512 +11, 768 -1.7, D=32 768 +0.5, 1280 -15, D=96 and 128 +4 to +9.
+static bool fwd_producer_stores_pay(int function, const Plan& p, int groups, int cached) {
+  const long cus = device_cus(), units = (long)groups * p.D;
+  if (function == FRNN_SLSTM) return units > (!cached ? 56 : p.waves <= 2 ? 40 : 28) * cus;
+  if (function == FRNN_LSTM) return cached ? units > 56 * cus : p.waves <= 4 && groups > (p.waves <= 2 ? 4 : 1) * cus;
+  return cached ? groups > cus && units >= 64 * cus : p.waves <= 4 && units > 128 * cus;
+}
+// The same for dWx in the reverse kernel (D = 32, 64 and 96).  Reverse pass, as above: LSTM D=64 192 groups +4.1, 232 +5.2, 288 -20 %, D=96 -1 to -5 at every
+// size, D=32 288 +1.7, 384 -2.7, 768 -11; sLSTM D=64 144 +1.2, 288 -23, D=96 -1 to -10 and D=32 -1 to -9 at every size; GRU D=64 232 +8.9, 288 -20, D=96 232
+// +1.8, 288 -16, D=32 512 +4.0, 768 -14; Elman, one value per element, D=32 +3.5 to +19 up to 1280, D=64 768 +4.5, 1280 -15, D=96 512 +4.8, 768 -11.
+// (With the stores issued in front of the loads of an iteration the same kernels lost up to 25 %: a wave's memory operations complete in
+// order, and the stores are acknowledged late.)  Recompute mode: at any size, the compute waves have the rebuild to do meanwhile (backward
+// pass, T = 256, compute-wave stores and producer stores: LSTM fp16 B33 T515 N8 D96 489 / 474 us, B16 N12 D64 153 / 148, B256 N24 D32 620 / 587, sLSTM B33 N8
+// D96 285 / 277, GRU 204 / 197), but not the GRU of 64 units (B16 N12 125 / 125, B256 N12 409 / 478).
+static bool bwd_producer_stores_pay(int function, const Plan& p, int groups, bool rc) {
+  const long cus = device_cus(), units = (long)groups * p.D;
+  if (rc) return !(function == FRNN_GRU && p.D == 64);
+  if (function == FRNN_ELMAN || function == FRNN_ELMAN_CLIP) return units > 256 * cus;
+  if (p.waves > 4 && function != FRNN_GRU) return true;
+  if (p.waves <= 2 && function != FRNN_LSTM) return function == FRNN_SLSTM || groups > 2 * cus;
+  return groups > cus;
+}
+
 // The tiling of a call: the table's default for the head dim, or the widest of its small-batch alternatives (variant 3, else 2) for
 // which all groups of the call fit one launch with 4-row tiles (not where FRNN_TILE_ROWS asks for taller tiles than it has).
 // FRNN_FUSED_VARIANT picks a variant by hand.
@@ -745,11 +775,8 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   a.poll_delay = env_int("FRNN_POLL_DELAY", fwd_poll_delay_default(fx, dtype, p, tr));
   a.h_clip = o.h_clip;
   a.mailbox = nullptr; a.inbox_off = a.outbox_off = a.in_slot = a.out_slot = 0; a.slots = 1; a.idle_limit = 0;
-  // producer-wave stores: for launches that put some load on the memory system (measured, bf16 T = 1024, forward kernel
-  // with the producer wave storing against the compute lanes storing: LSTM N12 D64 B256 0.82 against 1.03 ms, B128 0.50 / 0.65,
-  // B64 0.38 / 0.38, B16 0.30 / 0.295; sLSTM N12 D64 B128 0.68 / 0.97; GRU N12 D64 B256 0.66 / 0.78; LSTM N24 D32 B256
-  // 1.11 / 1.33); FRNN_PRODUCER_STORES=0/1 overrides
-  a.pst = step ? 0 : env_int("FRNN_PRODUCER_STORES", tr == 4 && p.kw == 1 && 2 * groups > device_cus() ? 1 : 0);
+  // (FRNN_PRODUCER_STORES=0/1 overrides)
+  a.pst = step ? 0 : env_int("FRNN_PRODUCER_STORES", tr == 4 && p.kw == 1 && fwd_producer_stores_pay(fx, p, groups, a.training) ? 1 : 0);
   a.trace = nullptr;
 #ifdef FRNN_TRACE
   a.trace = (long long*)((char*)workspace + w.zero_bytes);
@@ -887,15 +914,7 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
                        : p.kw <= 4 ? 0 : p.kw < 10 ? 2 : p.kw <= 16 ? 4 : p.kw <= 28 ? 6 : 2;
   a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", o.rc ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && dsp == 1 && tr == 4 || half && p.kw >= 32 ? 0 : p.kw == 40 ? 14 : wide_delay);
   a.g_clip = o.g_clip; a.cut = o.cut;
-  // producer-wave stores of dWx, under the same condition (reverse kernel: LSTM N12 D64 B256 1.16 against 1.26 ms, B128
-  // 0.64 / 0.76, B64 0.48 / 0.49, B16 0.41 / 0.41; GRU N12 D64 B256 0.79 / 0.97; sLSTM N12 D64 B128 0.80 / 1.00; LSTM N24 D32
-  // B256 1.22 / 1.53.  With the stores issued in front of the loads of an iteration the same kernels lost up to 25 %:
-  // a wave's memory operations complete in order, and the stores are acknowledged late)
-  // recompute mode: at any size, the compute waves have the rebuild to do meanwhile (backward pass, T = 256, compute-wave stores and producer
-  // stores: LSTM fp16 B33 T515 N8 D96 489 / 474 us, B16 N12 D64 153 / 148, B256 N24 D32 620 / 587, sLSTM B33 N8 D96 285 / 277, GRU 204 / 197), but not
-  // the GRU of 64 units (B16 N12 125 / 125, B256 N12 409 / 478)
-  const bool pst = o.rc ? !(function == FRNN_GRU && D == 64) : 2 * groups > device_cus();
-  a.pst = env_int("FRNN_PRODUCER_STORES", tr == 4 && p.kw == 1 && pst ? 1 : 0);
+  a.pst = env_int("FRNN_PRODUCER_STORES", tr == 4 && p.kw == 1 && bwd_producer_stores_pay(fx, p, groups, o.rc) ? 1 : 0);
   a.trace = nullptr;
 #ifdef FRNN_TRACE
   a.trace = (long long*)((char*)workspace + w.zero_bytes);
