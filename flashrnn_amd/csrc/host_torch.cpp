@@ -361,7 +361,7 @@ PYBIND11_MODULE(_host, m) {
     ring().take({kind, function, B, T, N, D}, reinterpret_cast<void*>(stream), o);
     return std::make_pair(reinterpret_cast<uintptr_t>(o.report), reinterpret_cast<uintptr_t>(o.report_any));
   });
-  m.def("status_poll", [](bool wait, uintptr_t stream) { ring().poll(wait, reinterpret_cast<void*>(stream)); }, py::call_guard<py::gil_scoped_release>());
+  m.def("status_poll", [](bool wait) { ring().poll(wait, c10::hip::getCurrentHIPStream().stream()); }, py::call_guard<py::gil_scoped_release>());
   m.def("status_last", [](int kind) { return ring().last_word(kind); }, py::call_guard<py::gil_scoped_release>());
   m.def("status_drain", []() {
     api.wait_launches();

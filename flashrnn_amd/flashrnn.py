@@ -201,7 +201,7 @@ class _StatusLog:
 
     def poll(self, wait: bool = False):
         if torch.cuda.is_initialized():
-            _lib.load_host().status_poll(wait, torch.cuda.current_stream().cuda_stream)
+            _lib.load_host().status_poll(wait)
 
     def last(self, kind: str) -> int:
         return _lib.load_host().status_last(int(kind == "backward"))

@@ -110,6 +110,22 @@ def test_autograd_meets_the_function_it_knows(gpu):
 
 
 @pytest.mark.gpu
+def test_compiled_caller(gpu):
+    """torch.compile of a caller: its graph breaks at the call, which takes the Python path."""
+    from flashrnn_amd import flashrnn
+
+    print("case host path compiled caller", flush=True)
+    leaves = _leaves(gpu)
+
+    def loss(*x):
+        return flashrnn(*x)[0].float().square().sum()
+
+    ref = torch.autograd.grad(loss(*leaves), leaves)
+    got = torch.autograd.grad(torch.compile(loss, backend="eager")(*leaves), leaves)
+    assert all(torch.equal(x, y) for x, y in zip(ref, got))
+
+
+@pytest.mark.gpu
 def test_threads_share_the_record_of_failed_waits(gpu):
     import threading
 
