@@ -13,6 +13,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <atomic>
+#include <cstring>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -181,6 +182,23 @@ CallPtr make_call(int function, int dtype, bool fused, double h_clip, double g_c
   return c;
 }
 
+// what the reverse pass needs of it, as whole numbers: an autograd node's record has to be hashable (compiled autograd keys its graphs by it)
+c10::List<int64_t> pack(const Call& c) {
+  int32_t h, g;
+  std::memcpy(&h, &c.o.forward_clipval, 4); std::memcpy(&g, &c.o.gradient_recurrent_clipval, 4);
+  return c10::List<int64_t>({c.function, c.dtype, c.fused, h, g, c.o.gradient_recurrent_cut, c.o.recompute, c.o.weight_grads});
+}
+Call unpack(const std::vector<int64_t>& p) {
+  Call c;
+  c.function = (int)p.at(0); c.dtype = (int)p.at(1); c.fused = p.at(2) != 0; c.amp = c.training = true;
+  c.o = frnn_options{};
+  c.o.struct_size = sizeof(frnn_options);
+  const int32_t h = (int32_t)p.at(3), g = (int32_t)p.at(4);
+  std::memcpy(&c.o.forward_clipval, &h, 4); std::memcpy(&c.o.gradient_recurrent_clipval, &g, 4);
+  c.o.gradient_recurrent_cut = (int)p.at(5); c.o.recompute = (int)p.at(6); c.o.weight_grads = (int)p.at(7);
+  return c;
+}
+
 Tensor cast(const Tensor& x, const char* name, const Call& c) {
   const auto k = kernel_type(c.dtype);
   TORCH_CHECK_TYPE(c.amp || x.scalar_type() == k, name, " is ", x.scalar_type(), ", the kernel type is ", k,
@@ -220,20 +238,20 @@ Saved run_forward(const Tensor& Wx_, const Tensor& R_, const Tensor& b_, const T
 struct Function : torch::autograd::Function<Function> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& Wx, const Tensor& R, const Tensor& b, const Tensor& s0, CallPtr c) {
     Saved v = run_forward(Wx, R, b, s0, *c);
-    ctx->saved_data["call"] = c10::IValue::make_capsule(c);
+    ctx->saved_data["call"] = pack(*c);
     // (recompute mode reads Wx again in the backward pass; it is the caller's tensor unless it was cast)
     ctx->save_for_backward({v.R, v.b, v.s0, v.states, v.cache, c->o.recompute ? v.Wx : v.cache});
     return v.states;
   }
 
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
-    const auto c = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
+    const Call c = unpack(ctx->saved_data["call"].toIntVector());
     const auto v = ctx->get_saved_variables();
     const bool again = torch::GradMode::is_enabled() && grads[0].requires_grad();
     torch::autograd::variable_list out;
     {
       torch::NoGradGuard no_grad;
-      out = run(*c, v, grads[0]);
+      out = run(c, v, grads[0]);
     }
     if (again) {  // the reverse scan is not differentiable: an error where a second derivative is asked for, not a silent zero
       auto err = std::make_shared<torch::autograd::DelayedError>(

@@ -126,6 +126,21 @@ def test_compiled_caller(gpu):
 
 
 @pytest.mark.gpu
+def test_compiled_autograd(gpu):
+    from flashrnn_amd import FlashRNNConfig, flashrnn
+
+    print("case host path compiled autograd", flush=True)
+    for options in ({}, {"gradient_recurrent_clipval": 0.25, "recompute_gates": True}):
+        cfg = FlashRNNConfig(head_dim=64, num_heads=2, **options)
+        leaves = _leaves(gpu)
+        ref = torch.autograd.grad(flashrnn(*leaves, config=cfg)[0].float().square().sum(), leaves)
+        value = flashrnn(*leaves, config=cfg)[0].float().square().sum()
+        with torch._dynamo.compiled_autograd._enable(torch.compile(backend="eager")):
+            value.backward()
+        assert all(torch.equal(x, y.grad) for x, y in zip(ref, leaves))
+
+
+@pytest.mark.gpu
 def test_threads_share_the_record_of_failed_waits(gpu):
     import threading
 
