@@ -705,18 +705,13 @@ fused_fwd_kernel(const FwdArgs a) {
 #pragma unroll
         for (int g = 0; g < GW; ++g) wx[g] = wxv[g][e];
         if constexpr (CXS >= 0) cc[NC] = s[u][e][CXS];  // (before the step overwrites it)
-        CM::fwd(ry, wx, bx[u][e], s[u][e], cc);
+        float mix[3];
+        CM::fwd(ry, wx, bx[u][e], s[u][e], cc, mix);
         s[u][e][0] = clamp_if(s[u][e][0], a.h_clip);
-        // (fp16: the states are rounded to fp32 first.  Left alone, some kernels round product and conversion at once
-        // (v_fma_mixlo_f16), and 4e-5 of their states differ in the last bit from those of a single step)
-        if constexpr (X::ID == FRNN_F16) {
-#pragma unroll
-          for (int k = 0; k < S; ++k) asm("" : "+v"(s[u][e][k]));
-        }
 #pragma unroll
         for (int c = 0; c < NCX; ++c) cv[c][e] = cc[c];
 #pragma unroll
-        for (int k = 0; k < S; ++k) so[k][e] = s[u][e][k];
+        for (int k = 0; k < S; ++k) so[k][e] = X::ID == FRNN_F16 && k == CM::ONCE ? fma_f16(mix) : s[u][e][k];
       }
       // the new h first: it is what the next step (of every workgroup of the head) waits for
       // (the own slice goes straight to the LDS buffer of the next step: the workgroup does not poll it)

@@ -44,20 +44,32 @@ __device__ __forceinline__ float mul(float a, float b) {
 // fwd:  ry[GR] recurrent pre-activations WITH the bias of their gate slot already added (the
 //       fused kernels fold it into the MFMA accumulator), wx[GW], bx = biases of the gate slots
 //       that have no recurrent input (gru: the n gate), s[S] in/out, cache[NC] out
+//       ONCE: the state that is a sum of products a * b + c (or -1); mix[3] = {a, b, c} where the caller asks for them
 // bwd:  cache[NC], sp[S] = s_{t-1}, sn[S] = s_t, dso[S] upstream cotangent of s_t,
 //       ds[S] in: running cotangent arriving from step t+1; out: cotangent for s_{t-1}
 //       WITHOUT the recurrent term R^T dgr (the caller adds it to ds[0]);
 //       dgr[GR] / dgw[GW] / dgb[GT]: cotangents of the R-side, Wx-side and bias pre-activations.
 template <int F, bool FAST> struct CellMath;
 
+// A state a * b + c as it is stored in fp16: rounded once, from the exact sum.  Through the fp32 state it would be rounded twice, and
+// 4e-5 of the stored values would be the farther of their two neighbours.  Written out because the compiler does it by
+// itself in most kernels but not in all, and every kernel has to store the same bits.
+__device__ __forceinline__ float fma_f16(const float* mix) {
+  half_t h;
+  asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(h) : "v"(mix[0]), "v"(mix[1]), "v"(mix[2]));
+  return (float)h;
+}
+
 template <bool FAST> struct CellMath<FRNN_LSTM, FAST> {
   typedef Math<FAST> M;
-  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float* cache) {
+  static constexpr int ONCE = 1;
+  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float* cache, float* mix = nullptr) {
     const float i = M::sigmoid(wx[0] + ry[0]);
     const float f = M::sigmoid(wx[1] + ry[1]);
     const float z = M::tanh(wx[2] + ry[2]);
     const float o = M::sigmoid(wx[3] + ry[3]);
-    const float c = __builtin_fmaf(i, z, mul(f, s[1]));
+    const float fc = mul(f, s[1]), c = __builtin_fmaf(i, z, fc);
+    if (mix) { mix[0] = i; mix[1] = z; mix[2] = fc; }
     s[1] = c;
     s[0] = mul(o, M::tanh(c));
     cache[0] = i; cache[1] = f; cache[2] = z; cache[3] = o;
@@ -81,7 +93,8 @@ template <bool FAST> struct CellMath<FRNN_LSTM, FAST> {
 
 template <bool FAST> struct CellMath<FRNN_SLSTM, FAST> {
   typedef Math<FAST> M;
-  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float* cache) {
+  static constexpr int ONCE = 1;
+  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float* cache, float* mix = nullptr) {
     const float ir = wx[0] + ry[0];
     const float fr = wx[1] + ry[1];
     const float z = M::tanh(wx[2] + ry[2]);
@@ -92,7 +105,8 @@ template <bool FAST> struct CellMath<FRNN_SLSTM, FAST> {
     const float mn = (s[2] == 0.0f) ? ir : fmaxf(ir, lfm);
     const float ig = M::exp(ir - mn);
     const float fg = M::exp(lfm - mn);
-    const float c = __builtin_fmaf(ig, z, mul(fg, s[1]));
+    const float fc = mul(fg, s[1]), c = __builtin_fmaf(ig, z, fc);
+    if (mix) { mix[0] = ig; mix[1] = z; mix[2] = fc; }
     const float n = fmaxf(__builtin_fmaf(fg, s[2], ig), 1.0f);
     s[0] = mul(mul(o, c), M::rcp(n));
     s[1] = c; s[2] = n; s[3] = mn;
@@ -118,8 +132,9 @@ template <bool FAST> struct CellMath<FRNN_SLSTM, FAST> {
 
 template <bool FAST> struct CellMath<FRNN_GRU, FAST> {
   typedef Math<FAST> M;
+  static constexpr int ONCE = -1;
   // R gates [g, r, z]; Wx gates [r, z, n]; bias gates [g, r, z, n]
-  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float* cache) {
+  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float* cache, float* = nullptr) {
     const float g = ry[0];
     const float r = M::sigmoid(wx[0] + ry[1]);
     const float z = M::sigmoid(wx[1] + ry[2]);
@@ -144,7 +159,8 @@ template <bool FAST> struct CellMath<FRNN_GRU, FAST> {
 
 template <bool FAST> struct CellMath<FRNN_ELMAN, FAST> {
   typedef Math<FAST> M;
-  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float*) {
+  static constexpr int ONCE = -1;
+  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float*, float* = nullptr) {
     s[0] = M::tanh(wx[0] + ry[0]);
   }
   static __device__ __forceinline__ void bwd(const float*, const float*, const float* sn, const float* dso,
@@ -159,7 +175,8 @@ template <bool FAST> struct CellMath<FRNN_ELMAN, FAST> {
 // Elman under forward_clipval: cache[0] is the unclamped tanh (the caller clamps s[0] after fwd)
 template <bool FAST> struct CellMath<FRNN_ELMAN_CLIP, FAST> {
   typedef Math<FAST> M;
-  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float* cache) {
+  static constexpr int ONCE = -1;
+  static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float* cache, float* = nullptr) {
     s[0] = M::tanh(wx[0] + ry[0]);
     cache[0] = s[0];
   }

@@ -113,11 +113,13 @@ __global__ void __launch_bounds__(256) fused_step_kernel(const StepArgs a) {
 #pragma unroll
     for (int g = 0; g < GR; ++g) ry[g] += bo[g];
   }
-  CM::fwd(ry, wx, bx, s, cc);
+  float mix[3];
+  CM::fwd(ry, wx, bx, s, cc, mix);
   s[0] = clamp_if(s[0], a.h_clip);
 #pragma unroll
   for (int k = 0; k < S; ++k) {
-    const Dw<1> v = pack<1>(&s[k], (T*)0);
+    const float so = X::ID == FRNN_F16 && k == CM::ONCE ? fma_f16(mix) : s[k];
+    const Dw<1> v = pack<1>(&so, (T*)0);
     reinterpret_cast<unsigned short*>(states)[((size_t)k * BS + b) * ND + idx] = (unsigned short)v.v[0];
     if (a.carry) a.carry[((size_t)k * B + b) * ND + idx] = s[k];
   }
