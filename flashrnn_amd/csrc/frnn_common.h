@@ -365,26 +365,27 @@ __device__ __forceinline__ unsigned ll_payload(half_t*, u64 w) { return ll_paylo
 __device__ __forceinline__ unsigned ll_payload(float*, u64 w) { return (unsigned)w; }
 
 // Partial sums of the backward exchange.  fp32 storage: (tag32 << 32 | f32 bits) as above.  16-bit
-// storage: one 32-bit word (tag8 << 24 | the sum rounded to sign, 8 exponent and 15 mantissa bits):
-// the operands of the sum carry 8 or 11 mantissa bits, and the exchange costs by the byte (measured:
-// -18 % per step against 8-byte words).  Tag of step t is never 0 and differs from that of step
-// t +- 2, the only older content a slot can hold.
+// storage: one 32-bit word (tag2 << 30 | the sum rounded to sign, 8 exponent and 21 mantissa bits): the exchange costs by
+// the byte (measured: -18 % per step against 8-byte words), and a tag needs no more than to tell step t from what a slot can
+// hold beside it, which is zero or the words of step t + 2 (every wave of the group has read those before anyone sends for step t).
+// So the sum keeps all but two of its bits: rounded to 15 mantissa bits under a tag of 8, the sums of the spread
+// tilings, twice to four times as many per element, lost more than those of the tilings that they stand in for.
 struct Part64 { typedef u64 Word; };
 struct Part32 { typedef unsigned Word; };
 __device__ __forceinline__ u64 part_pack(Part64*, float a, int t) { return (u64)__float_as_uint(a) | ((u64)(unsigned)(t + 1) << 32); }
 template <> struct TagMask<Part64> { static constexpr unsigned value = 0xffffffffu; };
 __device__ __forceinline__ unsigned ll_diff(Part64*, u64 w, int t) { return (unsigned)(w >> 32) ^ (unsigned)(t + 1); }
 __device__ __forceinline__ float part_value(Part64*, u64 w) { return __uint_as_float((unsigned)w); }
-__device__ __forceinline__ unsigned tag8(int t) { return (unsigned)(t % 255) + 1u; }
+__device__ __forceinline__ unsigned tag2(int t) { return ((unsigned)t >> 1) % 3u + 1u; }  // (a slot serves the steps of one parity)
 __device__ __forceinline__ unsigned part_pack(Part32*, float a, int t) {
-  // round to nearest on the 8 dropped bits; a NaN is left as it is (the rounding add would carry a large
+  // round to nearest on the 2 dropped bits; a NaN is left as it is (the rounding add would carry a large
   // NaN payload out of the word and turn the NaN into a zero)
   const unsigned bits = __float_as_uint(a);
-  return (tag8(t) << 24) | ((a != a ? bits : bits + 0x80u) >> 8);
+  return (tag2(t) << 30) | ((a != a ? bits : bits + 2u) >> 2);
 }
-template <> struct TagMask<Part32> { static constexpr unsigned value = 0xff000000u; };
-__device__ __forceinline__ unsigned ll_diff(Part32*, unsigned w, int t) { return w ^ (tag8(t) << 24); }
-__device__ __forceinline__ float part_value(Part32*, unsigned w) { return __uint_as_float(w << 8); }
+template <> struct TagMask<Part32> { static constexpr unsigned value = 0xc0000000u; };
+__device__ __forceinline__ unsigned ll_diff(Part32*, unsigned w, int t) { return w ^ (tag2(t) << 30); }
+__device__ __forceinline__ float part_value(Part32*, unsigned w) { return __uint_as_float(w << 2); }
 __device__ __forceinline__ unsigned ll_load(const unsigned* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -46,3 +46,33 @@ def test_fp16_cell_states_are_rounded_once(gpu, function, D, B):
     with torch.no_grad():
         seq, _ = flashrnn(wx(60000.0), R, b, s0, function=function, dtype="float16")
     assert torch.equal(seq[1, :, 0], want)
+
+
+@pytest.mark.parametrize("variant", ["", "1"])  # the tiling of a small call and the default one
+@pytest.mark.parametrize("function,B,N,D", [("lstm", 16, 4, 256), ("lstm", 16, 2, 512), ("slstm", 16, 3, 320), ("lstm", 16, 2, 768), ("slstm", 16, 2, 192)])
+def test_partial_sums_between_workgroups_keep_their_bits(gpu, monkeypatch, function, B, N, D, variant):
+    """ds0 of h is R^T dg, and dg is what dWx holds (the product takes it rounded).  fp32 sums of 4 D products are off by about sqrt(4 D)
+    2^-25 of the result, 2^-20 here, so about 2^-20 / 2^-11 = 0.2 % of them round to the farther of two fp16 values; if the workgroups' shares are
+    rounded to 15 mantissa bits on their way, 3 % do."""
+    from flashrnn_amd import flashrnn
+
+    print(f"case partial sums {function} B{B} N{N} D{D} variant={variant}", flush=True)
+    if variant:
+        monkeypatch.setenv("FRNN_FUSED_VARIANT", variant)
+    S = 2 if function == "lstm" else 4
+    gen = torch.Generator().manual_seed(85)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(gpu, torch.float16)
+    Wx, b, ds = mk(B, 1, 4, N, D).requires_grad_(True), mk(4, N, D) * 0.1, mk(S, B, 1, N, D)
+    R = (mk(4, N, D, D).float() / D ** 0.5).half()
+    s0 = mk(S, B, 1, N, D)
+    if function == "slstm":
+        s0[2] = s0[2].abs() + 1
+    s0.requires_grad_(True)
+    out, _ = flashrnn(Wx, R, b, s0, function=function, dtype="float16")
+    dwx, ds0 = torch.autograd.grad(out, [Wx, s0], grad_outputs=ds)
+    dg = dwx[:, 0].double().permute(1, 2, 0, 3).contiguous()             # [4, N, B, D]
+    want = torch.matmul(dg, R.double()).sum(0).transpose(0, 1)            # sum over gates and rows of R[g, n, row, col]
+    want = torch.from_numpy(want.cpu().numpy().astype("float16")).to(gpu)
+    wrong = float((ds0[0, :, 0] != want).float().mean())
+    print(f"rounded to the other neighbour: {wrong:.5f}", flush=True)
+    assert wrong < 5e-3
