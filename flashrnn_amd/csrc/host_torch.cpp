@@ -300,6 +300,11 @@ std::string shape(const Tensor& x) {  // as Python prints a tuple
   return s + (x.dim() == 1 ? ",)" : ")");
 }
 
+// (before anything is launched: a kernel that is handed memory of another device faults)
+void check_device(const char* name, const Tensor& x, const Tensor& Wx) {
+  TORCH_CHECK(x.device() == Wx.device(), "flashrnn_amd: ", name, " is on ", x.device(), ", Wx on ", Wx.device());
+}
+
 // flashrnn() on tensors in the kernels' layouts; None where the call needs the general path (two heads per head of 32 units,
 // ranges of the batch).
 py::object call(const Tensor& Wx, const Tensor& R, const Tensor& b, const std::optional<Tensor>& states, int function, int dtype, bool fused,
@@ -312,6 +317,8 @@ py::object call(const Tensor& Wx, const Tensor& R, const Tensor& b, const std::o
   TORCH_CHECK_VALUE(!states || states->sizes() == torch::IntArrayRef({S, B, 1, N, D}), "states must be [", S, ",", B, ",1,", N, ",", D, "], got ",
                     states ? shape(*states) : "");
   if (D == 16 || !Wx.is_cuda() || (rc && !fused) || B > INT_MAX || T > INT_MAX || N > INT_MAX || D > INT_MAX) return py::none();
+  check_device("R", R, Wx); check_device("b", b, Wx);
+  if (states) check_device("states", *states, Wx);
   auto c = make_call(function, dtype, fused, h_clip, g_clip, cut, rc, amp);
   c->training = torch::GradMode::is_enabled() &&
                 (Wx.requires_grad() || R.requires_grad() || b.requires_grad() || (states && states->requires_grad()));
@@ -352,6 +359,7 @@ Tensor step(const Tensor& Wx, const Tensor& R, const Tensor& b, const Tensor& st
   const std::pair<const char*, const Tensor&> in[] = {{"Wx", Wx}, {"R", R}, {"b", b}, {"states", states}};
   for (const auto& [name, x] : in) {
     TORCH_CHECK(x.is_cuda(), "flashrnn_amd runs on a GPU only (got a CPU tensor); there is no CPU fallback");
+    check_device(name, x, Wx);
     TORCH_CHECK_TYPE(x.scalar_type() == k && x.is_contiguous(), name, " must be a contiguous ", k, " tensor (the step path casts and copies nothing)");
   }
   TORCH_CHECK_TYPE(!carry || (carry->scalar_type() == torch::kFloat && carry->sizes() == torch::IntArrayRef({S, B, N, D}) &&

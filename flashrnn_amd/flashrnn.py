@@ -292,10 +292,18 @@ def fused_plan(function: str, dtype: str, B: int, N: int, D: int, backward: bool
     return tuple(o.value for o in out)
 
 
+def _check_device(device: torch.device, **tensors) -> None:
+    """Before anything is launched: a kernel that is handed memory of another device faults."""
+    for name, x in tensors.items():
+        if x.device != device:
+            raise RuntimeError(f"flashrnn_amd: {name} is on {x.device}, the call runs on {device}")
+
+
 def _cast_inputs(Wx, R, b, s0, cfg: FlashRNNConfig):
     """The inputs in the kernel type and the kernels' layouts, as the reference's custom_fwd(cast_inputs=...) does
     (flashrnn.py:690-695); s0 comes back as [S,B,N,D]."""
     kdt = DTYPE_DICT[cfg.dtype]
+    _check_device(Wx.device, R=R, b=b, states=s0)
     if not cfg.enable_automatic_mixed_precision:
         for name, x in (("Wx", Wx), ("R", R), ("b", b), ("states", s0)):
             if x.dtype != kdt:
@@ -682,6 +690,7 @@ class FlashRNNDecoder:
                 raise RuntimeError("flashrnn_amd runs on a GPU only (got a CPU tensor); there is no CPU fallback")
             if x.dtype != kdt or not x.is_contiguous():
                 raise TypeError(f"{name} must be a contiguous {kdt} tensor (the decode path casts and copies nothing)")
+        _check_device(states.device, R=R, b=b)
         self.config, self.function, self.kdt = config, function, kdt
         self.B, self.N, self.D, self.S, self.Gw, self.slots = B, N, D, S, Gw, slots
         self.device = states.device
@@ -721,8 +730,9 @@ class FlashRNNDecoder:
         with _on_device(self.device):
             if out is None:
                 out = torch.empty((self.S, self.B, C, self.N, self.D), dtype=self.kdt, device=self.device)
-            elif tuple(out.shape) != (self.S, self.B, C, self.N, self.D) or out.dtype != self.kdt or not out.is_contiguous():
-                raise TypeError(f"out must be a contiguous {self.kdt} tensor [{self.S},{self.B},{C},{self.N},{self.D}]")
+            elif (tuple(out.shape) != (self.S, self.B, C, self.N, self.D) or out.dtype != self.kdt or not out.is_contiguous()
+                  or out.device != self.device):
+                raise TypeError(f"out must be a contiguous {self.kdt} tensor [{self.S},{self.B},{C},{self.N},{self.D}] on {self.device}")
             rc = _lib.load_library().frnn_fused_decode_step(*self._ids, C, Wx.data_ptr(), out.data_ptr(), self.mailbox.data_ptr(),
                                                             self.mailbox.numel(), self.slots, _raw_stream(self.device))
             if rc != 0:

@@ -184,3 +184,37 @@ def test_a_failed_wait_is_named_behind_more_calls_than_the_ring_holds(gpu, monke
         flashrnn(*x)
     check_status()
     assert last_status("forward") == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["R", "b", "states"])
+def test_tensors_of_another_device_are_refused_on_the_host(gpu, monkeypatch, name):
+    """Weights or a state left on the CPU: an error before anything is launched, on every path."""
+    from flashrnn_amd import FlashRNNConfig, FlashRNNDecoder, flashrnn, flashrnn_step
+
+    print(f"case host path device {name}", flush=True)
+
+    def inputs(D, T=4):
+        x = dict(zip(("Wx", "R", "b", "states"), (v.detach() for v in _leaves(gpu, D=D, T=T))))
+        x[name] = x[name].cpu()
+        return x
+
+    refused = pytest.raises(RuntimeError, match="is on cpu|got a CPU tensor")
+    for D in (64, 16):  # (two heads of 16 units run as one)
+        with refused:
+            flashrnn(**inputs(D))
+    x = inputs(64)
+    with _Mode(), refused:
+        flashrnn(**x)
+    x["Wx"].requires_grad_()
+    with refused:
+        flashrnn(**x)
+    with refused:
+        flashrnn(**inputs(64), config=FlashRNNConfig(head_dim=64, num_heads=2, backend="hip"))
+    with refused:
+        flashrnn_step(**inputs(64, T=1))
+    with refused:
+        FlashRNNDecoder(*[inputs(64)[k] for k in ("R", "b", "states")])
+    monkeypatch.setenv("FRNN_TEST_MAX_BATCH", "2")  # (ranges of the batch)
+    with refused:
+        flashrnn(**inputs(64))
