@@ -16,6 +16,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/flashrnn_hip.h"
@@ -73,70 +74,112 @@ void check_rc(int rc, bool fused, const char* what) {
 // ---- failed waits -------------------------------------------------------------------------------------------------
 // A fused kernel whose bounded wait between workgroups ran out fills its outputs with NaN and sets the status word of its
 // workspace.  It also sets two words of pinned host memory that the call was given (frnn_options.report / report_any): one that
-// belongs to the call, in a ring of kSlots, and one that all calls share.  So nothing is copied or recorded per call: a later call
+// belongs to the call, out of kSlots, and one that all calls share.  So nothing is copied or recorded per call: a later call
 // reads the shared word, and only where it is set looks for the calls that set theirs, once the launches so far have ended.
-// A slot is used again after kSlots calls; the ring first waits for the launches so far there.
+// A word belongs to its call until the call's launches are known to have ended: when none is free, a call waits for what
+// was launched so far and frees those words, reading them as it does.  The words of calls that were not launched yet
+// (another thread, between take and the launch) stay theirs.
 constexpr int kSlots = 4096;
 const char* const kNames[4] = {"lstm", "slstm", "gru", "elman"};
 struct CallInfo { int kind, function, B, T, N, D; };
 struct StatusRing {
+  enum State : char { kFree, kTaken, kLaunched };
+  struct Slot { CallInfo call; State state = kFree; bool reported = false; long id = -1; };
   std::mutex mu;
   Tensor words;              // pinned: [kSlots] and the shared word
   std::atomic<int*> base{nullptr};  // its memory, for threads that look at the shared word without holding mu
-  std::vector<CallInfo> info;
+  std::vector<Slot> slots;
+  std::vector<int> free_slots;
   long taken = 0;
-  long last[2] = {-1, -1};   // the most recent call of each kind (forward, backward)
-  std::vector<std::string> older;  // failed calls whose slots were used again before anyone asked
+  struct { int slot = -1; long id = -1; int failed = 0; } last[2];  // the most recent call of each kind; failed: once its word is another call's
+  std::vector<std::string> found;  // failed calls whose words were freed before anyone asked
+
+  // a call's word, from take to behind its launches
+  struct Ticket {
+    StatusRing* ring = nullptr;
+    int slot = -1;
+    Ticket() = default;
+    Ticket(Ticket&& o) : ring(o.ring), slot(o.slot) { o.slot = -1; }
+    ~Ticket() { if (slot >= 0) ring->launched(slot); }
+  };
 
   volatile int* any() {
     int* const w = base.load(std::memory_order_acquire);
     return w ? w + kSlots : nullptr;
   }
   // the words of a call on `stream`; calls under capture are not recorded: a replay repeats the kernels, not this
-  void take(const CallInfo& c, void* stream, frnn_options& o) {
+  Ticket take(const CallInfo& c, void* stream, frnn_options& o) {
+    Ticket t;
     o.report = o.report_any = nullptr;
-    if (api.stream_capturing(stream)) return;
-    std::lock_guard<std::mutex> lk(mu);
+    if (api.stream_capturing(stream)) return t;
+    std::unique_lock<std::mutex> lk(mu);
     if (!words.defined()) {
       words = torch::zeros({kSlots + 1}, torch::TensorOptions().dtype(torch::kInt).pinned_memory(true));
-      info.resize(kSlots);
+      slots.assign(kSlots, Slot{});
+      for (int i = kSlots - 1; i >= 0; --i) free_slots.push_back(i);
       base.store(words.data_ptr<int>(), std::memory_order_release);
     }
-    const long s = taken++;
-    if (s >= kSlots && s % kSlots == 0) {
-      api.wait_launches();
-      gather(older);
-      *any() = older.empty() ? 0 : 1;
-      for (int i = 0; i < kSlots; ++i) words.data_ptr<int>()[i] = 0;
+    while (free_slots.empty()) {  // (again where other threads took them all meanwhile)
+      const auto ended = wait_for_launched(lk);
+      if (!words.defined()) return t;  // (drained meanwhile: the process ends)
+      for (const auto& [i, id] : ended) {
+        if (slots[i].state != kLaunched || slots[i].id != id) continue;  // (another thread freed it meanwhile)
+        read(i, found);
+        for (auto& l : last)
+          if (l.slot == i && l.id == id) { l.failed = word(i) != 0; l.slot = -1; }
+        word(i) = 0;
+        slots[i].state = kFree;
+        free_slots.push_back(i);
+      }
+      if (!found.empty()) *any() = 1;
     }
-    info[s % kSlots] = c;
-    last[c.kind] = s;
-    int* w = words.data_ptr<int>();
-    o.report = w + s % kSlots;
-    o.report_any = w + kSlots;
+    t.ring = this;
+    t.slot = free_slots.back();
+    free_slots.pop_back();
+    Slot& s = slots[t.slot];
+    s.call = c; s.state = kTaken; s.reported = false; s.id = taken++;
+    auto& l = last[c.kind];
+    l.slot = t.slot; l.id = s.id; l.failed = 0;
+    o.report = words.data_ptr<int>() + t.slot;
+    o.report_any = words.data_ptr<int>() + kSlots;
+    return t;
+  }
+  void launched(int slot) {
+    std::lock_guard<std::mutex> lk(mu);
+    if (slot < (int)slots.size() && slots[slot].state == kTaken) slots[slot].state = kLaunched;
   }
   // descriptions of the calls whose word is set, once each
   std::vector<std::string> collect() {
-    std::lock_guard<std::mutex> lk(mu);
+    std::unique_lock<std::mutex> lk(mu);
     std::vector<std::string> failed;
+    if (!words.defined() || *any() == 0) return failed;
+    *any() = 0;  // (in front of the wait: what ends behind it sets the word again)
+    const auto ended = wait_for_launched(lk);  // (the other workgroups of a call that reported may still be on their way out)
     if (!words.defined()) return failed;
-    if (*any() != 0) api.wait_launches();  // (the other workgroups of a call that reported may still be on their way out)
-    failed.swap(older);
-    gather(failed);
+    failed.swap(found);
+    for (const auto& [i, id] : ended)
+      if (slots[i].state == kLaunched && slots[i].id == id) read(i, failed);
+    for (int i = 0; i < kSlots; ++i)  // (calls launched behind the wait began: asked for again)
+      if (slots[i].state != kFree && !slots[i].reported && word(i) != 0) *any() = 1;
     return failed;
   }
-  void gather(std::vector<std::string>& failed) {  // (the launches so far have ended, mu is held)
-    if (*any() == 0) return;
-    *any() = 0;
-    volatile int* w = words.data_ptr<int>();
-    const long n = std::min<long>(taken, kSlots);
-    for (long i = taken - n; i < taken; ++i) {
-      if (w[i % kSlots] != 1) continue;
-      w[i % kSlots] = 2;  // (reported; still what last() returns)
-      const CallInfo& c = info[i % kSlots];
-      failed.push_back(std::string(c.kind ? "backward" : "forward") + " of " + kNames[c.function] + " B" + std::to_string(c.B) + " T" +
-                       std::to_string(c.T) + " N" + std::to_string(c.N) + " D" + std::to_string(c.D));
-    }
+  // Waits, without the lock, for the calls that are launched by now; returns them.
+  std::vector<std::pair<int, long>> wait_for_launched(std::unique_lock<std::mutex>& lk) {
+    std::vector<std::pair<int, long>> ended;
+    for (int i = 0; i < kSlots; ++i)
+      if (slots[i].state == kLaunched) ended.emplace_back(i, slots[i].id);
+    lk.unlock();
+    api.wait_launches();
+    lk.lock();
+    return ended;
+  }
+  volatile int& word(int i) { return words.data_ptr<int>()[i]; }
+  void read(int i, std::vector<std::string>& failed) {  // (the call has ended, mu is held)
+    if (slots[i].reported || word(i) == 0) return;
+    slots[i].reported = true;
+    const CallInfo& c = slots[i].call;
+    failed.push_back(std::string(c.kind ? "backward" : "forward") + " of " + kNames[c.function] + " B" + std::to_string(c.B) + " T" +
+                     std::to_string(c.T) + " N" + std::to_string(c.N) + " D" + std::to_string(c.D));
   }
   void poll(bool wait, void* stream) {
     const volatile int* a = any();
@@ -153,8 +196,18 @@ struct StatusRing {
   int last_word(int kind) {
     api.wait_launches();
     std::lock_guard<std::mutex> lk(mu);
-    if (last[kind] < 0 || taken - last[kind] > kSlots) return 0;
-    return words.data_ptr<int>()[last[kind] % kSlots] != 0 ? 1 : 0;
+    const auto& l = last[kind];
+    return l.slot >= 0 ? word(l.slot) != 0 : l.failed;
+  }
+  std::vector<std::string> drain() {
+    api.wait_launches();
+    auto failed = collect();
+    std::lock_guard<std::mutex> lk(mu);
+    base.store(nullptr);
+    words.reset();  // (pinned memory goes back while the HIP runtime is up)
+    slots.clear(); free_slots.clear();
+    for (auto& l : last) l = {};
+    return failed;
   }
 };
 StatusRing& ring() { static StatusRing* r = new StatusRing; return *r; }  // (never destroyed: calls may end after static destruction began)
@@ -227,7 +280,7 @@ Saved run_forward(const Tensor& Wx_, const Tensor& R_, const Tensor& b_, const T
   void* st = stream_of(v.Wx);
   frnn_options o = c.o;
   if (c.zero_s0) { o.clear = v.s0.data_ptr(); o.clear_bytes = v.s0.nbytes(); }
-  if (c.fused) ring().take({0, c.function, (int)B, (int)T, (int)N, (int)D}, st, o);
+  const auto ticket = !c.fused ? StatusRing::Ticket() : ring().take({0, c.function, (int)B, (int)T, (int)N, (int)D}, st, o);
   check_rc((c.fused ? api.fused_forward : api.alt_forward)(
                c.function, c.dtype, c.training, B, T, N, D, v.Wx.data_ptr(), v.R.data_ptr(), v.b.data_ptr(), v.s0.data_ptr(),
                v.states.data_ptr(), c.training ? v.cache.data_ptr() : nullptr, ws.data_ptr(), wsb, st, &o),
@@ -278,7 +331,7 @@ struct Function : torch::autograd::Function<Function> {
                                                      : api.alt_workspace_bytes(c.function, c.dtype, B, T, N, D, 1));
     const Tensor ws = torch::empty({(int64_t)wsb}, k.dtype(torch::kByte));
     frnn_options o = c.o;
-    if (c.fused) ring().take({1, c.function, (int)B, (int)T, (int)N, (int)D}, st, o);
+    const auto ticket = !c.fused ? StatusRing::Ticket() : ring().take({1, c.function, (int)B, (int)T, (int)N, (int)D}, st, o);
     int rc;
     if (c.o.recompute)
       rc = api.backward_recompute(c.function, c.dtype, B, T, N, D, Wx.data_ptr(), R.data_ptr(), b.data_ptr(), s0.data_ptr(), states.data_ptr(),
@@ -381,21 +434,14 @@ PYBIND11_MODULE(_host, m) {
   m.def("bind", &bind);
   m.def("call", &call);
   m.def("step", &step);
-  // (the general path's calls, made from Python: addresses of the two words, 0 under capture)
+  // (the general path's calls, made from Python: addresses of the two words, 0 under capture, and what status_launched gets behind the launches)
   m.def("status_take", [](int kind, int function, int B, int T, int N, int D, uintptr_t stream) {
     frnn_options o{};
-    ring().take({kind, function, B, T, N, D}, reinterpret_cast<void*>(stream), o);
-    return std::make_pair(reinterpret_cast<uintptr_t>(o.report), reinterpret_cast<uintptr_t>(o.report_any));
+    auto t = ring().take({kind, function, B, T, N, D}, reinterpret_cast<void*>(stream), o);
+    return std::make_tuple(reinterpret_cast<uintptr_t>(o.report), reinterpret_cast<uintptr_t>(o.report_any), std::exchange(t.slot, -1));
   });
+  m.def("status_launched", [](int slot) { if (slot >= 0) ring().launched(slot); });
   m.def("status_poll", [](bool wait) { ring().poll(wait, c10::hip::getCurrentHIPStream().stream()); }, py::call_guard<py::gil_scoped_release>());
   m.def("status_last", [](int kind) { return ring().last_word(kind); }, py::call_guard<py::gil_scoped_release>());
-  m.def("status_drain", []() {
-    api.wait_launches();
-    auto failed = ring().collect();
-    std::lock_guard<std::mutex> lk(ring().mu);
-    ring().base.store(nullptr);
-    ring().words.reset();  // (pinned memory goes back while the HIP runtime is up)
-    ring().taken = 0; ring().last[0] = ring().last[1] = -1;
-    return failed;
-  }, py::call_guard<py::gil_scoped_release>());
+  m.def("status_drain", []() { return ring().drain(); }, py::call_guard<py::gil_scoped_release>());
 }

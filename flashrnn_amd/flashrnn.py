@@ -13,6 +13,7 @@ for the backward pass (:746) or slice dWx (:789-796).
 from __future__ import annotations
 
 import atexit
+import contextlib
 import os
 from dataclasses import dataclass
 from typing import Optional, Sequence, Union
@@ -195,9 +196,18 @@ class _StatusLog:
     them, not the device) and does the same.  Calls under stream capture are not recorded: a replay repeats the kernels, not this
     bookkeeping."""
 
+    @contextlib.contextmanager
     def words(self, kind: str, cfg: "FlashRNNConfig", B: int, T: int, N: int, D: int, stream: int):
-        """The two words of a call (addresses; 0 under capture)."""
-        return _lib.load_host().status_take(int(kind == "backward"), _lib.FUNCTION_IDS[cfg.function], B, T, N, D, stream)
+        """The two words of a call (addresses; 0 under capture), the call's own until its launches have ended."""
+        if cfg.backend != "hip_fused":
+            yield None, None
+            return
+        host = _lib.load_host()
+        one, shared, slot = host.status_take(int(kind == "backward"), _lib.FUNCTION_IDS[cfg.function], B, T, N, D, stream)
+        try:
+            yield one, shared
+        finally:
+            host.status_launched(slot)
 
     def poll(self, wait: bool = False):
         if torch.cuda.is_initialized():
@@ -338,11 +348,11 @@ def _run_forward(Wx_k, R_k, b_k, s0_k, cfg: FlashRNNConfig, training: bool, out=
         ws_bytes = _workspace_bytes(cfg, f_id, d_id, B, T, N, D, 0)
         ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=Wx_k.device)
         stream = _raw_stream(Wx_k.device)
-        words = _status.words("forward", cfg, B, T, N, D, stream) if cfg.backend == "hip_fused" else (None, None)
-        rc = _entry(cfg.backend, "forward_opt")(
-            f_id, d_id, int(training), B, T, N, D, Wx_k.data_ptr(), R_k.data_ptr(), b_k.data_ptr(),
-            s0_k.data_ptr(), states.data_ptr(), cache.data_ptr() if training else None,
-            ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride, words))
+        with _status.words("forward", cfg, B, T, N, D, stream) as words:
+            rc = _entry(cfg.backend, "forward_opt")(
+                f_id, d_id, int(training), B, T, N, D, Wx_k.data_ptr(), R_k.data_ptr(), b_k.data_ptr(),
+                s0_k.data_ptr(), states.data_ptr(), cache.data_ptr() if training else None,
+                ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride, words))
         if rc != 0:
             _raise(rc, f"{cfg.backend} forward")
     return states, cache
@@ -365,17 +375,17 @@ def _run_backward(cfg: FlashRNNConfig, R_k, b_k, s0_k, states, cache, Wx_k, ds, 
         ws_bytes = _workspace_bytes(cfg, f_id, d_id, B, T, N, D, 1)
         ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
         stream = _raw_stream(dev)
-        words = _status.words("backward", cfg, B, T, N, D, stream) if cfg.backend == "hip_fused" else (None, None)
-        if cfg.recompute_gates:
-            rc = _lib.load_library().frnn_fused_backward_recompute(
-                f_id, d_id, B, T, N, D, Wx_k.data_ptr(), R_k.data_ptr(), b_k.data_ptr(), s0_k.data_ptr(),
-                states.data_ptr(), ds.data_ptr(), dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr(), db.data_ptr(),
-                ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride, words))
-        else:
-            rc = _entry(cfg.backend, "backward_opt")(
-                f_id, d_id, B, T, N, D, R_k.data_ptr(), b_k.data_ptr(), s0_k.data_ptr(), states.data_ptr(),
-                cache.data_ptr(), ds.data_ptr(), dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr(), db.data_ptr(),
-                ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride, words))
+        with _status.words("backward", cfg, B, T, N, D, stream) as words:
+            if cfg.recompute_gates:
+                rc = _lib.load_library().frnn_fused_backward_recompute(
+                    f_id, d_id, B, T, N, D, Wx_k.data_ptr(), R_k.data_ptr(), b_k.data_ptr(), s0_k.data_ptr(),
+                    states.data_ptr(), ds.data_ptr(), dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr(), db.data_ptr(),
+                    ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride, words))
+            else:
+                rc = _entry(cfg.backend, "backward_opt")(
+                    f_id, d_id, B, T, N, D, R_k.data_ptr(), b_k.data_ptr(), s0_k.data_ptr(), states.data_ptr(),
+                    cache.data_ptr(), ds.data_ptr(), dWx.data_ptr(), ds0.data_ptr(), dR.data_ptr(), db.data_ptr(),
+                    ws.data_ptr(), ws.numel(), stream, _options(cfg, batch_stride, words))
         if rc != 0:
             _raise(rc, f"{cfg.backend} backward")
     return dR, db, ds0

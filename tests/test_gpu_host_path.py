@@ -218,3 +218,47 @@ def test_tensors_of_another_device_are_refused_on_the_host(gpu, monkeypatch, nam
     monkeypatch.setenv("FRNN_TEST_MAX_BATCH", "2")  # (ranges of the batch)
     with refused:
         flashrnn(**inputs(64))
+
+
+@pytest.mark.gpu
+def test_the_last_result_of_a_kind_outlives_its_word(gpu, monkeypatch):
+    """A backward call that failed stays the last backward call, however many forward calls use the words behind it."""
+    from flashrnn_amd import check_status, flashrnn, last_status
+
+    print("case host path last status", flush=True)
+    leaves = _leaves(gpu, T=2, D=256)
+    out, _ = flashrnn(*leaves)
+    monkeypatch.setenv("FRNN_SPIN_LIMIT", "-2")
+    torch.autograd.grad(out.float().sum(), leaves)
+    monkeypatch.delenv("FRNN_SPIN_LIMIT")
+    with pytest.raises(RuntimeError, match="backward of lstm B5 T2 N2 D256"):
+        check_status()
+    with torch.no_grad():
+        for _ in range(4200):
+            flashrnn(*leaves)
+    assert last_status("backward") == 1 and last_status("forward") == 0
+    check_status()
+
+
+@pytest.mark.gpu
+def test_a_word_stays_with_its_call_until_that_is_launched(gpu):
+    """Another thread's call that took its words and is not launched yet, while this one makes more calls than there are words."""
+    import ctypes
+
+    from flashrnn_amd import _lib, check_status, flashrnn
+
+    print("case host path late launch", flush=True)
+    x = [v.detach() for v in _leaves(gpu, T=2, D=256)]
+    host, stream = _lib.load_host(), torch.cuda.current_stream().cuda_stream
+    one, shared, *late = host.status_take(1, 2, 7, 9, 3, 512, stream)
+    with torch.no_grad():
+        for _ in range(4200):
+            flashrnn(*x)
+    torch.cuda.synchronize()
+    for word in (one, shared):  # what its kernel does where a wait runs out
+        ctypes.c_int.from_address(word).value = 1
+    for slot in late:
+        host.status_launched(slot)
+    with pytest.raises(RuntimeError, match=r"earlier fused call \(backward of gru B7 T9 N3 D512\)"):
+        check_status()
+    check_status()
