@@ -439,8 +439,8 @@ PYBIND11_MODULE(_host, m) {
     frnn_options o{};
     auto t = ring().take({kind, function, B, T, N, D}, reinterpret_cast<void*>(stream), o);
     return std::make_tuple(reinterpret_cast<uintptr_t>(o.report), reinterpret_cast<uintptr_t>(o.report_any), std::exchange(t.slot, -1));
-  });
-  m.def("status_launched", [](int slot) { if (slot >= 0) ring().launched(slot); });
+  }, py::call_guard<py::gil_scoped_release>());  // (it waits for the device where no word is free)
+  m.def("status_launched", [](int slot) { if (slot >= 0) ring().launched(slot); }, py::call_guard<py::gil_scoped_release>());
   m.def("status_poll", [](bool wait) { ring().poll(wait, c10::hip::getCurrentHIPStream().stream()); }, py::call_guard<py::gil_scoped_release>());
   m.def("status_last", [](int kind) { return ring().last_word(kind); }, py::call_guard<py::gil_scoped_release>());
   m.def("status_drain", []() { return ring().drain(); }, py::call_guard<py::gil_scoped_release>());

@@ -262,3 +262,41 @@ def test_a_word_stays_with_its_call_until_that_is_launched(gpu):
     with pytest.raises(RuntimeError, match=r"earlier fused call \(backward of gru B7 T9 N3 D512\)"):
         check_status()
     check_status()
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_a_call_waits_for_a_word(gpu):
+    """Where every word is taken, a call of the general path waits for the device, and not with the interpreter lock."""
+    import threading
+    import time
+
+    from flashrnn_amd import _lib, flashrnn
+
+    print("case host path lock", flush=True)
+    x = [v.detach() for v in _leaves(gpu, T=4000, D=256)]
+    host, stream = _lib.load_host(), torch.cuda.current_stream().cuda_stream
+    gaps, done = [], threading.Event()
+
+    def tick():
+        last = time.perf_counter()
+        while not done.is_set():
+            time.sleep(0.001)
+            gaps.append(time.perf_counter() - last)
+            last += gaps[-1]
+
+    with torch.no_grad():
+        flashrnn(*x)
+        torch.cuda.synchronize()
+        for _ in range(100):  # (about 3 ms each)
+            flashrnn(*x)
+    thread, longest = threading.Thread(target=tick), 0.0
+    thread.start()
+    for _ in range(4200):
+        t = time.perf_counter()
+        host.status_launched(host.status_take(0, 0, 5, 4000, 2, 256, stream)[2])
+        longest = max(longest, time.perf_counter() - t)
+    done.set()
+    thread.join()
+    torch.cuda.synchronize()
+    print(f"longest wait for a word {longest * 1e3:.1f} ms, longest pause of the other thread {max(gaps) * 1e3:.1f} ms", flush=True)
+    assert longest > 0.05 and max(gaps) < longest / 2
