@@ -943,7 +943,7 @@ int frnn_fused_backward_opt(int function, int dtype, int B, int T, int N, int D,
                             const void* cache, const void* dstates,
                             void* dWx, void* ds0, float* dR, float* db,
                             void* workspace, size_t workspace_bytes, void* stream, const frnn_options* opt) {
-  if (opt && opt->struct_size >= sizeof(frnn_options) && opt->recompute && function != FRNN_ELMAN) {
+  if (opt && opt->struct_size >= offsetof(frnn_options, recompute) + sizeof(int) && opt->recompute && function != FRNN_ELMAN) {
     g_err[0] = 0;
     return fail(FRNN_E_ARG, "recompute mode has no gate cache: call frnn_fused_backward_recompute, which takes Wx");
   }

@@ -307,3 +307,11 @@ def test_options_carry_their_size(lib):
     assert lib.frnn_fused_cache_bytes_opt(L, 0, 4, 8, 2, 64, ctypes.byref(o)) == 0
     o.struct_size = 16                          # ... but the caller's build ends before that field: it is not read
     assert lib.frnn_fused_cache_bytes_opt(L, 0, 4, 8, 2, 64, ctypes.byref(o)) > 0
+
+
+@pytest.mark.parametrize("options", [_lib.Options, _lib.OptionsReport])
+def test_recompute_mode_is_refused_without_wx_whatever_the_size_of_the_options(lib, options):
+    """frnn_fused_backward_opt takes no Wx: with recompute set it says so, also to a caller whose struct ends before later fields."""
+    o = options(0.0, 0.0, 0, 1)
+    rc = lib.frnn_fused_backward_opt(_lib.FUNCTION_IDS["lstm"], 0, 4, 8, 2, 64, *[FAKE] * 11, 1 << 40, None, ctypes.byref(o))
+    assert rc == _lib.E_ARG and b"recompute mode has no gate cache" in lib.frnn_last_error()
