@@ -75,6 +75,7 @@ _SIGNATURES = {
     "frnn_fused_step": (c_int, [c_int] * 5 + [c_void_p] * 7 + [POINTER(Options)]),
     "frnn_alt_step": (c_int, [c_int] * 5 + [c_void_p] * 7 + [POINTER(Options)]),
     "frnn_streams_overlap": (c_int, [c_void_p, c_void_p]),
+    "frnn_fused_decode_workgroups": (c_int, [c_int] * 5 + [POINTER(c_int)] * 2),
     "frnn_fused_decode_mailbox_bytes": (c_size_t, _P6),
     "frnn_fused_decode_mailbox_layout": (c_int, _P6 + [POINTER(c_size_t)] * 4),
     "frnn_fused_decode_open": (c_int, [c_int] * 5 + [c_void_p] * 5 + [c_size_t, c_int, c_int, c_int, c_void_p, c_void_p, POINTER(Options)]),

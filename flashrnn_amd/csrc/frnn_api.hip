@@ -7,7 +7,10 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <atomic>
 #include <mutex>
+#include <optional>
+#include <shared_mutex>
 
 #include "frnn_alt.h"
 #include "frnn_fused_bwd.h"
@@ -158,6 +161,7 @@ static int fwd_poll_delay_default(int function, int dtype, const Plan& p, int ti
   // one to the L2 of an XCD (lstm fp32 D=1024, forward, 1024 steps: delay 0 6.09 ms, 8 4.81, 16 4.37, 24 3.92, 32 4.00, 48 4.36)
   // (the other cells and D = 768 also best at 24, within 1 %; 40 workgroups per head, D = 640: 18 2.64 ms, 24 2.74)
   if (p.kw > kXcdWorkgroups) return p.kw <= 40 ? 18 : 24;
+  if (p.order > 1 && dtype != FRNN_F32) return 1;  // (no product in front of the wait, see below)
   const bool elman = function == FRNN_ELMAN || function == FRNN_ELMAN_CLIP;
   // heads spread by splitting k between the waves of a tile (variants 2 and 3 of the tables), T = 256, B4 N1 and B16 N2, delays 0 to
   // 12 swept: fp32, fours: D=128 flat from 0 to 4 (6 +3 %), D=192 gru 6 (0.271 ms; 0 0.274), the others 0, D=256 lstm and gru 6 (0.311; 0
@@ -276,6 +280,85 @@ static bool pick_plan(int function, int dtype, int B, int N, int D, int backward
   }
   return true;
 }
+
+static bool stream_capturing(hipStream_t st);
+static int tile_split(const Plan& p) { return 16 * p.waves * p.utw * p.kw / p.D; }  // waves that share a tile (fwd_k_split, bwd_dest_split)
+// The tiling of a decode session, and of a sequence call while a session is open: a session keeps its workgroups on their compute units,
+// so neither takes more of them than the default tiling does.  LSTM 16-bit D = 768: 12 workgroups, and a second session or a sequence
+// call finds room for its 12 on the same XCD; in the spread tiling of 24 it does not, and its waits run out.  A tiling that
+// splits its tiles between waves is replaced by the default; forward the default then sums in the order of the tiling that it
+// replaces (Plan::order), so that tokens have the bits of a sequence call and those bits do not depend on what else is open.
+// The dense tilings take no more compute units than the default, and those without a split no more waves.
+static bool pick_beside(int function, int dtype, int B, int N, int D, int backward, Plan* p, bool dense = true) {
+  if (!pick_plan(function, dtype, B, N, D, backward, p, dense)) return false;
+  const int split = tile_split(*p);
+  if (p->variant < 2 || p->variant == kDenseVariant || split == 1) return true;
+  for (int v = p->variant - 1; ; --v) {
+    Plan q;
+    if (!find_plan(function, dtype, D, v, backward, &q)) return false;
+    if (q.variant != 0 && tile_split(q) > 1) continue;
+    if (!backward && split > tile_split(q)) q.order = split;
+    q.max_tr = 4;  // (as every tiling that is replaced: the same groups, and no more workspace)
+    *p = q;
+    return true;
+  }
+}
+
+// Decode sessions that may be running, by device.  A session is gone when its kernel has ended, whether it was closed, idled out or
+// served its tokens: the event behind the kernel tells.
+struct Session { const void* mailbox; hipEvent_t ended; };
+constexpr int kMaxSessions = 64;  // per device that are told apart; beyond that the device counts as never without one
+struct Sessions {
+  std::shared_mutex mu;
+  struct { Session s[kMaxSessions]; int n = 0; bool more = false; } of[64];
+  std::atomic<int> devices{0};  // > 0: some device has (had) a session, the lists have to be looked at
+  bool open(int dev) const { return of[dev].n > 0 || of[dev].more; }
+};
+static Sessions& g_sessions = *new Sessions;  // (never destroyed: calls may come while the process ends)
+static int current_device() {
+  int dev = 0;
+  return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 ? dev : -1;
+}
+// Takes the sessions out whose kernels have ended, and that of `mailbox` (mu is held alone).
+static void sessions_drop(int dev, const void* mailbox) {
+  auto& l = g_sessions.of[dev];
+  const bool was = g_sessions.open(dev);
+  for (int i = 0; i < l.n;) {
+    bool gone = l.s[i].mailbox == mailbox;
+    if (!gone && l.s[i].ended) {
+      gone = hipEventQuery(l.s[i].ended) == hipSuccess;
+      if (!gone) (void)hipGetLastError();
+    }
+    if (!gone) { ++i; continue; }
+    if (l.s[i].ended) (void)hipEventDestroy(l.s[i].ended);
+    l.s[i] = l.s[--l.n];
+  }
+  if (was && !g_sessions.open(dev)) --g_sessions.devices;
+}
+static void sessions_add(int dev, const void* mailbox, hipStream_t ks) {  // (behind the launch on ks, mu is held alone)
+  sessions_drop(dev, mailbox);
+  auto& l = g_sessions.of[dev];
+  if (!g_sessions.open(dev)) ++g_sessions.devices;
+  if (l.n == kMaxSessions) { l.more = true; return; }
+  Session s{mailbox, nullptr};
+  if (hipEventCreateWithFlags(&s.ended, hipEventDisableTiming) != hipSuccess) { s.ended = nullptr; (void)hipGetLastError(); }
+  if (s.ended && hipEventRecord(s.ended, ks) != hipSuccess) { (void)hipEventDestroy(s.ended); s.ended = nullptr; (void)hipGetLastError(); }
+  l.s[l.n++] = s;  // (without an event it counts until it is closed)
+}
+// A sequence call, from the choice of its tiling to its last launch: no session opens meanwhile, and `beside` stays true of what it launches.
+struct SequenceCall {
+  std::shared_lock<std::shared_mutex> lk;
+  bool beside = false;
+  explicit SequenceCall(hipStream_t st) {
+    int dev = g_sessions.devices.load() != 0 ? current_device() : -1;
+    if (dev >= 0 && !stream_capturing(st)) {  // (events are not asked under capture)
+      std::unique_lock<std::shared_mutex> alone(g_sessions.mu);
+      sessions_drop(dev, nullptr);
+    }
+    lk = std::shared_lock<std::shared_mutex>(g_sessions.mu);
+    if (g_sessions.devices.load() != 0 && (dev = current_device()) >= 0) beside = g_sessions.open(dev);
+  }
+};
 
 // Batch rows per group: 4, 8 or 16.  Fewer rows per tile mean less gate math per lane and fewer
 // words to poll per step (the larger costs of a step) at the price of more workgroups and copies
@@ -539,9 +622,8 @@ static int decode_plan(int function, int dtype, int B, int N, int D, int slots, 
   int e = check_problem(function, dtype, B, 1, N, D);
   if (e) return e;
   if (slots != 2 && slots != 4 && slots != 8 && slots != 16) return fail(FRNN_E_ARG, "slots must be 2, 4, 8 or 16 (got %d)", slots);
-  // (the tiling of a sequence call of this size: the order of a step's sums, and so the bits, are those of the sequence)
   // (never the dense tiling: it is for calls with more groups than a session may have)
-  if (!pick_plan(function, dtype, B, N, D, 0, &out->p, false))
+  if (!pick_beside(function, dtype, B, N, D, 0, &out->p, false))
     return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
   const Plan& p = out->p;
   out->groups = N * ((B + 3) / 4);
@@ -721,8 +803,11 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   e = parse_opts(opt, function, &o);
   if (e) return e;
   const int fx = o.fx;
+  hipStream_t st = (hipStream_t)stream;
+  std::optional<SequenceCall> call;
+  if (!step) call.emplace(st);  // (the workgroups of a single step wait for nobody)
   Plan p;
-  if (!pick_plan(fx, dtype, B, N, D, 0, &p, dense))
+  if (!(call && call->beside ? pick_beside : pick_plan)(fx, dtype, B, N, D, 0, &p, dense))
     return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
   e = check_fused_sizes(fx, dtype, B, T, N, D, o.bs, training && !o.rc);
   if (e) return e;
@@ -735,7 +820,6 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   }
   const bool need_cache = training && cell_dims(fx).NC > 0 && !o.rc;
   if (need_cache) CHECK_PTR(cache)
-  hipStream_t st = (hipStream_t)stream;
   if (step && dtype != FRNN_F32) {  // a kernel of its own, with the bits of this tiling
     prof_begin("fused_step_kernel", st);
     e = launch_fused_step(fx, dtype, p, tile_rows_for(B, N, p.kw, p.waves, p.max_tr, dtype), StepArgs{Wx, R, b, s0, states, carry, B, o.bs ? o.bs : B, N, D, o.h_clip}, st);
@@ -859,8 +943,10 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   if (e) return e;
   const int fx = o.fx;
   const CellDims c = cell_dims(fx);
+  hipStream_t st = (hipStream_t)stream;
+  SequenceCall call(st);
   Plan p;
-  if (!pick_plan(fx, dtype, B, N, D, o.rc ? 2 : 1, &p))
+  if (!(call.beside ? pick_beside : pick_plan)(fx, dtype, B, N, D, o.rc ? 2 : 1, &p, true))
     return fail(FRNN_E_UNSUPPORTED, "no fused%s kernel for function %d dtype %d head dim %d", o.rc ? " recompute-mode" : "",
                 function, dtype, D);
   e = check_fused_sizes(fx, dtype, B, T, N, D, o.bs, !o.rc);
@@ -871,7 +957,6 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   else if (c.NC > 0) CHECK_PTR(cache)
   const FusedBwdWs w = carve_fused_bwd(workspace, fx, dtype, B, T, N, D, p);
   if (workspace_bytes < w.total) return fail(FRNN_E_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, w.total);
-  hipStream_t st = (hipStream_t)stream;
   // (heads of several workgroups: the launch that transposes R clears the status word and the exchange words as well)
   prof_begin("transpose_r_kernel", st);
   e = launch_transpose_r(dtype, R, w.Rt, N, D, c.GR, st, workspace, p.kw > 1 ? w.zero_bytes : 0);
@@ -1003,6 +1088,16 @@ int frnn_streams_overlap(void* stream, void* kernel_stream) {
   return host[1] == 1 ? 1 : 0;
 }
 
+int frnn_fused_decode_workgroups(int function, int dtype, int B, int N, int D, int* waves, int* wgs) {
+  g_err[0] = 0;
+  DecodePlan dp;
+  int e = decode_plan(function, dtype, B, N, D, 2, &dp);
+  if (e) return e;
+  if (waves) *waves = dp.p.waves;
+  if (wgs) *wgs = dp.groups * dp.p.kw;
+  return 0;
+}
+
 size_t frnn_fused_decode_mailbox_bytes(int function, int dtype, int B, int N, int D, int slots) {
   DecodePlan dp;
   if (decode_plan(function, dtype, B, N, D, slots, &dp)) return 0;
@@ -1070,7 +1165,10 @@ int frnn_fused_decode_open(int function, int dtype, int B, int N, int D,
   a.mailbox = mailbox; a.inbox_off = dp.l.inbox_off; a.outbox_off = dp.l.outbox_off;
   a.in_slot = dp.l.in_slot; a.out_slot = dp.l.out_slot; a.slots = slots; a.idle_limit = idle_polls;
   a.trace = nullptr;
-  LaunchGate* gate = gate_enter(p.kw, ks);
+  // (sequence calls that chose their tiling before this one are launched, and those with waits queued, when the lock is given)
+  std::unique_lock<std::shared_mutex> alone(g_sessions.mu);
+  // (heads of one workgroup wait for nobody, but they too start behind what was launched in tilings for a device without sessions)
+  LaunchGate* gate = gate_enter(p.kw > 1 ? p.kw : 2, ks);
   switch (function) {
     case FRNN_LSTM:  e = fused_dec_dispatch<FRNN_LSTM>(dtype, p, a, ks); break;
     case FRNN_SLSTM: e = fused_dec_dispatch<FRNN_SLSTM>(dtype, p, a, ks); break;
@@ -1078,6 +1176,8 @@ int frnn_fused_decode_open(int function, int dtype, int B, int N, int D,
     default:         e = fused_dec_dispatch<FRNN_ELMAN>(dtype, p, a, ks); break;
   }
   gate_leave(gate, ks, e == 0, false);
+  const int dev = current_device();
+  if (e == 0 && dev >= 0) sessions_add(dev, mailbox, ks);
   return e ? hip_fail(e, "resident decode kernel launch") : 0;
 }
 
@@ -1113,6 +1213,12 @@ int frnn_fused_decode_close(void* mailbox, void* stream, void* kernel_stream) {
   int e = (int)hipGetLastError();
   if (e) return hip_fail(e, "stop word");
   e = order_streams(ks, st);  // what follows on the caller's stream sees the carry and the control block
+  {
+    std::unique_lock<std::shared_mutex> alone(g_sessions.mu);
+    for (int dev = 0; dev < 64; ++dev)
+      for (int i = 0; i < g_sessions.of[dev].n; ++i)
+        if (g_sessions.of[dev].s[i].mailbox == mailbox && !g_sessions.of[dev].s[i].ended) { sessions_drop(dev, mailbox); break; }
+  }
   return e ? hip_fail(e, "ordering the caller's stream behind the resident kernel") : 0;
 }
 

@@ -68,7 +68,7 @@ template <> __device__ __forceinline__ float load_frag<float>(const float* row, 
   return row[ks * 4 + kq];
 }
 
-template <int F, typename T, int D, int WAVES, int UTW, int KW, int TR, bool MB = false, bool PSTV = false>
+template <int F, typename T, int D, int WAVES, int UTW, int KW, int TR, bool MB = false, bool PSTV = false, int KO = 0>
 __global__ void __launch_bounds__((WAVES + (!MB && fwd_producer_wave(Cell<F>::GR, D, WAVES, UTW, KW, TR, (int)sizeof(T)) ? 1 : 0)) * 64)
 fused_fwd_kernel(const FwdArgs a) {
   static_assert(!MB || TR == 4, "the resident decode kernel runs on 4-row batch tiles");
@@ -81,9 +81,13 @@ fused_fwd_kernel(const FwdArgs a) {
   constexpr int GR = C::GR, GW = C::GW, GT = C::GT, S = C::S, NC = C::NC;
   // (KSP waves per tile, each with its part of k)
   constexpr int KSP = fwd_k_split(D, WAVES, UTW, KW), DK = D / KSP;
+  // (KO: k is summed in KO parts whatever KSP is, KOW of them by this wave: the bits of the tiling with KSP = KO in the workgroups
+  // of this one, for calls beside a decode session and for the sessions themselves)
+  constexpr int KOP = KO > 0 ? KO : KSP, KOW = KOP / KSP, DP = D / KOP;
+  static_assert(KOP % KSP == 0 && (KO == 0 || TR == 4) && (KO == 0 || sizeof(T) == 4 || (KSP == 1 && KO == 2)), "parts of k");
   constexpr int KS = D / X::KM, NT = WAVES * 64, UT_WG = WAVES * UTW / KSP;
   static_assert(UT_WG * KW * 16 == D && WAVES % KSP == 0, "tiling must cover the head");
-  static_assert(KSP == 1 || sizeof(T) == 2 || DK % 16 == 0, "fp32: a wave reads its part of h 16 k at a time");
+  static_assert(KOP == 1 || sizeof(T) == 2 || DP % 16 == 0, "fp32: a wave reads its part of h 16 k at a time");
   static_assert(KSP <= 2 || (sizeof(T) == 4 && UTW == 1), "more than two waves per tile: the fp32 4x4x1 form only");
   constexpr int LLW = 16 * D / X::EPW;  // 64-bit words per exchange slot
   // words a thread polls per step: the TR rows of the tile, without the workgroup's own slice
@@ -124,7 +128,7 @@ fused_fwd_kernel(const FwdArgs a) {
 #ifdef FRNN_NO_OWN_FIRST
   constexpr bool OWN_FIRST = false;
 #else
-  constexpr bool OWN_FIRST = fwd_own_slice_first(GR, D, WAVES, UTW, KW, TR, (int)sizeof(T));
+  constexpr bool OWN_FIRST = KO == 0 && fwd_own_slice_first(GR, D, WAVES, UTW, KW, TR, (int)sizeof(T));
 #endif
   constexpr int KSO = OWN_FIRST ? (D / KW) / X::KM : 0;
   __shared__ __attribute__((aligned(16))) T hbuf[2][16 * D];
@@ -147,7 +151,7 @@ fused_fwd_kernel(const FwdArgs a) {
   __shared__ __attribute__((aligned(16))) T obuf[PST ? 2 * OB : 1];
   // [wave][k-step][u][g][lane]: each lane reads back what it wrote
   __shared__ __attribute__((aligned(16))) Frag rlds[RLK > 0 ? WAVES * RLK * UTW * GR * 64 : 1];
-  __shared__ f32x4 psum[KSP > 1 ? UT_WG * (KS16 ? GR : KSP - 1) * 64 : 1];  // partial sums of the other waves of a tile: [tile][(gate | wave)][lane]
+  __shared__ f32x4 psum[KSP > 1 ? UT_WG * (KS16 ? GR : KOP - KOW) * 64 : 1];  // partial sums of the other waves of a tile: [tile][(gate | part)][lane]
 
   int grp_l, slice;
   if (!decode_block(a.groups, KW, grp_l, slice)) return;
@@ -464,7 +468,9 @@ fused_fwd_kernel(const FwdArgs a) {
     // independent MFMA chains are in flight (a dependent MFMA waits ~3x longer than an independent one)
     constexpr int NACC_ = UTW * GR >= 3 ? 1 : (UTW * GR == 2 ? 2 : 4);
     constexpr int NACC = NACC_ < KS ? NACC_ : KS;
-    f32x4 accp[M44 ? 1 : NACC][UTW][GR];
+    constexpr int PARTS = M44 ? 1 : KOW;  // (16-bit types, k summed in parts: a chain for each)
+    static_assert(PARTS == 1 || NACC == 1, "parts of a single chain");
+    f32x4 accp[M44 ? 1 : NACC * PARTS][UTW][GR];
     if constexpr (OWN_FIRST) {
       if (t > 0) lds_barrier();  // the own slice of h_(t-1), written by the gate math of every wave
       const Frag* hf = reinterpret_cast<const Frag*>(hbuf[cur]) + lane;
@@ -537,17 +543,22 @@ fused_fwd_kernel(const FwdArgs a) {
 #pragma unroll
       for (int v = 0; v < DK / 16; ++v) ha[v] = hf[64 * v];
       __builtin_amdgcn_sched_barrier(0);
-      f32x4 ac[UTW][4];  // 4 independent accumulation chains per tile
-#pragma unroll
-      for (int v = 0; v < DK / 16; ++v) {
-#pragma unroll
-        for (int u = 0; u < UTW; ++u) mfma_4x4x1_bcast16(ha[v], &rb[u][16 * v], ac[u], v == 0);
-      }
       f32x4 sum[UTW];
 #pragma unroll
-      for (int u = 0; u < UTW; ++u) {
-        sum[u] = (ac[u][0] + ac[u][1]) + (ac[u][2] + ac[u][3]);
-        if constexpr (KSP > 1) { if (kh != 0) psum[((wt * UTW + u) * (KSP - 1) + kh - 1) * 64 + lane] = sum[u]; }
+      for (int p = 0; p < KOW; ++p) {
+        f32x4 ac[UTW][4];  // 4 independent accumulation chains per tile
+#pragma unroll
+        for (int v = p * (DP / 16); v < (p + 1) * (DP / 16); ++v) {
+#pragma unroll
+          for (int u = 0; u < UTW; ++u) mfma_4x4x1_bcast16(ha[v], &rb[u][16 * v], ac[u], v == p * (DP / 16));
+        }
+#pragma unroll
+        for (int u = 0; u < UTW; ++u) {
+          const f32x4 part = (ac[u][0] + ac[u][1]) + (ac[u][2] + ac[u][3]);
+          if constexpr (KSP > 1) { if (kh != 0) psum[((wt * UTW + u) * (KOP - KOW) + (kh - 1) * KOW + p) * 64 + lane] = part; }
+          if (p == 0) sum[u] = part;
+          else sum[u] += part;
+        }
       }
       // (the buffer is free again before the second wave's next write: the barrier of the next step's exchange wait,
       // which every pair-split tiling has, lies in between)
@@ -557,7 +568,7 @@ fused_fwd_kernel(const FwdArgs a) {
         if constexpr (KSP > 1) {
           if (kh == 0) {
 #pragma unroll
-            for (int i = 0; i < KSP - 1; ++i) sum[u] += psum[((wt * UTW + u) * (KSP - 1) + i) * 64 + lane];
+            for (int i = 0; i < KOP - KOW; ++i) sum[u] += psum[((wt * UTW + u) * (KOP - KOW) + i) * 64 + lane];
           }
         }
         // lane 4*blk + j holds (gate j, unit blk) of batch rows 0..3; after the transpose lane 4*blk + b holds
@@ -594,7 +605,7 @@ fused_fwd_kernel(const FwdArgs a) {
       }
 #pragma unroll
       for (int k = 0; k < KC; ++k) {
-        const int ks = KSO + kc * KC + k, j = ks % NACC;
+        const int ks = KSO + kc * KC + k, j = PARTS > 1 ? ks / (KS / PARTS) : ks % NACC;
         // fragments kept in LDS: those of the next k-step are requested before this one's MFMAs
         Frag la[UTW][GR];
         if constexpr (RLK > 0) {
@@ -617,9 +628,9 @@ fused_fwd_kernel(const FwdArgs a) {
 #pragma unroll
           for (int g = 0; g < GR; ++g)
             accp[j][u][g] = X::mfma(ks < KSR ? rf[u][g][ks < KSR ? ks : 0] : la[u][g], hq[kc & 1][k],
-                                    ks < NACC ? ((BIAS_C && ks == 0) ? biasc[u][g] : f32x4{0.f, 0.f, 0.f, 0.f}) : accp[j][u][g]);
+                                    (PARTS > 1 ? ks % (KS / PARTS) == 0 : ks < NACC) ? ((BIAS_C && ks == 0) ? biasc[u][g] : f32x4{0.f, 0.f, 0.f, 0.f}) : accp[j][u][g]);
         // group by group: consecutive MFMAs then never depend on each other
-        if (j == NACC - 1) __builtin_amdgcn_sched_barrier(0);
+        if (PARTS > 1 || j == NACC - 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
 #pragma unroll
@@ -628,7 +639,7 @@ fused_fwd_kernel(const FwdArgs a) {
       for (int g = 0; g < GR; ++g) {
         acc[u][g] = accp[0][u][g];
 #pragma unroll
-        for (int j = 1; j < NACC; ++j) acc[u][g] += accp[j][u][g];
+        for (int j = 1; j < NACC * PARTS; ++j) acc[u][g] += accp[j][u][g];
       }
     if constexpr (KS16) {
       // the second wave of a pair hands its accumulators over (the buffer is free again before its next write: the

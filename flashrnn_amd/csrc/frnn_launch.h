@@ -79,3 +79,16 @@ bool find_plan(int function, int dtype, int D, int variant, int backward, Plan* 
 #endif
 #endif
 #endif
+
+#ifdef FRNN_TU_PLANS
+namespace frnn {
+// whether the tables of this cell and type have a forward tiling of D units whose waves sum k in `parts` parts (then the default tiling
+// of D is compiled with that order as well)
+constexpr bool order_compiled(int D, int parts) {
+#define FRNN_HAS(Dv, VAR, W, U, K, MTR) if (D == Dv && (VAR == 2 || VAR == 3) && fwd_k_split(Dv, W, U, K) == parts) return true;
+  FRNN_TU_PLANS(FRNN_HAS)
+#undef FRNN_HAS
+  return false;
+}
+}  // namespace frnn
+#endif

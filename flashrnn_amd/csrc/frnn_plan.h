@@ -24,6 +24,7 @@ struct Plan {
   int cooperative = 0;  // host side only: launch the kernel as a cooperative one (see fused_*_tu.hip)
   int recompute = 0;    // host side only: the reverse kernel of recompute mode
   int left_out = 0;     // host side only, tests of the failure path: workgroups at the end of the grid that are not launched
+  int order = 0;        // forward: > 1: sums over k in this many parts, as a tiling whose waves split k does (see pick_beside)
 };
 
 // Resident operand of the forward product: a wave holds UTW*G_r*KS fragments of R.  When they alone

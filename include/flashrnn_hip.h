@@ -299,7 +299,11 @@ int frnn_fused_forward_static(int function, int dtype, int training, int B, int 
  * unrounded state to `carry` ([S,B,N,D] fp32, optional; on entry, if given, it is the unrounded initial state as for
  * frnn_fused_step) and the reason to the control block; the collecting side gives up after FRNN_SPIN_LIMIT probes
  * and writes NaN.  Nothing is allocated.  While a session is open its workgroups occupy their compute units
- * (N * ceil(B / 4) * workgroups-per-head of them; FRNN_E_UNSUPPORTED if they do not fit at once), a device-wide
+ * (frnn_fused_decode_workgroups of them; FRNN_E_UNSUPPORTED if they do not fit at once).  A session takes the default tiling of
+ * its head dimension, and so do fused sequence calls made while a session is open on their device, not the wider ones that
+ * calls take that have the device for themselves, so that sessions and calls find room beside each other; the bits of a forward call do
+ * not depend on it (those of a backward call's sums between workgroups do).  A graph captured while no session is open
+ * keeps the wider tilings; to replay it beside a session, capture it while one is open, or under FRNN_FUSED_VARIANT=1.  A device-wide
  * synchronisation waits for the session to end, and `kernel_stream` must not share a hardware queue with `stream`
  * (a runtime maps streams onto a few queues; a post that queues behind the resident kernel is only served when the
  * kernel has idled out).  close orders `stream` behind the end of the resident kernel. */
@@ -309,6 +313,8 @@ int frnn_fused_forward_static(int function, int dtype, int training, int B, int 
  * kernel on `stream` sets.  Synchronises both streams; allocates nothing.  frnn_fused_decode_open runs it and refuses
  * a pair that returns 0 (FRNN_E_DEVICE). */
 int frnn_streams_overlap(void* stream, void* kernel_stream);
+/* workgroups of a session (a compute unit each, where the device has room) and waves per workgroup */
+int frnn_fused_decode_workgroups(int function, int dtype, int B, int N, int D, int* waves, int* workgroups);
 size_t frnn_fused_decode_mailbox_bytes(int function, int dtype, int B, int N, int D, int slots);
 /* byte offsets of the inbox and outbox rings and the sizes of one slot of each; the control block is the first 64 ints:
  * [0] status (1: a wait between workgroups ran out), [1] stop word, [2] why the kernel ended (1 wait ran out, 2 idle,

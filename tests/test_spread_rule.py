@@ -69,3 +69,47 @@ def test_calls_that_fit_the_static_scratch_keep_fitting():
         args = [FUNCTION_IDS[function], DTYPE_IDS["bfloat16"], 0, B, 4, N, 256] + [None] * 8
         rc = lib.frnn_fused_forward_static(*args)
         assert "static scratch" not in lib.frnn_last_error().decode(), (rc, lib.frnn_last_error())
+
+
+@pytest.mark.parametrize("function", list(FUNCTION_IDS))
+@pytest.mark.parametrize("dtype", list(DTYPE_IDS))
+def test_a_session_takes_no_more_than_the_default_tiling(monkeypatch, function, dtype):
+    """A decode session holds its workgroups for as long as it is open: those of the default tiling of its heads, also where a sequence
+    call of the same size spreads them over more (in tilings that split tiles; those that do not keep the number of waves)."""
+    lib, spread = load_library(), 0
+    for D in DIMS:
+        for B, N in ((1, 1), (4, 2), (8, 3), (33, 1)):
+            waves, wgs = ctypes.c_int(), ctypes.c_int()
+            if lib.frnn_fused_decode_workgroups(FUNCTION_IDS[function], DTYPE_IDS[dtype], B, N, D, ctypes.byref(waves), ctypes.byref(wgs)):
+                continue  # (does not fit the device at once)
+            monkeypatch.setenv("FRNN_FUSED_VARIANT", "1")  # (no such entry: the default)
+            monkeypatch.setenv("FRNN_TILE_ROWS", "4")
+            q = _plan(function, dtype, B, N, D, 0)
+            monkeypatch.delenv("FRNN_FUSED_VARIANT")
+            monkeypatch.delenv("FRNN_TILE_ROWS")
+            p = _plan(function, dtype, B, N, D, 0)
+            spread += p[0] * p[3] > q[0] * q[3]
+            assert wgs.value * waves.value <= q[0] * q[3], (D, B, N)
+    assert spread > 0 or function == "elman"
+
+
+@pytest.mark.parametrize("function", list(FUNCTION_IDS))
+@pytest.mark.parametrize("dtype", list(DTYPE_IDS))
+def test_the_workspace_of_a_call_serves_its_tiling_beside_a_session(monkeypatch, function, dtype):
+    """Workspace is asked for before a call, which may meet a session that was opened since: the default tiling at 4-row tiles needs no
+    more of it than the spread tiling that it replaces."""
+    lib = load_library()
+    for D in DIMS:
+        for backward in (0, 1):
+            for B, N in ((1, 1), (5, 2), (16, 4), (33, 3), (64, 1)):
+                p = _plan(function, dtype, B, N, D, backward)
+                if p is None or 16 * p[0] * p[1] * p[2] == D:  # (no wave shares a tile: kept beside a session)
+                    continue
+                args = (FUNCTION_IDS[function], DTYPE_IDS[dtype], B, 7, N, D, backward)
+                asked = lib.frnn_fused_workspace_bytes(*args)
+                monkeypatch.setenv("FRNN_FUSED_VARIANT", "1")
+                default = _plan(function, dtype, B, N, D, backward)
+                monkeypatch.setenv("FRNN_TILE_ROWS", "4")
+                assert p[:3] == default[:3] or 0 < lib.frnn_fused_workspace_bytes(*args) <= asked, (D, backward, B, N)
+                monkeypatch.delenv("FRNN_FUSED_VARIANT")
+                monkeypatch.delenv("FRNN_TILE_ROWS")
