@@ -17,8 +17,8 @@ namespace frnn {
 
 // Which product of a sum is contracted into a fused multiply-add is written out in the forward math, not left to the compiler
 // (whose choice between f * c + (i * z) and (f * c) + i * z differs from kernel to kernel): a step then rounds the same way in every
-// tiling, tile height and kernel, and single steps give the bits of a sequence whichever kernels run them.  The product that is ready
-// first is the one that is rounded.
+// tiling, tile height and kernel, and single steps give the bits of a sequence whichever kernels run them.  The forms are those that
+// it had chosen for nearly all of them: the product with the carried state is the one that is not rounded.
 template <bool FAST> struct Math {
   static __device__ __forceinline__ float exp(float x) { return FAST ? __expf(x) : expf(x); }
   static __device__ __forceinline__ float rcp(float x) { return FAST ? __builtin_amdgcn_rcpf(x) : 1.0f / x; }
@@ -68,8 +68,8 @@ template <bool FAST> struct CellMath<FRNN_LSTM, FAST> {
     const float f = M::sigmoid(wx[1] + ry[1]);
     const float z = M::tanh(wx[2] + ry[2]);
     const float o = M::sigmoid(wx[3] + ry[3]);
-    const float fc = mul(f, s[1]), c = __builtin_fmaf(i, z, fc);
-    if (mix) { mix[0] = i; mix[1] = z; mix[2] = fc; }
+    const float iz = mul(i, z), c = __builtin_fmaf(f, s[1], iz);
+    if (mix) { mix[0] = f; mix[1] = s[1]; mix[2] = iz; }
     s[1] = c;
     s[0] = mul(o, M::tanh(c));
     cache[0] = i; cache[1] = f; cache[2] = z; cache[3] = o;
@@ -105,8 +105,8 @@ template <bool FAST> struct CellMath<FRNN_SLSTM, FAST> {
     const float mn = (s[2] == 0.0f) ? ir : fmaxf(ir, lfm);
     const float ig = M::exp(ir - mn);
     const float fg = M::exp(lfm - mn);
-    const float fc = mul(fg, s[1]), c = __builtin_fmaf(ig, z, fc);
-    if (mix) { mix[0] = ig; mix[1] = z; mix[2] = fc; }
+    const float iz = mul(ig, z), c = __builtin_fmaf(fg, s[1], iz);
+    if (mix) { mix[0] = fg; mix[1] = s[1]; mix[2] = iz; }
     const float n = fmaxf(__builtin_fmaf(fg, s[2], ig), 1.0f);
     s[0] = mul(mul(o, c), M::rcp(n));
     s[1] = c; s[2] = n; s[3] = mn;
@@ -139,7 +139,7 @@ template <bool FAST> struct CellMath<FRNN_GRU, FAST> {
     const float r = M::sigmoid(wx[0] + ry[1]);
     const float z = M::sigmoid(wx[1] + ry[2]);
     const float nv = M::tanh(__builtin_fmaf(r, g, wx[2] + b[0]));
-    s[0] = __builtin_fmaf(1.0f - z, nv, mul(z, s[0]));
+    s[0] = __builtin_fmaf(z, s[0], mul(1.0f - z, nv));
     cache[0] = g; cache[1] = r; cache[2] = z; cache[3] = nv;  // the candidate itself: the adjoint needs no tanh
   }
   static __device__ __forceinline__ void bwd(const float* cache, const float* sp, const float* sn, const float* dso,

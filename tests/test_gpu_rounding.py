@@ -76,3 +76,42 @@ def test_partial_sums_between_workgroups_keep_their_bits(gpu, monkeypatch, funct
     wrong = float((ds0[0, :, 0] != want).float().mean())
     print(f"rounded to the other neighbour: {wrong:.5f}", flush=True)
     assert wrong < 5e-3
+
+
+@pytest.mark.parametrize("function", ["lstm", "gru"])
+@pytest.mark.parametrize("D", [64, 256])
+def test_the_sum_of_two_products_is_fused_with_the_carried_state(gpu, function, D):
+    """c = fma(f, c', i z) and h = fma(z, h', (1 - z) n), the second product rounded: the bits that calls have always had.  The gates come out
+    of steps that leave one of them alone (an fp32 state is stored as it is); 64 bits of mantissa hold the exact sums."""
+    import numpy as np
+
+    from flashrnn_amd import flashrnn, flashrnn_step
+
+    print(f"case fused sum {function} D{D}", flush=True)
+    B, N, big, S = 16, 2, 1e4, 2 if function == "lstm" else 1
+    G = 4 if function == "lstm" else 3
+    gen = torch.Generator().manual_seed(86)
+    R, b = torch.zeros(G, N, D, D, device=gpu), torch.zeros(4, N, D, device=gpu)
+    pre, prev = torch.randn(G, B, N, D, generator=gen), torch.randn(B, N, D, generator=gen)
+
+    def step(gates, carried, run=None):
+        x = torch.zeros(B, 1, G, N, D)
+        for g, v in enumerate(gates):
+            x[:, 0, g] = v
+        s0 = torch.zeros(S, B, 1, N, D)
+        s0[S - 1, :, 0] = carried
+        args = (x.to(gpu), R, b, s0.to(gpu))
+        with torch.no_grad():
+            out = flashrnn_step(*args, function=function, dtype="float32") if run is None else flashrnn(*args, function=function, dtype="float32")[0]
+        return out[S - 1, :, 0].cpu().numpy()
+
+    if function == "lstm":  # gates i, f, z, o
+        i, f, z = step((pre[0], -big, big, 0), 0.0), step((-big, pre[1], 0, 0), 1.0), step((big, -big, pre[2], 0), 0.0)
+        gates, plain = (pre[0], pre[1], pre[2], 0), i * z
+    else:                   # gates r, z, n
+        f, z = step((0, pre[1], 0), 1.0), step((0, -big, pre[2]), 0.0)
+        gates, plain = (0, pre[1], pre[2]), (np.float32(1) - f) * z
+    carried = prev.numpy()
+    want = (f.astype(np.longdouble) * carried.astype(np.longdouble) + plain.astype(np.longdouble)).astype(np.float32)
+    assert (want != f * carried + plain).any()
+    assert np.array_equal(step(gates, prev), want) and np.array_equal(step(gates, prev, run="sequence"), want)
