@@ -55,6 +55,8 @@ WAITS = [(f, t, b, d, None) for f, t, b, d in (("lstm", "bfloat16", 8, 320), ("s
 WAITS += [(f, t, b, d, "1") for f, t, b, d in (("lstm", "bfloat16", 8, 256), ("slstm", "bfloat16", 8, 192), ("gru", "bfloat16", 5, 1024),
                                                ("gru", "float32", 4, 256), ("lstm", "float32", 4, 384), ("gru", "float32", 4, 512))]
 WAITS += [("lstm", "float32", 4, 320, "2")]
+# (a producer wave beside pairs that split k: it counts the barrier at which the pairs hand their sums over, and leaves with the others)
+WAITS += [("lstm", "bfloat16", 8, 512, None), ("slstm", "float16", 5, 384, None)]
 
 
 @pytest.mark.parametrize("function,dtype,B,D,variant", WAITS)
