@@ -2,17 +2,18 @@
 // (gate-row count, storage type), forward and backward.  Replaces the reference's constraint
 // solver + JIT bisection (flashrnn/flashrnn/flashrnn.py:429-589, cuda_init_parametric.py:92-358).
 //
-// X(D, VARIANT, WAVES, UTW, KW, MTR):  D = 16 * UTW * WAVES * KW;  MTR = the largest batch tile (4, 8 or 16 rows)
+// X(D, VARIANT, WAVES, UTW, KW, MTR):  D = 16 * UTW * WAVES * KW, or half or a quarter of that where two or four waves share
+// every unit tile (fwd_k_split, bwd_dest_split);  MTR = the largest batch tile (4, 8 or 16 rows)
 // this tiling is compiled for: taller tiles keep more state per lane, and where that would spill registers to
 // scratch memory the tile height stops below (a large batch then runs as more groups, in several launches if
 // the workgroups of a head wait for each other).  No compiled kernel uses scratch memory; a test checks the
 // compiler's resource report of every instantiation.
-//   R registers per lane = UTW * G_r * D / 8 (bf16) or UTW * G_r * D / 4 (f32); a workgroup of
+//   R registers per lane = UTW * G_r * D / 8 (bf16) or UTW * G_r * D / 4 (f32), over the waves that share a tile; a workgroup of
 //   4 waves (one per SIMD) may use up to 512 VGPRs per lane, one of 8 waves 256, of 16 waves 128.
 // VARIANT 0 is the default.  VARIANTS 2 and 3, where a head dim has them, spread the head over more workgroups: 3, the
 // wider one, or else 2, is used instead of the default while all groups of the call fit one launch with 4-row
 // batch tiles (measured faster up to a launch that fills the device, slower where the default still takes one launch and
-// they would take two).  VARIANT 4 packs the head into half the workgroups of the default, two waves per SIMD: a large batch then
+// they would take two; not while a decode session runs, see pick_beside).  VARIANT 4 packs the head into half the workgroups of the default, two waves per SIMD: a large batch then
 // runs on tiles of half the height (see pick_plan).  To try another tiling add an X(D, 1, ...) entry and run with FRNN_FUSED_VARIANT=1.  The alternatives that were measured and lost (4 waves x 2 tiles for
 // D = 128, 8 x 2 waves for D = 256, ...) are not compiled in.
 // Forward and backward tile independently (the gate cache layout does not depend on the plan).
@@ -84,8 +85,8 @@ constexpr bool fwd_producer_wave(int GR, int D, int WAVES, int UTW, int KW, int 
 }
 // Forward kernel: may the producer wave also store the outputs of a step (16-byte pieces, one step late) instead of the
 // compute lanes (2 bytes per state and lane at 4-row tiles)?  Exists for the heads that run as one workgroup with a
-// producer wave; the host picks these instantiations for launches that fill the device (measured: LSTM B256 N12 D64
-// forward -20 %, but +5-9 % at B = 16, where the stores of the compute lanes are hidden anyway).
+// producer wave; the host picks these instantiations by cell, cache and number of groups (fwd_producer_stores_pay; measured: LSTM
+// B256 N12 D64 forward -20 %, but +5-9 % at B = 16, where the stores of the compute lanes are hidden anyway).
 constexpr bool fwd_producer_stores(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize) {
   return KW == 1 && fwd_producer_wave(GR, D, WAVES, UTW, KW, TR, esize);
 }
@@ -194,7 +195,7 @@ constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, in
   X(32, 0, 2, 1, 1, 16) X(64, 0, 4, 1, 1, 8) X(96, 0, 2, 1, 3, 16) X(128, 0, 4, 1, 2, 16) X(160, 0, 2, 1, 5, 16) X(192, 0, 4, 1, 3, 16) X(256, 0, 4, 1, 4, 8) \
   X(320, 0, 4, 1, 5, 8) X(384, 0, 4, 1, 12, 4) X(448, 0, 4, 1, 14, 4) X(512, 0, 4, 1, 16, 4) \
   X(640, 0, 4, 1, 40, 4) X(768, 0, 4, 1, 48, 4) X(1024, 0, 4, 1, 64, 4)
-// slstm fp32 backward: the same without the 20-workgroup tiling of D = 320 (with four states its kernel spills)
+// slstm fp32 backward: the same, from the same measurements
 #define FRNN_BWD_PLANS_SLSTM_F32(X) \
   X(64, 2, 2, 1, 2, 16) X(64, 3, 4, 1, 4, 4) X(96, 3, 4, 1, 6, 4) X(128, 2, 4, 1, 4, 4) X(128, 3, 4, 1, 8, 4) X(160, 2, 4, 1, 5, 4) X(160, 3, 4, 1, 10, 4) X(192, 2, 4, 1, 6, 4) X(192, 3, 4, 1, 12, 4) \
   X(256, 2, 4, 1, 8, 4) X(256, 3, 4, 1, 16, 4) X(320, 2, 4, 1, 10, 4) X(320, 3, 4, 1, 20, 4) X(384, 3, 4, 1, 24, 4) X(448, 3, 4, 1, 28, 4) X(512, 3, 4, 1, 32, 4) \

@@ -1,7 +1,7 @@
 // One time step with carried state, fused backend, 16-bit types (frnn_fused_step).
 //
 // The scan kernel can run a single step, but it first loads its whole slice of R into registers, D * G_r / 8 fragments per wave, and
-// a head has few workgroups so that they exchange little: LSTM B8 N3 D256, 24 workgroups that read 128 KB each, 7.3 us.  A single
+// a head has few workgroups so that they exchange little: LSTM B8 N3 D256, 24 workgroups that read 128 KB each, 7.8 us.  A single
 // step exchanges nothing, so here R is spread over as many waves as it has (unit tile, gate) rows of fragments.  Kernel time, scan
 // kernel's step -> this one (4-row tiles unless noted): LSTM N12 D64 B1 4.0 -> 3.7 us, N6 D128 B16 7.1 -> 4.5, N3 D256 B8 7.8 -> 5.0, D512 B8
 // 11.6 -> 7.3, D768 B8 22.3 -> 10.9, D1024 B4 18.9 -> 11.6, B64 (16 rows) 21.9 -> 13.8; GRU D1024 B4 22.4 -> 11.2; Elman D1024 B4 11.0 -> 4.4, N12

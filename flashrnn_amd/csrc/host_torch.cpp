@@ -1,10 +1,10 @@
 // _host.so: the host side of flashrnn() and flashrnn_step() for the usual call (see flashrnn.py: plain tensors in the kernels'
 // layouts, no transform, tracing or dispatch mode active), and the record of failed waits of every fused call.
 //
-// A short call is bound by the host: LSTM bf16 B5 T19 N3 D256, forward and backward, takes ~70 us on the device.  With an
-// autograd function and ctypes calls in Python it took 300 us of host time (a copy, an event and a tensor view per call to fetch
-// its status word, a dozen ctypes calls, the interpreter on the autograd worker thread); here it takes 111, of which an autograd
-// node of torch's own takes 42.  The forward alone 57 -> 18 us, flashrnn_step 9.6 -> 5.8 us a call.
+// A short call is bound by the host: LSTM bf16 B5 T19 N3 D256, forward and backward, takes ~60 us on the device.  With an
+// autograd function and ctypes calls in Python a pass took 300 us (a copy, an event and a tensor view per call to fetch
+// its status word, a dozen ctypes calls, the interpreter on the autograd worker thread); here it takes 87 to 107 alone and 64 to 95
+// behind others, by process.  The forward alone 57 -> 17 us of host time, flashrnn_step 9.6 -> 7 us a call.
 // The entry points of libflashrnn_hip.so are handed over as addresses (bind), so the library that FLASHRNN_HIP_LIBRARY names is
 // the one that runs, and this file needs no HIP symbol of its own.
 #include <torch/extension.h>
