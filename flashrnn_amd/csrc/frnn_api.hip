@@ -211,6 +211,17 @@ static int device_cus() {
 // of the device: with KW = 12 an XCD of 32 compute units holds 2 groups, the device 16, not 256 / 12 = 21.
 // Heads of more than 32 workgroups (kXcdWorkgroups) spread over the whole device: what counts is the device.
 static int groups_per_launch(int kw) { return kw > kXcdWorkgroups ? device_cus() / kw : 8 * ((device_cus() / 8) / kw); }
+// Workgroups per XCD that fetch the operands of a scan into its L2 (frnn_prefetch.h): one for each group of the XCD, as far as compute units
+// are left.  Not beside a decode session, whose workgroups need the compute units that are left.
+// FRNN_PREFETCH caps them.
+static int helpers_for(const Plan& p, int groups, int T) {
+  if (p.left_out || T <= kPrefetchMinSteps) return 0;
+  const int per_xcd = (groups + 7) / 8, idle = device_cus() / 8 - p.kw * per_xcd;
+  int h = env_int("FRNN_PREFETCH", per_xcd);
+  h = h < per_xcd ? h : per_xcd;
+  h = h < idle ? h : idle;
+  return h > 0 ? h : 0;
+}
 // (such groups never share an XCD: no handshake, every exchange store at agent scope)
 static bool near_stores_possible(const Plan& p) { return p.kw > 1 && p.kw <= kXcdWorkgroups; }
 
@@ -858,6 +869,7 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   p.cooperative = env_int("FRNN_COOPERATIVE", 0);
   a.poll_delay = env_int("FRNN_POLL_DELAY", fwd_poll_delay_default(fx, dtype, p, tr));
   a.h_clip = o.h_clip;
+  a.helpers = 0;
   a.mailbox = nullptr; a.inbox_off = a.outbox_off = a.in_slot = a.out_slot = 0; a.slots = 1; a.idle_limit = 0;
   // (FRNN_PRODUCER_STORES=0/1 overrides)
   a.pst = step ? 0 : env_int("FRNN_PRODUCER_STORES", tr == 4 && p.kw == 1 && fwd_producer_stores_pay(fx, p, groups, a.training) ? 1 : 0);
@@ -868,6 +880,7 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   LaunchGate* gate = gate_enter(step ? 1 : p.kw, st);  // (the workgroups of a single step never wait for each other)
   for (int g0 = 0; g0 < groups; g0 += per_launch) {
     a.grp0 = g0; a.groups = groups - g0 < per_launch ? groups - g0 : per_launch;
+    a.helpers = step || call->beside || !fwd_prefetched(cell_dims(fx).GR, p.kw) ? 0 : helpers_for(p, a.groups, T);
     prof_begin("fused_fwd_kernel", st);
     switch (fx) {
       case FRNN_LSTM:  e = fused_fwd_dispatch<FRNN_LSTM>(dtype, p, a, st); break;
@@ -1162,6 +1175,7 @@ int frnn_fused_decode_open(int function, int dtype, int B, int N, int D,
   a.spin_limit = env_int("FRNN_SPIN_LIMIT", 1 << 22);
   a.poll_delay = env_int("FRNN_POLL_DELAY", fwd_poll_delay_default(function, dtype, p, 4));
   a.h_clip = o.h_clip; a.pst = 0;
+  a.helpers = 0;
   a.mailbox = mailbox; a.inbox_off = dp.l.inbox_off; a.outbox_off = dp.l.outbox_off;
   a.in_slot = dp.l.in_slot; a.out_slot = dp.l.out_slot; a.slots = slots; a.idle_limit = idle_polls;
   a.trace = nullptr;

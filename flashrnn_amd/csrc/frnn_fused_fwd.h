@@ -21,6 +21,7 @@
 #include "frnn_exchange.h"
 #include "frnn_mailbox.h"
 #include "frnn_plan.h"
+#include "frnn_prefetch.h"
 #include "frnn_pointwise.h"
 
 namespace frnn {
@@ -48,6 +49,7 @@ struct FwdArgs {
   // from the inbox of `mailbox` and the new states go to its outbox (frnn_mailbox.h); a wait for a token gives up after
   // idle_limit probes or when the stop word of the control block is set, and the kernel then ends normally
   void* mailbox; size_t inbox_off, outbox_off, in_slot, out_slot; int slots, idle_limit;
+  int helpers;       // workgroups per XCD behind those of the scan that fetch Wx into its L2 (frnn_prefetch.h)
   long long* trace;  // phase cycle sums per workgroup; only written by -DFRNN_TRACE builds
 };
 
@@ -154,6 +156,18 @@ fused_fwd_kernel(const FwdArgs a) {
   __shared__ f32x4 psum[KSP > 1 ? UT_WG * (KS16 ? GR : KOP - KOW) * 64 : 1];  // partial sums of the other waves of a tile: [tile][(gate | part)][lane]
 
   int grp_l, slice;
+  if constexpr (fwd_prefetched(GR, KW) && !MB) {
+    static_assert(KW <= kXcdWorkgroups, "groups within an XCD");
+    const int scan = 8 * KW * ((a.groups + 7) / 8);  // workgroups of the scan (see decode_block), then 8 of those that prefetch for each of a.helpers
+    if (a.helpers && (int)blockIdx.x >= scan) {
+      static_assert(2 * 16 * D * (int)sizeof(T) >= 1024, "room for what is fetched");
+      const auto pa = own_args<FwdArgs>();
+      prefetch_wx<T, GW, D, TR, LLW>(pa->Wx, pa->ll, pa->status, (int)blockIdx.x - scan, 8 * pa->helpers, pa->groups, pa->grp0, pa->N, pa->B, pa->T,
+                                     __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)blockDim.x >> 6, threadIdx.x & 63, pa->spin_limit,
+                                     (unsigned)(size_t)&hbuf[0][0]);
+      return;
+    }
+  }
   if (!decode_block(a.groups, KW, grp_l, slice)) return;
   const int grp = a.grp0 + grp_l;
   const int N = a.N, Tn = a.T, B = a.B, BS = a.BS;

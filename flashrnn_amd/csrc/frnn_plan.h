@@ -57,6 +57,9 @@ constexpr int fwd_lds_ksteps(int GR, int D, int WAVES, int UTW, int esize) {
 constexpr int fwd_k_split(int D, int WAVES, int UTW, int KW) { return 16 * WAVES * UTW * KW / D; }
 // the dense alternatives of the tables (host: pick_plan; not for the resident decode kernel, whose groups all have 4 rows)
 constexpr int kDenseVariant = 4;
+// Forward kernels whose launch may get workgroups that fetch Wx into L2 (frnn_prefetch.h): the gated cells, heads of several workgroups within
+// an XCD.  (Elman, one load per step: -1.4 to +1.0 % at any batch.)
+constexpr bool fwd_prefetched(int GR, int KW) { return GR >= 3 && KW > 1 && KW <= 32; }
 // Forward kernel, fp32 at 4-row tiles, cells with 3 or 4 recurrent gates: the product runs on v_mfma_f32_4x4x1_16B_f32
 // (see the kernel), when the whole operand, D / KSP registers per tile in that form, fits the registers of a wave (512 in
 // workgroups of up to 4 waves, 256 with up to 8: D = 96 as 6 waves).

@@ -1,0 +1,120 @@
+// Workgroups that fetch the operands of the coming steps into the L2 of an XCD (heads of several workgroups).
+//
+// A compute unit's vector memory returns in the order in which it was asked, whichever wave asked.  A scan whose workgroups exchange
+// words in every step therefore waits, with its words, for every operand that some wave of the same compute unit has requested
+// from HBM meanwhile, a producer wave's included: ~1900 cycles, more the more the device moves, against ~700 for the words.  (Forward, T = 1024,
+// a build whose Wx is always the same two steps', i.e. in L2: LSTM B8 N3 D256 0.874 -> 0.833 ms, B256 1.783 -> 1.481.)  The scans leave
+// compute units idle, and those of the same XCD share its L2.  So a launch gets a few more workgroups, each on a compute unit of its
+// own, which request what the scan will need some steps later; the scan's own requests find it in L2.
+// They follow the groups (a group's step is read off the words that its workgroups exchange, in passing), nobody waits for
+// them, and they end with the last step requested, or when their groups stop: a failed wait, or no step for kPrefetchPolls probes.
+//
+// Forward kernel, bf16, T = 1024, without and with: LSTM N3 D256 B8 0.883 -> 0.840 ms, B16 0.900 -> 0.842, B64 0.965 -> 0.854, B128 1.231 ->
+// 1.083, B256 1.787 -> 1.527; sLSTM N4 D192 B16 0.905 -> 0.832, B256 2.805 -> 2.401; GRU N3 D256 B16 0.839 -> 0.773, B256 1.492 -> 1.243;
+// LSTM B16 N1 D512 1.157 -> 1.148, D768 1.409 -> 1.402 (steps longer than a trip to HBM).
+#pragma once
+#include "frnn_common.h"
+
+namespace frnn {
+
+// Steps ahead of the one that is being computed.  3 are too few where the device moves much (forward, B64 N3 D256 -0.3 % instead of -13 %, B256
+// -9 instead of -18), 12 are as good as 6 but for B256 (-15: 12 steps of 12 groups no longer stay in an L2 beside what is stored).
+constexpr int kPrefetchAhead = 6;
+constexpr int kPrefetchPolls = 1 << 15;    // probes that see no step before such a workgroup ends
+constexpr int kPrefetchMinSteps = 16;      // sequences up to this length go without
+
+__device__ __forceinline__ u32x4 make_rsrc4(const void* p, size_t bytes) {  // (make_rsrc as a register tuple, for inline asm)
+  const u64 a = (u64)p;
+  return u32x4{(unsigned)a, (unsigned)(a >> 32) & 0xffffu, (unsigned)(bytes > 0x7fffffffu ? 0x7fffffffu : bytes), 0x00020000u};
+}
+// The kernel's arguments through a pointer that the compiler knows nothing about: what one role of a kernel reads through it is loaded
+// where that role needs it.  Read as the kernel's parameter, the loads are shared with the scan's, in front of the branches between the
+// roles, and stay in scalar registers over the time loop; the scans at the limit then move masks and pointers to vector registers
+// and back in every step.
+template <typename Args> __device__ __forceinline__ const __attribute__((address_space(4))) Args* own_args() {
+  typedef const __attribute__((address_space(4))) Args* args_t;
+  args_t p = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+// 16 bytes per lane to the LDS address `lds` + 16 * lane (out of range: no memory traffic)
+__device__ __forceinline__ void load_to_lds(u32x4 r, unsigned voff, unsigned soff, unsigned lds) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "s"(lds) : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
+// The loop of such a workgroup.  Its groups are first, first + stride, ... below `groups`; its waves share them out, or share one.
+// begun(group): the number of steps that the group has begun, as far as is known; request(group, step, part, parts): fetch this
+// wave's part of the operands of a step.
+template <typename Begun, typename Request>
+__device__ __forceinline__ void prefetch_follow(int first, int stride, int groups, int Tn, int wave, int waves, const int* status, int spin_limit, Begun begun, Request request) {
+  const int mine = first < groups ? (groups - first + stride - 1) / stride : 0;  // groups of this workgroup
+  const int parts = mine > 0 && waves >= mine ? waves / mine : 1;                // waves per group
+  const int part = wave % parts;
+  int next[2], grp[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int i = wave / parts + k * waves;
+    grp[k] = first + i * stride;
+    next[k] = i < mine ? 0 : Tn;
+  }
+  for (int polls = 0; polls <= min(spin_limit, kPrefetchPolls); ++polls) {
+    if (next[0] >= Tn && next[1] >= Tn) break;
+    bool did = false;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (next[k] >= Tn) continue;
+      const int b = begun(grp[k], next[k]), goal = min(b + kPrefetchAhead, Tn);
+      next[k] = max(next[k], min(b, Tn));  // (late: what is behind is of no use any more)
+      for (; next[k] < goal; ++next[k]) {
+        request(grp[k], next[k], part, parts);
+        did = true;
+      }
+    }
+    if (did) { polls = 0; continue; }
+    __builtin_amdgcn_s_sleep(4);
+    if ((polls & 63) == 63 && __builtin_amdgcn_readfirstlane(__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != STATUS_OK) break;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (none may land in the LDS of a workgroup that comes later)
+}
+
+// Steps begun, off the first word of a forward group's two exchange slots (`slots`, LLW words each): h of step t carries the tag of t.
+// `known`: steps requested so far; the group is at most kPrefetchAhead behind that.
+template <typename T, int LLW> __device__ __forceinline__ int forward_steps_begun(const u64* slots, int known) {
+  int begun = 0;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const u64 v = ll_load(slots + s * LLW);
+    int t1;  // t + 1, or 0
+    if constexpr (sizeof(T) == 4) t1 = (int)(v >> 32);
+    else {
+      const int tag = (int)((unsigned)v >> 16), base = max(known - kPrefetchAhead - 2, 0);  // (tag: t % 65535 + 1)
+      t1 = tag == 0 ? 0 : base + (tag - 1 + 65535 - base % 65535) % 65535 + 1;
+    }
+    begun = max(begun, t1);
+  }
+  return __builtin_amdgcn_readfirstlane(begun);
+}
+
+// The forward scan's Wx: TR rows x GW gates x D units of a step.  `junk`: LDS address of 1 KB that nobody reads.
+template <typename T, int GW, int D, int TR, int LLW>
+__device__ __forceinline__ void prefetch_wx(const void* Wx, const u64* ll, const int* status, int first, int stride, int groups, int grp0, int N, int B, int Tn, int wave, int waves,
+                                            int lane, int spin_limit, unsigned junk) {
+  constexpr int ES = (int)sizeof(T), PPR = D * ES / 16, NP = TR * GW * PPR, NI = (NP + 63) / 64;  // 16-byte pieces per row, per step; instructions
+  const unsigned ND = (unsigned)N * D;
+  const u32x4 r = make_rsrc4(Wx, (size_t)B * Tn * GW * ND * ES);
+  prefetch_follow(first, stride, groups, Tn, wave, waves, status, spin_limit,
+    [&](int g, int known) { return forward_steps_begun<T, LLW>(ll + (size_t)(grp0 + g) * 3 * LLW, known); },
+    [&](int g, int t, int part, int parts) {
+      const int n = (grp0 + g) % N, bt = (grp0 + g) / N, rows = min(TR, B - bt * TR);
+      const unsigned so = (((unsigned)bt * TR * Tn + t) * GW * ND + n * D) * ES;
+      for (int i = part; i < NI; i += parts) {
+        const int c = lane + 64 * i, q = c % PPR, row = c / PPR % TR, gate = c / (PPR * TR);
+        load_to_lds(r, c < NP && row < rows ? (((unsigned)row * Tn * GW + gate) * ND) * ES + q * 16 : kInvalidOff, so, junk);
+      }
+    });
+}
+
+}  // namespace frnn

@@ -25,21 +25,31 @@ template <int Dv, int VAR, int W, int U, int K, int MTR> static void (*fwd_kerne
   return nullptr;
 }
 
+// dynamic LDS with which two workgroups of a kernel do not fit one compute unit
+static size_t alone_on_a_compute_unit(const void* kern) {
+  hipFuncAttributes at;
+  if (hipFuncGetAttributes(&at, kern) != hipSuccess) { (void)hipGetLastError(); return 0; }
+  const size_t half = 80 * 1024 + 512, more = at.sharedSizeBytes < half ? half - at.sharedSizeBytes : 0;
+  if (more > 65536 && hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)more) != hipSuccess) { (void)hipGetLastError(); return 0; }
+  return more;
+}
+
 template <>
 int fused_fwd_launch<FRNN_F, FRNN_DT>(const Plan& p, const FwdArgs& a, hipStream_t st) {
-  const dim3 grid(grid_for(a.groups, p.kw) - p.left_out);
+  const dim3 grid(grid_for(a.groups, p.kw) - p.left_out + 8 * a.helpers);
 #define FRNN_CASE(Dv, VAR, W, U, K, MTR)                                                     \
   if (p.D == Dv && p.waves == W && p.utw == U && p.kw == K) {                                 \
     auto kern = fwd_kernel_for<Dv, VAR, W, U, K, MTR>(a.tile_rows, a.pst, p.order);                                \
     if (!kern) return FRNN_E_UNSUPPORTED;                                                     \
     /* (one more wave where the kernel has a producer wave: the same predicate as in the kernel) */ \
     const dim3 block((W + (fwd_producer_wave(Cell<FRNN_F>::GR, Dv, W, U, K, a.tile_rows, (int)sizeof(FRNN_TU_T)) ? 1 : 0)) * 64); \
+    const size_t lds = K > 1 && a.helpers ? alone_on_a_compute_unit((const void*)kern) : 0;         \
     if (K > 1 && p.cooperative) {                                                             \
       FwdArgs aa = a;                                                                         \
       void* args[] = {(void*)&aa};                                                            \
-      return (int)hipLaunchCooperativeKernel((const void*)kern, grid, block, args, 0, st);    \
+      return (int)hipLaunchCooperativeKernel((const void*)kern, grid, block, args, lds, st);    \
     }                                                                                         \
-    hipLaunchKernelGGL(kern, grid, block, 0, st, a);                                          \
+    hipLaunchKernelGGL(kern, grid, block, lds, st, a);                                          \
     return (int)hipGetLastError();                                                            \
   }
   FRNN_TU_PLANS(FRNN_CASE)
