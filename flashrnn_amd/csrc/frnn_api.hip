@@ -180,6 +180,8 @@ static int fwd_poll_delay_default(int function, int dtype, const Plan& p, int ti
   if (fwd_own_slice_first(cell_dims(function).GR, p.D, p.waves, p.utw, p.kw, tile_rows, dtype == FRNN_F32 ? 4 : 2)) {
     if (elman) return p.kw <= 8 && p.waves <= 4 && tile_rows == 4 && dtype != FRNN_F32 ? 1 : 0;
     if (p.kw > 8) return p.kw >= 16 ? 6 : p.kw < 12 ? 1 : function == FRNN_GRU ? 1 : 0;
+    // (8-row tiles that store behind the probe: lstm B128 D=256 1.018 ms with 0, 1.044 with 2, slstm B256 D=192 2.218 / 2.246)
+    if (tile_rows == 8 && function != FRNN_GRU && fwd_stores_behind_probe(4, p.D, p.waves, p.utw, p.kw, 8, dtype == FRNN_F32 ? 4 : 2)) return 0;
     return tile_rows >= 8 ? 2 : (function == FRNN_GRU || p.kw > 5) ? 1 : 0;
   }
   if (elman) return p.waves > 4 ? 2 : 6;

@@ -22,6 +22,7 @@
 //   elements instead of 4.
 //   4-row tiles: one more DPP move (row_shr:4) leaves one element per lane.
 #pragma once
+#include <type_traits>
 #include "frnn_common.h"
 
 namespace frnn {
@@ -216,21 +217,47 @@ __device__ __forceinline__ void report_failure(int* one, int* any) {
   if (any) __hip_atomic_store(any, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// `behind`: memory operations that the wave does not wait for, issued while the first probe is on its way.  In front of it they cost the
+// chain of dependent steps their issue, and the probe, which returns in order, theirs as well.  (The first probe is tested outside
+// the loop of the later ones: where both paths meet, the compiler would wait for these operations too.)
+struct NothingBehind {};
+// sends a probe, does what goes behind the first one, tests it, and carries on probing
+template <typename Probe, typename Test, typename Behind>
+__device__ __forceinline__ void probe_until(Probe probe, Test arrived, Wait& w, Behind behind) {
+  if constexpr (std::is_same_v<Behind, NothingBehind>) {
+    for (int spins = 0;; ++spins) {
+      probe();
+      if (__builtin_expect(arrived(), 1)) break;
+      if (give_up(w, spins)) break;
+    }
+  } else {
+    probe();
+    __builtin_amdgcn_sched_barrier(0);
+    behind();
+    __builtin_amdgcn_sched_barrier(0);
+    if (__builtin_expect(arrived(), 1)) return;
+    for (int spins = 0; !give_up(w, spins); ++spins) {
+      probe();
+      if (__builtin_expect(arrived(), 1)) break;
+    }
+  }
+}
+
 // Poll NW tagged words (addresses base + off[i]; every lane polls NW words, lanes or entries
 // with nothing to wait for pass need[i] = false and may point anywhere valid) until all carry the
 // tag of step t.  Loads are unconditional and the exit test is a wave vote.
-template <typename TAG, int NW, bool BITS>
-__device__ __forceinline__ void poll_words(const u64* base, const int* off, const bool* need, int t, u64* out, Wait& w, int first_delay) {
+template <typename TAG, int NW, bool BITS, typename Behind>
+__device__ __forceinline__ void poll_words(const u64* base, const int* off, const bool* need, int t, u64* out, Wait& w, int first_delay, Behind behind) {
   // (one probe of the set in flight: more only add congestion, measured again with exact waits)
   // the producers finish their step at about the same time as this wave: a probe sent at once
   // reaches memory before their stores and costs a whole extra round trip
   for (int i = 0; i < first_delay; ++i) __builtin_amdgcn_s_sleep(1);
-  for (int spins = 0;; ++spins) {
+  probe_until(
+    [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NW; ++i) out[i] = ll_load(base + off[i]);
-    if (__builtin_expect(all_arrived<TAG, NW, BITS>(out, need, t), 1)) break;
-    if (give_up(w, spins)) break;
-  }
+      for (int i = 0; i < NW; ++i) out[i] = ll_load(base + off[i]);
+    },
+    [&]() __attribute__((always_inline)) { return all_arrived<TAG, NW, BITS>(out, need, t); }, w, behind);
 }
 
 // The same wait in two halves: the first probe is sent by poll_issue, the caller does work that needs no
@@ -268,20 +295,20 @@ __device__ __forceinline__ void poll_words_reload(const W* base, const int* off,
 // The same wait for pairs of adjacent words, each pair fetched with one 16-byte agent-scope load
 // (raw buffer load, cache policy sc1): half the memory instructions per probe.  A 16-byte load is
 // not one atomic access, which the protocol does not need: every 32-bit half carries its own tag.
-template <typename TAG, int NW, bool BITS>
-__device__ __forceinline__ void poll_pairs(rsrc_t slot, unsigned soff, const int* off, const bool* need, int t, u64* out, Wait& w, int first_delay) {
+template <typename TAG, int NW, bool BITS, typename Behind>
+__device__ __forceinline__ void poll_pairs(rsrc_t slot, unsigned soff, const int* off, const bool* need, int t, u64* out, Wait& w, int first_delay, Behind behind) {
   static_assert(NW % 2 == 0, "pairs");
   for (int i = 0; i < first_delay; ++i) __builtin_amdgcn_s_sleep(1);
-  for (int spins = 0;; ++spins) {
+  probe_until(
+    [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NW; i += 2) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(slot, (unsigned)off[i] * 8u, soff, 16 /* sc1 */);
-      out[i] = (u64)v.x | ((u64)v.y << 32);
-      out[i + 1] = (u64)v.z | ((u64)v.w << 32);
-    }
-    if (__builtin_expect(all_arrived<TAG, NW, BITS>(out, need, t), 1)) break;
-    if (give_up(w, spins)) break;
-  }
+      for (int i = 0; i < NW; i += 2) {
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(slot, (unsigned)off[i] * 8u, soff, 16 /* sc1 */);
+        out[i] = (u64)v.x | ((u64)v.y << 32);
+        out[i + 1] = (u64)v.z | ((u64)v.w << 32);
+      }
+    },
+    [&]() __attribute__((always_inline)) { return all_arrived<TAG, NW, BITS>(out, need, t); }, w, behind);
 }
 // Word `off` of a vector of `tot` words in an LDS copy that starts `rot` words into the vector and wraps around
 // (tot = 0: no rotation)
@@ -289,9 +316,9 @@ __device__ __forceinline__ unsigned lds_rotated(int off, int rot, int tot) {
   const unsigned d = (unsigned)(off - rot);
   return tot ? min(d, d + (unsigned)tot) : (unsigned)off;  // (off < rot: d wraps, d + tot is the index)
 }
-template <typename T, int NP, bool BITS>
+template <typename T, int NP, bool BITS, typename Behind>
 __device__ __forceinline__ void ll_gather_pairs(rsrc_t slots, unsigned soff, const int* q, int t, T* lds_dst, Wait& w,
-                                                int first_delay, int rot = 0, int tot = 0) {
+                                                int first_delay, int rot, int tot, Behind behind) {
   constexpr int CH = NP < 16 ? NP : 16;  // words polled together
   static_assert(NP % CH == 0 && CH % 2 == 0, "poll list must split into whole chunks of pairs");
 #pragma unroll
@@ -299,7 +326,8 @@ __device__ __forceinline__ void ll_gather_pairs(rsrc_t slots, unsigned soff, con
     int off[CH]; bool need[CH]; u64 v[CH];
 #pragma unroll
     for (int i = 0; i < CH; ++i) { need[i] = q[c0 + i] >= 0; off[i] = need[i] ? q[c0 + i] : 0; }
-    poll_pairs<T, CH, BITS>(slots, soff, off, need, t, v, w, c0 == 0 ? first_delay : 0);
+    if (c0 == 0) poll_pairs<T, CH, BITS>(slots, soff, off, need, t, v, w, first_delay, behind);
+    else poll_pairs<T, CH, BITS>(slots, soff, off, need, t, v, w, 0, NothingBehind());
     // (the list is a whole number of pairs: its length, rows x columns / 2, is even)
 #pragma unroll
     for (int i = 0; i < CH; i += 2)
@@ -311,9 +339,9 @@ __device__ __forceinline__ void ll_gather_pairs(rsrc_t slots, unsigned soff, con
 
 // Forward gather: poll the planned words of slot, then copy their payloads to LDS.
 // C4: the LDS vector is kept as [k][4 rows] (the fp32 4-row tiles, see lds_index4) instead of fragment order
-template <typename T, int NP, bool BITS, bool C4 = false>
+template <typename T, int NP, bool BITS, bool C4, typename Behind>
 __device__ __forceinline__ void ll_gather(const u64* slot, const int* q, int t, T* lds_dst, Wait& w,
-                                          int first_delay, int rot = 0, int tot = 0) {
+                                          int first_delay, int rot, int tot, Behind behind) {
   constexpr int CH = NP < 16 ? NP : 16;  // words polled together
   static_assert(NP % CH == 0, "poll list must split into whole chunks");
 #pragma unroll
@@ -321,7 +349,8 @@ __device__ __forceinline__ void ll_gather(const u64* slot, const int* q, int t, 
     int off[CH]; bool need[CH]; u64 v[CH];
 #pragma unroll
     for (int i = 0; i < CH; ++i) { need[i] = q[c0 + i] >= 0; off[i] = need[i] ? q[c0 + i] : 0; }
-    poll_words<T, CH, BITS>(slot, off, need, t, v, w, c0 == 0 ? first_delay : 0);
+    if (c0 == 0) poll_words<T, CH, BITS>(slot, off, need, t, v, w, first_delay, behind);
+    else poll_words<T, CH, BITS>(slot, off, need, t, v, w, 0, NothingBehind());
 #pragma unroll
     for (int i = 0; i < CH; ++i)
       if (need[i]) reinterpret_cast<unsigned*>(lds_dst)[C4 ? lds_index4_of_word(off[i]) : lds_rotated(off[i], rot, tot)] = ll_payload((T*)0, v[i]);

@@ -472,6 +472,17 @@ fused_fwd_kernel(const FwdArgs a) {
   long long tr[3] = {0, 0, 0};
   const long long tr_begin = clock64();
 #endif
+  constexpr bool DEFER = !MB && KO == 0 && fwd_stores_behind_probe(GR, D, WAVES, UTW, KW, TR, (int)sizeof(T));
+  Dw<ND_> out_s[DEFER ? UTW : 1][S];
+  Dw<NWC> out_c[DEFER ? UTW : 1];
+  auto store_outputs = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < (DEFER ? UTW : 0); ++u) {
+#pragma unroll
+      for (int k = 0; k < S; ++k) buf_store<ND_, SB>(out_s[u][k], rSt, st_v[u], ((unsigned)k * BS * Tn + t) * ND * ES);
+      if constexpr (NC > 0) buf_store_wide<NWC>(out_c[u], rCa, ca_v[u], (((unsigned)t * N + n) * (D / 16)) * Bpad * 16 * NCP * ES);
+    }
+  };
   bool dead = near_i < 0;
   bool stopped = false;  // resident decode kernel: a wait for a token gave up (idle bound or stop word)
   // one time step: consumes `wc` (Wx of step t), prefetches Wx of step t+PD into `wn`
@@ -507,8 +518,12 @@ fused_fwd_kernel(const FwdArgs a) {
     if (t > 0) {
       if (KW > 1) {
         Wait w{a.status, &dead_flag, a.spin_limit};
-        if constexpr (PAIRS) ll_gather_pairs<T, NP, !LANE_TESTS>(rLL, (unsigned)((t - 1) & 1) * LLW * 8u, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
-        else ll_gather<T, NP, !LANE_TESTS, M44>(llbase + (size_t)((t - 1) & 1) * LLW, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0);
+        auto gather = [&](auto behind) __attribute__((always_inline)) {
+          if constexpr (PAIRS) ll_gather_pairs<T, NP, !LANE_TESTS>(rLL, (unsigned)((t - 1) & 1) * LLW * 8u, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0, behind);
+          else ll_gather<T, NP, !LANE_TESTS, M44>(llbase + (size_t)((t - 1) & 1) * LLW, qpoll, t - 1, hbuf[cur], w, a.poll_delay, rot_w, OWN_FIRST ? LLW : 0, behind);
+        };
+        if constexpr (DEFER) gather([&]() __attribute__((always_inline)) { store_outputs(t - 1); });
+        else gather(NothingBehind());
         if (barrier_or(&dead_flag)) { dead = true; return; }
       } else {
         lds_barrier();
@@ -763,6 +778,10 @@ fused_fwd_kernel(const FwdArgs a) {
             for (int i = 0; i < NWC; ++i) dst[i] = cw.v[i];
           }
         }
+      } else if constexpr (DEFER) {
+#pragma unroll
+        for (int k = 0; k < S; ++k) out_s[u][k] = pack<E>(so[k], (T*)0);
+        if constexpr (NC > 0) out_c[u] = cache_pack<T, NCA, E>(cv);
       } else {
 #pragma unroll
       for (int k = 0; k < S; ++k)
@@ -813,6 +832,7 @@ fused_fwd_kernel(const FwdArgs a) {
   for (int j = 0; j < PD; ++j)
     if (!MB && !dead && t + j < Tn) step(t + j, wx[j], wx[(j + PD) % (PD + 1)]);
 
+  if constexpr (DEFER) { if (!dead) store_outputs(Tn - 1); }
   if constexpr (PST) lds_barrier();  // (the last step's outputs are in LDS: the producer wave stores them behind this barrier)
 #ifdef FRNN_TRACE
   if (lane == 0 && a.trace) {

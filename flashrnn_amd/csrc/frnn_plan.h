@@ -149,6 +149,16 @@ constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, in
          (fwd_lds_ksteps(GR, D, WAVES, UTW, esize) == 0 || KW <= 12) && (D / KW) % KM == 0 &&
          !(esize == 4 && UTW * GR * KS >= 256 && TR >= (KW > 8 ? 8 : 16));
 }
+// Forward kernel: the outputs of a step are stored behind the first probe of the next step, while it is on its way, instead of in front
+// of it.  For the gated cells in the 16-bit types whose product over the own slice comes before the probe: workgroups of 4 waves, up to 8
+// per head at 4-row tiles and 5 at 8-row tiles; their first probe mostly finds the words.  (A second one has to wait for the stores.)  Forward, T =
+// 384: LSTM N3 D256 B16 0.325 -> 0.302 ms, B64 0.338 -> 0.314, B128 0.422 -> 0.404, N2 D320 B16 0.341 -> 0.333, sLSTM N4 D192 B16 0.321 -> 0.297, B128
+// 0.474 -> 0.441, GRU N3 D256 B16 0.314 -> 0.296, N2 D384 0.350 -> 0.337, D512 0.397 -> 0.394.  Elsewhere the words come later than the first probe:
+// 8-row tiles of 6 and more workgroups +2 to +6 %, waves that split k +4 to +10, 10 workgroups and more +5 to +8, 16-row tiles and the
+// dense tilings +2 to +9, fp32 +4 to +9; the Elman cell -1.5 to +0.5.
+constexpr bool fwd_stores_behind_probe(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize) {
+  return esize == 2 && GR >= 3 && WAVES == 4 && KW <= (TR == 4 ? 8 : TR == 8 ? 5 : 0) && fwd_own_slice_first(GR, D, WAVES, UTW, KW, TR, esize);
+}
 }
 
 // Measured on MI355X (T = 1024, bf16): when the head fits one workgroup, one tile per wave and
