@@ -224,6 +224,12 @@ static int helpers_for(const Plan& p, int groups, int T) {
   h = h < idle ? h : idle;
   return h > 0 ? h : 0;
 }
+// The same for a reverse scan, which gets one for each group or none: one for several, bf16, T = 512, against none, LSTM B64 N3 D256 +25 %, GRU B256 +19, sLSTM B16
+// N4 D192 +7 (the backward pass; the kernels that such a launch takes rely on operands in L2)
+static int reverse_helpers_for(const Plan& p, int groups, int T) {
+  const int h = helpers_for(p, groups, T);
+  return h == (groups + 7) / 8 ? h : 0;
+}
 // (such groups never share an XCD: no handshake, every exchange store at agent scope)
 static bool near_stores_possible(const Plan& p) { return p.kw > 1 && p.kw <= kXcdWorkgroups; }
 
@@ -1012,7 +1018,7 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   const int dsp = bwd_dest_split(p.D, p.waves, p.utw, p.kw);
   const int wide_delay = half && dsp > 1 ? (p.kw <= 4 || p.kw >= 16 ? 0 : p.kw == 8 ? 1 : 2) : half || dsp != 4 ? 2
                        : p.kw <= 4 ? 0 : p.kw < 10 ? 2 : p.kw <= 16 ? 4 : p.kw <= 28 ? 6 : 2;
-  a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", o.rc ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && dsp == 1 && tr == 4 || half && p.kw >= 32 ? 0 : p.kw == 40 ? 14 : wide_delay);
+  const int poll_delay = o.rc ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && dsp == 1 && tr == 4 || half && p.kw >= 32 ? 0 : p.kw == 40 ? 14 : wide_delay;
   a.g_clip = o.g_clip; a.cut = o.cut;
   a.pst = env_int("FRNN_PRODUCER_STORES", tr == 4 && p.kw == 1 && bwd_producer_stores_pay(fx, p, groups, o.rc) ? 1 : 0);
   a.trace = nullptr;
@@ -1022,6 +1028,9 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   LaunchGate* gate = gate_enter(a.cut ? 1 : p.kw, st);  // (the truncated reverse scan exchanges nothing)
   for (int g0 = 0; g0 < groups; g0 += per_launch) {
     a.grp0 = g0; a.groups = groups - g0 < per_launch ? groups - g0 : per_launch;
+    a.helpers = a.cut || call.beside || !bwd_prefetched(c.GR, p.D, p.waves, p.utw, p.kw, tr, dtype == FRNN_F32 ? 4 : 2, o.rc != 0) ? 0 : reverse_helpers_for(p, a.groups, T);
+    // (with the operands in L2, LSTM B8 N3 D256: 0 942 us, 2 950, sLSTM B16 N4 D192 900 / 918, D=384 585 / 574; 8- and 16-row tiles, GRU B256 N3 D256: 0 938, 2 953, 4 915)
+    a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", !a.helpers ? poll_delay : tr > 4 ? (fx == FRNN_GRU ? 4 : poll_delay) : p.kw <= 8 ? 0 : poll_delay);
     prof_begin("fused_bwd_kernel", st);
     switch (fx) {
       case FRNN_LSTM:  e = fused_bwd_dispatch<FRNN_LSTM>(dtype, p, a, st); break;

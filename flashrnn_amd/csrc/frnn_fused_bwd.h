@@ -56,6 +56,7 @@ struct BwdArgs {
   // recompute mode (kernels instantiated with RC = true): no gate cache; the gates of step t are rebuilt from
   // Wx_t, b and R h_(t-1), with h_(t-1) read back from the stored states
   const void* Wx; const void* R; const void* b;
+  int helpers;   // workgroups per XCD behind those of the scan that fetch its operands into the XCD's L2 (frnn_prefetch.h)
   int pst;  // host side only: launch the instantiation whose producer wave stores dWx (bwd_producer_stores)
 };
 
@@ -177,6 +178,22 @@ fused_bwd_kernel(const BwdArgs a) {
   __shared__ float rsum[RSP ? NPOS * (DSP - 1) * UTW * O::E * 64 : 1];  // sums of the sources polled by the other waves: [position][wave - 1][tile][element][lane]
 
   int grp_l, slice;
+  // FETCHED (an instantiation of its own): the launch has workgroups that fetch the operands into L2, and the groups say how far they are
+  constexpr bool FETCHED = PSTV && KW > 1;
+  static_assert(!FETCHED || bwd_prefetched(GR, D, WAVES, UTW, KW, TR, (int)sizeof(T), RC), "instantiated without need");
+  if constexpr (FETCHED) {
+    const int scan = 8 * KW * ((a.groups + 7) / 8);  // workgroups of the scan, then 8 of those that prefetch for each of a.helpers
+    if ((int)blockIdx.x >= scan) {
+      static_assert(KW <= kXcdWorkgroups, "groups within an XCD");
+      static_assert(2 * 16 * KDL * (int)sizeof(T) >= 1024, "room for what is fetched");
+      const auto pa = own_args<BwdArgs>();
+      prefetch_reverse<T, S, CacheBlk<T, NCA>::NCP, CXS >= 0 ? C::SPM & ~(1 << (CXS >= 0 ? CXS : 0)) : C::SPM, C::DSM, D, TR>(
+        pa->cache, pa->states, pa->dstates, reinterpret_cast<const unsigned*>(pa->ll) + 2 * INW, 3 * INW, pa->status, (int)blockIdx.x - scan, 8 * pa->helpers,
+        pa->groups, pa->grp0, pa->N, pa->B, pa->BS, pa->T, __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)blockDim.x >> 6, threadIdx.x & 63, pa->spin_limit,
+        (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem_raw);
+      return;
+    }
+  }
   if (!decode_block(a.groups, KW, grp_l, slice)) return;
   const int grp = a.grp0 + grp_l;
   const int N = a.N, Tn = a.T, B = a.B, BS = a.BS;
@@ -548,6 +565,13 @@ fused_bwd_kernel(const BwdArgs a) {
   typedef typename PT::Word IW;
   IW* const inbox = reinterpret_cast<IW*>(a.ll) + (size_t)grp * 3 * INW;
 
+  // steps begun, for the workgroups that prefetch: the first word of the third area, which no padded lane has (lane 0 is row 0).  Stored by the
+  // second wave of the first pair, which has nothing else to do by then, in kernels without pairs by the first wave
+  constexpr bool TELL_IDLE = FETCHED && DSP > 1;
+  unsigned* const begun_word = reinterpret_cast<unsigned*>(inbox + 2 * INW);
+  const rsrc_t rBegun = make_rsrc(begun_word, FETCHED && !TELL_IDLE ? 4 : 0);
+  const unsigned begun_v = tid == 0 && slice == 0 ? 0u : kInvalidOff;
+
   // operands of one step.  s_t is not among them: it is the s_(t-1) of the step before (kept in
   // registers, `sn` below), so only the first step loads it
   // recompute mode: h_(t-1) of the whole head (TR rows x D) goes from the stored states to LDS in pieces of HC
@@ -582,7 +606,10 @@ fused_bwd_kernel(const BwdArgs a) {
 #ifdef FRNN_PD
   constexpr int PD = RC ? 2 : KW == 1 ? FRNN_PD : 1;
 #else
-  constexpr int PD = RC ? 2 : KW > 1 || WAVES >= 8 || PW ? 1 : 3;  // measured: with 8 waves and more, other waves hide the fetch
+  constexpr bool DEFER = FETCHED && bwd_operands_behind_probe(GR, TR);
+  static_assert(!FETCHED || !RSP, "the second wave of a pair has nothing to wait for");
+  static_assert(!DEFER || ROUNDS == 1, "one round of polling: a second one would wait for what goes behind the first probe");
+  constexpr int PD = RC || DEFER ? 2 : KW > 1 || WAVES >= 8 || PW ? 1 : 3;  // measured: with 8 waves and more, other waves hide the fetch
 #endif
   Pre pre[PD + 1];
   auto load_pre = [&](Pre& p, int t) __attribute__((always_inline)) {
@@ -627,6 +654,8 @@ fused_bwd_kernel(const BwdArgs a) {
   }
   __syncthreads();
   const int near_i = KW > 1 ? __builtin_amdgcn_readfirstlane(near_word) : 0;  // 1: stores stay in the XCD's L2, -1: wait ran out
+  // (a group that has come to run on several XCDs: nothing to fetch for)
+  if constexpr (FETCHED) { if (near_i <= 0) __hip_atomic_store(begun_word, (unsigned)Tn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
   u64 near_m;  // lane mask for ll_store_sel: all ones or zero, in scalar registers
   asm("s_cmp_gt_i32 %1, 0\n\ts_cselect_b64 %0, -1, 0" : "=s"(near_m) : "s"(near_i) : "scc");
 
@@ -736,7 +765,7 @@ fused_bwd_kernel(const BwdArgs a) {
     FRNN_STAMP(c0);
     // (readfirstlane: the compiler otherwise forms max(t - PD, 0) with a saturating VALU subtract
     // and then wraps a buffer load that uses it as a scalar offset into a waterfall loop)
-    if constexpr (!(PW && !cut)) { if (DSP == 1 || hf == 0) load_pre(pn, __builtin_amdgcn_readfirstlane(t >= PD ? t - PD : 0)); }
+    if constexpr (!((PW || DEFER) && !cut)) { if (DSP == 1 || hf == 0) load_pre(pn, __builtin_amdgcn_readfirstlane(t >= PD ? t - PD : 0)); }
     // dWx_t (and the GRU's g-gate cotangent).  With an exchange the stores are issued after the
     // partial sums are sent, where they fill the wait for the other workgroups instead of delaying
     // the barrier (a vector memory instruction costs ~30 cycles to issue)
@@ -751,6 +780,13 @@ fused_bwd_kernel(const BwdArgs a) {
 #pragma unroll
       for (int g = 0; g < GW; ++g) buf_store<ND_, SB>(dwp[u][g], rDw, wx_v[u], ((unsigned)t * GW + g) * ND * ES);
       if (F == FRNN_GRU) buf_store<ND_, SB>(dxp[u], rDx, st_v[u], (unsigned)t * ND * ES);
+    };
+    auto tell = [&]() __attribute__((always_inline)) {
+      if constexpr (TELL_IDLE) {
+        if (w_u == 1 && slice == 0 && lane == 0) __hip_atomic_store(begun_word, (unsigned)(Tn - t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      } else if constexpr (FETCHED) {
+        __builtin_amdgcn_raw_buffer_store_b32((unsigned)(Tn - t), rBegun, begun_v, 0, 0);
+      }
     };
     if (DSP == 1 || hf == 0) {  // (wave-uniform: the second wave of a pair owns no element)
 #pragma unroll
@@ -1121,10 +1157,11 @@ fused_bwd_kernel(const BwdArgs a) {
             ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * EW, sslot, wv, near_m);
         }
       }
-      if constexpr (DW_LATE) {
+      if constexpr (DW_LATE && !DEFER) {
         if (DSP == 1 || hf == 0) {
 #pragma unroll
           for (int u = 0; u < UTW; ++u) store_dw(u);
+          if constexpr (!TELL_IDLE) tell();
         }
       }
       if constexpr (OWN_LAST) {
@@ -1159,6 +1196,14 @@ fused_bwd_kernel(const BwdArgs a) {
       const IW* const mine = inbox + (size_t)(t & 1) * INW + ((size_t)(slice * NPOS + wp) * UTW) * KW * EW + lane;
       // fp32 wave pairs of the GRU, 14 and 16 workgroups per head: asked in front of the next probe (reverse kernel, T = 256, B8 N2, next
       // probe first against this: D = 512 0.668 -> 0.659 ms, where the shorter waits had cost 2 %, D = 448 0.605 -> 0.590)
+      // what goes behind the first probe (bwd_operands_behind_probe)
+      auto behind_probe = [&]() __attribute__((always_inline)) {
+        load_pre(pn, __builtin_amdgcn_readfirstlane(t >= PD ? t - PD : 0));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UTW; ++u) store_dw(u);
+        if constexpr (!TELL_IDLE) tell();
+      };
       constexpr bool SEND_FIRST = !(F == FRNN_GRU && sizeof(T) == 4 && DSP == 2 && KW >= 14);
       if constexpr (RSP) {
         const int rbeg = 1 + hf * SRC_W;  // (uniform) this wave's sources: rbeg .. rbeg + SRC_W - 1, below KW
@@ -1186,7 +1231,7 @@ fused_bwd_kernel(const BwdArgs a) {
           // (groups that span the device probe memory: the shorter waits had them probe more often, at D = 640 in front of the words;
           // a pause between the probes 0.4 to 1.5 % at every batch size, two units less, four and eight slower; see also the
           // first-probe delay)
-          poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0);
+          poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0, NothingBehind());
 #pragma unroll
           for (int rr = 0; rr < PSRC_W; ++rr) {
             const bool in = k0 + rr < SRC_W && rbeg + k0 + rr < KW;
@@ -1250,7 +1295,8 @@ fused_bwd_kernel(const BwdArgs a) {
             if (never()) { dead = true; return; }  // (without an exit here the sLSTM's D = 128 kernel spills)
           }
         } else {
-          poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0);
+          if constexpr (DEFER) poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, a.poll_delay, behind_probe);
+          else poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0, NothingBehind());
         }
 #pragma unroll
         for (int rr = 0; rr < PSRC; ++rr)
@@ -1261,7 +1307,7 @@ fused_bwd_kernel(const BwdArgs a) {
               for (int e = 0; e < E; ++e) ds[u][e][0] += part_value((PT*)0, v[(rr * UTW + u) * E + e]);
           }
       }
-      }
+      } else if constexpr (TELL_IDLE) tell();
     }
     if constexpr (RCP) rebuild_math(pn, racc);  // (behind step 0: of nothing, unused)
     else if constexpr (RC && KW == 1) {
@@ -1302,7 +1348,7 @@ fused_bwd_kernel(const BwdArgs a) {
       }
     };
     if (a.cut) run(std::true_type{}); else run(std::false_type{});
-  } else if (a.cut) {
+  } else if (!FETCHED && a.cut) {
     for (; t >= PD; t -= PD + 1) {
 #pragma unroll
       for (int j = 0; j <= PD; ++j) step(std::true_type{}, t - j, pre[j], pre[j], pre[(j + PD) % (PD + 1)]);

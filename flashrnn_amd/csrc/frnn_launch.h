@@ -2,6 +2,8 @@
 #pragma once
 #include "frnn_common.h"
 #include "frnn_plan.h"
+#include <mutex>
+#include <unordered_map>
 
 namespace frnn {
 
@@ -19,6 +21,27 @@ template <int F, int DT> int fused_dec_launch(const Plan& p, const FwdArgs& a, h
 // plan table lookup: function, dtype, D, variant -> plan; false if none.
 // backward: 0 forward, 1 reverse scan with gate cache, 2 reverse scan in recompute mode
 bool find_plan(int function, int dtype, int D, int variant, int backward, Plan* out);
+
+// dynamic LDS with which two workgroups of a kernel do not fit one compute unit (its static LDS, a constant of the code object, is asked once:
+// the question takes longer than the rest of a launch)
+inline size_t alone_on_a_compute_unit(const void* kern) {
+  static std::mutex lock;
+  static std::unordered_map<const void*, size_t> known;
+  size_t more;
+  {
+    std::lock_guard<std::mutex> g(lock);
+    const auto it = known.find(kern);
+    if (it != known.end()) more = it->second;
+    else {
+      hipFuncAttributes at;
+      if (hipFuncGetAttributes(&at, kern) != hipSuccess) { (void)hipGetLastError(); return 0; }
+      const size_t half = 80 * 1024 + 512;
+      more = known[kern] = at.sharedSizeBytes < half ? half - at.sharedSizeBytes : 0;
+    }
+  }
+  if (more > 65536 && hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)more) != hipSuccess) { (void)hipGetLastError(); return 0; }
+  return more;
+}
 
 }  // namespace frnn
 

@@ -159,6 +159,22 @@ constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, in
 constexpr bool fwd_stores_behind_probe(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize) {
   return esize == 2 && GR >= 3 && WAVES == 4 && KW <= (TR == 4 ? 8 : TR == 8 ? 5 : 0) && fwd_own_slice_first(GR, D, WAVES, UTW, KW, TR, esize);
 }
+// Reverse kernels with an instantiation for launches that have workgroups which fetch its operands into L2 (frnn_prefetch.h): 16-bit types, gated
+// cells, and either pairs of waves that split the destinations (4-row tiles, up to 16 workgroups per head) or 8- and 16-row tiles of up to 5
+// workgroups per head.  Whole backward pass, bf16, T = 512, without and with: LSTM B8 T1024 N3 D256 958 -> 942 us, B16 N4 D192 463 -> 451, N1 D384 589 ->
+// 575, D512 674 -> 655, sLSTM B16 T1024 N4 D192 933 -> 900, D512 694 -> 668, GRU B16 N1 D512 650 -> 610; taller tiles: LSTM B256 N3 D256 1240 -> 1189, sLSTM
+// B128 N4 D192 886 -> 813, B256 1411 -> 1350, GRU B128 N3 D256 700 -> 663, B256 995 -> 911.  Elsewhere: taller tiles of 6 to 10 workgroups -0.5 to
+// +2.7 %, 4-row tiles without pairs +-1 (LSTM B64 N3 D256), GRU +6 at D = 768 (20 workgroups and more, whose second waves poll), fours of waves
+// (sLSTM D = 256) 0, fp32 -0.3 to +4, recompute mode +-1.
+constexpr bool bwd_prefetched(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize, bool rc) {
+  return esize == 2 && GR >= 3 && KW > 1 && !rc && UTW == 1 &&
+         (TR == 4 ? bwd_dest_split(D, WAVES, UTW, KW) == 2 && KW <= 16 : bwd_dest_split(D, WAVES, UTW, KW) == 1 && KW <= 5);
+}
+// Of these, the kernels that store dWx and request the operands of the step after next behind the first probe, while it is on its way, instead of in front
+// of it and at the head of a step: what a wave asks of memory costs it ~30 cycles each and a probe returns behind it.  Only with operands
+// that are in L2 (from HBM a second probe waits for them: LSTM B8 N3 D256 964 -> 1073 us), and with registers for one more set of them: 4-row tiles, and 8-row
+// tiles of the GRU (the others' and the 16-row ones spill).
+constexpr bool bwd_operands_behind_probe(int GR, int TR) { return TR <= (GR == 3 ? 8 : 4); }
 }
 
 // Measured on MI355X (T = 1024, bf16): when the head fits one workgroup, one tile per wave and

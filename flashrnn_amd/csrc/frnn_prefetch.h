@@ -6,8 +6,8 @@
 // a build whose Wx is always the same two steps', i.e. in L2: LSTM B8 N3 D256 0.874 -> 0.833 ms, B256 1.783 -> 1.481.)  The scans leave
 // compute units idle, and those of the same XCD share its L2.  So a launch gets a few more workgroups, each on a compute unit of its
 // own, which request what the scan will need some steps later; the scan's own requests find it in L2.
-// They follow the groups (a group's step is read off the words that its workgroups exchange, in passing), nobody waits for
-// them, and they end with the last step requested, or when their groups stop: a failed wait, or no step for kPrefetchPolls probes.
+// They follow the groups (forward: a group's step is read off the words that its workgroups exchange, in passing; reverse: the group writes it down, as
+// the 2 bits of a step that its words carry are lost as soon as such a workgroup falls 6 steps behind), nobody waits for them, and they end with the last step requested, or when their groups stop: a failed wait, or no step for kPrefetchPolls probes.
 //
 // Forward kernel, bf16, T = 1024, without and with: LSTM N3 D256 B8 0.883 -> 0.840 ms, B16 0.900 -> 0.842, B64 0.965 -> 0.854, B128 1.231 ->
 // 1.083, B256 1.787 -> 1.527; sLSTM N4 D192 B16 0.905 -> 0.832, B256 2.805 -> 2.401; GRU N3 D256 B16 0.839 -> 0.773, B256 1.492 -> 1.243;
@@ -21,7 +21,8 @@ namespace frnn {
 // -9 instead of -18), 12 are as good as 6 but for B256 (-15: 12 steps of 12 groups no longer stay in an L2 beside what is stored).
 constexpr int kPrefetchAhead = 6;
 constexpr int kPrefetchPolls = 1 << 15;    // probes that see no step before such a workgroup ends
-constexpr int kPrefetchMinSteps = 16;      // sequences up to this length go without
+// Sequences up to this length go without (training pass, bf16: B256 N3 D256 T19 130.7 -> 131.9 us, T32 189.5 -> 180.1; B5 T19 93.0 -> 93.5, T64 141.8 -> 139.1)
+constexpr int kPrefetchMinSteps = 24;
 
 __device__ __forceinline__ u32x4 make_rsrc4(const void* p, size_t bytes) {  // (make_rsrc as a register tuple, for inline asm)
   const u64 a = (u64)p;
@@ -98,11 +99,22 @@ template <typename T, int LLW> __device__ __forceinline__ int forward_steps_begu
   return __builtin_amdgcn_readfirstlane(begun);
 }
 
+// One wave's part of `planes` planes of `rows` (of up to TR) rows of PPR 16-byte pieces; k: the instruction that is next for this wave
+template <int PPR, int PLANES, int TR>
+__device__ __forceinline__ void fetch_rows(u32x4 r, unsigned so, unsigned row_bytes, unsigned plane_bytes, int rows, int lane, int& k, int parts, unsigned junk) {
+  constexpr int NP = PLANES * TR * PPR, NI = (NP + 63) / 64;
+  for (; k < NI; k += parts) {
+    const int c = lane + 64 * k, q = c % PPR, row = c / PPR % TR, plane = c / (PPR * TR);
+    load_to_lds(r, c < NP && row < rows ? row * row_bytes + plane * plane_bytes + q * 16 : kInvalidOff, so, junk);
+  }
+  k -= NI;
+}
+
 // The forward scan's Wx: TR rows x GW gates x D units of a step.  `junk`: LDS address of 1 KB that nobody reads.
 template <typename T, int GW, int D, int TR, int LLW>
 __device__ __forceinline__ void prefetch_wx(const void* Wx, const u64* ll, const int* status, int first, int stride, int groups, int grp0, int N, int B, int Tn, int wave, int waves,
                                             int lane, int spin_limit, unsigned junk) {
-  constexpr int ES = (int)sizeof(T), PPR = D * ES / 16, NP = TR * GW * PPR, NI = (NP + 63) / 64;  // 16-byte pieces per row, per step; instructions
+  constexpr int ES = (int)sizeof(T);
   const unsigned ND = (unsigned)N * D;
   const u32x4 r = make_rsrc4(Wx, (size_t)B * Tn * GW * ND * ES);
   prefetch_follow(first, stride, groups, Tn, wave, waves, status, spin_limit,
@@ -110,9 +122,31 @@ __device__ __forceinline__ void prefetch_wx(const void* Wx, const u64* ll, const
     [&](int g, int t, int part, int parts) {
       const int n = (grp0 + g) % N, bt = (grp0 + g) / N, rows = min(TR, B - bt * TR);
       const unsigned so = (((unsigned)bt * TR * Tn + t) * GW * ND + n * D) * ES;
-      for (int i = part; i < NI; i += parts) {
-        const int c = lane + 64 * i, q = c % PPR, row = c / PPR % TR, gate = c / (PPR * TR);
-        load_to_lds(r, c < NP && row < rows ? (((unsigned)row * Tn * GW + gate) * ND) * ES + q * 16 : kInvalidOff, so, junk);
+      int k = part;
+      fetch_rows<D * ES / 16, GW, TR>(r, so, Tn * GW * ND * ES, ND * ES, rows, lane, k, parts, junk);
+    });
+}
+
+// The reverse scan's operands of a step: the gate cache (NCP values per element), the planes DSM of the cotangent and SPM of the states before
+// the step.  `begun`: where group 0 keeps its number of steps begun, the others `stride_words` apart.
+template <typename T, int S, int NCP, int SPM, int DSM, int D, int TR>
+__device__ __forceinline__ void prefetch_reverse(const void* cache, const void* states, const void* dstates, const unsigned* begun, size_t stride_words, const int* status, int first,
+                                                 int stride, int groups, int grp0, int N, int B, int BS, int Tn, int wave, int waves, int lane, int spin_limit, unsigned junk) {
+  constexpr int ES = (int)sizeof(T), PPR = D * ES / 16;
+  const unsigned ND = (unsigned)N * D;
+  const u32x4 rSt = make_rsrc4(states, ((size_t)(S - 1) * BS + B) * Tn * ND * ES), rDs = make_rsrc4(dstates, ((size_t)(S - 1) * BS + B) * Tn * ND * ES);
+  const u32x4 rCa = make_rsrc4(cache, (size_t)Tn * N * B * D * NCP * ES);
+  prefetch_follow(first, stride, groups, Tn, wave, waves, status, spin_limit,
+    [&](int g, int) { return __builtin_amdgcn_readfirstlane((int)ll_load(begun + (size_t)(grp0 + g) * stride_words)); },
+    [&](int g, int i, int part, int parts) {
+      const int t = Tn - 1 - i, n = (grp0 + g) % N, bt = (grp0 + g) / N, rows = min(TR, B - bt * TR);
+      int k = part;
+      fetch_rows<NCP * ES, D / 16, TR>(rCa, (((unsigned)t * N + n) * (D / 16) * B + bt * TR) * 16 * NCP * ES, 16 * NCP * ES, (unsigned)B * 16 * NCP * ES, rows, lane, k, parts, junk);
+#pragma unroll
+      for (int p = 0; p < S; ++p) {
+        const unsigned so = (((unsigned)(p * BS + bt * TR) * Tn + t) * ND + n * D) * ES;
+        if ((DSM >> p) & 1) fetch_rows<PPR, 1, TR>(rDs, so, Tn * ND * ES, 0, rows, lane, k, parts, junk);
+        if ((SPM >> p) & 1 && t > 0) fetch_rows<PPR, 1, TR>(rSt, so - ND * ES, Tn * ND * ES, 0, rows, lane, k, parts, junk);
       }
     });
 }

@@ -7,33 +7,40 @@ namespace frnn {
 
 // the kernel for a tile height, or null if the tiling is not compiled that tall (a template, so that the
 // taller kernels of such a tiling are never instantiated)
-template <int Dv, int W, int U, int K, int MTR, bool RCV> static void (*bwd_kernel_for(int tile_rows, bool pst))(const BwdArgs) {
-  if constexpr (bwd_producer_stores(Cell<FRNN_F>::GR, Cell<FRNN_F>::NC, Dv, W, U, K, 4, (int)sizeof(FRNN_TU_T), RCV)) {
-    if (tile_rows == 4 && pst) return fused_bwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, 4, RCV, true>;
+// (alt: the instantiation whose producer wave stores dWx, or the one whose launch has workgroups that prefetch)
+template <int Dv, int W, int U, int K, int MTR, bool RCV, int TR> static void (*bwd_kernel_tall(bool alt))(const BwdArgs) {
+  constexpr int GR = Cell<FRNN_F>::GR, ES = (int)sizeof(FRNN_TU_T);
+  if constexpr (TR > MTR) return nullptr;
+  else {
+    if constexpr ((TR == 4 && bwd_producer_stores(GR, Cell<FRNN_F>::NC, Dv, W, U, K, 4, ES, RCV)) || bwd_prefetched(GR, Dv, W, U, K, TR, ES, RCV)) {
+      if (alt) return fused_bwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, TR, RCV, true>;
+    }
+    return fused_bwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, TR, RCV>;
   }
-  if (tile_rows == 4) return fused_bwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, 4, RCV>;
-  if constexpr (MTR >= 8) { if (tile_rows == 8) return fused_bwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, 8, RCV>; }
-  if constexpr (MTR >= 16) { if (tile_rows == 16) return fused_bwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, 16, RCV>; }
-  return nullptr;
+}
+template <int Dv, int W, int U, int K, int MTR, bool RCV> static void (*bwd_kernel_for(int tile_rows, bool alt))(const BwdArgs) {
+  return tile_rows == 4 ? bwd_kernel_tall<Dv, W, U, K, MTR, RCV, 4>(alt) : tile_rows == 8 ? bwd_kernel_tall<Dv, W, U, K, MTR, RCV, 8>(alt)
+       : tile_rows == 16 ? bwd_kernel_tall<Dv, W, U, K, MTR, RCV, 16>(alt) : nullptr;
 }
 
 template <>
 int fused_bwd_launch<FRNN_F, FRNN_DT>(const Plan& p, const BwdArgs& a, hipStream_t st) {
-  const dim3 grid(grid_for(a.groups, p.kw) - p.left_out);
+  const dim3 grid(grid_for(a.groups, p.kw) - p.left_out + 8 * a.helpers);
   const bool rc = p.recompute != 0;
   // (one more wave and its hand-over buffers where the kernel has a producer wave: the same predicate as in the kernel)
   const bool pw = bwd_producer_wave(Cell<FRNN_F>::GR, Cell<FRNN_F>::NC, p.D, p.waves, p.utw, p.kw, a.tile_rows, (int)sizeof(FRNN_TU_T), rc);
   const bool pst = a.pst && !a.cut && bwd_producer_stores(Cell<FRNN_F>::GR, Cell<FRNN_F>::NC, p.D, p.waves, p.utw, p.kw, a.tile_rows, (int)sizeof(FRNN_TU_T), rc);  // (the truncated scan has no barrier per step to hand over at)
   // (wave pairs that split the destinations keep every fragment in registers: the two dg buffers only)
   const bool ds16 = sizeof(FRNN_TU_T) == 2 && bwd_dest_split(p.D, p.waves, p.utw, p.kw) > 1;
-  const size_t lds = (ds16 ? (size_t)2 * 16 * Cell<FRNN_F>::GR * (p.D / p.kw) * sizeof(FRNN_TU_T)
+  const size_t own_lds = (ds16 ? (size_t)2 * 16 * Cell<FRNN_F>::GR * (p.D / p.kw) * sizeof(FRNN_TU_T)
                            : bwd_lds_bytes(Cell<FRNN_F>::GR, p.D, p.waves, p.utw, p.kw, (int)sizeof(FRNN_TU_T), rc)) + 16 +
                      (pw ? bwd_producer_bytes(rc ? Cell<FRNN_F>::GW : Cell<FRNN_F>::NC + (cache_carried_state(FRNN_F, (int)sizeof(FRNN_TU_T), p.D) >= 0 ? 1 : 0), Cell<FRNN_F>::S, p.waves * p.utw, a.tile_rows, (int)sizeof(FRNN_TU_T)) : 0) +
                      (pst ? bwd_producer_store_bytes(Cell<FRNN_F>::GW, FRNN_F == FRNN_GRU, p.D, a.tile_rows, (int)sizeof(FRNN_TU_T)) : 0);
 #define FRNN_CASE_(RCV, Dv, VAR, W, U, K, MTR)                                                          \
   if (rc == RCV && p.D == Dv && p.waves == W && p.utw == U && p.kw == K) {                               \
-    auto kern = bwd_kernel_for<Dv, W, U, K, MTR, RCV>(a.tile_rows, pst);                                      \
+    auto kern = bwd_kernel_for<Dv, W, U, K, MTR, RCV>(a.tile_rows, pst || a.helpers);                                      \
     if (!kern) return FRNN_E_UNSUPPORTED;                                                                \
+    const size_t alone = K > 1 && a.helpers ? alone_on_a_compute_unit((const void*)kern) : 0, lds = alone > own_lds ? alone : own_lds; \
     if (lds > 65536) {                                                                                   \
       hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
       if (e != hipSuccess) return (int)e;                                                                \

@@ -25,15 +25,6 @@ template <int Dv, int VAR, int W, int U, int K, int MTR> static void (*fwd_kerne
   return nullptr;
 }
 
-// dynamic LDS with which two workgroups of a kernel do not fit one compute unit
-static size_t alone_on_a_compute_unit(const void* kern) {
-  hipFuncAttributes at;
-  if (hipFuncGetAttributes(&at, kern) != hipSuccess) { (void)hipGetLastError(); return 0; }
-  const size_t half = 80 * 1024 + 512, more = at.sharedSizeBytes < half ? half - at.sharedSizeBytes : 0;
-  if (more > 65536 && hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)more) != hipSuccess) { (void)hipGetLastError(); return 0; }
-  return more;
-}
-
 template <>
 int fused_fwd_launch<FRNN_F, FRNN_DT>(const Plan& p, const FwdArgs& a, hipStream_t st) {
   const dim3 grid(grid_for(a.groups, p.kw) - p.left_out + 8 * a.helpers);

@@ -8,10 +8,13 @@ from test_gpu_decode import _device_inputs
 
 pytestmark = pytest.mark.gpu
 
-# T: 16 is the longest sequence that goes without.  B250 N3 D256: 12 groups of an XCD share 8 such workgroups, B120 N4 the 15 groups of an XCD 2
-CASES = [("lstm", "bfloat16", 5, 16, 3, 256), ("lstm", "bfloat16", 5, 17, 3, 256), ("slstm", "float16", 9, 18, 4, 192), ("gru", "bfloat16", 250, 23, 3, 256),
-         ("lstm", "float16", 250, 25, 3, 256), ("lstm", "bfloat16", 517, 19, 2, 256), ("slstm", "bfloat16", 120, 21, 4, 192), ("lstm", "bfloat16", 9, 29, 1, 768),
-         ("elman", "bfloat16", 17, 31, 1, 1024), ("gru", "float32", 6, 27, 3, 160), ("lstm", "float32", 33, 22, 2, 256), ("gru", "bfloat16", 131, 24, 2, 384)]
+# T: 24 is the longest sequence that goes without.  B250 N3 D256: 12 groups of an XCD share 8 such workgroups, B120 N4 the 15 groups of an XCD 2
+CASES = [("lstm", "bfloat16", 5, 24, 3, 256), ("lstm", "bfloat16", 5, 25, 3, 256), ("slstm", "float16", 9, 26, 4, 192), ("gru", "bfloat16", 250, 31, 3, 256),
+         ("lstm", "float16", 250, 33, 3, 256), ("lstm", "bfloat16", 517, 27, 2, 256), ("slstm", "bfloat16", 120, 29, 4, 192), ("lstm", "bfloat16", 9, 37, 1, 768),
+         ("elman", "bfloat16", 17, 39, 1, 1024), ("gru", "float32", 6, 35, 3, 160), ("lstm", "float32", 33, 30, 2, 256), ("gru", "bfloat16", 131, 32, 2, 384),
+         # reverse: pairs of waves at both ends of their rule, ragged 8- and 16-row tiles, several launches
+         ("lstm", "float16", 7, 45, 1, 512), ("slstm", "bfloat16", 3, 25, 1, 448), ("gru", "bfloat16", 18, 49, 2, 512), ("lstm", "bfloat16", 99, 28, 4, 192),
+         ("gru", "float16", 67, 26, 3, 256), ("slstm", "float16", 131, 27, 3, 256), ("gru", "bfloat16", 517, 25, 2, 256)]
 
 
 @pytest.mark.parametrize("function,dtype,B,T,N,D", CASES)
@@ -35,7 +38,8 @@ def test_same_bits_with_and_without(gpu, monkeypatch, function, dtype, B, T, N, 
         assert all(torch.equal(a, b) for a, b in zip(out[0], other))
 
 
-@pytest.mark.parametrize("function,dtype,B,T,N,D", [("lstm", "bfloat16", 7, 33, 3, 256), ("gru", "float16", 131, 18, 2, 256), ("slstm", "float32", 5, 20, 2, 128)])
+@pytest.mark.parametrize("function,dtype,B,T,N,D", [("lstm", "bfloat16", 7, 41, 3, 256), ("gru", "float16", 131, 26, 2, 256), ("slstm", "float32", 5, 28, 2, 128),
+                                                  ("gru", "bfloat16", 6, 26, 1, 512), ("slstm", "bfloat16", 99, 25, 4, 192)])
 def test_matches_the_oracle(gpu, function, dtype, B, T, N, D):
     print(f"case prefetch oracle {function} {dtype} B{B} T{T} N{N} D{D}", flush=True)
     check_case(gpu, function, B, T, N, D, dtype, "hip_fused", seed=47)
