@@ -180,7 +180,7 @@ fused_bwd_kernel(const BwdArgs a) {
   int grp_l, slice;
   // FETCHED (an instantiation of its own): the launch has workgroups that fetch the operands into L2, and the groups say how far they are
   constexpr bool FETCHED = PSTV && KW > 1;
-  static_assert(!FETCHED || bwd_prefetched(GR, D, WAVES, UTW, KW, TR, (int)sizeof(T), RC), "instantiated without need");
+  static_assert(!FETCHED || bwd_prefetched(GR, NC, D, WAVES, UTW, KW, TR, (int)sizeof(T), RC), "instantiated without need");
   if constexpr (FETCHED) {
     const int scan = 8 * KW * ((a.groups + 7) / 8);  // workgroups of the scan, then 8 of those that prefetch for each of a.helpers
     if ((int)blockIdx.x >= scan) {
@@ -606,10 +606,8 @@ fused_bwd_kernel(const BwdArgs a) {
 #ifdef FRNN_PD
   constexpr int PD = RC ? 2 : KW == 1 ? FRNN_PD : 1;
 #else
-  constexpr bool DEFER = FETCHED && bwd_operands_behind_probe(GR, TR);
   static_assert(!FETCHED || !RSP, "the second wave of a pair has nothing to wait for");
-  static_assert(!DEFER || ROUNDS == 1, "one round of polling: a second one would wait for what goes behind the first probe");
-  constexpr int PD = RC || DEFER ? 2 : KW > 1 || WAVES >= 8 || PW ? 1 : 3;  // measured: with 8 waves and more, other waves hide the fetch
+  constexpr int PD = RC ? 2 : KW > 1 || WAVES >= 8 || PW ? 1 : 3;  // measured: with 8 waves and more, other waves hide the fetch
 #endif
   Pre pre[PD + 1];
   auto load_pre = [&](Pre& p, int t) __attribute__((always_inline)) {
@@ -750,6 +748,54 @@ fused_bwd_kernel(const BwdArgs a) {
     rebuild_gates(pre[0], Tn - 1);
   }
 
+  // The half of the adjoint of a step that does not depend on the running cotangent (operands unpacked, tanh(c), the products of the gates).
+  // EARLY: done for the step to come while the first probe of the wait is on its way, off the chain of dependent steps.
+  constexpr bool EARLY = KW > 1 && !RC && (RSP ? ROUNDS_W : ROUNDS) == 1 && bwd_adjoint_early(GR, NC, UTW, KW, TR, (int)sizeof(T), FETCHED);
+  constexpr bool TWIN = bwd_prefetched(GR, NC, D, WAVES, UTW, KW, TR, (int)sizeof(T), RC);  // one of two kernels that differ in FETCHED
+  float prep[EARLY ? UTW : 1][E][CM::NP];
+  auto prepare = [&](const Pre& p, int u, float (&out)[E][CM::NP]) __attribute__((always_inline)) {
+    float cv[NCA][E], spv[S][E], snv[S][E], dsov[S][E];
+    if constexpr (NC > 0 && !RC) cache_unpack<T, NCA, E>(p.cache[u], cv);
+    if constexpr (NC > 0 && RC) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int e = 0; e < E; ++e) cv[c][e] = gc[u][c][e];
+    }
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      unpack<E>(sn[u][k], snv[k], (T*)0); unpack<E>(p.dso[u][k], dsov[k], (T*)0);
+      if (CXU && k == CXS) {  // (from the cache line; packed again, exactly, for the next step)
+#pragma unroll
+        for (int e = 0; e < E; ++e) spv[k][e] = cv[NC][e];
+        sn[u][k] = pack<E>(cv[NC], (T*)0);
+        continue;
+      }
+      unpack<E>(p.sp[u][k], spv[k], (T*)0);
+      sn[u][k] = p.sp[u][k];  // s_(t-1) is the s_t of the next step
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      float cc[NCA], sp1[S], sn1[S], dso1[S];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) cc[c] = cv[c][e];
+#pragma unroll
+      for (int k = 0; k < S; ++k) { sp1[k] = spv[k][e]; sn1[k] = snv[k][e]; dso1[k] = dsov[k][e]; }
+      CM::prepare(cc, sp1, sn1, dso1, out[e]);
+      // (EARLY: left alone, the compiler sinks it to its use.  TWIN, fp16: the same products and sums in both kernels)
+      if constexpr (EARLY || (TWIN && std::is_same_v<T, half_t>)) {
+#pragma unroll
+        for (int i = 0; i < CM::NP; ++i) asm volatile("" : "+v"(out[e][i]));
+      }
+    }
+  };
+  if constexpr (EARLY) {
+    if (!a.cut) {
+#pragma unroll
+      for (int u = 0; u < UTW; ++u) prepare(pre[0], u, prep[u]);
+    }
+  }
+
   bool dead = near_i < 0;
   // does a step look at the workgroup's flag of a failed wait?  Heads of one workgroup never wait, and nobody sets it
   constexpr bool FLAG = KW > 1;
@@ -765,7 +811,7 @@ fused_bwd_kernel(const BwdArgs a) {
     FRNN_STAMP(c0);
     // (readfirstlane: the compiler otherwise forms max(t - PD, 0) with a saturating VALU subtract
     // and then wraps a buffer load that uses it as a scalar offset into a waterfall loop)
-    if constexpr (!((PW || DEFER) && !cut)) { if (DSP == 1 || hf == 0) load_pre(pn, __builtin_amdgcn_readfirstlane(t >= PD ? t - PD : 0)); }
+    if constexpr (!(PW && !cut)) { if (DSP == 1 || hf == 0) load_pre(pn, __builtin_amdgcn_readfirstlane(t >= PD ? t - PD : 0)); }
     // dWx_t (and the GRU's g-gate cotangent).  With an exchange the stores are issued after the
     // partial sums are sent, where they fill the wait for the other workgroups instead of delaying
     // the barrier (a vector memory instruction costs ~30 cycles to issue)
@@ -791,36 +837,21 @@ fused_bwd_kernel(const BwdArgs a) {
     if (DSP == 1 || hf == 0) {  // (wave-uniform: the second wave of a pair owns no element)
 #pragma unroll
     for (int u = 0; u < UTW; ++u) {
-      float cv[NCA][E], spv[S][E], snv[S][E], dsov[S][E];
-      if constexpr (NC > 0 && !RC) cache_unpack<T, NCA, E>(pc.cache[u], cv);
-      if constexpr (NC > 0 && RC) {
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-#pragma unroll
-          for (int e = 0; e < E; ++e) cv[c][e] = gc[u][c][e];
-      }
-#pragma unroll
-      for (int k = 0; k < S; ++k) {
-        unpack<E>(sn[u][k], snv[k], (T*)0); unpack<E>(pc.dso[u][k], dsov[k], (T*)0);
-        if (CXU && k == CXS) {  // (from the cache line; packed again, exactly, for the next step)
-#pragma unroll
-          for (int e = 0; e < E; ++e) spv[k][e] = cv[NC][e];
-          sn[u][k] = pack<E>(cv[NC], (T*)0);
-          continue;
-        }
-        unpack<E>(pc.sp[u][k], spv[k], (T*)0);
-        sn[u][k] = pc.sp[u][k];  // s_(t-1) is the s_t of the next step
-      }
+      if constexpr (!EARLY || cut) prepare(pc, u, prep[EARLY ? u : 0]);
       float dgr[GR][E], dgw[GW][E];
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        float cc[NCA], sp[S], sn[S], dso[S], gr[GR], gw[GW], gb_[GT];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) cc[c] = cv[c][e];
-#pragma unroll
-        for (int k = 0; k < S; ++k) { sp[k] = spv[k][e]; sn[k] = snv[k][e]; dso[k] = dsov[k][e]; }
+        float gr[GR], gw[GW], gb_[GT];
         ds[u][e][0] = clamp_if(ds[u][e][0], a.g_clip);
-        CM::bwd(cc, sp, sn, dso, ds[u][e], gr, gw, gb_);
+        CM::finish(prep[EARLY ? u : 0][e], ds[u][e], gr, gw, gb_);
+        // (fp16: rounded to fp32 first in both, where the compiler takes the conversion into the product in one of them)
+        if constexpr (TWIN && std::is_same_v<T, half_t>) {
+#pragma unroll
+          for (int g = 0; g < GR; ++g) asm("" : "+v"(gr[g]));
+          if constexpr (F == FRNN_GRU) { asm("" : "+v"(gw[2])); gw[0] = gr[1]; gw[1] = gr[2]; gb_[3] = gw[2]; }
+#pragma unroll
+          for (int g = 0; g < GR; ++g) { gb_[g] = gr[g]; if constexpr (GR == 4) gw[g] = gr[g]; }
+        }
         // padded batch rows contribute nothing (selects, not branches)
 #pragma unroll
         for (int g = 0; g < GR; ++g) dgr[g][e] = bvalid ? gr[g] : 0.f;
@@ -1157,7 +1188,7 @@ fused_bwd_kernel(const BwdArgs a) {
             ll_store_sel<E, 64 * (int)sizeof(IW)>(inbox + (size_t)(((x * NPOS + wp_u) * UTW + u) * KW + slice) * EW, sslot, wv, near_m);
         }
       }
-      if constexpr (DW_LATE && !DEFER) {
+      if constexpr (DW_LATE) {
         if (DSP == 1 || hf == 0) {
 #pragma unroll
           for (int u = 0; u < UTW; ++u) store_dw(u);
@@ -1196,13 +1227,10 @@ fused_bwd_kernel(const BwdArgs a) {
       const IW* const mine = inbox + (size_t)(t & 1) * INW + ((size_t)(slice * NPOS + wp) * UTW) * KW * EW + lane;
       // fp32 wave pairs of the GRU, 14 and 16 workgroups per head: asked in front of the next probe (reverse kernel, T = 256, B8 N2, next
       // probe first against this: D = 512 0.668 -> 0.659 ms, where the shorter waits had cost 2 %, D = 448 0.605 -> 0.590)
-      // what goes behind the first probe (bwd_operands_behind_probe)
+      // what goes behind the first probe
       auto behind_probe = [&]() __attribute__((always_inline)) {
-        load_pre(pn, __builtin_amdgcn_readfirstlane(t >= PD ? t - PD : 0));
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < UTW; ++u) store_dw(u);
-        if constexpr (!TELL_IDLE) tell();
+        for (int u = 0; u < (EARLY ? UTW : 0); ++u) prepare(pm, u, prep[u]);
       };
       constexpr bool SEND_FIRST = !(F == FRNN_GRU && sizeof(T) == 4 && DSP == 2 && KW >= 14);
       if constexpr (RSP) {
@@ -1231,7 +1259,8 @@ fused_bwd_kernel(const BwdArgs a) {
           // (groups that span the device probe memory: the shorter waits had them probe more often, at D = 640 in front of the words;
           // a pause between the probes 0.4 to 1.5 % at every batch size, two units less, four and eight slower; see also the
           // first-probe delay)
-          poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0, NothingBehind());
+          if constexpr (EARLY) poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, a.poll_delay, behind_probe);
+          else poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0, NothingBehind());
 #pragma unroll
           for (int rr = 0; rr < PSRC_W; ++rr) {
             const bool in = k0 + rr < SRC_W && rbeg + k0 + rr < KW;
@@ -1295,7 +1324,7 @@ fused_bwd_kernel(const BwdArgs a) {
             if (never()) { dead = true; return; }  // (without an exit here the sLSTM's D = 128 kernel spills)
           }
         } else {
-          if constexpr (DEFER) poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, a.poll_delay, behind_probe);
+          if constexpr (EARLY) poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, a.poll_delay, behind_probe);
           else poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0, NothingBehind());
         }
 #pragma unroll
@@ -1360,22 +1389,22 @@ fused_bwd_kernel(const BwdArgs a) {
     // (written out: in the general form below the register allocation of the largest kernels,
     // which sit at the 256-register limit, comes out with spills)
     for (; t >= 1 && !dead; t -= 2) {
-      step(std::false_type{}, t, pre[0], pre[0], pre[1]);
+      step(std::false_type{}, t, pre[0], pre[1], pre[1]);
       if (dead) break;
-      step(std::false_type{}, t - 1, pre[1], pre[1], pre[0]);
+      step(std::false_type{}, t - 1, pre[1], pre[0], pre[0]);
     }
-    if (!dead && t == 0) step(std::false_type{}, 0, pre[0], pre[0], pre[1]);
+    if (!dead && t == 0) step(std::false_type{}, 0, pre[0], pre[1], pre[1]);
   } else {
     for (; t >= PD && !dead; t -= PD + 1) {
 #pragma unroll
       for (int j = 0; j <= PD; ++j) {
-        step(std::false_type{}, t - j, pre[j], pre[j], pre[(j + PD) % (PD + 1)]);
+        step(std::false_type{}, t - j, pre[j], pre[(j + 1) % (PD + 1)], pre[(j + PD) % (PD + 1)]);
         if (dead) break;
       }
     }
 #pragma unroll
     for (int j = 0; j < PD; ++j)
-      if (!dead && t - j >= 0) step(std::false_type{}, t - j, pre[j], pre[j], pre[(j + PD) % (PD + 1)]);
+      if (!dead && t - j >= 0) step(std::false_type{}, t - j, pre[j], pre[(j + 1) % (PD + 1)], pre[(j + PD) % (PD + 1)]);
   }
   if constexpr (!FLAG) lds_barrier();  // (the producer wave takes part in it)
   else { if (!dead && barrier_or(dead_flag)) dead = true; }

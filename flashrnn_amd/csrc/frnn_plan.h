@@ -159,22 +159,28 @@ constexpr bool fwd_own_slice_first(int GR, int D, int WAVES, int UTW, int KW, in
 constexpr bool fwd_stores_behind_probe(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize) {
   return esize == 2 && GR >= 3 && WAVES == 4 && KW <= (TR == 4 ? 8 : TR == 8 ? 5 : 0) && fwd_own_slice_first(GR, D, WAVES, UTW, KW, TR, esize);
 }
-// Reverse kernels with an instantiation for launches that have workgroups which fetch its operands into L2 (frnn_prefetch.h): 16-bit types, gated
-// cells, and either pairs of waves that split the destinations (4-row tiles, up to 16 workgroups per head) or 8- and 16-row tiles of up to 5
-// workgroups per head.  Whole backward pass, bf16, T = 512, without and with: LSTM B8 T1024 N3 D256 958 -> 942 us, B16 N4 D192 463 -> 451, N1 D384 589 ->
-// 575, D512 674 -> 655, sLSTM B16 T1024 N4 D192 933 -> 900, D512 694 -> 668, GRU B16 N1 D512 650 -> 610; taller tiles: LSTM B256 N3 D256 1240 -> 1189, sLSTM
-// B128 N4 D192 886 -> 813, B256 1411 -> 1350, GRU B128 N3 D256 700 -> 663, B256 995 -> 911.  Elsewhere: taller tiles of 6 to 10 workgroups -0.5 to
-// +2.7 %, 4-row tiles without pairs +-1 (LSTM B64 N3 D256), GRU +6 at D = 768 (20 workgroups and more, whose second waves poll), fours of waves
-// (sLSTM D = 256) 0, fp32 -0.3 to +4, recompute mode +-1.
-constexpr bool bwd_prefetched(int GR, int D, int WAVES, int UTW, int KW, int TR, int esize, bool rc) {
-  return esize == 2 && GR >= 3 && KW > 1 && !rc && UTW == 1 &&
-         (TR == 4 ? bwd_dest_split(D, WAVES, UTW, KW) == 2 && KW <= 16 : bwd_dest_split(D, WAVES, UTW, KW) == 1 && KW <= 5);
+// Reverse kernels with an instantiation for launches that have workgroups which fetch its operands into L2 (frnn_prefetch.h): gated cells in the 16-bit
+// types, 8- and 16-row tiles of up to 5 workgroups per head (the GRU 8-row tiles), and the sLSTM's pairs of 6 workgroups (nc: values of the gate cache).
+// Whole backward pass, bf16, T = 512, without and with: LSTM B128 N3 D256 784 -> 752 us, B256 1261 -> 1174, sLSTM B128 N3 D256 879 -> 813, B256 N4
+// D192 1385 -> 1285, B16 T1024 N4 D192 915 -> 890, GRU B128 N2 D320 736 -> 717, N3 D256 714 -> 708, B256 918 -> 915.  Elsewhere: GRU B16 N1 D512 592 -> 596, LSTM B8 T1024 N3 D256 912 -> 930, B16 N1 D384 551
+// -> 562, D512 650 -> 649, sLSTM B16 N4 D128 400 -> 415, D512 659 -> 655, taller tiles of 6 to 10 workgroups -0.5 to +2.7 %, fp32 -0.3 to +4, recompute mode +-1.
+constexpr bool bwd_prefetched(int GR, int nc, int D, int WAVES, int UTW, int KW, int TR, int esize, bool rc) {
+  return esize == 2 && (GR == 4 || (GR == 3 && TR == 8)) && KW > 1 && !rc && UTW == 1 &&
+         (TR == 4 ? nc == 5 && bwd_dest_split(D, WAVES, UTW, KW) == 2 && KW == 6 : bwd_dest_split(D, WAVES, UTW, KW) == 1 && KW <= 5);
 }
-// Of these, the kernels that store dWx and request the operands of the step after next behind the first probe, while it is on its way, instead of in front
-// of it and at the head of a step: what a wave asks of memory costs it ~30 cycles each and a probe returns behind it.  Only with operands
-// that are in L2 (from HBM a second probe waits for them: LSTM B8 N3 D256 964 -> 1073 us), and with registers for one more set of them: 4-row tiles, and 8-row
-// tiles of the GRU (the others' and the 16-row ones spill).
-constexpr bool bwd_operands_behind_probe(int GR, int TR) { return TR <= (GR == 3 ? 8 : 4); }
+// Reverse kernel, heads of several workgroups: the half of a step's adjoint that does not depend on the running cotangent is done behind the
+// first probe of the step before, while the words travel.  16-bit gated cells at any tiling that waits in one round (backward pass, bf16, T = 512: LSTM B8 T1024 N3
+// D256 959 -> 912 us, B16 N4 D192 462 -> 431, N1 D384 588 -> 551, D512 680 -> 650, D640 830 -> 751, D768 937 -> 847, D1024 1094 -> 1043, sLSTM D512 695 -> 659,
+// GRU N3 D256 502 -> 460, D512 648 -> 592, D1024 1008 -> 963), but at tiles of 8 and 16 rows of up to 5 workgroups, whose probes come back sooner than 2 or 4 elements
+// are done, only where the operands are in L2 (LSTM B256 N3 D256 1250 without either, 1261 with this, 1174 with both) or the cell is the GRU (1030
+// -> 954); the LSTM in fp32 from 16 workgroups on (D512 1205 -> 1159, D256 716 -> 698, but N3 D128 -1 %, sLSTM D256 +3, D128 +9, taller tiles +5 to +6); not the
+// Elman cell, which has no more to prepare than a product (+-1 to +8 %).
+constexpr bool bwd_adjoint_early(int GR, int nc, int UTW, int KW, int TR, int esize, bool fetched) {
+  if (UTW != 1) return false;
+  if (GR == 1) return false;
+  if (esize == 4) return GR == 4 && nc == 4 && KW >= 16 && TR == 4;
+  return GR == 3 || TR == 4 || KW > 5 || fetched;
+}
 }
 
 // Measured on MI355X (T = 1024, bf16): when the head fits one workgroup, one tile per wave and

@@ -12,7 +12,7 @@ template <int Dv, int W, int U, int K, int MTR, bool RCV, int TR> static void (*
   constexpr int GR = Cell<FRNN_F>::GR, ES = (int)sizeof(FRNN_TU_T);
   if constexpr (TR > MTR) return nullptr;
   else {
-    if constexpr ((TR == 4 && bwd_producer_stores(GR, Cell<FRNN_F>::NC, Dv, W, U, K, 4, ES, RCV)) || bwd_prefetched(GR, Dv, W, U, K, TR, ES, RCV)) {
+    if constexpr ((TR == 4 && bwd_producer_stores(GR, Cell<FRNN_F>::NC, Dv, W, U, K, 4, ES, RCV)) || bwd_prefetched(GR, Cell<FRNN_F>::NC, Dv, W, U, K, TR, ES, RCV)) {
       if (alt) return fused_bwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, TR, RCV, true>;
     }
     return fused_bwd_kernel<FRNN_F, FRNN_TU_T, Dv, W, U, K, TR, RCV>;
