@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(256) alt_step_bwd_kernel(const AltStepBwdArgs 
   // (c, not to be seen through: the compiler moved the first steps of tanh(c) up to its load and waited there, a trip to HBM in
   // front of the product; fp32 LSTM B8, backward of 96 steps with that wait and without: N4 D32 0.460 and 0.443 ms, N3 D256 0.853 and 0.833)
   if constexpr (sizeof(T) == 4 && F == FRNN_LSTM) asm volatile("" : "+v"(sn[1]));
-  cell_bwd<CM>(cc, sp, sn, dso, ds, gr, gw, gb);
+  CM::bwd(cc, sp, sn, dso, ds, gr, gw, gb);
 #pragma unroll
   for (int k = 0; k < S; ++k) a.dsr[(size_t)k * BND + idx] = ds[k];
   T* dg = static_cast<T*>(a.dg_out) + ((size_t)b * N + n) * GR * D + d;

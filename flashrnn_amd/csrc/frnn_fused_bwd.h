@@ -752,43 +752,41 @@ fused_bwd_kernel(const BwdArgs a) {
   // EARLY: done for the step to come while the first probe of the wait is on its way, off the chain of dependent steps.
   constexpr bool EARLY = KW > 1 && !RC && (RSP ? ROUNDS_W : ROUNDS) == 1 && bwd_adjoint_early(GR, NC, UTW, KW, TR, (int)sizeof(T), FETCHED);
   constexpr bool TWIN = bwd_prefetched(GR, NC, D, WAVES, UTW, KW, TR, (int)sizeof(T), RC);  // one of two kernels that differ in FETCHED
+  constexpr bool SPLIT = EARLY || (TWIN && std::is_same_v<T, half_t>);  // the two halves apart
   float prep[EARLY ? UTW : 1][E][CM::NP];
-  auto prepare = [&](const Pre& p, int u, float (&out)[E][CM::NP]) __attribute__((always_inline)) {
-    float cv[NCA][E], spv[S][E], snv[S][E], dsov[S][E];
-    if constexpr (NC > 0 && !RC) cache_unpack<T, NCA, E>(p.cache[u], cv);
-    if constexpr (NC > 0 && RC) {
+  // (Only there: a closure with references to a step's registers, even one that nobody calls, has the compiler order the steps of other kernels worse, and a
+  // function for what both unpack those of the sLSTM: reverse pass, Elman D = 160 and 192 +2 to +6 %, sLSTM D = 192 +3 to +7.)
+  auto prepare = [&]() __attribute__((always_inline)) {
+    if constexpr (!SPLIT) return 0;
+    else return [&](const Pre& p, int u, float (&out)[E][CM::NP]) __attribute__((always_inline)) {
+      float cv[NCA][E], spv[S][E], snv[S][E], dsov[S][E];
+      if constexpr (NC > 0) cache_unpack<T, NCA, E>(p.cache[u], cv);
 #pragma unroll
-      for (int c = 0; c < NC; ++c)
+      for (int k = 0; k < S; ++k) {
+        unpack<E>(sn[u][k], snv[k], (T*)0); unpack<E>(p.dso[u][k], dsov[k], (T*)0);
+        if (CXU && k == CXS) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) cv[c][e] = gc[u][c][e];
-    }
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
-      unpack<E>(sn[u][k], snv[k], (T*)0); unpack<E>(p.dso[u][k], dsov[k], (T*)0);
-      if (CXU && k == CXS) {  // (from the cache line; packed again, exactly, for the next step)
-#pragma unroll
-        for (int e = 0; e < E; ++e) spv[k][e] = cv[NC][e];
-        sn[u][k] = pack<E>(cv[NC], (T*)0);
-        continue;
+          for (int e = 0; e < E; ++e) spv[k][e] = cv[NC][e];
+          sn[u][k] = pack<E>(cv[NC], (T*)0);
+          continue;
+        }
+        unpack<E>(p.sp[u][k], spv[k], (T*)0);
+        sn[u][k] = p.sp[u][k];
       }
-      unpack<E>(p.sp[u][k], spv[k], (T*)0);
-      sn[u][k] = p.sp[u][k];  // s_(t-1) is the s_t of the next step
-    }
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      float cc[NCA], sp1[S], sn1[S], dso1[S];
+      for (int e = 0; e < E; ++e) {
+        float cc[NCA], sp1[S], sn1[S], dso1[S];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) cc[c] = cv[c][e];
+        for (int c = 0; c < NC; ++c) cc[c] = cv[c][e];
 #pragma unroll
-      for (int k = 0; k < S; ++k) { sp1[k] = spv[k][e]; sn1[k] = snv[k][e]; dso1[k] = dsov[k][e]; }
-      CM::prepare(cc, sp1, sn1, dso1, out[e]);
-      // (EARLY: left alone, the compiler sinks it to its use.  TWIN, fp16: the same products and sums in both kernels)
-      if constexpr (EARLY || (TWIN && std::is_same_v<T, half_t>)) {
+        for (int k = 0; k < S; ++k) { sp1[k] = spv[k][e]; sn1[k] = snv[k][e]; dso1[k] = dsov[k][e]; }
+        CM::prepare(cc, sp1, sn1, dso1, out[e]);
+        // (EARLY: left alone, the compiler sinks it to its use.  TWIN, fp16: the same products and sums in both kernels)
 #pragma unroll
         for (int i = 0; i < CM::NP; ++i) asm volatile("" : "+v"(out[e][i]));
       }
-    }
-  };
+    };
+  }();
   if constexpr (EARLY) {
     if (!a.cut) {
 #pragma unroll
@@ -804,7 +802,7 @@ fused_bwd_kernel(const BwdArgs a) {
   // CUT (a std::bool_constant): truncated backpropagation, the step ends with the pointwise carry;
   // it is a compile-time variant of the step so that the full step carries no trace of it
   // (a run-time early exit cost 8 % at D = 128)
-  // Recompute mode: `pm` holds the operands of step t-1, whose gates are rebuilt during this step.
+  // `pm` holds the operands of step t-1: recompute mode rebuilds its gates during this step, EARLY does the first half of its adjoint.
   auto step = [&](auto CUT, const int t, Pre& pc, Pre& pm, Pre& pn) __attribute__((always_inline)) {
     constexpr bool cut = decltype(CUT)::value;
     T* const gb = (t & 1) ? gbuf1 : gbuf0;
@@ -837,13 +835,44 @@ fused_bwd_kernel(const BwdArgs a) {
     if (DSP == 1 || hf == 0) {  // (wave-uniform: the second wave of a pair owns no element)
 #pragma unroll
     for (int u = 0; u < UTW; ++u) {
-      if constexpr (!EARLY || cut) prepare(pc, u, prep[EARLY ? u : 0]);
+      float cv[NCA][E], spv[S][E], snv[S][E], dsov[S][E];
+      if constexpr (!SPLIT) {
+        if constexpr (NC > 0 && !RC) cache_unpack<T, NCA, E>(pc.cache[u], cv);
+        if constexpr (NC > 0 && RC) {
+#pragma unroll
+          for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < E; ++e) cv[c][e] = gc[u][c][e];
+        }
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+          unpack<E>(sn[u][k], snv[k], (T*)0); unpack<E>(pc.dso[u][k], dsov[k], (T*)0);
+          if (CXU && k == CXS) {  // (from the cache line; packed again, exactly, for the next step)
+#pragma unroll
+            for (int e = 0; e < E; ++e) spv[k][e] = cv[NC][e];
+            sn[u][k] = pack<E>(cv[NC], (T*)0);
+            continue;
+          }
+          unpack<E>(pc.sp[u][k], spv[k], (T*)0);
+          sn[u][k] = pc.sp[u][k];  // s_(t-1) is the s_t of the next step
+        }
+      } else if constexpr (!EARLY || cut) prepare(pc, u, prep[EARLY ? u : 0]);
       float dgr[GR][E], dgw[GW][E];
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         float gr[GR], gw[GW], gb_[GT];
-        ds[u][e][0] = clamp_if(ds[u][e][0], a.g_clip);
-        CM::finish(prep[EARLY ? u : 0][e], ds[u][e], gr, gw, gb_);
+        if constexpr (!SPLIT) {
+          float cc[NCA], sp1[S], sn1[S], dso1[S];
+#pragma unroll
+          for (int c = 0; c < NC; ++c) cc[c] = cv[c][e];
+#pragma unroll
+          for (int k = 0; k < S; ++k) { sp1[k] = spv[k][e]; sn1[k] = snv[k][e]; dso1[k] = dsov[k][e]; }
+          ds[u][e][0] = clamp_if(ds[u][e][0], a.g_clip);
+          CM::bwd(cc, sp1, sn1, dso1, ds[u][e], gr, gw, gb_);
+        } else {
+          ds[u][e][0] = clamp_if(ds[u][e][0], a.g_clip);
+          CM::finish(prep[EARLY ? u : 0][e], ds[u][e], gr, gw, gb_);
+        }
         // (fp16: rounded to fp32 first in both, where the compiler takes the conversion into the product in one of them)
         if constexpr (TWIN && std::is_same_v<T, half_t>) {
 #pragma unroll
@@ -1227,11 +1256,6 @@ fused_bwd_kernel(const BwdArgs a) {
       const IW* const mine = inbox + (size_t)(t & 1) * INW + ((size_t)(slice * NPOS + wp) * UTW) * KW * EW + lane;
       // fp32 wave pairs of the GRU, 14 and 16 workgroups per head: asked in front of the next probe (reverse kernel, T = 256, B8 N2, next
       // probe first against this: D = 512 0.668 -> 0.659 ms, where the shorter waits had cost 2 %, D = 448 0.605 -> 0.590)
-      // what goes behind the first probe
-      auto behind_probe = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < (EARLY ? UTW : 0); ++u) prepare(pm, u, prep[u]);
-      };
       constexpr bool SEND_FIRST = !(F == FRNN_GRU && sizeof(T) == 4 && DSP == 2 && KW >= 14);
       if constexpr (RSP) {
         const int rbeg = 1 + hf * SRC_W;  // (uniform) this wave's sources: rbeg .. rbeg + SRC_W - 1, below KW
@@ -1259,8 +1283,14 @@ fused_bwd_kernel(const BwdArgs a) {
           // (groups that span the device probe memory: the shorter waits had them probe more often, at D = 640 in front of the words;
           // a pause between the probes 0.4 to 1.5 % at every batch size, two units less, four and eight slower; see also the
           // first-probe delay)
-          if constexpr (EARLY) poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, a.poll_delay, behind_probe);
-          else poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0, NothingBehind());
+          if constexpr (EARLY) {
+            poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, a.poll_delay, [&]() __attribute__((always_inline)) {
+#pragma unroll
+              for (int u = 0; u < UTW; ++u) prepare(pm, u, prep[u]);
+            });
+          } else {
+            poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0, NothingBehind());
+          }
 #pragma unroll
           for (int rr = 0; rr < PSRC_W; ++rr) {
             const bool in = k0 + rr < SRC_W && rbeg + k0 + rr < KW;
@@ -1324,8 +1354,14 @@ fused_bwd_kernel(const BwdArgs a) {
             if (never()) { dead = true; return; }  // (without an exit here the sLSTM's D = 128 kernel spills)
           }
         } else {
-          if constexpr (EARLY) poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, a.poll_delay, behind_probe);
-          else poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0, NothingBehind());
+          if constexpr (EARLY) {
+            poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, a.poll_delay, [&]() __attribute__((always_inline)) {
+#pragma unroll
+              for (int u = 0; u < UTW; ++u) prepare(pm, u, prep[u]);
+            });
+          } else {
+            poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0, NothingBehind());
+          }
         }
 #pragma unroll
         for (int rr = 0; rr < PSRC; ++rr)

@@ -49,13 +49,11 @@ __device__ __forceinline__ float mul(float a, float b) {
 //       ds[S] in: running cotangent arriving from step t+1; out: cotangent for s_{t-1}
 //       WITHOUT the recurrent term R^T dgr (the caller adds it to ds[0]);
 //       dgr[GR] / dgw[GW] / dgb[GT]: cotangents of the R-side, Wx-side and bias pre-activations.
-//       In two halves: prepare(), what does not depend on the running cotangent, into NP values, and finish(), which needs only those and ds.
+// prepare, finish: bwd in two halves, for reverse kernels that do the first ahead of time: what does not depend on the running cotangent, into NP
+//       values, and the rest, which needs only those and ds.  bwd stays beside them: composed of the two, or with the values computed where
+//       finish uses them, the same instructions come in another order (reverse pass, Elman B64 N2 D192 T256 112.6 -> 117.4 us, D160 105.8 -> 111.2,
+//       recompute mode, sLSTM B64 N2 D128 331 -> 336).
 template <int F, bool FAST> struct CellMath;
-template <typename CM> __device__ __forceinline__ void cell_bwd(const float* cache, const float* sp, const float* sn, const float* dso, float* ds, float* dgr, float* dgw, float* dgb) {
-  float p[CM::NP];
-  CM::prepare(cache, sp, sn, dso, p);
-  CM::finish(p, ds, dgr, dgw, dgb);
-}
 
 // A state a * b + c as it is stored in fp16: rounded once, from the exact sum.  Through the fp32 state it would be rounded twice, and
 // 4e-5 of the stored values would be the farther of their two neighbours.  Written out because the compiler does it by
@@ -79,6 +77,21 @@ template <bool FAST> struct CellMath<FRNN_LSTM, FAST> {
     s[1] = c;
     s[0] = mul(o, M::tanh(c));
     cache[0] = i; cache[1] = f; cache[2] = z; cache[3] = o;
+  }
+  static __device__ __forceinline__ void bwd(const float* cache, const float* sp, const float* sn, const float* dso,
+                                             float* ds, float* dgr, float* dgw, float* dgb) {
+    const float i = cache[0], f = cache[1], z = cache[2], o = cache[3];
+    const float dy = dso[0] + ds[0];
+    const float tc = M::tanh(sn[1]);
+    const float dc = dso[1] + ds[1] + (1.0f - tc * tc) * o * dy;
+    dgr[0] = i * (1.0f - i) * z * dc;
+    dgr[1] = f * (1.0f - f) * sp[1] * dc;
+    dgr[2] = (1.0f - z * z) * i * dc;
+    dgr[3] = o * (1.0f - o) * tc * dy;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) { dgw[g] = dgr[g]; dgb[g] = dgr[g]; }
+    ds[0] = 0.0f;
+    ds[1] = f * dc;
   }
   static constexpr int NP = 8;
   static __device__ __forceinline__ void prepare(const float* cache, const float* sp, const float* sn, const float* dso, float* p) {
@@ -126,6 +139,22 @@ template <bool FAST> struct CellMath<FRNN_SLSTM, FAST> {
     s[1] = c; s[2] = n; s[3] = mn;
     cache[0] = ig; cache[1] = fg; cache[2] = z; cache[3] = o; cache[4] = M::sigmoid(-fr);
   }
+  static __device__ __forceinline__ void bwd(const float* cache, const float* sp, const float* sn, const float* dso,
+                                             float* ds, float* dgr, float* dgw, float* dgb) {
+    const float ig = cache[0], fg = cache[1], z = cache[2], o = cache[3], omf = cache[4];
+    const float dy = dso[0] + ds[0];
+    const float dyi = dy * M::rcp(sn[2]);
+    const float dc = dso[1] + ds[1] + dyi * o;
+    const float dn = dso[2] + ds[2] - dyi * sn[0];
+    dgr[0] = ig * (z * dc + dn);
+    dgr[1] = fg * (dc * sp[1] + dn * sp[2]) * omf;
+    dgr[2] = dc * ig * (1.0f - z * z);
+    dgr[3] = (1.0f - o) * sn[0] * dy;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) { dgw[g] = dgr[g]; dgb[g] = dgr[g]; }
+    // the stabiliser m is held constant (slstm_pointwise.cu:205): no cotangent flows into it
+    ds[0] = 0.0f; ds[1] = fg * dc; ds[2] = fg * dn; ds[3] = 0.0f;
+  }
   static constexpr int NP = 14;
   static __device__ __forceinline__ void prepare(const float* cache, const float* sp, const float* sn, const float* dso, float* p) {
     const float ig = cache[0], fg = cache[1], z = cache[2], o = cache[3], omf = cache[4];
@@ -163,6 +192,19 @@ template <bool FAST> struct CellMath<FRNN_GRU, FAST> {
     s[0] = __builtin_fmaf(z, s[0], mul(1.0f - z, nv));
     cache[0] = g; cache[1] = r; cache[2] = z; cache[3] = nv;  // the candidate itself: the adjoint needs no tanh
   }
+  static __device__ __forceinline__ void bwd(const float* cache, const float* sp, const float* sn, const float* dso,
+                                             float* ds, float* dgr, float* dgw, float* dgb) {
+    const float g = cache[0], r = cache[1], z = cache[2], nv = cache[3];
+    const float dy = dso[0] + ds[0];
+    const float dz = z * (1.0f - z) * dy * (sp[0] - nv);
+    const float dn = dy * (1.0f - z) * (1.0f - nv * nv);
+    const float dr = dn * g * r * (1.0f - r);
+    const float dg = dn * r;
+    dgr[0] = dg; dgr[1] = dr; dgr[2] = dz;
+    dgw[0] = dr; dgw[1] = dz; dgw[2] = dn;
+    dgb[0] = dg; dgb[1] = dr; dgb[2] = dz; dgb[3] = dn;
+    ds[0] = z * dy;
+  }
   static constexpr int NP = 9;
   static __device__ __forceinline__ void prepare(const float* cache, const float* sp, const float* sn, const float* dso, float* p) {
     const float g = cache[0], r = cache[1], z = cache[2], nv = cache[3];
@@ -188,17 +230,14 @@ template <bool FAST> struct CellMath<FRNN_ELMAN, FAST> {
   static __device__ __forceinline__ void fwd(const float* ry, const float* wx, const float* b, float* s, float*, float* = nullptr) {
     s[0] = M::tanh(wx[0] + ry[0]);
   }
-  static constexpr int NP = 2;
-  static __device__ __forceinline__ void prepare(const float*, const float*, const float* sn, const float* dso, float* p) {
-    p[0] = 1.0f - sn[0] * sn[0];
-    p[1] = dso[0];
-  }
-  static __device__ __forceinline__ void finish(const float* p, float* ds, float* dgr, float* dgw, float* dgb) {
-    const float dy = p[1] + ds[0];
-    dgr[0] = p[0] * dy;
+  static __device__ __forceinline__ void bwd(const float*, const float*, const float* sn, const float* dso,
+                                             float* ds, float* dgr, float* dgw, float* dgb) {
+    const float dy = dso[0] + ds[0];
+    dgr[0] = (1.0f - sn[0] * sn[0]) * dy;
     dgw[0] = dgr[0]; dgb[0] = dgr[0];
     ds[0] = 0.0f;
   }
+  static constexpr int NP = 1;  // (never split: one product would move)
 };
 
 // Elman under forward_clipval: cache[0] is the unclamped tanh (the caller clamps s[0] after fwd)
@@ -209,17 +248,14 @@ template <bool FAST> struct CellMath<FRNN_ELMAN_CLIP, FAST> {
     s[0] = M::tanh(wx[0] + ry[0]);
     cache[0] = s[0];
   }
-  static constexpr int NP = 2;
-  static __device__ __forceinline__ void prepare(const float* cache, const float*, const float*, const float* dso, float* p) {
-    p[0] = 1.0f - cache[0] * cache[0];
-    p[1] = dso[0];
-  }
-  static __device__ __forceinline__ void finish(const float* p, float* ds, float* dgr, float* dgw, float* dgb) {
-    const float dy = p[1] + ds[0];
-    dgr[0] = p[0] * dy;
+  static __device__ __forceinline__ void bwd(const float* cache, const float*, const float*, const float* dso,
+                                             float* ds, float* dgr, float* dgw, float* dgb) {
+    const float dy = dso[0] + ds[0];
+    dgr[0] = (1.0f - cache[0] * cache[0]) * dy;
     dgw[0] = dgr[0]; dgb[0] = dgr[0];
     ds[0] = 0.0f;
   }
+  static constexpr int NP = 1;  // (never split: one product would move)
 };
 
 }  // namespace frnn

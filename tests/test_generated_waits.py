@@ -75,3 +75,14 @@ def test_alternating_lstm_step_in_fp32_requests_its_product_before_it_waits(tmp_
     waits = [i for i, t in enumerate(code[:first]) if re.search(r"vmcnt\(", t)]
     early = [i for i in waits if first - i > 20]
     assert not early, code[early[0] - 5:early[0] + 3]
+
+
+def test_operands_of_an_elman_step_stay_where_they_arrive(tmp_path):
+    """Reverse kernels of 10 and 12 waves: of the operands that a step requests, few are moved to another register, each behind a
+    wait for its load (with a closure beside the step that nobody calls there was one more in each of the two loops)."""
+    kernels = {k: v for k, v in _functions("fused_bwd_3_0.o", tmp_path).items() if re.search(r"fused_bwd_kernelILi3E\w+?Li(160ELi10|192ELi12)ELi1ELi1ELi4E", k)}
+    assert len(kernels) == 2, sorted(kernels)
+    for name, code in kernels.items():
+        arrive = {m.group(1) for t in code for m in [re.match(r"buffer_load_ushort (v\d+),", t)] if m}
+        moved = [t for t in code for m in [re.match(r"v_mov_b32_e32 v\d+, (v\d+)$", t)] if m and m.group(1) in arrive]
+        assert arrive and len(moved) <= 8, (name, moved)
