@@ -284,21 +284,18 @@ __device__ __forceinline__ void poll_finish(const W* base, const int* off, const
 }
 
 // The two halves back to back.
-template <typename TAG, int NW, bool BITS, bool SEND_FIRST, int PAUSE = 0, typename W, typename Behind>
-__device__ __forceinline__ void poll_words_reload(const W* base, const int* off, const bool* need, int t, W* v, Wait& w, int first_delay, Behind behind) {
+template <typename TAG, int NW, bool BITS, bool SEND_FIRST, int PAUSE = 0, typename W>
+__device__ __forceinline__ void poll_words_reload(const W* base, const int* off, const bool* need, int t, W* v, Wait& w, int first_delay) {
   for (int i = 0; i < first_delay; ++i) __builtin_amdgcn_s_sleep(1);
-  if constexpr (std::is_same_v<Behind, NothingBehind>) {
-#pragma unroll
-    for (int i = 0; i < NW; ++i) v[i] = ll_load(base + off[i]);
-    poll_finish<TAG, NW, BITS, SEND_FIRST, PAUSE>(base, off, need, t, v, w);
-  } else {
-    probe_until(
-      [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < NW; ++i) v[i] = ll_load(base + off[i]);
-      },
-      [&]() __attribute__((always_inline)) { return all_arrived<TAG, NW, BITS>(v, need, t); }, w, behind);
-  }
+  poll_issue<NW>(base, off, v);
+  poll_finish<TAG, NW, BITS, SEND_FIRST, PAUSE>(base, off, need, t, v, w);
+}
+// The same with work behind the first probe (see probe_until).
+template <typename TAG, int NW, bool BITS, typename W, typename Behind>
+__device__ __forceinline__ void poll_words_behind(const W* base, const int* off, const bool* need, int t, W* v, Wait& w, int first_delay, Behind behind) {
+  for (int i = 0; i < first_delay; ++i) __builtin_amdgcn_s_sleep(1);
+  probe_until([&]() __attribute__((always_inline)) { poll_issue<NW>(base, off, v); },
+              [&]() __attribute__((always_inline)) { return all_arrived<TAG, NW, BITS>(v, need, t); }, w, behind);
 }
 
 // The same wait for pairs of adjacent words, each pair fetched with one 16-byte agent-scope load

@@ -750,7 +750,7 @@ fused_bwd_kernel(const BwdArgs a) {
 
   // The half of the adjoint of a step that does not depend on the running cotangent (operands unpacked, tanh(c), the products of the gates).
   // EARLY: done for the step to come while the first probe of the wait is on its way, off the chain of dependent steps.
-  constexpr bool EARLY = KW > 1 && !RC && (RSP ? ROUNDS_W : ROUNDS) == 1 && bwd_adjoint_early(GR, NC, UTW, KW, TR, (int)sizeof(T), FETCHED);
+  constexpr bool EARLY = KW > 1 && !RC && (RSP ? ROUNDS_W : ROUNDS) == 1 && bwd_adjoint_early(GR, NC, D, WAVES, UTW, KW, TR, (int)sizeof(T), std::is_same_v<T, half_t>, FETCHED);
   constexpr bool TWIN = bwd_prefetched(GR, NC, D, WAVES, UTW, KW, TR, (int)sizeof(T), RC);  // one of two kernels that differ in FETCHED
   constexpr bool SPLIT = EARLY || (TWIN && std::is_same_v<T, half_t>);  // the two halves apart
   float prep[EARLY ? UTW : 1][E][CM::NP];
@@ -1284,12 +1284,13 @@ fused_bwd_kernel(const BwdArgs a) {
           // a pause between the probes 0.4 to 1.5 % at every batch size, two units less, four and eight slower; see also the
           // first-probe delay)
           if constexpr (EARLY) {
-            poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, a.poll_delay, [&]() __attribute__((always_inline)) {
+            // (no pause here: D640 794 us without and 796 with one, D768 878 and 880, B4 T256)
+            poll_words_behind<PT, NWR, true>(mine, off, need, t, v, wait, a.poll_delay, [&]() __attribute__((always_inline)) {
 #pragma unroll
               for (int u = 0; u < UTW; ++u) prepare(pm, u, prep[u]);
             });
           } else {
-            poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0, NothingBehind());
+            poll_words_reload<PT, NWR, true, SEND_FIRST, (KW > kXcdWorkgroups ? 1 : 0)>(mine, off, need, t, v, wait, k0 == 0 ? a.poll_delay : 0);
           }
 #pragma unroll
           for (int rr = 0; rr < PSRC_W; ++rr) {
@@ -1355,12 +1356,12 @@ fused_bwd_kernel(const BwdArgs a) {
           }
         } else {
           if constexpr (EARLY) {
-            poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, a.poll_delay, [&]() __attribute__((always_inline)) {
+            poll_words_behind<PT, NWR, !LANES>(mine, off, need, t, v, wait, a.poll_delay, [&]() __attribute__((always_inline)) {
 #pragma unroll
               for (int u = 0; u < UTW; ++u) prepare(pm, u, prep[u]);
             });
           } else {
-            poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0, NothingBehind());
+            poll_words_reload<PT, NWR, !LANES, !LANES>(mine, off, need, t, v, wait, r0 == 1 ? a.poll_delay : 0);
           }
         }
 #pragma unroll

@@ -169,17 +169,29 @@ constexpr bool bwd_prefetched(int GR, int nc, int D, int WAVES, int UTW, int KW,
          (TR == 4 ? nc == 5 && bwd_dest_split(D, WAVES, UTW, KW) == 2 && KW == 6 : bwd_dest_split(D, WAVES, UTW, KW) == 1 && KW <= 5);
 }
 // Reverse kernel, heads of several workgroups: the half of a step's adjoint that does not depend on the running cotangent is done behind the
-// first probe of the step before, while the words travel.  16-bit gated cells at any tiling that waits in one round (backward pass, bf16, T = 512: LSTM B8 T1024 N3
-// D256 959 -> 912 us, B16 N4 D192 462 -> 431, N1 D384 588 -> 551, D512 680 -> 650, D640 830 -> 751, D768 937 -> 847, D1024 1094 -> 1043, sLSTM D512 695 -> 659,
-// GRU N3 D256 502 -> 460, D512 648 -> 592, D1024 1008 -> 963), but at tiles of 8 and 16 rows of up to 5 workgroups, whose probes come back sooner than 2 or 4 elements
-// are done, only where the operands are in L2 (LSTM B256 N3 D256 1250 without either, 1261 with this, 1174 with both) or the cell is the GRU (1030
-// -> 954); the LSTM in fp32 from 16 workgroups on (D512 1205 -> 1159, D256 716 -> 698, but N3 D128 -1 %, sLSTM D256 +3, D128 +9, taller tiles +5 to +6); not the
-// Elman cell, which has no more to prepare than a product (+-1 to +8 %).
-constexpr bool bwd_adjoint_early(int GR, int nc, int UTW, int KW, int TR, int esize, bool fetched) {
-  if (UTW != 1) return false;
-  if (GR == 1) return false;
-  if (esize == 4) return GR == 4 && nc == 4 && KW >= 16 && TR == 4;
-  return GR == 3 || TR == 4 || KW > 5 || fetched;
+// first probe of the step before, while the words travel.  16-bit gated cells at tilings that wait in one round (backward pass, bf16, T = 512: LSTM B8 T1024 N3
+// D256 959 -> 912 us, B16 N4 D192 462 -> 431, N1 D384 588 -> 551, D512 680 -> 650, D640 830 -> 751, D768 937 -> 847, D1024 1094 -> 1043,
+// GRU N3 D256 502 -> 460, D512 648 -> 592, D1024 1008 -> 963).  Not where it loses (kernels of the same tree that differ in nothing else):
+// - the sLSTM's pairs of 4 and of more than 12 workgroups, but in bf16 20 and 24.  It needs a step's operands one wait earlier, and has the most of them: as soon
+//   as a call has more to read than the last-level cache holds they come from memory, and these steps wait for them (fp16, T = 2000, B32 D128 1540 -> 1782, D448
+//   2562 -> 2716, D512 2698 -> 3248, D640 T1046 1711 -> 1813, D768 3616 -> 3826, D1024 T653 1478 -> 1559, bf16 D512 2938 -> 3261, D1024 1214 -> 1239; where the
+//   cache holds them, D448 +5 %, D128 and D512 to D1024 -2 to -6).  6 to 12 gain either way (D320 -4 to -7 %, D384 T4096 -10), as do bf16 at 20 (D640 -3 to -6)
+//   and 24 (D768 -7 to +0.9), its fours (D256) and its single waves.
+// - the GRU's single waves at 10 and 12 workgroups, 4-row tiles (D640, D768: +2.2 and +2.3 % at B1, -1.3 to +1.0 else; at 7 -3.2 to +0.4),
+// - four gates at 3 workgroups or less, 4-row tiles (LSTM B160 N2 D192 T256 328 -> 333, T1024 1175 -> 1203, sLSTM 0 to +0.9 %; the GRU -3),
+// - tiles of 8 and 16 rows of up to 5 workgroups, whose probes come back sooner than 2 or 4 elements are done, unless the operands are in
+//   L2 (LSTM B256 N3 D256 1250 without either, 1261 with this, 1174 with both) or the cell is the GRU (1030 -> 954),
+// - fp32, but for the LSTM's 4-row tiles of 16 to 48 workgroups (T = 256, B16 D256 359 -> 351, D384 537 -> 532, D512 625 -> 603, D640 1073 -> 1054, D768
+//   1280 -> 1263; D1024, 64 workgroups, B1 1097 -> 1136, B4 1052 -> 1100; N3 D128 -1 %, sLSTM D256 +3, D128 +9, taller tiles +5 to +6),
+// - the Elman cell, which has no more to prepare than a product (+-1 to +8 %).
+constexpr bool bwd_adjoint_early(int GR, int nc, int D, int WAVES, int UTW, int KW, int TR, int esize, bool fp16, bool fetched) {
+  const int dsp = bwd_dest_split(D, WAVES, UTW, KW);
+  if (UTW != 1 || GR == 1) return false;
+  if (esize == 4) return GR == 4 && nc == 4 && KW >= 16 && KW <= 48 && TR == 4;
+  if (TR > 4) return GR == 3 || KW > 5 || fetched;
+  if (GR == 3) return dsp > 1 || KW < 10;
+  if (nc == 5 && dsp == 2) return (KW >= 6 && KW <= 12) || (!fp16 && KW > 16 && KW < 32);
+  return KW > 3;
 }
 }
 
