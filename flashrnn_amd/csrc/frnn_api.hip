@@ -888,7 +888,7 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   LaunchGate* gate = gate_enter(step ? 1 : p.kw, st);  // (the workgroups of a single step never wait for each other)
   for (int g0 = 0; g0 < groups; g0 += per_launch) {
     a.grp0 = g0; a.groups = groups - g0 < per_launch ? groups - g0 : per_launch;
-    a.helpers = step || call->beside || !fwd_prefetched(cell_dims(fx).GR, p.kw) ? 0 : helpers_for(p, a.groups, T);
+    a.helpers = step || call->beside || !fwd_prefetched(cell_dims(fx).GR, p.kw) || (dtype != FRNN_F32 && T > kPrefetchMaxSteps) ? 0 : helpers_for(p, a.groups, T);
     prof_begin("fused_fwd_kernel", st);
     switch (fx) {
       case FRNN_LSTM:  e = fused_fwd_dispatch<FRNN_LSTM>(dtype, p, a, st); break;

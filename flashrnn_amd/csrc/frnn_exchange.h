@@ -117,6 +117,12 @@ template <int E> __device__ __forceinline__ void ll_write(float*, const void* ba
   ll_store_sel<E, 128>(base, slot_off + (unsigned)ST<float>::frag_elem(row, k0) * 8u, wv, near);
 }
 
+// The XCD that this wave runs on, + 1
+__device__ __forceinline__ int own_xcd() {
+  unsigned x;
+  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(x));
+  return (int)(x & 15u) + 1;
+}
 // Do the KW workgroups of one group run on one XCD?  The launch places them on workgroup ids that are congruent
 // mod 8, which the dispatcher hands to one XCD; this handshake checks it where it matters, once per launch: every
 // workgroup publishes the id of its XCD (agent scope, visible anywhere) in the group's `words` (KW of them, zero at
@@ -126,9 +132,7 @@ template <int KW>
 __device__ __forceinline__ int xcd_handshake(int* words, int slice, int lane, int* status, int spin_limit) {
   static_assert(KW <= 64, "one lane per workgroup of the group");
   if (spin_limit < -1) return -1;  // host-side test hook: every wait gives up at once
-  unsigned x;
-  asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(x));
-  const int mine = (int)(x & 15u) + 1;
+  const int mine = own_xcd();
   if (lane == 0) __hip_atomic_store(words + slice, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   int v = mine;
   for (int spins = 0;; ++spins) {

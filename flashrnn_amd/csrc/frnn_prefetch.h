@@ -7,22 +7,17 @@
 // compute units idle, and those of the same XCD share its L2.  So a launch gets a few more workgroups, each on a compute unit of its
 // own, which request what the scan will need some steps later; the scan's own requests find it in L2.
 // They follow the groups (forward: a group's step is read off the words that its workgroups exchange, in passing; reverse: the group writes it down, as
-// the 2 bits of a step that its words carry are lost as soon as such a workgroup falls 6 steps behind), nobody waits for them, and they end with the last step requested, or when their groups stop: a failed wait, or no step for kPrefetchPolls probes.
+// the 2 bits of a step that its words carry are lost as soon as such a workgroup falls 6 steps behind), nobody waits for them, and they end with the last step requested, when their groups turn out to run on another XCD, or
+// when these stop: a failed wait, or no step for kPrefetchPolls probes.
 //
 // Forward kernel, bf16, T = 1024, without and with: LSTM N3 D256 B8 0.883 -> 0.840 ms, B16 0.900 -> 0.842, B64 0.965 -> 0.854, B128 1.231 ->
 // 1.083, B256 1.787 -> 1.527; sLSTM N4 D192 B16 0.905 -> 0.832, B256 2.805 -> 2.401; GRU N3 D256 B16 0.839 -> 0.773, B256 1.492 -> 1.243;
 // LSTM B16 N1 D512 1.157 -> 1.148, D768 1.409 -> 1.402 (steps longer than a trip to HBM).
 #pragma once
-#include "frnn_common.h"
+#include "frnn_exchange.h"
+#include "frnn_follow.h"
 
 namespace frnn {
-
-// Steps ahead of the one that is being computed.  3 are too few where the device moves much (forward, B64 N3 D256 -0.3 % instead of -13 %, B256
-// -9 instead of -18), 12 are as good as 6 but for B256 (-15: 12 steps of 12 groups no longer stay in an L2 beside what is stored).
-constexpr int kPrefetchAhead = 6;
-constexpr int kPrefetchPolls = 1 << 15;    // probes that see no step before such a workgroup ends
-// Sequences up to this length go without (training pass, bf16: B256 N3 D256 T19 130.7 -> 131.9 us, T32 189.5 -> 180.1; B5 T19 93.0 -> 93.5, T64 141.8 -> 139.1)
-constexpr int kPrefetchMinSteps = 24;
 
 __device__ __forceinline__ u32x4 make_rsrc4(const void* p, size_t bytes) {  // (make_rsrc as a register tuple, for inline asm)
   const u64 a = (u64)p;
@@ -46,57 +41,15 @@ __device__ __forceinline__ void load_to_lds(u32x4 r, unsigned voff, unsigned sof
 #pragma clang diagnostic pop
 }
 
-// The loop of such a workgroup.  Its groups are first, first + stride, ... below `groups`; its waves share them out, or share one.
-// begun(group): the number of steps that the group has begun, as far as is known; request(group, step, part, parts): fetch this
-// wave's part of the operands of a step.
-template <typename Begun, typename Request>
-__device__ __forceinline__ void prefetch_follow(int first, int stride, int groups, int Tn, int wave, int waves, const int* status, int spin_limit, Begun begun, Request request) {
-  const int mine = first < groups ? (groups - first + stride - 1) / stride : 0;  // groups of this workgroup
-  const int parts = mine > 0 && waves >= mine ? waves / mine : 1;                // waves per group
-  const int part = wave % parts;
-  int next[2], grp[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int i = wave / parts + k * waves;
-    grp[k] = first + i * stride;
-    next[k] = i < mine ? 0 : Tn;
-  }
-  for (int polls = 0; polls <= min(spin_limit, kPrefetchPolls); ++polls) {
-    if (next[0] >= Tn && next[1] >= Tn) break;
-    bool did = false;
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if (next[k] >= Tn) continue;
-      const int b = begun(grp[k], next[k]), goal = min(b + kPrefetchAhead, Tn);
-      next[k] = max(next[k], min(b, Tn));  // (late: what is behind is of no use any more)
-      for (; next[k] < goal; ++next[k]) {
-        request(grp[k], next[k], part, parts);
-        did = true;
-      }
-    }
-    if (did) { polls = 0; continue; }
-    __builtin_amdgcn_s_sleep(4);
-    if ((polls & 63) == 63 && __builtin_amdgcn_readfirstlane(__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != STATUS_OK) break;
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (none may land in the LDS of a workgroup that comes later)
-}
+// (none may land in the LDS of a workgroup that comes later)
+__device__ __forceinline__ void all_fetched() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// Steps begun, off the first word of a forward group's two exchange slots (`slots`, LLW words each): h of step t carries the tag of t.
-// `known`: steps requested so far; the group is at most kPrefetchAhead behind that.
-template <typename T, int LLW> __device__ __forceinline__ int forward_steps_begun(const u64* slots, int known) {
-  int begun = 0;
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const u64 v = ll_load(slots + s * LLW);
-    int t1;  // t + 1, or 0
-    if constexpr (sizeof(T) == 4) t1 = (int)(v >> 32);
-    else {
-      const int tag = (int)((unsigned)v >> 16), base = max(known - kPrefetchAhead - 2, 0);  // (tag: t % 65535 + 1)
-      t1 = tag == 0 ? 0 : base + (tag - 1 + 65535 - base % 65535) % 65535 + 1;
-    }
-    begun = max(begun, t1);
-  }
-  return __builtin_amdgcn_readfirstlane(begun);
+// Steps begun, off the first word of a forward group's two exchange slots (`slots`, LLW words each): h of step t carries the tag of t, which
+// is t + 1 in sequences that get such workgroups.
+template <typename T, int LLW> __device__ __forceinline__ int forward_steps_begun(const u64* slots) {
+  const u64 v0 = ll_load(slots), v1 = ll_load(slots + LLW);
+  const int t0 = sizeof(T) == 4 ? (int)(v0 >> 32) : (int)((unsigned)v0 >> 16), t1 = sizeof(T) == 4 ? (int)(v1 >> 32) : (int)((unsigned)v1 >> 16);
+  return __builtin_amdgcn_readfirstlane(max(t0, t1));
 }
 
 // One wave's part of `planes` planes of `rows` (of up to TR) rows of PPR 16-byte pieces; k: the instruction that is next for this wave
@@ -112,32 +65,33 @@ __device__ __forceinline__ void fetch_rows(u32x4 r, unsigned so, unsigned row_by
 
 // The forward scan's Wx: TR rows x GW gates x D units of a step.  `junk`: LDS address of 1 KB that nobody reads.
 template <typename T, int GW, int D, int TR, int LLW>
-__device__ __forceinline__ void prefetch_wx(const void* Wx, const u64* ll, const int* status, int first, int stride, int groups, int grp0, int N, int B, int Tn, int wave, int waves,
+__device__ __forceinline__ void prefetch_wx(const void* Wx, const u64* ll, const int* status, const int* xcd, int first, int stride, int groups, int grp0, int N, int B, int Tn, int wave, int waves,
                                             int lane, int spin_limit, unsigned junk) {
   constexpr int ES = (int)sizeof(T);
   const unsigned ND = (unsigned)N * D;
   const u32x4 r = make_rsrc4(Wx, (size_t)B * Tn * GW * ND * ES);
-  prefetch_follow(first, stride, groups, Tn, wave, waves, status, spin_limit,
-    [&](int g, int known) { return forward_steps_begun<T, LLW>(ll + (size_t)(grp0 + g) * 3 * LLW, known); },
+  prefetch_follow(first, stride, groups, Tn, wave, waves, status, xcd ? xcd + (size_t)grp0 * 32 : nullptr, own_xcd(), spin_limit,
+    [&](int g) { return forward_steps_begun<T, LLW>(ll + (size_t)(grp0 + g) * 3 * LLW); },
     [&](int g, int t, int part, int parts) {
       const int n = (grp0 + g) % N, bt = (grp0 + g) / N, rows = min(TR, B - bt * TR);
       const unsigned so = (((unsigned)bt * TR * Tn + t) * GW * ND + n * D) * ES;
       int k = part;
       fetch_rows<D * ES / 16, GW, TR>(r, so, Tn * GW * ND * ES, ND * ES, rows, lane, k, parts, junk);
     });
+  all_fetched();
 }
 
 // The reverse scan's operands of a step: the gate cache (NCP values per element), the planes DSM of the cotangent and SPM of the states before
 // the step.  `begun`: where group 0 keeps its number of steps begun, the others `stride_words` apart.
 template <typename T, int S, int NCP, int SPM, int DSM, int D, int TR>
-__device__ __forceinline__ void prefetch_reverse(const void* cache, const void* states, const void* dstates, const unsigned* begun, size_t stride_words, const int* status, int first,
+__device__ __forceinline__ void prefetch_reverse(const void* cache, const void* states, const void* dstates, const unsigned* begun, size_t stride_words, const int* status, const int* xcd, int first,
                                                  int stride, int groups, int grp0, int N, int B, int BS, int Tn, int wave, int waves, int lane, int spin_limit, unsigned junk) {
   constexpr int ES = (int)sizeof(T), PPR = D * ES / 16;
   const unsigned ND = (unsigned)N * D;
   const u32x4 rSt = make_rsrc4(states, ((size_t)(S - 1) * BS + B) * Tn * ND * ES), rDs = make_rsrc4(dstates, ((size_t)(S - 1) * BS + B) * Tn * ND * ES);
   const u32x4 rCa = make_rsrc4(cache, (size_t)Tn * N * B * D * NCP * ES);
-  prefetch_follow(first, stride, groups, Tn, wave, waves, status, spin_limit,
-    [&](int g, int) { return __builtin_amdgcn_readfirstlane((int)ll_load(begun + (size_t)(grp0 + g) * stride_words)); },
+  prefetch_follow(first, stride, groups, Tn, wave, waves, status, xcd ? xcd + (size_t)grp0 * 32 : nullptr, own_xcd(), spin_limit,
+    [&](int g) { return __builtin_amdgcn_readfirstlane((int)ll_load(begun + (size_t)(grp0 + g) * stride_words)); },
     [&](int g, int i, int part, int parts) {
       const int t = Tn - 1 - i, n = (grp0 + g) % N, bt = (grp0 + g) / N, rows = min(TR, B - bt * TR);
       int k = part;
@@ -149,6 +103,7 @@ __device__ __forceinline__ void prefetch_reverse(const void* cache, const void* 
         if ((SPM >> p) & 1 && t > 0) fetch_rows<PPR, 1, TR>(rSt, so - ND * ES, Tn * ND * ES, 0, rows, lane, k, parts, junk);
       }
     });
+  all_fetched();
 }
 
 }  // namespace frnn
