@@ -16,11 +16,10 @@ constexpr int kPrefetchMaxSteps = 65535;
 
 // Its groups are first, first + stride, ... below `groups`; its waves share them out, or share one.
 // begun(group): the number of steps that the group has begun, as far as is known; request(group, step, part, parts): fetch this
-// wave's part of the operands of a step.  `xcd`: 32 words per group, the first the XCD + 1 that the group's first workgroup runs on, zero until it
-// does (or null: not known); `own`: the same of this workgroup.  What it fetches is of use on its own XCD only, and a group on another one may keep
-// its words to itself.
-template <typename Begun, typename Request>
-__device__ __forceinline__ void prefetch_follow(int first, int stride, int groups, int Tn, int wave, int waves, const int* status, const int* xcd, int own, int spin_limit, Begun begun,
+// wave's part of the operands of a step.  here(group): 1 if the group runs on the XCD of this workgroup, -1 if not, 0 as long as that is not
+// known.  What is fetched is of use on this XCD only, and a group on another one keeps its words there.
+template <typename Here, typename Begun, typename Request>
+__device__ __forceinline__ void prefetch_follow(int first, int stride, int groups, int Tn, int wave, int waves, const int* status, int spin_limit, Here here, Begun begun,
                                                 Request request) {
   const int mine = first < groups ? (groups - first + stride - 1) / stride : 0;  // groups of this workgroup
   const int parts = mine > 0 && waves >= mine ? waves / mine : 1;                // waves per group
@@ -32,7 +31,7 @@ __device__ __forceinline__ void prefetch_follow(int first, int stride, int group
     const int i = wave / parts + k * waves;
     grp[k] = first + i * stride;
     next[k] = i < mine ? 0 : Tn;
-    placed[k] = !xcd;
+    placed[k] = false;
   }
   for (int polls = 0; polls <= min(spin_limit, kPrefetchPolls); ++polls) {
     if (next[0] >= Tn && next[1] >= Tn) break;
@@ -41,9 +40,9 @@ __device__ __forceinline__ void prefetch_follow(int first, int stride, int group
     for (int k = 0; k < 2; ++k) {
       if (next[k] >= Tn) continue;
       if (!placed[k]) {
-        const int at = __builtin_amdgcn_readfirstlane(__hip_atomic_load(xcd + (size_t)grp[k] * 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        placed[k] = at != 0;
-        if (placed[k] && at != own) { next[k] = Tn; continue; }
+        const int at = here(grp[k]);
+        placed[k] = at > 0;
+        if (at < 0) { next[k] = Tn; continue; }
       }
       const int b = begun(grp[k]), goal = min(b + kPrefetchAhead, Tn);
       next[k] = max(next[k], min(b, Tn));  // (late: what is behind is of no use any more)

@@ -187,7 +187,7 @@ fused_bwd_kernel(const BwdArgs a) {
       static_assert(KW <= kXcdWorkgroups, "groups within an XCD");
       static_assert(2 * 16 * KDL * (int)sizeof(T) >= 1024, "room for what is fetched");
       const auto pa = own_args<BwdArgs>();
-      prefetch_reverse<T, S, CacheBlk<T, NCA>::NCP, CXS >= 0 ? C::SPM & ~(1 << (CXS >= 0 ? CXS : 0)) : C::SPM, C::DSM, D, TR>(
+      prefetch_reverse<T, KW, S, CacheBlk<T, NCA>::NCP, CXS >= 0 ? C::SPM & ~(1 << (CXS >= 0 ? CXS : 0)) : C::SPM, C::DSM, D, TR>(
         pa->cache, pa->states, pa->dstates, reinterpret_cast<const unsigned*>(pa->ll) + 2 * INW, 3 * INW, pa->status, pa->xcd, (int)blockIdx.x - scan, 8 * pa->helpers,
         pa->groups, pa->grp0, pa->N, pa->B, pa->BS, pa->T, __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)blockDim.x >> 6, threadIdx.x & 63, pa->spin_limit,
         (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem_raw);
@@ -570,6 +570,7 @@ fused_bwd_kernel(const BwdArgs a) {
   constexpr bool TELL_IDLE = FETCHED && DSP > 1;
   unsigned* const begun_word = reinterpret_cast<unsigned*>(inbox + 2 * INW);
   const rsrc_t rBegun = make_rsrc(begun_word, FETCHED && !TELL_IDLE ? 4 : 0);
+  const unsigned begun_v = tid == 0 && slice == 0 ? 0u : kInvalidOff;
 
   // operands of one step.  s_t is not among them: it is the s_(t-1) of the step before (kept in
   // registers, `sn` below), so only the first step loads it
@@ -651,10 +652,6 @@ fused_bwd_kernel(const BwdArgs a) {
   }
   __syncthreads();
   const int near_i = KW > 1 ? __builtin_amdgcn_readfirstlane(near_word) : 0;  // 1: stores stay in the XCD's L2, -1: wait ran out
-  // (a group that has come to run on several XCDs, or whose wait ran out: nothing to fetch for, said once and for all)
-  if constexpr (FETCHED) { if (near_i <= 0 && slice == 0 && tid == 0) __hip_atomic_store(begun_word, (unsigned)Tn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-  const bool tells = slice == 0 && near_i > 0;
-  const unsigned begun_v = tid == 0 && tells ? 0u : kInvalidOff;
   u64 near_m;  // lane mask for ll_store_sel: all ones or zero, in scalar registers
   asm("s_cmp_gt_i32 %1, 0\n\ts_cselect_b64 %0, -1, 0" : "=s"(near_m) : "s"(near_i) : "scc");
 
@@ -828,7 +825,7 @@ fused_bwd_kernel(const BwdArgs a) {
     };
     auto tell = [&]() __attribute__((always_inline)) {
       if constexpr (TELL_IDLE) {
-        if (w_u == 1 && tells && lane == 0) __hip_atomic_store(begun_word, (unsigned)(Tn - t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (w_u == 1 && slice == 0 && lane == 0) __hip_atomic_store(begun_word, (unsigned)(Tn - t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       } else if constexpr (FETCHED) {
         __builtin_amdgcn_raw_buffer_store_b32((unsigned)(Tn - t), rBegun, begun_v, 0, 0);
       }

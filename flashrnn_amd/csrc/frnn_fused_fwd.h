@@ -162,7 +162,7 @@ fused_fwd_kernel(const FwdArgs a) {
     if (a.helpers && (int)blockIdx.x >= scan) {
       static_assert(2 * 16 * D * (int)sizeof(T) >= 1024, "room for what is fetched");
       const auto pa = own_args<FwdArgs>();
-      prefetch_wx<T, GW, D, TR, LLW>(pa->Wx, pa->ll, pa->status, pa->xcd, (int)blockIdx.x - scan, 8 * pa->helpers, pa->groups, pa->grp0, pa->N, pa->B, pa->T,
+      prefetch_wx<T, KW, GW, D, TR, LLW>(pa->Wx, pa->ll, pa->status, pa->xcd, (int)blockIdx.x - scan, 8 * pa->helpers, pa->groups, pa->grp0, pa->N, pa->B, pa->T,
                                      __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)blockDim.x >> 6, threadIdx.x & 63, pa->spin_limit,
                                      (unsigned)(size_t)&hbuf[0][0]);
       return;

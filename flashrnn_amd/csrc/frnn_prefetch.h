@@ -44,6 +44,13 @@ __device__ __forceinline__ void load_to_lds(u32x4 r, unsigned voff, unsigned sof
 // (none may land in the LDS of a workgroup that comes later)
 __device__ __forceinline__ void all_fetched() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// Does a group run on this XCD?  (prefetch_follow's here(); `words`: its words of xcd_handshake, or null: as the launch has placed it)
+template <int KW> __device__ __forceinline__ int group_here(const int* words, int lane) {
+  if (!words) return 1;
+  const int own = own_xcd(), v = lane < KW ? __hip_atomic_load(words + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : own;
+  return __any(v != 0 && v != own) ? -1 : __all(v != 0) ? 1 : 0;
+}
+
 // Steps begun, off the first word of a forward group's two exchange slots (`slots`, LLW words each): h of step t carries the tag of t, which
 // is t + 1 in sequences that get such workgroups.
 template <typename T, int LLW> __device__ __forceinline__ int forward_steps_begun(const u64* slots) {
@@ -64,13 +71,14 @@ __device__ __forceinline__ void fetch_rows(u32x4 r, unsigned so, unsigned row_by
 }
 
 // The forward scan's Wx: TR rows x GW gates x D units of a step.  `junk`: LDS address of 1 KB that nobody reads.
-template <typename T, int GW, int D, int TR, int LLW>
+template <typename T, int KW, int GW, int D, int TR, int LLW>
 __device__ __forceinline__ void prefetch_wx(const void* Wx, const u64* ll, const int* status, const int* xcd, int first, int stride, int groups, int grp0, int N, int B, int Tn, int wave, int waves,
                                             int lane, int spin_limit, unsigned junk) {
   constexpr int ES = (int)sizeof(T);
   const unsigned ND = (unsigned)N * D;
   const u32x4 r = make_rsrc4(Wx, (size_t)B * Tn * GW * ND * ES);
-  prefetch_follow(first, stride, groups, Tn, wave, waves, status, xcd ? xcd + (size_t)grp0 * 32 : nullptr, own_xcd(), spin_limit,
+  prefetch_follow(first, stride, groups, Tn, wave, waves, status, spin_limit,
+    [&](int g) { return group_here<KW>(xcd ? xcd + (size_t)(grp0 + g) * 32 : nullptr, lane); },
     [&](int g) { return forward_steps_begun<T, LLW>(ll + (size_t)(grp0 + g) * 3 * LLW); },
     [&](int g, int t, int part, int parts) {
       const int n = (grp0 + g) % N, bt = (grp0 + g) / N, rows = min(TR, B - bt * TR);
@@ -83,14 +91,15 @@ __device__ __forceinline__ void prefetch_wx(const void* Wx, const u64* ll, const
 
 // The reverse scan's operands of a step: the gate cache (NCP values per element), the planes DSM of the cotangent and SPM of the states before
 // the step.  `begun`: where group 0 keeps its number of steps begun, the others `stride_words` apart.
-template <typename T, int S, int NCP, int SPM, int DSM, int D, int TR>
+template <typename T, int KW, int S, int NCP, int SPM, int DSM, int D, int TR>
 __device__ __forceinline__ void prefetch_reverse(const void* cache, const void* states, const void* dstates, const unsigned* begun, size_t stride_words, const int* status, const int* xcd, int first,
                                                  int stride, int groups, int grp0, int N, int B, int BS, int Tn, int wave, int waves, int lane, int spin_limit, unsigned junk) {
   constexpr int ES = (int)sizeof(T), PPR = D * ES / 16;
   const unsigned ND = (unsigned)N * D;
   const u32x4 rSt = make_rsrc4(states, ((size_t)(S - 1) * BS + B) * Tn * ND * ES), rDs = make_rsrc4(dstates, ((size_t)(S - 1) * BS + B) * Tn * ND * ES);
   const u32x4 rCa = make_rsrc4(cache, (size_t)Tn * N * B * D * NCP * ES);
-  prefetch_follow(first, stride, groups, Tn, wave, waves, status, xcd ? xcd + (size_t)grp0 * 32 : nullptr, own_xcd(), spin_limit,
+  prefetch_follow(first, stride, groups, Tn, wave, waves, status, spin_limit,
+    [&](int g) { return group_here<KW>(xcd ? xcd + (size_t)(grp0 + g) * 32 : nullptr, lane); },
     [&](int g) { return __builtin_amdgcn_readfirstlane((int)ll_load(begun + (size_t)(grp0 + g) * stride_words)); },
     [&](int g, int i, int part, int parts) {
       const int t = Tn - 1 - i, n = (grp0 + g) % N, bt = (grp0 + g) / N, rows = min(TR, B - bt * TR);

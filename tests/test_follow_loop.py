@@ -17,27 +17,25 @@ using std::max; using std::min;
 #define __forceinline__ inline
 #define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_s_sleep(x) ++now
-#define __hip_atomic_load(p, order, scope) (*(p))
+#define __hip_atomic_load(p, order, scope) (*(p))  // (the status word)
 static int now = 0;  // pauses of the loop: the clock of the scan that is played
 #include "frnn_follow.h"
 
 // groups, T, pauses per step, start (pause at which the scan begins), stop (step at which it stops, -1: none), fails (pause at which the status word is set, -1: never),
-// at (XCD + 1 of the groups, 0: never known), known (are there words of the XCDs?), spin_limit, wave, waves
+// at (where the groups run: 1 here, -1 elsewhere, 0 never known), spin_limit, wave, waves
 int main(int, char** v) {
-  const int groups = atoi(v[1]), T = atoi(v[2]), per = atoi(v[3]), start = atoi(v[4]), stop = atoi(v[5]), fails = atoi(v[6]), at = atoi(v[7]), known = atoi(v[8]), limit = atoi(v[9]),
-            wave = atoi(v[10]), waves = atoi(v[11]);
+  const int groups = atoi(v[1]), T = atoi(v[2]), per = atoi(v[3]), start = atoi(v[4]), stop = atoi(v[5]), fails = atoi(v[6]), at = atoi(v[7]), limit = atoi(v[8]),
+            wave = atoi(v[9]), waves = atoi(v[10]);
   int status = 0;
-  std::vector<int> xcd(groups * 32, 0);
   std::vector<std::vector<int>> got(groups);
   int ahead = 0;
   auto steps = [&]() {
     if (fails >= 0 && now >= fails) status = 1;
-    if (now >= start) for (int g = 0; g < groups; ++g) xcd[g * 32] = at;
     const int b = now < start ? 0 : min(T, (now - start) / per);
     return stop >= 0 ? min(b, stop) : b;
   };
   steps();
-  frnn::prefetch_follow(0, 1, groups, T, wave, waves, &status, known ? xcd.data() : nullptr, 3, limit, [&](int) { return steps(); },
+  frnn::prefetch_follow(0, 1, groups, T, wave, waves, &status, limit, [&](int) { return now >= start ? at : 0; }, [&](int) { return steps(); },
                         [&](int g, int t, int, int) { got[g].push_back(t); ahead = max(ahead, t + 1 - steps()); });
   bool rising = true;
   long n = 0;
@@ -54,18 +52,18 @@ def play(tmp_path_factory):
     exe = str(src.with_suffix(""))
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, "-o", exe, str(src)], check=True)
 
-    def run(groups=1, T=100, per=3, start=0, stop=-1, fails=-1, at=3, known=1, limit=1 << 22, wave=0, waves=4):
-        args = [str(a) for a in (groups, T, per, start, stop, fails, at, known, limit, wave, waves)]
+    def run(groups=1, T=100, per=3, start=0, stop=-1, fails=-1, at=1, limit=1 << 22, wave=0, waves=4):
+        args = [str(a) for a in (groups, T, per, start, stop, fails, at, limit, wave, waves)]
         out = subprocess.run([exe, *args], check=True, capture_output=True, text=True, timeout=60).stdout.split()
         return dict(zip(("pauses", "fetched", "ahead", "rising", "last"), map(int, out)))
 
     return run
 
 
-@pytest.mark.parametrize("known", [0, 1])
+@pytest.mark.parametrize("at", [0, 1])
 @pytest.mark.parametrize("T", [25, 100, 65535])
-def test_every_step_is_fetched_once_and_some_steps_ahead(play, T, known):
-    r = play(T=T, known=known)
+def test_every_step_is_fetched_once_and_some_steps_ahead(play, T, at):
+    r = play(T=T, at=at)
     assert r == dict(pauses=r["pauses"], fetched=T, ahead=6, rising=1, last=T - 1)
 
 
@@ -84,12 +82,12 @@ def test_a_group_that_has_ended_is_not_waited_for(play):
 
 def test_a_group_of_another_xcd_is_let_go(play):
     """Its words need never become visible here: a loop that waited for them would hold its launch for as long as its bound of probes lasts."""
-    assert play(at=5, stop=0)["pauses"] <= 1
-    r = play(at=5, start=20, stop=0)  # not known at first
+    assert play(at=-1, stop=0)["pauses"] <= 1
+    r = play(at=-1, start=20, stop=0)  # not known at first
     assert r["fetched"] == 6 and r["pauses"] <= 22
 
 
-@pytest.mark.parametrize("at", [0, 3])
+@pytest.mark.parametrize("at", [0, 1])
 def test_the_loop_ends_with_a_scan_that_stops(play, at):
     assert play(at=at, stop=4, fails=500)["pauses"] <= 500 + 64 + 3  # the status word says so
     assert play(at=at, stop=4)["pauses"] <= (1 << 15) + 32           # nobody says so
