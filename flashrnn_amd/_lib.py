@@ -53,6 +53,7 @@ _SIGNATURES = {
     "frnn_function_dims": (c_int, [c_int] + [POINTER(c_int)] * 5),
     "frnn_fused_supported": (c_int, [c_int] * 5),
     "frnn_fused_plan": (c_int, [c_int] * 6 + [POINTER(c_int)] * 4),
+    "frnn_fused_fetch_workgroups": (c_int, _P6 + [c_int]),
     "frnn_fused_cache_bytes": (c_size_t, _P6),
     "frnn_fused_workspace_bytes": (c_size_t, _P6 + [c_int]),
     "frnn_fused_forward": (c_int, [c_int] * 7 + [c_void_p] * 7 + [c_size_t, c_void_p]),

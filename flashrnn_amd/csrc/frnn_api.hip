@@ -214,21 +214,31 @@ static int device_cus() {
 // Heads of more than 32 workgroups (kXcdWorkgroups) spread over the whole device: what counts is the device.
 static int groups_per_launch(int kw) { return kw > kXcdWorkgroups ? device_cus() / kw : 8 * ((device_cus() / 8) / kw); }
 // Workgroups per XCD that fetch the operands of a scan into its L2 (frnn_prefetch.h): one for each group of the XCD, as far as compute units
-// are left.  Not beside a decode session, whose workgroups need the compute units that are left.
+// are left.  Not beside a decode session, whose workgroups need the compute units that are left.  Fewer than one for each group only where one has no
+// more than 32 KB a step to fetch (`step_bytes`: of a group), about what a compute unit takes in while a step of 1 us lasts.  Forward, bf16, N3, without and with: 4
+// for 7 groups (B70 D256 T = 512, 14 KB) LSTM 453 -> 397 us, sLSTM 478 -> 428, B140 (28 KB) 537 -> 497 and 617 -> 590, GRU 506 -> 495, 8 for 12 (B256, 24 KB)
+// 721 -> 692, 945 -> 847, 595 -> 572.  With more they are late and only in the way of the scan's start: 2 for 6 (B128 D320, 60 KB) LSTM T = 28 50.2 -> 52.9, T = 128
+// +1.9 %, T = 512 568 -> 570, 2 for 3 (B256 D640, 60 KB) T = 28 +6.8 %, T = 512 +0.6, 2 for 5 (B256 D384, 120 KB) T = 28 +4.3, T = 512 -0.5.
 // FRNN_PREFETCH caps them.
-static int helpers_for(const Plan& p, int groups, int T) {
+static int helpers_for(const Plan& p, int groups, int T, long step_bytes) {
   if (p.left_out || T <= kPrefetchMinSteps) return 0;
   const int per_xcd = (groups + 7) / 8, idle = device_cus() / 8 - p.kw * per_xcd;
-  int h = env_int("FRNN_PREFETCH", per_xcd);
-  h = h < per_xcd ? h : per_xcd;
-  h = h < idle ? h : idle;
-  return h > 0 ? h : 0;
+  const int most = idle < per_xcd ? idle : per_xcd;
+  if (most <= 0 || (most < per_xcd && per_xcd * step_bytes > most * 32768l)) return 0;
+  const int h = env_int("FRNN_PREFETCH", most);
+  return h < 0 ? 0 : h < most ? h : most;
 }
 // The same for a reverse scan, which gets one for each group or none: one for several, bf16, T = 512, against none, LSTM B64 N3 D256 +25 %, GRU B256 +19, sLSTM B16
 // N4 D192 +7 (the backward pass; the kernels that such a launch takes rely on operands in L2)
-static int reverse_helpers_for(const Plan& p, int groups, int T) {
-  const int h = helpers_for(p, groups, T);
+static int reverse_helpers_for(int fx, int dtype, const Plan& p, int tile_rows, int groups, int T) {
+  const CellDims c = cell_dims(fx);
+  if (!bwd_prefetched(c.GR, c.NC, p.D, p.waves, p.utw, p.kw, tile_rows, dtype == FRNN_F32 ? 4 : 2, p.recompute != 0)) return 0;
+  const int h = helpers_for(p, groups, T, 0);
   return h == (groups + 7) / 8 ? h : 0;
+}
+static int forward_helpers_for(int fx, int dtype, const Plan& p, int tile_rows, int groups, int T) {
+  const CellDims c = cell_dims(fx);
+  return fwd_prefetched(c.GR, p.kw) && (dtype == FRNN_F32 || T <= kPrefetchMaxSteps) ? helpers_for(p, groups, T, (long)tile_rows * c.GW * p.D * (dtype == FRNN_F32 ? 4 : 2)) : 0;
 }
 // (such groups never share an XCD: no handshake, every exchange store at agent scope)
 static bool near_stores_possible(const Plan& p) { return p.kw > 1 && p.kw <= kXcdWorkgroups; }
@@ -753,6 +763,17 @@ int frnn_fused_plan(int function, int dtype, int B, int N, int D, int backward,
   return 0;
 }
 
+int frnn_fused_fetch_workgroups(int function, int dtype, int B, int T, int N, int D, int backward) {
+  const int e = check_problem(function, dtype, B, T, N, D);
+  if (e) return e;
+  Plan p;
+  if (!pick_plan(function, dtype, B, N, D, backward, &p))
+    return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
+  const int tr = tile_rows_for(B, N, p.kw, p.waves, p.max_tr, dtype), groups = N * ((B + tr - 1) / tr), most = p.kw > 1 ? groups_per_launch(p.kw) : groups;
+  const int first = groups < most ? groups : most;
+  return 8 * (p.kw <= 1 ? 0 : backward ? reverse_helpers_for(function, dtype, p, tr, first, T) : forward_helpers_for(function, dtype, p, tr, first, T));
+}
+
 size_t frnn_fused_cache_bytes(int function, int dtype, int B, int T, int N, int D) {
   if (check_problem(function, dtype, B, T, N, D)) return 0;
   return fused_cache_bytes_of(function, dtype, B, T, N, D);
@@ -888,7 +909,7 @@ static int fused_forward_impl(int function, int dtype, int training, int B, int 
   LaunchGate* gate = gate_enter(step ? 1 : p.kw, st);  // (the workgroups of a single step never wait for each other)
   for (int g0 = 0; g0 < groups; g0 += per_launch) {
     a.grp0 = g0; a.groups = groups - g0 < per_launch ? groups - g0 : per_launch;
-    a.helpers = step || call->beside || !fwd_prefetched(cell_dims(fx).GR, p.kw) || (dtype != FRNN_F32 && T > kPrefetchMaxSteps) ? 0 : helpers_for(p, a.groups, T);
+    a.helpers = step || call->beside ? 0 : forward_helpers_for(fx, dtype, p, tr, a.groups, T);
     prof_begin("fused_fwd_kernel", st);
     switch (fx) {
       case FRNN_LSTM:  e = fused_fwd_dispatch<FRNN_LSTM>(dtype, p, a, st); break;
@@ -1029,7 +1050,7 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   LaunchGate* gate = gate_enter(a.cut ? 1 : p.kw, st);  // (the truncated reverse scan exchanges nothing)
   for (int g0 = 0; g0 < groups; g0 += per_launch) {
     a.grp0 = g0; a.groups = groups - g0 < per_launch ? groups - g0 : per_launch;
-    a.helpers = a.cut || call.beside || !bwd_prefetched(c.GR, c.NC, p.D, p.waves, p.utw, p.kw, tr, dtype == FRNN_F32 ? 4 : 2, o.rc != 0) ? 0 : reverse_helpers_for(p, a.groups, T);
+    a.helpers = a.cut || call.beside ? 0 : reverse_helpers_for(fx, dtype, p, tr, a.groups, T);
     a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", tr > 4 && (a.helpers || (fx == FRNN_GRU && p.kw == 2)) ? 0 : poll_delay);
     prof_begin("fused_bwd_kernel", st);
     switch (fx) {

@@ -85,6 +85,10 @@ int frnn_fused_supported(int function, int dtype, int B, int N, int D);
 int frnn_fused_plan(int function, int dtype, int B, int N, int D, int backward,
                     int* waves, int* tiles_per_wave, int* wgs_per_head, int* active_wgs);
 
+/* Workgroups that the (first) launch of such a call gets beside those of the plan, on compute units which these leave idle, and which only
+ * fetch the scan's operands into L2; 0: none, < 0: FRNN_E_*.  Calls beside a decode session and truncated backward calls never have any. */
+int frnn_fused_fetch_workgroups(int function, int dtype, int B, int T, int N, int D, int backward);
+
 /* Bytes of the private gate cache written by a training forward and read by backward
  * (reference: gate_cache_r / gate_cache_i, fused/flashrnn.cc:97-112). */
 size_t frnn_fused_cache_bytes(int function, int dtype, int B, int T, int N, int D);
