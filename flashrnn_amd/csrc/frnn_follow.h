@@ -10,7 +10,7 @@ constexpr int kPrefetchAhead = 6;
 constexpr int kPrefetchPolls = 1 << 15;    // probes that see no step before such a workgroup ends
 // Sequences up to this length go without (training pass, bf16: B256 N3 D256 T19 130.7 -> 131.9 us, T32 189.5 -> 180.1; B5 T19 93.0 -> 93.5, T64 141.8 -> 139.1)
 constexpr int kPrefetchMinSteps = 24;
-// Forward scans in the 16-bit types beyond this length as well: the tag of a word, t % 65535 + 1, which tells how far a group is, then says nothing
+// Forward scans beyond this length as well: the tag of a word, t % 65535 + 1, which tells how far a group is, then says nothing
 // to a workgroup that starts late.
 constexpr int kPrefetchMaxSteps = 65535;
 

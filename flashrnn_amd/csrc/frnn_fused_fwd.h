@@ -156,13 +156,13 @@ fused_fwd_kernel(const FwdArgs a) {
   __shared__ f32x4 psum[KSP > 1 ? UT_WG * (KS16 ? GR : KOP - KOW) * 64 : 1];  // partial sums of the other waves of a tile: [tile][(gate | part)][lane]
 
   int grp_l, slice;
-  if constexpr (fwd_prefetched(GR, KW) && !MB) {
+  if constexpr (fwd_prefetched(GR, KW, (int)sizeof(T)) && !MB) {
     static_assert(KW <= kXcdWorkgroups, "groups within an XCD");
     const int scan = 8 * KW * ((a.groups + 7) / 8);  // workgroups of the scan (see decode_block), then 8 of those that prefetch for each of a.helpers
     if (a.helpers && (int)blockIdx.x >= scan) {
       static_assert(2 * 16 * D * (int)sizeof(T) >= 1024, "room for what is fetched");
       const auto pa = own_args<FwdArgs>();
-      prefetch_wx<T, KW, GW, D, TR, LLW>(pa->Wx, pa->ll, pa->status, pa->xcd, (int)blockIdx.x - scan, 8 * pa->helpers, pa->groups, pa->grp0, pa->N, pa->B, pa->T,
+      prefetch_wx<KW, GW, D, TR, LLW>(pa->Wx, pa->ll, pa->status, pa->xcd, (int)blockIdx.x - scan, 8 * pa->helpers, pa->groups, pa->grp0, pa->N, pa->B, pa->T,
                                      __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)blockDim.x >> 6, threadIdx.x & 63, pa->spin_limit,
                                      (unsigned)(size_t)&hbuf[0][0]);
       return;

@@ -57,9 +57,12 @@ constexpr int fwd_lds_ksteps(int GR, int D, int WAVES, int UTW, int esize) {
 constexpr int fwd_k_split(int D, int WAVES, int UTW, int KW) { return 16 * WAVES * UTW * KW / D; }
 // the dense alternatives of the tables (host: pick_plan; not for the resident decode kernel, whose groups all have 4 rows)
 constexpr int kDenseVariant = 4;
-// Forward kernels whose launch may get workgroups that fetch Wx into L2 (frnn_prefetch.h): the gated cells, heads of several workgroups within
-// an XCD.  (Elman, one load per step: -1.4 to +1.0 % at any batch.)
-constexpr bool fwd_prefetched(int GR, int KW) { return GR >= 3 && KW > 1 && KW <= 32; }
+// Forward kernels whose launch may get workgroups that fetch Wx into L2 (frnn_prefetch.h): the gated cells in the 16-bit types, 2 to 8 workgroups per head.
+// (Forward, T = 512, all sizes from B1 N1 to B256 N3, without and with: those -2 to -15 % where the call has more to move than the last-level cache holds, +-0.5 where
+// not.  10 to 24 workgroups, whose steps last longer than a trip to HBM, -0.4 to +0.1, fp32, 3 to 28 workgroups, -0.5 to +0.8; and the role itself, a branch and its
+// registers, made their scans 1 to 2 % slower: LSTM bf16 B64 N3 D768 T = 256 935 -> 948 us, GRU B256 N3 D640 1034 -> 1050, fp32 LSTM B8 N3 D448 429 -> 439, sLSTM D160
+// 313 -> 318.  Elman, one load per step: -1.4 to +1.0 % at any batch.)
+constexpr bool fwd_prefetched(int GR, int KW, int esize) { return esize == 2 && GR >= 3 && KW > 1 && KW <= 8; }
 // Forward kernel, fp32 at 4-row tiles, cells with 3 or 4 recurrent gates: the product runs on v_mfma_f32_4x4x1_16B_f32
 // (see the kernel), when the whole operand, D / KSP registers per tile in that form, fits the registers of a wave (512 in
 // workgroups of up to 4 waves, 256 with up to 8: D = 96 as 6 waves).

@@ -11,8 +11,7 @@
 // when these stop: a failed wait, or no step for kPrefetchPolls probes.
 //
 // Forward kernel, bf16, T = 1024, without and with: LSTM N3 D256 B8 0.883 -> 0.840 ms, B16 0.900 -> 0.842, B64 0.965 -> 0.854, B128 1.231 ->
-// 1.083, B256 1.787 -> 1.527; sLSTM N4 D192 B16 0.905 -> 0.832, B256 2.805 -> 2.401; GRU N3 D256 B16 0.839 -> 0.773, B256 1.492 -> 1.243;
-// LSTM B16 N1 D512 1.157 -> 1.148, D768 1.409 -> 1.402 (steps longer than a trip to HBM).
+// 1.083, B256 1.787 -> 1.527; sLSTM N4 D192 B16 0.905 -> 0.832, B256 2.805 -> 2.401; GRU N3 D256 B16 0.839 -> 0.773, B256 1.492 -> 1.243.
 #pragma once
 #include "frnn_exchange.h"
 #include "frnn_follow.h"
@@ -53,10 +52,9 @@ template <int KW> __device__ __forceinline__ int group_here(const int* words, in
 
 // Steps begun, off the first word of a forward group's two exchange slots (`slots`, LLW words each): h of step t carries the tag of t, which
 // is t + 1 in sequences that get such workgroups.
-template <typename T, int LLW> __device__ __forceinline__ int forward_steps_begun(const u64* slots) {
-  const u64 v0 = ll_load(slots), v1 = ll_load(slots + LLW);
-  const int t0 = sizeof(T) == 4 ? (int)(v0 >> 32) : (int)((unsigned)v0 >> 16), t1 = sizeof(T) == 4 ? (int)(v1 >> 32) : (int)((unsigned)v1 >> 16);
-  return __builtin_amdgcn_readfirstlane(max(t0, t1));
+template <int LLW> __device__ __forceinline__ int forward_steps_begun(const u64* slots) {
+  const unsigned v0 = (unsigned)ll_load(slots), v1 = (unsigned)ll_load(slots + LLW);
+  return __builtin_amdgcn_readfirstlane((int)(max(v0, v1) >> 16));
 }
 
 // One wave's part of `planes` planes of `rows` (of up to TR) rows of PPR 16-byte pieces; k: the instruction that is next for this wave
@@ -70,16 +68,16 @@ __device__ __forceinline__ void fetch_rows(u32x4 r, unsigned so, unsigned row_by
   k -= NI;
 }
 
-// The forward scan's Wx: TR rows x GW gates x D units of a step.  `junk`: LDS address of 1 KB that nobody reads.
-template <typename T, int KW, int GW, int D, int TR, int LLW>
+// The forward scan's Wx (16-bit types): TR rows x GW gates x D units of a step.  `junk`: LDS address of 1 KB that nobody reads.
+template <int KW, int GW, int D, int TR, int LLW>
 __device__ __forceinline__ void prefetch_wx(const void* Wx, const u64* ll, const int* status, const int* xcd, int first, int stride, int groups, int grp0, int N, int B, int Tn, int wave, int waves,
                                             int lane, int spin_limit, unsigned junk) {
-  constexpr int ES = (int)sizeof(T);
+  constexpr int ES = 2;
   const unsigned ND = (unsigned)N * D;
   const u32x4 r = make_rsrc4(Wx, (size_t)B * Tn * GW * ND * ES);
   prefetch_follow(first, stride, groups, Tn, wave, waves, status, spin_limit,
     [&](int g) { return group_here<KW>(xcd ? xcd + (size_t)(grp0 + g) * 32 : nullptr, lane); },
-    [&](int g) { return forward_steps_begun<T, LLW>(ll + (size_t)(grp0 + g) * 3 * LLW); },
+    [&](int g) { return forward_steps_begun<LLW>(ll + (size_t)(grp0 + g) * 3 * LLW); },
     [&](int g, int t, int part, int parts) {
       const int n = (grp0 + g) % N, bt = (grp0 + g) / N, rows = min(TR, B - bt * TR);
       const unsigned so = (((unsigned)bt * TR * Tn + t) * GW * ND + n * D) * ES;
