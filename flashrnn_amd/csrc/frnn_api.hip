@@ -229,10 +229,15 @@ static int helpers_for(const Plan& p, int groups, int T, long step_bytes) {
   return h < 0 ? 0 : h < most ? h : most;
 }
 // The same for a reverse scan, which gets one for each group or none: one for several, bf16, T = 512, against none, LSTM B64 N3 D256 +25 %, GRU B256 +19, sLSTM B16
-// N4 D192 +7 (the backward pass; the kernels that such a launch takes rely on operands in L2)
-static int reverse_helpers_for(int fx, int dtype, const Plan& p, int tile_rows, int groups, int T) {
+// N4 D192 +7 (the backward pass; the kernels that such a launch takes rely on operands in L2).  At 4-row tiles only calls that move more than the last-level cache
+// holds (`bytes`: states, cotangents, gate cache and dWx): below that the forward pass has left the operands there, a step of 4 rows does not wait for them, and
+// the workgroups are in its way.  sLSTM D192 bf16 and fp16, backward pass against none, by MB moved: 80 and 200 +2.2 to +3.1 %, 260 +2.3 to -2.4, 310 -1.8 to -4.4, 600
+// and 900 -2.4 to -4.8; before the line B16 N4 T256 242 -> 247 us, T2048 1814 -> 1738.  Taller tiles gain at any size (LSTM B128 N3 D256 T = 28 -3 %, T = 512 -6).
+constexpr size_t kLastLevelCache = (size_t)256 << 20;
+static int reverse_helpers_for(int fx, int dtype, const Plan& p, int tile_rows, int groups, int T, size_t bytes) {
   const CellDims c = cell_dims(fx);
   if (!bwd_prefetched(c.GR, c.NC, p.D, p.waves, p.utw, p.kw, tile_rows, dtype == FRNN_F32 ? 4 : 2, p.recompute != 0)) return 0;
+  if (tile_rows == 4 && bytes <= kLastLevelCache) return 0;
   const int h = helpers_for(p, groups, T, 0);
   return h == (groups + 7) / 8 ? h : 0;
 }
@@ -506,6 +511,11 @@ static size_t fused_cache_bytes_of(int function, int dtype, int B, int T, int N,
   const int ncp = dtype_size(dtype) == 2 ? (nc + 1) / 2 * 2 : nc;
   return (size_t)T * N * B * D * ncp * dtype_size(dtype);
 }
+// what a reverse scan reads and writes: gate cache, states, their cotangents, dWx
+static size_t reverse_bytes(int function, int dtype, int B, int T, int N, int D) {
+  const CellDims c = cell_dims(function);
+  return fused_cache_bytes_of(function, dtype, B, T, N, D) + (size_t)B * T * N * D * (2 * c.S + c.GW) * dtype_size(dtype);
+}
 // the fused kernels address each tensor with 32-bit byte offsets
 // bs: rows between the state planes (0: B)
 static int check_fused_sizes(int function, int dtype, int B, int T, int N, int D, int bs = 0, bool with_cache = true) {
@@ -771,7 +781,7 @@ int frnn_fused_fetch_workgroups(int function, int dtype, int B, int T, int N, in
     return fail(FRNN_E_UNSUPPORTED, "no fused kernel for function %d dtype %d head dim %d", function, dtype, D);
   const int tr = tile_rows_for(B, N, p.kw, p.waves, p.max_tr, dtype), groups = N * ((B + tr - 1) / tr), most = p.kw > 1 ? groups_per_launch(p.kw) : groups;
   const int first = groups < most ? groups : most;
-  return 8 * (p.kw <= 1 ? 0 : backward ? reverse_helpers_for(function, dtype, p, tr, first, T) : forward_helpers_for(function, dtype, p, tr, first, T));
+  return 8 * (p.kw <= 1 ? 0 : backward ? reverse_helpers_for(function, dtype, p, tr, first, T, reverse_bytes(function, dtype, B, T, N, D)) : forward_helpers_for(function, dtype, p, tr, first, T));
 }
 
 size_t frnn_fused_cache_bytes(int function, int dtype, int B, int T, int N, int D) {
@@ -1047,10 +1057,11 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
 #ifdef FRNN_TRACE
   a.trace = (long long*)((char*)workspace + w.zero_bytes);
 #endif
+  const size_t moved = reverse_bytes(fx, dtype, B, T, N, D);
   LaunchGate* gate = gate_enter(a.cut ? 1 : p.kw, st);  // (the truncated reverse scan exchanges nothing)
   for (int g0 = 0; g0 < groups; g0 += per_launch) {
     a.grp0 = g0; a.groups = groups - g0 < per_launch ? groups - g0 : per_launch;
-    a.helpers = a.cut || call.beside ? 0 : reverse_helpers_for(fx, dtype, p, tr, a.groups, T);
+    a.helpers = a.cut || call.beside ? 0 : reverse_helpers_for(fx, dtype, p, tr, a.groups, T, moved);
     a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", tr > 4 && (a.helpers || (fx == FRNN_GRU && p.kw == 2)) ? 0 : poll_delay);
     prof_begin("fused_bwd_kernel", st);
     switch (fx) {

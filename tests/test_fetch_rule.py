@@ -16,5 +16,13 @@ def test_forward(function, B, N, D, want):
     assert fetch_workgroups(function, "bfloat16", B, 24, N, D, 0) == 0
 
 
+# backward: one for each group or none, 4-row tiles only beyond the last-level cache (36 bytes a unit and step: B16 N4 D192 T606 and T607)
+@pytest.mark.parametrize("function,B,T,N,D,want", [("lstm", 128, 28, 3, 256, 48), ("lstm", 256, 64, 3, 256, 48), ("lstm", 8, 1024, 3, 256, 0), ("slstm", 16, 606, 4, 192, 0),
+                                                   ("slstm", 16, 607, 4, 192, 16), ("slstm", 16, 2048, 2, 384, 0), ("lstm", 16, 4096, 4, 192, 0), ("gru", 128, 512, 3, 256, 48)])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_backward(function, dtype, B, T, N, D, want):
+    assert fetch_workgroups(function, dtype, B, T, N, D, 1) == want
+
+
 def test_errors():
     assert fetch_workgroups("lstm", "bfloat16", 0, 8, 1, 256, 0) < 0 and fetch_workgroups("lstm", "bfloat16", 1, 8, 1, 100, 0) < 0
