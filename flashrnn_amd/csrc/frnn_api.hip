@@ -1043,14 +1043,17 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   // 7.37 / 7.31, gru 0.797 / 0.760, 2.02 / 1.99, 6.76 / 6.68); with 48 and 64 the best place differs by batch size (D = 1024: B8 N1 -4 %
   // with 24, B4 N1 +10 %)
   // heads spread by splitting the destinations (variants 2 and 3 of the tables), swept as in the forward call: 16-bit pairs 2 up to
-  // 14 workgroups (lstm B8 T1024 N3 D=256, backward pass, 912 us with 2, 920 with 1; 3 at 10 for slstm and gru, N2 D=320 526 and 488, with 2 537 and 510), 1 at 16 (lstm
-  // D=512 650 us, with 0 657, gru 592 / 606, but slstm 667 / 659), 0 above (D=768 847, with 2 876); 8- and 16-row tiles whose operands
-  // are fetched into L2 0 (B256, lstm D=256 1174, with 2 1179, slstm D=192 1285 / 1297), and the gru's 2 workgroups (B256 D=256 918 / 954); fp32 fours 4 from 10 to 16 workgroups, 6 from 20 to 28 (D=320 0.443 ms, with 2 0.450), 0 at 4, else 2
+  // 8 workgroups (lstm B8 T1024 N3 D=256, backward pass, 912 us with 2, 920 with 1), 3 from 10 to 14 where half of the adjoint is done behind the probe (T = 512, with 2 and 3,
+  // bf16 and fp16: N2 D=320 slstm 536 / 530 and 545 / 528, gru 497 / 482 and 505 / 488, D=384 slstm 596 / 583 and 594 / 587, lstm 588 / 566 and 592 / 576, D=448 lstm
+  // 635 / 625 and 654 / 635) but not the lstm's 10 (514 / 520 and 528 / 517), 2 where it is not (D=448 slstm 719 / 734 and 680 / 690), 1 at 16 (lstm D=512 650 us, with 0 657,
+  // gru 592 / 606, but slstm 667 / 659), 0 above (D=768 847, with 2 876); 8- and 16-row tiles of up to 5 workgroups 0 (B256, with 2: gru D=256 908 / 948, D=320 1180 / 1193,
+  // slstm D=256 1364 / 1373, D=320 1452 / 1465, lstm +-0.3 %); fp32 fours 4 from 10 to 16 workgroups, 6 from 20 to 28 (D=320 0.443 ms, with 2 0.450), 0 at 4, else 2
   const bool half = dtype != FRNN_F32;
   const int dsp = bwd_dest_split(p.D, p.waves, p.utw, p.kw);
-  const int wide_delay = half && dsp > 1 ? (p.kw <= 4 || p.kw > 16 ? 0 : p.kw == 16 ? (fx == FRNN_SLSTM ? 0 : 1) : p.kw == 10 && fx != FRNN_LSTM ? 3 : 2) : half || dsp != 4 ? 2
+  const bool early = bwd_adjoint_early(c.GR, c.NC, p.D, p.waves, p.utw, p.kw, tr, half ? 2 : 4, dtype == FRNN_F16, false);
+  const int wide_delay = half && dsp > 1 ? (p.kw <= 4 || p.kw > 16 ? 0 : p.kw == 16 ? (fx == FRNN_SLSTM ? 0 : 1) : early && p.kw >= 10 && !(fx == FRNN_LSTM && p.kw == 10) ? 3 : 2) : half || dsp != 4 ? 2
                        : p.kw <= 4 ? 0 : p.kw < 10 ? 2 : p.kw <= 16 ? 4 : p.kw <= 28 ? 6 : 2;
-  const int poll_delay = o.rc ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && dsp == 1 && tr == 4 || half && p.kw >= 32 ? 0 : p.kw == 40 ? 14 : wide_delay;
+  a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", o.rc || (half && c.GR > 1 && tr > 4 && p.kw <= 5) ? 0 : c.GR == 1 ? (half && p.waves <= 4 ? 2 : p.kw > 4 ? 8 : 4) : half && p.kw >= 10 && dsp == 1 && tr == 4 || half && p.kw >= 32 ? 0 : p.kw == 40 ? 14 : wide_delay);
   a.g_clip = o.g_clip; a.cut = o.cut;
   a.pst = env_int("FRNN_PRODUCER_STORES", tr == 4 && p.kw == 1 && bwd_producer_stores_pay(fx, p, groups, o.rc) ? 1 : 0);
   a.trace = nullptr;
@@ -1062,7 +1065,6 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   for (int g0 = 0; g0 < groups; g0 += per_launch) {
     a.grp0 = g0; a.groups = groups - g0 < per_launch ? groups - g0 : per_launch;
     a.helpers = a.cut || call.beside ? 0 : reverse_helpers_for(fx, dtype, p, tr, a.groups, T, moved);
-    a.poll_delay = env_int("FRNN_POLL_DELAY_BWD", tr > 4 && (a.helpers || (fx == FRNN_GRU && p.kw == 2)) ? 0 : poll_delay);
     prof_begin("fused_bwd_kernel", st);
     switch (fx) {
       case FRNN_LSTM:  e = fused_bwd_dispatch<FRNN_LSTM>(dtype, p, a, st); break;
