@@ -243,7 +243,7 @@ static int reverse_helpers_for(int fx, int dtype, const Plan& p, int tile_rows, 
 }
 static int forward_helpers_for(int fx, int dtype, const Plan& p, int tile_rows, int groups, int T) {
   const CellDims c = cell_dims(fx);
-  return fwd_prefetched(c.GR, p.kw, dtype == FRNN_F32 ? 4 : 2) && T <= kPrefetchMaxSteps ? helpers_for(p, groups, T, 2l * tile_rows * c.GW * p.D) : 0;
+  return fwd_prefetched(c.GR, p.D, p.waves, p.utw, p.kw, dtype == FRNN_F32 ? 4 : 2) && T <= kPrefetchMaxSteps ? helpers_for(p, groups, T, 2l * tile_rows * c.GW * p.D) : 0;
 }
 // (such groups never share an XCD: no handshake, every exchange store at agent scope)
 static bool near_stores_possible(const Plan& p) { return p.kw > 1 && p.kw <= kXcdWorkgroups; }

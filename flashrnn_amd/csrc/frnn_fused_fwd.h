@@ -156,7 +156,7 @@ fused_fwd_kernel(const FwdArgs a) {
   __shared__ f32x4 psum[KSP > 1 ? UT_WG * (KS16 ? GR : KOP - KOW) * 64 : 1];  // partial sums of the other waves of a tile: [tile][(gate | part)][lane]
 
   int grp_l, slice;
-  if constexpr (fwd_prefetched(GR, KW, (int)sizeof(T)) && !MB) {
+  if constexpr (fwd_prefetched(GR, D, WAVES, UTW, KW, (int)sizeof(T)) && !MB) {
     static_assert(KW <= kXcdWorkgroups, "groups within an XCD");
     const int scan = 8 * KW * ((a.groups + 7) / 8);  // workgroups of the scan (see decode_block), then 8 of those that prefetch for each of a.helpers
     if (a.helpers && (int)blockIdx.x >= scan) {

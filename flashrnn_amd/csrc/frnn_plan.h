@@ -57,12 +57,15 @@ constexpr int fwd_lds_ksteps(int GR, int D, int WAVES, int UTW, int esize) {
 constexpr int fwd_k_split(int D, int WAVES, int UTW, int KW) { return 16 * WAVES * UTW * KW / D; }
 // the dense alternatives of the tables (host: pick_plan; not for the resident decode kernel, whose groups all have 4 rows)
 constexpr int kDenseVariant = 4;
-// Forward kernels whose launch may get workgroups that fetch Wx into L2 (frnn_prefetch.h): the gated cells in the 16-bit types, 2 to 8 workgroups per head.
+// Forward kernels whose launch may get workgroups that fetch Wx into L2 (frnn_prefetch.h): the gated cells in the 16-bit types, 2 to 8 workgroups per head, and from
+// 20 on those whose waves split k (training pass, Wx from memory, bf16 T = 1024: B16 N1 LSTM D640 2773 -> 2756 us, D768 3054 -> 3046, GRU 2591 -> 2578, 2832 -> 2804).
 // (Forward, T = 512, all sizes from B1 N1 to B256 N3, without and with: those -2 to -15 % where the call has more to move than the last-level cache holds, +-0.5 where
-// not.  10 to 24 workgroups, whose steps last longer than a trip to HBM, -0.4 to +0.1, fp32, 3 to 28 workgroups, -0.5 to +0.8; and the role itself, a branch and its
+// not.  10 to 16 workgroups, whose steps last longer than a trip to HBM, -0.4 to +0.1, fp32, 3 to 28 workgroups, -0.5 to +0.8; and the role itself, a branch and its
 // registers, made their scans 1 to 2 % slower: LSTM bf16 B64 N3 D768 T = 256 935 -> 948 us, GRU B256 N3 D640 1034 -> 1050, fp32 LSTM B8 N3 D448 429 -> 439, sLSTM D160
 // 313 -> 318.  Elman, one load per step: -1.4 to +1.0 % at any batch.)
-constexpr bool fwd_prefetched(int GR, int KW, int esize) { return esize == 2 && GR >= 3 && KW > 1 && KW <= 8; }
+constexpr bool fwd_prefetched(int GR, int D, int WAVES, int UTW, int KW, int esize) {
+  return esize == 2 && GR >= 3 && KW > 1 && (KW <= 8 || (KW >= 20 && KW < 32 && fwd_k_split(D, WAVES, UTW, KW) > 1));
+}
 // Forward kernel, fp32 at 4-row tiles, cells with 3 or 4 recurrent gates: the product runs on v_mfma_f32_4x4x1_16B_f32
 // (see the kernel), when the whole operand, D / KSP registers per tile in that form, fits the registers of a wave (512 in
 // workgroups of up to 4 waves, 256 with up to 8: D = 96 as 6 waves).
@@ -165,8 +168,12 @@ constexpr bool fwd_stores_behind_probe(int GR, int D, int WAVES, int UTW, int KW
 // Reverse kernels with an instantiation for launches that have workgroups which fetch its operands into L2 (frnn_prefetch.h): gated cells in the 16-bit
 // types, 8- and 16-row tiles of up to 5 workgroups per head (the GRU 8-row tiles), and the sLSTM's pairs of 6 workgroups (nc: values of the gate cache).
 // Whole backward pass, bf16, T = 512, without and with: LSTM B128 N3 D256 784 -> 752 us, B256 1261 -> 1174, sLSTM B128 N3 D256 879 -> 813, B256 N4
-// D192 1385 -> 1285, B16 T1024 N4 D192 915 -> 890, GRU B128 N2 D320 736 -> 717, N3 D256 714 -> 708, B256 918 -> 915.  Elsewhere: GRU B16 N1 D512 592 -> 596, LSTM B8 T1024 N3 D256 912 -> 930, B16 N1 D384 551
-// -> 562, D512 650 -> 649, sLSTM B16 N4 D128 400 -> 415, D512 659 -> 655, taller tiles of 6 to 10 workgroups -0.5 to +2.7 %, fp32 -0.3 to +4, recompute mode +-1.
+// D192 1385 -> 1285, GRU B128 N2 D320 736 -> 717, N3 D256 714 -> 708, in its dense tiling of 2 (65 to 80 groups; training pass) B171 and B200 N3 D256 T = 256 742 -> 729, 760 -> 744, T = 1024
+// 2783 -> 2799, 2848 -> 2866; the pairs of 6 beyond the last-level cache: bf16 and fp16 B16 N4 T2048 D192 1809 -> 1746, 1819 -> 1751.
+// Elsewhere: GRU B16 N1 D512 592 -> 596, LSTM B8 T1024 N3 D256 912 -> 930, B16
+// N1 D384 551 -> 562, D512 650 -> 649, sLSTM B16 N4 D128 400 -> 415, taller tiles of 6 to 10 workgroups -0.5 to +2.7 %, fp32 -0.3 to +4, recompute mode +-1.  The
+// sLSTM's other pairs, beyond the last-level cache: 10 and 12 workgroups, bf16, whose steps are longer, -0.4 and -0.7 %, which is no second kernel's worth; 14 -3 % in
+// bf16, -2 in fp16, 16 -2.5 and +7.5, 20 +1.8, 24 -8.5 and +2.4: one type's gain is the other's loss, and they are left without.
 constexpr bool bwd_prefetched(int GR, int nc, int D, int WAVES, int UTW, int KW, int TR, int esize, bool rc) {
   return esize == 2 && (GR == 4 || (GR == 3 && TR == 8)) && KW > 1 && !rc && UTW == 1 &&
          (TR == 4 ? nc == 5 && bwd_dest_split(D, WAVES, UTW, KW) == 2 && KW == 6 : bwd_dest_split(D, WAVES, UTW, KW) == 1 && KW <= 5);

@@ -20,9 +20,9 @@ CASES = [("lstm", "bfloat16", 5, 24, 3, 256), ("lstm", "bfloat16", 5, 25, 3, 256
 
 # forward and backward launches that have them (in the first launch of the call): all, 8 for 12 groups of an XCD, 4 for 7, 5 for 10
 FORWARD = [("lstm", "bfloat16", 5, 25, 3, 256), ("gru", "bfloat16", 250, 31, 3, 256), ("lstm", "float16", 70, 33, 3, 256), ("slstm", "float16", 130, 26, 4, 192), ("gru", "float16", 131, 32, 2, 384)]
-# 16-row tiles, 8-row tiles of each cell, pairs of waves beyond the last-level cache
+# 16-row tiles, 8-row tiles of each cell, the GRU's dense tiling, pairs of waves beyond the last-level cache
 BACKWARD = [("lstm", "float16", 250, 33, 3, 256), ("lstm", "bfloat16", 99, 28, 4, 192), ("slstm", "bfloat16", 120, 29, 4, 192), ("gru", "float16", 101, 40, 3, 256), ("gru", "bfloat16", 77, 26, 3, 320),
-            ("slstm", "float16", 9, 1100, 4, 192), ("slstm", "bfloat16", 6, 6500, 1, 192)]
+            ("gru", "bfloat16", 199, 27, 3, 256), ("gru", "float16", 171, 26, 3, 256), ("slstm", "float16", 9, 1100, 4, 192), ("slstm", "bfloat16", 6, 6500, 1, 192)]
 
 
 @pytest.mark.parametrize("function,dtype,B,T,N,D", CASES + [c for c in FORWARD + BACKWARD if c not in CASES])
