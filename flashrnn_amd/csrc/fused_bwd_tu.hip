@@ -41,7 +41,7 @@ int fused_bwd_launch<FRNN_F, FRNN_DT>(const Plan& p, const BwdArgs& a, hipStream
     auto kern = bwd_kernel_for<Dv, W, U, K, MTR, RCV>(a.tile_rows, pst || a.helpers);                                      \
     if (!kern) return FRNN_E_UNSUPPORTED;                                                                \
     const size_t alone = K > 1 && a.helpers ? alone_on_a_compute_unit((const void*)kern) : 0, lds = alone > own_lds ? alone : own_lds; \
-    if (lds > 65536) {                                                                                   \
+    if (lds > 65536 && lds != alone) {  /* (alone_on_a_compute_unit has asked) */                         \
       hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
       if (e != hipSuccess) return (int)e;                                                                \
     }                                                                                                    \
