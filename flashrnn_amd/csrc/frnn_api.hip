@@ -221,7 +221,7 @@ static int groups_per_launch(int kw) { return kw > kXcdWorkgroups ? device_cus()
 // +1.9 %, T = 512 568 -> 570, 2 for 3 (B256 D640, 60 KB) T = 28 +6.8 %, T = 512 +0.6, 2 for 5 (B256 D384, 120 KB) T = 28 +4.3, T = 512 -0.5.
 // FRNN_PREFETCH caps them.
 static int helpers_for(const Plan& p, int groups, int T, long step_bytes) {
-  if (p.left_out || T <= kPrefetchMinSteps) return 0;
+  if (T <= kPrefetchMinSteps) return 0;
   const int per_xcd = (groups + 7) / 8, idle = device_cus() / 8 - p.kw * per_xcd;
   const int most = idle < per_xcd ? idle : per_xcd;
   if (most <= 0 || (most < per_xcd && per_xcd * step_bytes > most * 32768l)) return 0;
@@ -243,6 +243,7 @@ static int reverse_helpers_for(int fx, int dtype, const Plan& p, int tile_rows, 
 }
 static int forward_helpers_for(int fx, int dtype, const Plan& p, int tile_rows, int groups, int T) {
   const CellDims c = cell_dims(fx);
+  if (p.left_out) return 0;  // (the forward kernel has no place for both: the branch cost LSTM B256 N3 D256 1 %)
   return fwd_prefetched(c.GR, p.D, p.waves, p.utw, p.kw, dtype == FRNN_F32 ? 4 : 2) && T <= kPrefetchMaxSteps ? helpers_for(p, groups, T, 2l * tile_rows * c.GW * p.D) : 0;
 }
 // (such groups never share an XCD: no handshake, every exchange store at agent scope)
@@ -1065,6 +1066,7 @@ static int fused_backward_impl(int function, int dtype, int B, int T, int N, int
   for (int g0 = 0; g0 < groups; g0 += per_launch) {
     a.grp0 = g0; a.groups = groups - g0 < per_launch ? groups - g0 : per_launch;
     a.helpers = a.cut || call.beside ? 0 : reverse_helpers_for(fx, dtype, p, tr, a.groups, T, moved);
+    a.scan_blocks = grid_for(a.groups, p.kw) - p.left_out;
     prof_begin("fused_bwd_kernel", st);
     switch (fx) {
       case FRNN_LSTM:  e = fused_bwd_dispatch<FRNN_LSTM>(dtype, p, a, st); break;

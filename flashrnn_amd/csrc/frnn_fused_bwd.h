@@ -57,6 +57,8 @@ struct BwdArgs {
   // Wx_t, b and R h_(t-1), with h_(t-1) read back from the stored states
   const void* Wx; const void* R; const void* b;
   int helpers;   // workgroups per XCD behind those of the scan that fetch its operands into the XCD's L2 (frnn_prefetch.h)
+  int scan_blocks;  // blocks of the grid that do the scan; behind them, in tests of the failure path, those left out of it, then the helpers
+                    // (worked out in the kernel it costs the fp16 sLSTM's pairs 5 %: registers)
   int pst;  // host side only: launch the instantiation whose producer wave stores dWx (bwd_producer_stores)
 };
 
@@ -182,11 +184,12 @@ fused_bwd_kernel(const BwdArgs a) {
   constexpr bool FETCHED = PSTV && KW > 1;
   static_assert(!FETCHED || bwd_prefetched(GR, NC, D, WAVES, UTW, KW, TR, (int)sizeof(T), RC), "instantiated without need");
   if constexpr (FETCHED) {
-    const int scan = 8 * KW * ((a.groups + 7) / 8);  // workgroups of the scan, then 8 of those that prefetch for each of a.helpers
-    if ((int)blockIdx.x >= scan) {
+    if ((int)blockIdx.x >= a.scan_blocks) {
       static_assert(KW <= kXcdWorkgroups, "groups within an XCD");
       static_assert(2 * 16 * KDL * (int)sizeof(T) >= 1024, "room for what is fetched");
       const auto pa = own_args<BwdArgs>();
+      const int scan = 8 * KW * ((pa->groups + 7) / 8);  // workgroups of the whole scan, then 8 of those that prefetch for each of a.helpers
+      if ((int)blockIdx.x < scan) return;
       prefetch_reverse<T, KW, S, CacheBlk<T, NCA>::NCP, CXS >= 0 ? C::SPM & ~(1 << (CXS >= 0 ? CXS : 0)) : C::SPM, C::DSM, D, TR>(
         pa->cache, pa->states, pa->dstates, reinterpret_cast<const unsigned*>(pa->ll) + 2 * INW, 3 * INW, pa->status, pa->xcd, (int)blockIdx.x - scan, 8 * pa->helpers,
         pa->groups, pa->grp0, pa->N, pa->B, pa->BS, pa->T, __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)blockDim.x >> 6, threadIdx.x & 63, pa->spin_limit,

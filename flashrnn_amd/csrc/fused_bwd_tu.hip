@@ -25,7 +25,7 @@ template <int Dv, int W, int U, int K, int MTR, bool RCV> static void (*bwd_kern
 
 template <>
 int fused_bwd_launch<FRNN_F, FRNN_DT>(const Plan& p, const BwdArgs& a, hipStream_t st) {
-  const dim3 grid(grid_for(a.groups, p.kw) - p.left_out + 8 * a.helpers);
+  const dim3 grid(a.helpers ? grid_for(a.groups, p.kw) + 8 * a.helpers : a.scan_blocks);
   const bool rc = p.recompute != 0;
   // (one more wave and its hand-over buffers where the kernel has a producer wave: the same predicate as in the kernel)
   const bool pw = bwd_producer_wave(Cell<FRNN_F>::GR, Cell<FRNN_F>::NC, p.D, p.waves, p.utw, p.kw, a.tile_rows, (int)sizeof(FRNN_TU_T), rc);
